@@ -1,0 +1,104 @@
+"""decode_stream.hip: fp16 queries over fp16 caches at head_dim 64 to 128, as one
+workgroup per (row, kv head) (short tables) and in equal slices (long tables).
+
+Every unattended slot of the pool holds NaN, so a read of one that reaches the
+result shows.  Reference: the oracle on the same pool (NaN replaced there: the
+oracle reads attended slots only)."""
+import numpy as np
+import pytest
+
+from helpers import F16_ATOL, F16_RTOL, assert_close, to_dev, to_np
+
+pytestmark = pytest.mark.gpu
+
+# (H, Hkv, D, block size): each head dimension, both head tiles, groups of one,
+# block sizes that are no power of two or shorter than a step
+SHAPES = [(14, 2, 64, 16), (2, 2, 64, 1), (34, 2, 64, 24), (4, 4, 80, 16), (32, 2, 80, 12), (33, 33, 80, 16),
+          (3, 3, 96, 32), (16, 1, 96, 5), (16, 16, 112, 16), (34, 2, 112, 16), (32, 2, 128, 16), (32, 1, 128, 16),
+          (8, 2, 128, 8), (8, 8, 128, 48)]
+# contexts at the edges of a step (32 tokens), of a wave's share and of a slice
+CONTEXTS = [1, 31, 0, 32, 33, 64, 65, 257, 0, 700]
+
+
+def _case(rng, H, Hkv, D, bs, ctx, table_tokens):
+    from vllm_kv_amd import workloads
+    lay = workloads.make_layout(np.asarray(ctx, np.int32), bs, rng, max_blocks_per_seq=-(-table_tokens // bs))
+    shape = (lay.num_blocks, bs, Hkv, D)
+    pools = [(rng.standard_normal(shape, dtype=np.float32) * 0.7).astype(np.float16) for _ in range(2)]
+    used = np.zeros((lay.num_blocks, bs), bool)
+    for s, n in enumerate(ctx):
+        pos = np.arange(n)
+        used[lay.block_tables[s, pos // bs], pos % bs] = True
+    for p in pools:
+        p[~used] = np.nan
+    q = (rng.standard_normal((len(ctx), H, D), dtype=np.float32) * 0.7).astype(np.float16)
+    return lay, pools, q
+
+
+@pytest.mark.parametrize("table", [1024, 6000], ids=["rows", "slices"])
+@pytest.mark.parametrize("H,Hkv,D,bs", SHAPES)
+def test_stream_edges_vs_oracle(vkv, oracle, cuda, H, Hkv, D, bs, table):
+    import torch
+    rng = np.random.default_rng(D * 100 + H + bs)
+    lay, (k, v), q = _case(rng, H, Hkv, D, bs, CONTEXTS, table)
+    scale = -float(D) ** -0.5 if bs == 24 else float(D) ** -0.5
+    ref = oracle.paged_decode(q.astype(np.float32), np.nan_to_num(k).view(np.uint16), np.nan_to_num(v).view(np.uint16),
+                              lay.block_tables, lay.context_lens, scale)
+    args = (to_dev(q, cuda), to_dev(k, cuda), to_dev(v, cuda), to_dev(lay.block_tables, cuda),
+            to_dev(lay.context_lens, cuda), scale)
+    for size in (0, 64):  # the library's slices, and the caller's
+        out = torch.full((len(CONTEXTS), H, D), 7.0, dtype=torch.float16, device=cuda)
+        vkv.paged_decode(out, *args, partition_size=size)
+        torch.cuda.synchronize()
+        assert_close(to_np(out).astype(np.float32), ref, F16_ATOL, F16_RTOL, f"{H}/{Hkv}/{D}/bs{bs} size {size}")
+    acc = torch.ones((len(CONTEXTS), H, D), dtype=torch.float16, device=cuda)
+    vkv.paged_decode(acc, *args, accumulate=True)
+    torch.cuda.synchronize()
+    assert_close(to_np(acc).astype(np.float32), ref + 1.0, F16_ATOL, F16_RTOL, "accumulate")
+
+
+@pytest.mark.parametrize("table", [1024, 6000], ids=["rows", "slices"])
+@pytest.mark.parametrize("H,Hkv,D,bs", [(4, 4, 80, 16), (34, 2, 112, 24), (32, 2, 128, 16), (14, 2, 64, 8)])
+def test_stream_fused_append(vkv, cuda, H, Hkv, D, bs, table):
+    """The fused step against the append and the decode as two calls: same bits."""
+    import torch
+    rng = np.random.default_rng(D + bs)
+    ctx = [1, 32, 33, 300, 31]
+    lay, (k, v), q = _case(rng, H, Hkv, D, bs, ctx, table)
+    new = [(rng.standard_normal((len(ctx), Hkv, D), dtype=np.float32) * 0.7).astype(np.float16) for _ in range(2)]
+    slots = lay.slots(lay.context_lens - 1, np.arange(len(ctx)))
+    slots[3] = -1  # skipped: the cache keeps its rows and the decode reads them
+    got = []
+    for fused in (True, False):
+        kc, vc = to_dev(k, cuda), to_dev(v, cuda)
+        out = torch.zeros((len(ctx), H, D), dtype=torch.float16, device=cuda)
+        args = (out, to_dev(q, cuda), kc, vc, to_dev(lay.block_tables, cuda), to_dev(lay.context_lens, cuda), D ** -0.5)
+        rows = (to_dev(new[0], cuda), to_dev(new[1], cuda))
+        if fused:
+            vkv.paged_decode_append(*args, *rows, to_dev(slots, cuda))
+        else:
+            vkv.reshape_and_cache(*rows, kc, vc, to_dev(slots, cuda))
+            vkv.paged_decode(*args)
+        torch.cuda.synchronize()
+        got.append([to_np(x).view(np.uint16) for x in (out, kc, vc)])
+    for a, b in zip(*got):
+        assert np.array_equal(a, b)
+
+
+def test_stream_noalloc_without_room_for_slices(vkv, oracle, cuda):
+    """A call whose slices would not fit the library's array, but whose plain
+    partitions do: accepted, and as right as the call with a workspace."""
+    import torch
+    H, Hkv, D, bs, S = 32, 2, 128, 16, 400
+    rng = np.random.default_rng(3)
+    ctx = rng.integers(1, 40, S)
+    lay, (k, v), q = _case(rng, H, Hkv, D, bs, ctx, 4096)
+    out = torch.zeros((S, H, D), dtype=torch.float16, device=cuda)
+    args = (out, to_dev(q, cuda), to_dev(k, cuda), to_dev(v, cuda), to_dev(lay.block_tables, cuda),
+            to_dev(lay.context_lens, cuda), D ** -0.5)
+    assert vkv.decode_workspace_size(*args) > 64 << 20
+    vkv.paged_decode_noalloc(*args)
+    torch.cuda.synchronize()
+    ref = oracle.paged_decode(q.astype(np.float32), np.nan_to_num(k).view(np.uint16), np.nan_to_num(v).view(np.uint16),
+                              lay.block_tables, lay.context_lens, D ** -0.5)
+    assert_close(to_np(out).astype(np.float32), ref, F16_ATOL, F16_RTOL, "noalloc")

@@ -70,6 +70,8 @@ constexpr int kOneChunkAboveGFp8 = VKV_DECODE_ONE_CHUNK_ABOVE_G_FP8;
 constexpr int64_t kMinItems = 2048;
 // Small batches stop splitting before a row could have more partitions than this.
 constexpr int64_t kMaxSplitParts = 64;
+// Shortest slices that equal-slice split calls (decode_stream.hip) hold partials for.
+constexpr int64_t kSliceTokens = 128;
 // Per-call partition choice (library default only).  Candidates relative to
 // the default size P0 (block multiples, at most 64 blocks): 3/4, 7/8, 1, 5/4,
 // 5/3, 2 x P0 (at P0 = 768: 576, 672, 768, 960, 1 280 and 1 536 tokens with
@@ -874,8 +876,8 @@ __global__ __launch_bounds__(DT ? DT : 1024) void decode_reduce_kernel(DecodeArg
     if (a.qsl && a.qsl[s + 1] - a.qsl[s] != 1) return;
     load_batch(0);
     const int ctx = row_context(a, s);
-    const int P = a.num_cands > 1 ? __builtin_amdgcn_readfirstlane(a.counters[kChosenPartitionSlot]) : a.P;
-    const int np = ctx > 0 ? (ctx + P - 1) / P : 0;
+    const int P = a.num_cands > 1 && !a.row_parts ? __builtin_amdgcn_readfirstlane(a.counters[kChosenPartitionSlot]) : a.P;
+    const int np = a.row_parts ? a.row_parts[s] : ctx > 0 ? (ctx + P - 1) / P : 0;
     float m = -INFINITY, l = 0.0f, acc = 0.0f;
     for (int i0 = 0; i0 < np; i0 += kMergeBatch) {
         if (i0 > 0) load_batch(i0);
@@ -915,6 +917,8 @@ void launch_g(DecodeArgs& args, int grid_x, int grid_y, int grid_z, size_t lds, 
     // Matrix-core QK^T for fp16 query and keys at D = 128 with blocks of a
     // multiple of 16 tokens; the VALU variant covers everything else.
     constexpr bool kMfmaShape = std::is_same<IO, _Float16>::value && KVT != kF32 && D == 128;
+    // fp16 over fp16 at head_dim 64 and 128 runs on decode_stream.hip otherwise.
+    constexpr bool kStreamed = mfma_enabled() && std::is_same<IO, _Float16>::value && KVT == kF16 && D <= 128;
     // grid_x arrives as the number of item groups (an upper bound).  One workgroup per resident slot: the variant's workgroups per CU by
     // registers (queried once per variant), bounded by the LDS the rows'
     // prefix takes, and never more than there are item groups.  Groups
@@ -969,7 +973,7 @@ void launch_g(DecodeArgs& args, int grid_x, int grid_y, int grid_z, size_t lds, 
     if (kMfmaShape && args.bs_log2 >= 4 && args.mfma_enabled)
         run(decode_partition_kernel<IO, KVT, D, G, kMfmaShape, false>,
             decode_partition_kernel<IO, KVT, D, G, kMfmaShape, kStatic>, 1);
-    else
+    else if constexpr (!kStreamed)
         run(decode_partition_kernel<IO, KVT, D, G, false, false>, decode_partition_kernel<IO, KVT, D, G, false, kStatic>, 0);
 }
 
@@ -1024,8 +1028,8 @@ __global__ __launch_bounds__(kWave) void decode_reduce_wave_kernel(DecodeArgs a)
     const float* o = a.part_o + slot0 * DT + d;
     if (a.qsl && a.qsl[s + 1] - a.qsl[s] != 1) return;
     const int ctx = row_context(a, s);
-    const int P = a.num_cands > 1 ? __builtin_amdgcn_readfirstlane(a.counters[kChosenPartitionSlot]) : a.P;
-    const int np = ctx > 0 ? (ctx + P - 1) / P : 0;
+    const int P = a.num_cands > 1 && !a.row_parts ? __builtin_amdgcn_readfirstlane(a.counters[kChosenPartitionSlot]) : a.P;
+    const int np = a.row_parts ? a.row_parts[s] : ctx > 0 ? (ctx + P - 1) / P : 0;
     // partials of batch i0 (slots past np are neither loaded nor read)
     float bm[B], bl[B];
     fE bo[B];
@@ -1099,6 +1103,11 @@ int launch_reduce(int D, const DecodeArgs& args, int H, int S, hipStream_t st) {
     return launch_reduce_b<IO, 64>(D, args, H, S, st);
 }
 
+bool stream_shape(const vkv_decode_params* p) {
+    return mfma_enabled() && stream_decode_shape(p->head_dim, p->num_heads / p->num_kv_heads, p->key_cache, p->value_cache,
+                                                 p->io_dtype == VKV_DTYPE_F16, p->kv_dtype == VKV_DTYPE_F16);
+}
+
 int ilog2(int x) {
     int r = 0;
     while ((1 << r) < x) ++r;
@@ -1169,8 +1178,27 @@ DecodePlan plan_decode(const vkv_decode_params* p) {
     }
     plan.max_parts = int((max_ctx + smallest - 1) / smallest);
     if (plan.max_parts < 1) plan.max_parts = 1;
-    plan.workspace_bytes = kWorkspaceHeader + size_t(launch_rows_max(p->num_seqs)) * p->num_heads * plan.max_parts *
-                                                  (p->head_dim + 2) * sizeof(float);
+    const size_t rows = size_t(launch_rows_max(p->num_seqs));
+    const size_t part_bytes = rows * p->num_heads * (p->head_dim + 2) * sizeof(float);  // one partial of every row
+    plan.base_bytes = plan.workspace_bytes = kWorkspaceHeader + part_bytes * plan.max_parts;
+    plan.whole_rows = false;
+    plan.stream = stream_shape(p);
+    if (plan.stream && !matrix_split_shape(p->head_dim, p->num_heads / p->num_kv_heads, bs, p->key_cache, p->value_cache)) {
+        // Equal slices (decode_stream.hip): partials for slices of down to
+        // kSliceTokens tokens, at most kMaxSplitParts of a row and one more (a
+        // row's first and last slice are shared with its neighbours).  A
+        // caller's size is rounded up to whole steps of 32 tokens.
+        const bool own = p->partition_size <= 0;
+        const int64_t slice = own ? kSliceTokens : (int64_t(P) + 31) / 32 * 32;
+        int64_t parts = (max_ctx + slice - 1) / slice;
+        if (own && parts > kMaxSplitParts) parts = kMaxSplitParts;
+        parts = parts < 1 ? 2 : parts + 1;
+        if (own && parts < plan.max_parts) parts = plan.max_parts;
+        plan.partition_size = int(slice);
+        plan.num_candidates = own ? 2 : 1;  // 2: the kernel sizes the slices
+        plan.max_parts = int(parts);
+        plan.workspace_bytes = kWorkspaceHeader + part_bytes * plan.max_parts + rows * sizeof(int32_t);
+    }
     return plan;
 }
 
@@ -1244,6 +1272,9 @@ int launch_rows(const vkv_decode_params* p, const DecodePlan& plan, void* worksp
     const int D = p->head_dim;
     const int io_eb = p->io_dtype == VKV_DTYPE_F32 ? 4 : 2;
     const bool fixed = fixed_decode_shape(D, G, p->block_size, p->key_cache, p->value_cache);
+    const bool split_streams = plan.stream && !matrix_split_shape(D, G, p->block_size, p->key_cache, p->value_cache);
+    a.row_parts = split_streams ? reinterpret_cast<int32_t*>(a.part_ml + size_t(rows) * p->num_heads * plan.max_parts * 2)
+                                : nullptr;
     a.head_dim = D;
     a.block_size = p->block_size;
     set_block_div(a, p->block_size);
@@ -1260,10 +1291,12 @@ int launch_rows(const vkv_decode_params* p, const DecodePlan& plan, void* worksp
         const int n = p->num_seqs - r0 < kMaxRowsPerLaunch ? p->num_seqs - r0 : kMaxRowsPerLaunch;
         DecodeArgs c = a;
         c.num_rows = n;
+        const bool whole_rows = plan.stream && (plan.whole_rows || stream_decode_rows(n, p->num_kv_heads, D, c.max_ctx, !split_streams));
+        const bool streamed = whole_rows || split_streams;
         // Small plain decode calls (at most one (row, kv head) pair per CU):
         // a static grid over the partitions of the default size, if its waves
         // are all resident at once (decided at launch).
-        if (fixed && !qsl && !row_seq && p->io_dtype == VKV_DTYPE_F16 &&
+        if (fixed && !streamed && !qsl && !row_seq && p->io_dtype == VKV_DTYPE_F16 &&
             int64_t(n) * p->num_kv_heads <= device_cu_count())
             c.static_parts = int32_t((int64_t(c.max_ctx) + c.P - 1) / c.P > 0 ? (int64_t(c.max_ctx) + c.P - 1) / c.P : 1);
         if (qsl) {
@@ -1296,7 +1329,10 @@ int launch_rows(const vkv_decode_params* p, const DecodePlan& plan, void* worksp
         const int grid_x = int(item_wgs < 1 ? 1 : item_wgs);
         const size_t lds = (size_t(n) + 1) * sizeof(int) + lpt_lds_bytes(n);
         int rc;
-        if (!fixed) {
+        if (streamed) {
+            rc = launch_decode_stream(c, whole_rows, (size_t(n) + 1) * sizeof(int), st);
+            if (!rc && !whole_rows) rc = launch_reduce<_Float16>(D, c, p->num_heads, n, st);
+        } else if (!fixed) {
             rc = launch_decode_generic(c, p->kv_dtype, int64_t(n) * plan.max_parts, lds, st);
             if (!rc) rc = p->io_dtype == VKV_DTYPE_F32 ? launch_reduce<float>(D, c, p->num_heads, n, st)
                                                        : launch_reduce<_Float16>(D, c, p->num_heads, n, st);
@@ -1338,8 +1374,8 @@ bool decode_append_fusable(const vkv_append_params* ap, const vkv_decode_params*
            ap->num_kv_heads == p->num_kv_heads && ap->head_dim == p->head_dim &&
            ap->block_size == p->block_size && ap->num_blocks == p->num_blocks && (src & 15u) == 0 &&
            ks % 16 == 0 && vs % 16 == 0 &&
-           fixed_decode_shape(p->head_dim, p->num_heads / p->num_kv_heads, p->block_size, p->key_cache,
-                              p->value_cache);
+           (stream_shape(p) || fixed_decode_shape(p->head_dim, p->num_heads / p->num_kv_heads, p->block_size,
+                                                  p->key_cache, p->value_cache));
 }
 
 int launch_decode_append(const vkv_append_params* ap, const vkv_decode_params* p, const DecodePlan& plan,

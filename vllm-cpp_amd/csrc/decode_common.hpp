@@ -90,6 +90,10 @@ struct DecodeArgs {
     // prefix scan, no claims, and items request their block ids together with
     // the context length.  0: the persistent claim loop.
     int32_t static_parts;
+    // decode_stream.hip's split calls: partials of each row (written by the
+    // partition launch, read by the merge), nullptr for the other kernels
+    // (whose rows have ceil(context / P)).
+    int32_t* row_parts;
     // Append fused into the call (source rows in the cache's element type,
     // fp16 or fp32; fixed shapes): row s's new token is fkey / fval + s *
     // stride (bytes), bound for cache slot fslots[s].  The partition kernel
@@ -123,6 +127,24 @@ inline bool fixed_decode_shape(int head_dim, int group, int block_size, const vo
     const bool aligned = ((reinterpret_cast<uintptr_t>(kc) | reinterpret_cast<uintptr_t>(vc)) & 15u) == 0;
     return (head_dim == 64 || head_dim == 128 || head_dim == 256) && group >= 1 && group <= 8 && pow2_bs && aligned;
 }
+
+// The shapes of decode_stream.hip: fp16 queries over fp16 caches at these head
+// dimensions, groups of up to 32 heads and any block size.  Split-K calls at
+// head_dim 128, groups of up to 8 and power-of-two blocks of 16 tokens and more
+// stay on decode.hip's matrix-core kernel (matrix_split_shape).
+inline bool stream_decode_shape(int head_dim, int group, const void* kc, const void* vc, bool f16_io, bool f16_kv) {
+    const bool aligned = ((reinterpret_cast<uintptr_t>(kc) | reinterpret_cast<uintptr_t>(vc)) & 15u) == 0;
+    return f16_io && f16_kv && aligned && head_dim >= 64 && head_dim <= 128 && head_dim % 16 == 0 && group >= 1 &&
+           group <= 32;
+}
+inline bool matrix_split_shape(int head_dim, int group, int block_size, const void* kc, const void* vc) {
+    return head_dim == 128 && block_size >= 16 && fixed_decode_shape(head_dim, group, block_size, kc, vc);
+}
+// Whether a launch of num_rows rows runs as one workgroup per (row, kv head),
+// merged in LDS, instead of split-K.
+bool stream_decode_rows(int num_rows, int num_kv_heads, int head_dim, int max_ctx, bool matrix_split);
+// The call's partition launch (or, with rows, its only launch).  0 or VKV_ERR_*.
+int launch_decode_stream(DecodeArgs& a, bool rows, size_t lds, hipStream_t st);
 
 // Partition kernel of the generic variant (decode_generic.hip) for one launch
 // of rows; max_pairs bounds the (row, partition) pairs.  0 or VKV_ERR_*.

@@ -50,12 +50,14 @@ int scratch_address(void** out) {
 extern "C" int vkv_paged_decode_noalloc(const vkv_decode_params* p, vkv_stream_t stream) {
     int rc = vkv::check_decode_args(p);
     if (rc != VKV_OK || p->num_seqs == 0) return rc;
-    const vkv::DecodePlan plan = vkv::plan_decode(p);
-    if (plan.workspace_bytes > kScratchBytes)
+    vkv::DecodePlan plan = vkv::plan_decode(p);
+    if (plan.base_bytes > kScratchBytes)
         return vkv::report_error(VKV_ERR_WORKSPACE,
                                  "vkv_paged_decode_noalloc: the call needs %zu bytes of split-K scratch, more than "
                                  "the %zu the library holds; use vkv_paged_decode with a workspace",
-                                 plan.workspace_bytes, kScratchBytes);
+                                 plan.base_bytes, kScratchBytes);
+    // a finer split than the array holds: one workgroup per (row, kv head), which needs no scratch
+    plan.whole_rows = plan.workspace_bytes > kScratchBytes;
     void* ws = nullptr;
     rc = scratch_address(&ws);
     if (rc != VKV_OK) return rc;

@@ -1,0 +1,619 @@
+// decode_stream.hip — paged decode attention for fp16 queries over fp16 caches
+// at head_dim 64, 80, 96, 112 or 128 with groups of up to 32 query heads, both
+// products on the matrix cores (gfx950).  Semantics as in decode.hip (the
+// reference's src/attention/paged_attention.cu:13-82).
+//
+// A wave streams the K and V rows of its tokens through LDS, 32 tokens a step,
+// with direct global->LDS loads (global_load_lds_dwordx4, 1 KiB per wave
+// instruction) into a ring that is the wave's own: no barrier, no registers
+// held by loads in flight, and a load waits only for its own stage
+// (s_waitcnt vmcnt counted in asm).  A step then costs, whatever the group:
+//   S^T = K Q^T   v_mfma_f32_16x16x32_f16 (and one 16x16x16 when head_dim is
+//                 an odd multiple of 16): A = K rows from LDS, B = Q in
+//                 registers (columns = the group's heads, 16 per tile);
+//   softmax       lane-local on the S^T layout (lane l: head l % 16, keys
+//                 4 (l / 16) + e of each 16-key half), the running max raised
+//                 lazily (only when a score passes it by 2^8);
+//   O^T += V^T P^T  A = V^T by ds_read_b64_tr_b16 from the row-major tile,
+//                 B = P^T straight from the S^T registers, so the weights
+//                 never leave the lane and the accumulators are head_dim / 4
+//                 registers per 16 heads.
+// The VALU kernels that served these shapes spent ~300 instructions per 16
+// tokens and held 4 KiB of loads per wave, waited for in turn.
+#include <atomic>
+#include <type_traits>
+
+#include "common.hpp"
+#include "decode_common.hpp"
+#include "launch.hpp"
+
+namespace vkv {
+namespace dec {
+namespace {
+
+typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
+typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
+typedef float float4_t __attribute__((ext_vector_type(4)));
+typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+
+constexpr int kStep = 32;            // tokens per step (the k of the P V products)
+constexpr float kLazyLog2 = 8.0f;    // the running max is raised when passed by 2^8
+
+// LDS tile of a step's K (or V) rows: row-major, unpadded (a direct load
+// writes lane L's 16 bytes at 16 L).  Where a row is a power of two of 16-byte
+// chunks, chunk c of row r sits at slot c ^ (r % CH): the operand reads take
+// one chunk column of 16 rows, which would otherwise meet in the same banks.
+// (Rows of 160, 192 or 224 bytes are spread by their own stride.)
+template <int D>
+struct Tile {
+    static constexpr int ROW = 2 * D;
+    static constexpr int CH = ROW / 16;
+    static constexpr int NI = kStep * CH / 64;  // direct loads per tile
+    static constexpr int BYTES = kStep * ROW;
+    static constexpr bool SWZ = (CH & (CH - 1)) == 0;
+    static constexpr int KS = D / 32;       // 32-dim MFMA steps of K Q^T
+    static constexpr bool HALF = D % 32 != 0;  // and a 16-dim one
+    static constexpr int DT = D / 16;       // dim tiles of O^T
+    static_assert(D % 16 == 0 && kStep * CH % 64 == 0, "whole loads");
+    __device__ static __forceinline__ int slot(int row, int chunk) { return SWZ ? chunk ^ (row % CH) : chunk; }
+    __device__ static __forceinline__ int off(int row, int chunk) { return row * ROW + slot(row, chunk) * 16; }
+};
+
+__device__ __forceinline__ uint32_t lds_addr(const char* p) {
+    typedef const __attribute__((address_space(3))) char* lds_cptr;
+    return uint32_t(size_t((lds_cptr)p));
+}
+// One 16-byte direct load per lane to LDS bytes lds + 16 lane (s_nop 0: the
+// wait state between the M0 write and the load that reads it).
+// Rows of whole 128-byte lines stream past the caches (nt); other rows share
+// lines with the neighbouring heads, whose waves read them soon after.
+template <bool NT>
+__device__ __forceinline__ void dma16(const char* g, const uint32_t lds) {
+    const uint32_t l = __builtin_amdgcn_readfirstlane(lds);
+    if constexpr (NT)
+        asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off nt" : : "v"(g), "s"(l) : "memory", "m0");
+    else
+        asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(g), "s"(l) : "memory", "m0");
+}
+template <int N>
+__device__ __forceinline__ void wait_loads() {
+    static_assert(N >= 0 && N < 64, "vmcnt is 6 bits");
+    asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory");
+}
+// This wave's LDS operations have completed (before a load overwrites what they read).
+__device__ __forceinline__ void wait_lds() { asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory"); }
+
+__device__ __forceinline__ u32x2 tr_read(const char* lds) {
+    typedef __fp16 fp16x4_t __attribute__((__vector_size__(4 * sizeof(__fp16))));
+    typedef __attribute__((address_space(3))) fp16x4_t* lds_ptr;
+    return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4f16((lds_ptr)(lds)));
+}
+
+// Attention state of one wave: CT tiles of 16 heads.
+template <int D, int CT>
+struct State {
+    using T = Tile<D>;
+    half8_t q[CT][T::KS];
+    half4_t qh[CT];
+    float m[CT];              // running max of head 16 ct + l % 16, raw logits
+    float4_t l[CT];           // weight sums (every element the same)
+    float4_t o[CT][T::DT];    // O^T: lane l holds dims 16 t + 4 (l / 16) + e of head l % 16
+};
+
+// Q as the B operand and an empty state.  Columns past the group read head 0
+// and are zeroed; a negative scale is moved into Q (exact sign flip).
+template <int D, int CT>
+__device__ __forceinline__ void init_state(const DecodeArgs& a, State<D, CT>& st, const int s, const int kvh,
+                                           const int G, const int lane) {
+    using T = Tile<D>;
+    const int col = lane & 15, grp = lane >> 4;
+    const uint32_t flip = a.scale_log2 < 0.0f ? 0x80008000u : 0u;
+#pragma unroll
+    for (int c = 0; c < CT; ++c) {
+        const int h = 16 * c + col;
+        const uint32_t keep = h < G ? 0xFFFFFFFFu : 0u;
+        const char* qrow = static_cast<const char*>(a.q) +
+                           (query_row(a, s) * a.q_stride + int64_t(kvh * G + (h < G ? h : 0)) * D) * 2;
+#pragma unroll
+        for (int i = 0; i < T::KS; ++i) {
+            u32x4 w = load16(qrow + (32 * i + 8 * grp) * 2);
+            w = (w ^ u32x4{flip, flip, flip, flip}) & u32x4{keep, keep, keep, keep};
+            st.q[c][i] = __builtin_bit_cast(half8_t, w);
+        }
+        if constexpr (T::HALF) {
+            u32x2 w = *reinterpret_cast<const u32x2*>(qrow + (32 * T::KS + 4 * grp) * 2);
+            w = (w ^ u32x2{flip, flip}) & u32x2{keep, keep};
+            st.qh[c] = __builtin_bit_cast(half4_t, w);
+        }
+        st.m[c] = -INFINITY;
+        st.l[c] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int t = 0; t < T::DT; ++t) st.o[c][t] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+}
+
+// Attends tokens [t0, t0 + n) (n >= 1) of row s at kv head kvh.  ring: NST
+// stages of a K and a V tile, this wave's own.  my_block: block ids of
+// [win, win + 64) in the row's table, one per lane (0 where out of the pool).
+template <int D, int CT, int NST>
+__device__ __forceinline__ void stream_tokens(const DecodeArgs& a, State<D, CT>& st, char* ring, const int s,
+                                              const int32_t* table, const int ctx, const int kvh, const int t0,
+                                              const int n, int win, int my_block, const int lane) {
+    using T = Tile<D>;
+    constexpr int kStage = 2 * T::BYTES;
+    constexpr int kLoads = 2 * T::NI;  // vector-memory operations per stage
+    const int col = lane & 15, grp = lane >> 4;
+    const uint32_t slot_stride = uint32_t(a.num_kv_heads) * T::ROW;
+    const uint32_t ring_lds = lds_addr(ring);
+    const float sc = a.scale_log2 < 0.0f ? -a.scale_log2 : a.scale_log2;
+    const float lazy = kLazyLog2 / sc;
+    const int steps = (n + kStep - 1) / kStep;
+    // The fused append: the row's last position reads the new token's rows
+    // when the append targets that position's slot.
+    const bool fused = a.fkey && t0 + n == ctx;
+    const int64_t fslot = fused ? int64_t(a.fslots[s]) : -1;
+
+    auto issue = [&](const int step, const int stage) __attribute__((always_inline)) {
+        const int last = min(step * kStep + kStep, n) - 1;
+        if (block_div(a, t0 + last) - win >= kWave) {  // (wave-uniform)
+            win = block_div(a, t0 + step * kStep);
+            my_block = 0;
+            if (win + lane < a.max_blocks_per_seq) {
+                my_block = table[win + lane];
+                if (a.num_blocks > 0 && unsigned(my_block) >= unsigned(a.num_blocks)) my_block = 0;
+            }
+        }
+        const bool has_new = fused && step == steps - 1;
+        const uint32_t dst = ring_lds + uint32_t(stage * kStage);
+#pragma unroll
+        for (int i = 0; i < T::NI; ++i) {
+            const int row = (i * 64 + lane) / T::CH;
+            const uint32_t chunk = uint32_t(T::slot(row, (i * 64 + lane) % T::CH)) * 16;  // (slot is its own inverse)
+            // tokens past the end read the last one again (masked below)
+            const int tok = t0 + min(step * kStep + row, n - 1);
+            const int blk = block_div(a, tok);
+            const int64_t slot = int64_t(__shfl(my_block, blk - win, kWave)) * a.block_size + (tok - blk * a.block_size);
+            const uint64_t off = uint64_t(slot) * slot_stride + (uint32_t(kvh * T::ROW) + chunk);
+            const char* kp = a.kc + off;
+            const char* vp = a.vc + off;
+            if (has_new && tok == ctx - 1 && slot == fslot) {
+                kp = a.fkey + s * a.fkey_stride + kvh * T::ROW + chunk;
+                vp = a.fval + s * a.fval_stride + kvh * T::ROW + chunk;
+            }
+            dma16<T::ROW % 128 == 0>(kp, dst + i * 1024);
+            dma16<T::ROW % 128 == 0>(vp, dst + T::BYTES + i * 1024);
+        }
+    };
+
+    const half8_t ones = {1.0f16, 1.0f16, 1.0f16, 1.0f16, 1.0f16, 1.0f16, 1.0f16, 1.0f16};
+    auto compute = [&](const int step, const int stage) __attribute__((always_inline)) {
+        char* kb = ring + stage * kStage;
+        char* vb = kb + T::BYTES;
+        const bool tail = step * kStep + kStep > n;
+        if (tail) {
+            // rows past the end: V zero whatever the slots hold (their weight is 0)
+#pragma unroll
+            for (int i = 0; i < T::NI; ++i)
+                if (step * kStep + (i * 64 + lane) / T::CH >= n) store16(vb + i * 1024 + lane * 16, u32x4{0u, 0u, 0u, 0u});
+            wave_lds_sync();
+        }
+        float4_t sv[CT][2];
+        [[maybe_unused]] float4_t half_sv[CT][2];
+#pragma unroll
+        for (int c = 0; c < CT; ++c) sv[c][0] = sv[c][1] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int hh = 0; hh < 2; ++hh) {
+#pragma unroll
+            for (int i = 0; i < T::KS; ++i) {
+                const half8_t k = __builtin_bit_cast(half8_t, load16(kb + T::off(16 * hh + col, 4 * i + grp)));
+#pragma unroll
+                for (int c = 0; c < CT; ++c)
+                    sv[c][hh] = __builtin_amdgcn_mfma_f32_16x16x32_f16(k, st.q[c][i], sv[c][hh], 0, 0, 0);
+            }
+            if constexpr (T::HALF) {
+                // A product of its own, added on the VALU: accumulated onto the
+                // 16x16x32 result right behind it (no wait state between the
+                // two shapes in the compiler's code), head_dim 112 gave wrong
+                // scores.
+                const half4_t k = __builtin_bit_cast(
+                    half4_t, *reinterpret_cast<const u32x2*>(kb + (16 * hh + col) * T::ROW + 64 * T::KS + 8 * grp));
+#pragma unroll
+                for (int c = 0; c < CT; ++c) {
+                    const float4_t zero = {0.0f, 0.0f, 0.0f, 0.0f};
+                    half_sv[c][hh] = __builtin_amdgcn_mfma_f32_16x16x16f16(k, st.qh[c], zero, 0, 0, 0);
+                }
+            }
+        }
+        if constexpr (T::HALF) {
+#pragma unroll
+            for (int c = 0; c < CT; ++c)
+#pragma unroll
+                for (int hh = 0; hh < 2; ++hh) sv[c][hh] += half_sv[c][hh];
+        }
+        half8_t p[CT];
+#pragma unroll
+        for (int c = 0; c < CT; ++c) {
+            float x[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) x[e] = sv[c][e >> 2][e & 3];
+            if (tail) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+                    if (step * kStep + 16 * (e >> 2) + 4 * grp + (e & 3) >= n) x[e] = -INFINITY;
+            }
+            const float mx = fmaxf(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])), fmaxf(fmaxf(x[4], x[5]), fmaxf(x[6], x[7])));
+            // Below m + lazy the weights stay under 2^8, exact enough in fp16
+            // as any others; the first step always sets m.
+            if (__builtin_amdgcn_ballot_w64(mx > st.m[c] + lazy)) {
+                const float mn = fmaxf(st.m[c], xor_max<32>(xor_max<16>(mx)));
+                const float alpha = mn > st.m[c] ? __builtin_amdgcn_exp2f((st.m[c] - mn) * sc) : 1.0f;
+                st.m[c] = mn;
+                st.l[c] *= alpha;
+#pragma unroll
+                for (int t = 0; t < T::DT; ++t) st.o[c][t] *= alpha;
+            }
+            const float msc = st.m[c] == -INFINITY ? 0.0f : st.m[c] * sc;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) p[c][e] = static_cast<_Float16>(__builtin_amdgcn_exp2f(fmaf(x[e], sc, -msc)));
+            // sums of the rounded weights, on the matrix pipe
+            st.l[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ones, p[c], st.l[c], 0, 0, 0);
+        }
+        // V^T operand: within each 16-lane group, lane i receives element i % 4
+        // of the 8-byte chunks addressed by lanes i / 4 + 4 e, so lane (col,
+        // grp) addresses key 4 grp + col / 4 (+ 16), dims 16 t + 4 (col % 4)
+        const int vrow = 4 * grp + (col >> 2);
+#pragma unroll
+        for (int t = 0; t < T::DT; ++t) {
+            const int chunk = 2 * t + ((col & 3) >> 1);
+            const u32x2 lo = tr_read(vb + T::off(vrow, chunk) + 8 * (col & 1));
+            const u32x2 hi = tr_read(vb + T::off(16 + vrow, chunk) + 8 * (col & 1));
+            const half8_t v = __builtin_bit_cast(half8_t, u32x4{lo[0], lo[1], hi[0], hi[1]});
+#pragma unroll
+            for (int c = 0; c < CT; ++c) st.o[c][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(v, p[c], st.o[c][t], 0, 0, 0);
+        }
+    };
+
+    if constexpr (NST == 1) {
+        for (int step = 0; step < steps; ++step) {
+            wait_lds();
+            issue(step, 0);
+            wait_loads<0>();
+            compute(step, 0);
+        }
+    } else {
+        static_assert(NST == 2, "one or two stages");
+        wait_lds();
+        issue(0, 0);
+        for (int step = 0; step < steps; ++step) {
+            if (step + 1 < steps) {
+                wait_lds();  // (the stage's reads, two steps ago in program order, are done)
+                issue(step + 1, (step + 1) & 1);
+                wait_loads<kLoads>();
+            } else {
+                wait_loads<0>();
+            }
+            compute(step, step & 1);
+        }
+    }
+}
+
+__device__ __forceinline__ int load_block(const DecodeArgs& a, const int32_t* table, const int i) {
+    int id = 0;
+    if (i < a.max_blocks_per_seq) {
+        id = table[i];
+        if (a.num_blocks > 0 && unsigned(id) >= unsigned(a.num_blocks)) id = 0;
+    }
+    return id;
+}
+
+// ---------------------------------------------------------------------------
+// A workgroup of W waves per (row, kv head): each wave attends a contiguous
+// share of the context and the shares are merged in LDS, so the call is one
+// launch with no workspace.
+template <int D, int CT, int W, int NST>
+__global__ __launch_bounds__(64 * W) void decode_rows_kernel(const DecodeArgs a) {
+    using T = Tile<D>;
+    constexpr int kRing = NST * 2 * T::BYTES;
+    constexpr int kMergeBytes = W * 16 * CT * (D + 2) * 4;
+    __shared__ __attribute__((aligned(1024))) char lds[W * kRing > kMergeBytes ? W * kRing : kMergeBytes];
+    const int lane = threadIdx.x & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    // Rows that are not whole 128-byte lines share lines with the neighbouring
+    // heads (four heads are whole lines): four adjacent heads go to one XCD
+    // (workgroups are dealt to the 8 XCDs in turn), next to each other there.
+    int pair = int(blockIdx.x);
+    if (T::ROW % 128 != 0 && pair < int(gridDim.x) / 32 * 32)
+        pair = pair / 32 * 32 + (pair % 8) * 4 + pair % 32 / 8;
+    const int s = pair / a.num_kv_heads;
+    const int kvh = pair - s * a.num_kv_heads;
+    const int G = a.num_heads / a.num_kv_heads;
+    const int seq = a.row_seq ? a.row_seq[s] : s;
+    const int32_t* table = a.bt + int64_t(seq) * a.max_blocks_per_seq;
+    if (a.qsl && a.qsl[s + 1] - a.qsl[s] != 1) return;  // (a prefill sequence of a mixed call)
+    // requested together with the context length: Q, and the block ids while
+    // the table fits one id per lane
+    const bool whole = a.max_blocks_per_seq <= kWave;
+    int ids = whole ? load_block(a, table, lane) : 0;
+    State<D, CT> st;
+    init_state(a, st, s, kvh, G, lane);
+    const int ctx = row_context(a, s);
+    const int per = ((ctx + W - 1) / W + kStep - 1) / kStep * kStep;
+    const int t0 = wave * per;
+    const int n = min(ctx - t0, per);
+    if (n > 0) {
+        int win = 0;
+        if (!whole) {
+            win = block_div(a, t0);
+            ids = load_block(a, table, win + lane);
+        }
+        stream_tokens<D, CT, NST>(a, st, lds + wave * kRing, s, table, ctx, kvh, t0, n, win, ids, lane);
+    }
+    // ---------------- merge
+    const float sc = a.scale_log2 < 0.0f ? -a.scale_log2 : a.scale_log2;
+    const int col = lane & 15, grp = lane >> 4;
+    float* mo = reinterpret_cast<float*>(lds);      // [W][16 CT][D]
+    float* mml = mo + W * 16 * CT * D;              // [W][16 CT][2]
+    __syncthreads();
+    if (n > 0) {
+#pragma unroll
+        for (int c = 0; c < CT; ++c) {
+            const int h = 16 * c + col;
+            if (h >= G) continue;
+            float* row = mo + (wave * 16 * CT + h) * D;
+#pragma unroll
+            for (int t = 0; t < T::DT; ++t) *reinterpret_cast<float4_t*>(row + 16 * t + 4 * grp) = st.o[c][t];
+            if (grp == 0) {
+                mml[(wave * 16 * CT + h) * 2] = st.m[c] * sc;
+                mml[(wave * 16 * CT + h) * 2 + 1] = st.l[c][0];
+            }
+        }
+    } else if (lane < 16 * CT) {
+        mml[(wave * 16 * CT + lane) * 2] = -INFINITY;  // (no share: weight 0 below)
+        mml[(wave * 16 * CT + lane) * 2 + 1] = 0.0f;
+    }
+    __syncthreads();
+    _Float16* out = static_cast<_Float16*>(a.out) + (query_row(a, s) * a.num_heads + kvh * G) * D;
+    const int shares = ctx > 0 ? (ctx + per - 1) / per : 0;
+    for (int i = threadIdx.x; i < G * (D / 2); i += 64 * W) {
+        const int h = i / (D / 2), d = (i - h * (D / 2)) * 2;
+        float mx = -INFINITY;
+#pragma unroll
+        for (int w = 0; w < W; ++w) mx = fmaxf(mx, mml[(w * 16 * CT + h) * 2]);
+        float l = 0.0f, x0 = 0.0f, x1 = 0.0f;
+#pragma unroll
+        for (int w = 0; w < W; ++w) {
+            if (w < shares) {
+                const float f = __builtin_amdgcn_exp2f(mml[(w * 16 * CT + h) * 2] - mx);
+                const float* row = mo + (w * 16 * CT + h) * D + d;
+                l = fmaf(f, mml[(w * 16 * CT + h) * 2 + 1], l);
+                x0 = fmaf(f, row[0], x0);
+                x1 = fmaf(f, row[1], x1);
+            }
+        }
+        float r0 = shares > 0 ? x0 / l : 0.0f, r1 = shares > 0 ? x1 / l : 0.0f;
+        _Float16* o = out + h * D + d;
+        if (a.accumulate) {
+            r0 += static_cast<float>(o[0]);
+            r1 += static_cast<float>(o[1]);
+        }
+        o[0] = static_cast<_Float16>(r0);
+        o[1] = static_cast<_Float16>(r1);
+    }
+    // Fused append: this workgroup alone reads the new token's slot at this kv
+    // head, and has.
+    if (a.fkey) {
+        const int64_t slot = a.fslots[s];
+        if (slot >= 0 && slot < a.fnum_slots && threadIdx.x < 2 * T::CH) {
+            const bool v = threadIdx.x >= T::CH;
+            const int64_t c = int64_t(kvh) * T::ROW + (threadIdx.x - (v ? T::CH : 0)) * 16;
+            const char* src = v ? a.fval + s * a.fval_stride + c : a.fkey + s * a.fkey_stride + c;
+            char* dst = const_cast<char*>(v ? a.vc : a.kc) + slot * a.num_kv_heads * T::ROW + c;
+            store16(dst, load16(src));
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Split-K in equal slices.  The rows' contexts are laid end to end in steps of
+// 32 tokens and cut into slices of the same number of steps (a slice may end
+// in the middle of a row and begin another), one (slice, kv head) per resident
+// wave, kv heads fastest: every wave streams the same amount, whatever the
+// context lengths, where partitions of a fixed size leave some waves a second
+// one (256 rows of head_dim 64, contexts up to 4 096: 66 to 78 us over sizes
+// 128 to 512, 57 at the best of them).  A row's partials are its slices in
+// order; row_parts holds their number for the merge kernel.  Slices are at
+// least so long that no row has more than max_parts of them.
+constexpr int kMinSliceSteps = 2;
+// Building with -DVKV_STREAM_ROWS=1 (2) runs every launch as one workgroup per
+// (row, kv head) (in equal slices): an A/B switch.
+#ifndef VKV_STREAM_ROWS
+#define VKV_STREAM_ROWS 0
+#endif
+
+template <int D, int CT, int NST>
+__global__ __launch_bounds__(256) void decode_stream_kernel(const DecodeArgs a) {
+    using T = Tile<D>;
+    constexpr int kRing = NST * 2 * T::BYTES;
+    __shared__ __attribute__((aligned(1024))) char lds[kWavesPerBlock * kRing];
+    __shared__ int wave_total[kWavesPerBlock], wave_longest[kWavesPerBlock];
+    extern __shared__ int prefix[];  // [num_rows + 1] exclusive prefix of the rows' steps
+    const int lane = threadIdx.x & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int G = a.num_heads / a.num_kv_heads;
+    const int nrows = a.num_rows;
+    // Prefix scan: each thread sums a contiguous tile of rows, the tile sums
+    // are scanned across the workgroup, then each thread writes its entries.
+    auto steps_of = [&](int r) {
+        const int ctx = row_context(a, r);
+        return ctx > 0 ? (ctx + kStep - 1) / kStep : 0;
+    };
+    {
+        const int per = (nrows + kBlockThreads - 1) / kBlockThreads;
+        const int r0 = int(threadIdx.x) * per;
+        int local = 0, longest = 0;
+        for (int i = 0; i < per; ++i) {
+            const int x = r0 + i < nrows ? steps_of(r0 + i) : 0;
+            local += x;
+            longest = x > longest ? x : longest;
+        }
+        const int incl = wave_incl_scan(local);
+        for (int o = 32; o > 0; o >>= 1) longest = max(longest, __shfl_xor(longest, o, kWave));
+        if (lane == kWave - 1) {
+            wave_total[wave] = incl;
+            wave_longest[wave] = longest;
+        }
+        __syncthreads();
+        int run = incl - local;
+        for (int w = 0; w < wave; ++w) run += wave_total[w];
+        for (int i = 0; i < per; ++i) {
+            if (r0 + i < nrows) {
+                prefix[r0 + i] = run;
+                run += steps_of(r0 + i);
+            }
+        }
+        if (threadIdx.x == kBlockThreads - 1) prefix[nrows] = run;
+        __syncthreads();
+    }
+    const int total = __builtin_amdgcn_readfirstlane(prefix[nrows]);
+    int longest = 0;
+    for (int w = 0; w < kWavesPerBlock; ++w) longest = max(longest, wave_longest[w]);
+    // Steps per slice: an equal share of every resident wave (a size the
+    // caller asked for instead, a.P), within max_parts partials per row.
+    const int waves = int(gridDim.x) * kWavesPerBlock;
+    const int share = waves / a.num_kv_heads > 0 ? waves / a.num_kv_heads : 1;
+    int R = a.num_cands > 1 ? max((total + share - 1) / share, kMinSliceSteps) : a.P / kStep;
+    R = max(R, (longest + a.max_parts - 2) / (a.max_parts - 1));
+    R = __builtin_amdgcn_readfirstlane(max(R, 1));
+    if (blockIdx.x == 0) {
+        for (int r = int(threadIdx.x); r < nrows; r += kBlockThreads) {
+            const int b = prefix[r], e = prefix[r + 1];
+            a.row_parts[r] = e > b ? (e - 1) / R - b / R + 1 : 0;
+        }
+    }
+    const int items = (total + R - 1) / R * a.num_kv_heads;
+    const float sc = a.scale_log2 < 0.0f ? -a.scale_log2 : a.scale_log2;
+    const int col = lane & 15, grp = lane >> 4;
+    for (int it = int(blockIdx.x) * kWavesPerBlock + wave; it < items; it += waves) {
+        const int slice = it / a.num_kv_heads;
+        const int kvh = it - slice * a.num_kv_heads;
+        const int end = min((slice + 1) * R, total);
+        int at = slice * R;
+        int lo = 0, hi = nrows - 1;  // row = last r with prefix[r] <= at
+        while (lo < hi) {
+            const int mid = (lo + hi + 1) >> 1;
+            if (prefix[mid] <= at) lo = mid;
+            else hi = mid - 1;
+        }
+        for (int s = lo; at < end; ++s) {
+            const int b = prefix[s], e = min(prefix[s + 1], end);
+            if (e <= at) continue;  // (a row without keys)
+            const int seq = a.row_seq ? a.row_seq[s] : s;
+            const int32_t* table = a.bt + int64_t(seq) * a.max_blocks_per_seq;
+            const int ctx = row_context(a, s);
+            const int t0 = (at - b) * kStep;
+            const int n = min(ctx - t0, (e - at) * kStep);
+            const int win = block_div(a, t0);
+            const int ids = load_block(a, table, win + lane);
+            State<D, CT> st;
+            init_state(a, st, s, kvh, G, lane);
+            stream_tokens<D, CT, NST>(a, st, lds + wave * kRing, s, table, ctx, kvh, t0, n, win, ids, lane);
+            const int64_t slot = (int64_t(s) * a.num_kv_heads + kvh) * a.max_parts + (slice - b / R);
+#pragma unroll
+            for (int c = 0; c < CT; ++c) {
+                const int h = 16 * c + col;
+                if (h >= G) continue;
+                float* row = a.part_o + (slot * G + h) * D;
+#pragma unroll
+                for (int t = 0; t < T::DT; ++t) *reinterpret_cast<float4_t*>(row + 16 * t + 4 * grp) = st.o[c][t];
+                if (grp == 0) {
+                    a.part_ml[(slot * G + h) * 2] = st.m[c] * sc;
+                    a.part_ml[(slot * G + h) * 2 + 1] = st.l[c][0];
+                }
+            }
+            at = e;
+        }
+    }
+}
+
+// One workgroup per resident slot (occupancy queried once per variant).
+template <int D, int CT, int NST>
+void launch_split(DecodeArgs& a, size_t lds, hipStream_t st) {
+    static std::atomic<int> cached{0};
+    auto kernel = decode_stream_kernel<D, CT, NST>;
+    int per_cu = cached.load(std::memory_order_relaxed);
+    if (per_cu <= 0) {
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kBlockThreads, 0) != hipSuccess || per_cu <= 0) per_cu = 1;
+        cached.store(per_cu, std::memory_order_relaxed);
+    }
+    const int by_lds = kLdsPerCu / int(lds + 1024 + kWavesPerBlock * NST * 2 * Tile<D>::BYTES);
+    if (by_lds < per_cu) per_cu = by_lds > 0 ? by_lds : 1;
+    hipLaunchKernelGGL(kernel, dim3(device_cu_count() * per_cu), dim3(kBlockThreads), lds, st, a);
+}
+
+template <int D, int CT>
+void launch_shape(DecodeArgs& a, bool rows, size_t lds, hipStream_t st) {
+    if (rows) {
+        const int64_t pairs = int64_t(a.num_rows) * a.num_kv_heads;
+        const dim3 grid{unsigned(pairs)};
+        if (pairs <= device_cu_count())
+            hipLaunchKernelGGL((decode_rows_kernel<D, CT, 8, D == 64 ? 2 : 1>), grid, dim3(512), 0, st, a);
+        else
+            hipLaunchKernelGGL((decode_rows_kernel<D, CT, 4, D == 64 ? 2 : 1>), grid, dim3(256), 0, st, a);
+        return;
+    }
+    // (calls over thousands of rows leave LDS for one stage only)
+    if constexpr (D > 80) {
+        if (lds > (16 << 10)) {
+            launch_split<D, CT, 1>(a, lds, st);
+            return;
+        }
+    }
+    launch_split<D, CT, D == 80 ? 1 : 2>(a, lds, st);
+}
+
+template <int D>
+void launch_dim(DecodeArgs& a, int G, bool rows, size_t lds, hipStream_t st) {
+    if (G <= 16) launch_shape<D, 1>(a, rows, lds, st);
+    else launch_shape<D, 2>(a, rows, lds, st);
+}
+
+}  // namespace
+
+// One workgroup per (row, kv head) saves the merge launch and the scan of the
+// rows, but the longest row's workgroup streams alone at the end, at about 54
+// bytes per ns.  Measured both ways over contexts U[1, max_ctx] (us per
+// appending step, workgroup per row against equal slices; host-bound at ~13):
+//   head_dim 64,   64 pairs: max 2 048: 15.6 / 16.7   4 096: 26.1 / 21.8
+//                 512 pairs:     2 048: 33.1 / 36.3   4 096: 57.3 / 53.9
+//                2048 pairs:     2 048: 102 / 110     4 096: 189 / 192
+//   head_dim 128,  64 pairs:     1 024: 16.7 / 18.7   2 048: 27.8 / 22.7
+//     (group 16) 1024 pairs:     1 024: 63.0 / 74.6   2 048: 114 / 119     4 096: 207 / 205
+//   head_dim 80,   64 pairs:     1 024: 13.2 / 16.9   2 048: 20.6 / 18.6
+//                1024 pairs:       512: 23.8 / 25.4   1 024: 42.6 / 38.9
+//                2048 pairs:       256: 27.8 / 28.2     512: 48.1 / 47.6
+// Against decode.hip's split (head_dim 128, group 4): 256 pairs, 1 024: 18.6 /
+// 24.3; 2 048: 36.3 / 36.8; 1 024 pairs, 1 024: 53.9 / 79.1.
+bool stream_decode_rows(int num_rows, int num_kv_heads, int head_dim, int max_ctx, bool matrix_split) {
+#if VKV_STREAM_ROWS
+    return VKV_STREAM_ROWS == 1;
+#endif
+    const int64_t pairs = int64_t(num_rows) * num_kv_heads, cus = device_cu_count();
+    if (head_dim % 64 != 0) return max_ctx <= (pairs < 2 * cus ? 1056 : pairs < 8 * cus ? 528 : 264);
+    const int64_t row_bytes = int64_t(max_ctx) * head_dim * 4;
+    return max_ctx <= 2112 && (row_bytes <= 528 << 10 || (pairs >= cus && !matrix_split));
+}
+
+int launch_decode_stream(DecodeArgs& a, bool rows, size_t lds, hipStream_t st) {
+    const int G = a.num_heads / a.num_kv_heads;
+    switch (a.head_dim) {
+        case 64: launch_dim<64>(a, G, rows, lds, st); return 0;
+        case 80: launch_dim<80>(a, G, rows, lds, st); return 0;
+        case 96: launch_dim<96>(a, G, rows, lds, st); return 0;
+        case 112: launch_dim<112>(a, G, rows, lds, st); return 0;
+        case 128: launch_dim<128>(a, G, rows, lds, st); return 0;
+        default: return VKV_ERR_UNSUPPORTED;
+    }
+}
+
+}  // namespace dec
+}  // namespace vkv

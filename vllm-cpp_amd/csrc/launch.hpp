@@ -33,6 +33,12 @@ struct DecodePlan {
     size_t workspace_bytes;
     int num_candidates;
     int candidates[kMaxPartitionCandidates];
+    // decode_stream.hip's shapes.  base_bytes: the workspace without their
+    // finer split (workspace_bytes for every other shape); whole_rows: run
+    // every launch as one workgroup per (row, kv head), which needs none.
+    bool stream;
+    bool whole_rows;
+    size_t base_bytes;
 };
 DecodePlan plan_decode(const vkv_decode_params* p);
 int launch_decode(const vkv_decode_params* p, const DecodePlan& plan, void* workspace, hipStream_t st);
