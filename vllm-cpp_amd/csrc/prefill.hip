@@ -7,16 +7,13 @@
 // sequence's paged cache, i.e. causal attention over the prior context plus
 // the chunk.  Keys are gathered through the block table like decode.
 //
-// The kernels share the matrix-core layout below: prefill_w64_kernel (fp16
-// caches at head_dim 128) and prefill_wide_kernel (fp16 caches at head_dim 64
-// with groups below 4 heads): work items of (token, head) rows, tiles staged
-// by direct global->LDS loads; prefill_wide8_kernel for FP8 caches at head_dim
-// 128 (the same, with the code tiles converted to fp16 in LDS once per
-// workgroup); prefill_mfma_kernel for the rest of head_dim 64.  In the last a
-// workgroup owns (sequence, kv head, block of kBQ = 32 query tokens); wave w
-// computes query head kvh * G + w for those 32 tokens as two 16-row MFMA
-// tiles, so the G heads that share a kv head share every K/V tile staged in
-// LDS.  In both, keys are staged kBK = 64 at a time and computed in 32-key
+// The kernels share the matrix-core layout below; their work items are blocks
+// of (query token, head) rows of one sequence and kv head, with K/V tiles staged
+// by direct global->LDS loads: prefill_split_kernel (blocks of 64 to 256 rows,
+// the keys split over groups of waves: head_dim 64, and head_dim 128 in calls
+// that give few 256-row blocks), prefill_w64_kernel (fp16 caches at head_dim
+// 128), prefill_wide8_kernel (FP8 caches at head_dim 128, the code tiles
+// converted to fp16 in LDS once per workgroup).  Keys are computed in 32-key
 // steps:
 //   S^T = K Q^T   v_mfma_f32_16x16x32_f16, A = K rows (LDS), B = Q (registers);
 //                 lane l holds row (query token) l % 16 for keys 4 (l / 16) + e
@@ -27,14 +24,8 @@
 //                 runs over keys in the order the S^T layout holds them), so P
 //                 never leaves the wave.
 // The output tile is O^T, again one row per lane, normalised at the end.
-//
-// Staging of FP8 caches (prefill_mfma_kernel): each of the first 256 threads
-// loads its share of the next tile's K and V rows into registers while the
-// current tile is computed, then writes them row-major into LDS (rows padded
-// by 16 bytes to spread the banks), dequantised on the way (code x per-token
-// scale, fp32 -> fp16).  Block ids of the sequence are cached in LDS, 1024 at
-// a time.
 #include <algorithm>
+#include <atomic>
 #include <functional>
 #include <queue>
 #include <utility>
@@ -49,12 +40,6 @@
 #ifndef VKV_PREFILL_W64
 #define VKV_PREFILL_W64 1
 #endif
-// Building with -DVKV_PREFILL_D64_WIDE=1 runs fp16 caches at head_dim 64 on
-// the 8-wave direct-load kernel for every group size (an A/B switch; by
-// default groups of 4 and more take the register-staged kernel).
-#ifndef VKV_PREFILL_D64_WIDE
-#define VKV_PREFILL_D64_WIDE 0
-#endif
 
 namespace vkv {
 namespace {
@@ -63,12 +48,8 @@ typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 typedef float float4_t __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 
-constexpr int kBQ = 32;        // query tokens per workgroup
-constexpr int kRT = kBQ / 16;  // 16-row MFMA tiles per wave
 constexpr int kBK = 64;        // keys staged per tile (computed 32 at a time)
-constexpr int kMaxWaves = 8;   // heads per workgroup (more: grid.z splits the group)
-constexpr int kMinWaves = 4;   // staging always has >= 256 threads
-constexpr int kBtCache = 1024; // block ids cached in LDS at a time
+constexpr int kMaxGroup = 504; // query heads per kv head
 
 struct PrefillArgs {
     _Float16* out;
@@ -84,7 +65,6 @@ struct PrefillArgs {
     int32_t num_heads;
     int32_t num_kv_heads;
     int32_t group;  // G = H / Hkv
-    int32_t heads_per_wg;
     int32_t bs_log2;
     int32_t max_blocks_per_seq;
     int32_t num_blocks;
@@ -92,7 +72,7 @@ struct PrefillArgs {
     int32_t qblocks;  // row blocks per sequence, at most (bounds the number of items)
     int32_t num_seqs;
     const int2* items;       // work list (s, b * Hkv + kvh), b the sequence's row block
-    int32_t* item_count;     // [0] items, [1 + z] claim counter of head group z (zeroed by the list kernel)
+    int32_t* item_count;     // items
     float scale_log2;
     // direct-load kernels, calls of at most kInlineBlocks row blocks: every
     // workgroup orders the blocks itself (no list kernel)
@@ -120,55 +100,23 @@ struct PrefillItem {
     int s, b, kvh, q0, qlen, prior;
 };
 
-template <int D, int KVT>
-struct Stage {
-    static constexpr int EB = KvTraits<KVT>::bytes;
-    static constexpr int COLS = D / 8;                // 8-dim columns per token row
-    static constexpr int UNITS = kBK * COLS;          // (key, column) units of a K or V tile
-    static constexpr int UPT = UNITS / (64 * kMinWaves);  // units per staging thread
-    static constexpr int STR = D * 2 + 16;            // bytes per K or V row in LDS
-    static_assert(UNITS % (64 * kMinWaves) == 0, "a tile must split evenly over 256 threads");
-    // fp16: the 16 loaded bytes; FP8: 8 code bytes in .xy and the token's scale
-    // (bits) in .z, dequantised only when written to LDS so that the loads stay
-    // in flight while the current tile is computed.
-    u32x4 k[UPT];
-    u32x4 v[UPT];
-};
-
-// Eight elements of one token as loaded: 16 fp16 bytes, or 8 FP8 code bytes
-// with the token's scale beside them.
-template <int KVT>
-__device__ __forceinline__ u32x4 load8(const char* p, const float* scale) {
-    if constexpr (KVT == kF16) {
-        return load16_nt(p);
-    } else {
-        const u32x2 w = __builtin_nontemporal_load(reinterpret_cast<const u32x2*>(p));
-        return u32x4{w[0], w[1], __builtin_bit_cast(uint32_t, *scale), 0u};
-    }
-}
-
-// Eight fp16 values for LDS: fp16 bytes as they are, FP8 codes dequantised with
-// the token's scale (code * scale in fp32, rounded to fp16).  The codes widen
-// exactly to fp32 two at a time (gfx950's v_cvt_pk_f32_fp8, OCP e4m3fn).
-template <int KVT>
+// Eight FP8 codes (raw[0], raw[1]) of one token dequantised with its scale
+// (bits in raw[2]) for LDS: code * scale in fp32, rounded to fp16.  The codes
+// widen exactly to fp32 two at a time (gfx950's v_cvt_pk_f32_fp8, OCP e4m3fn).
 __device__ __forceinline__ u32x4 to_half8(u32x4 raw) {
-    if constexpr (KVT == kF16) {
-        return raw;
-    } else {
-        typedef float float2_t __attribute__((ext_vector_type(2)));
-        const float sc = as_f32(raw[2]);
-        u32x4 r;
+    typedef float float2_t __attribute__((ext_vector_type(2)));
+    const float sc = as_f32(raw[2]);
+    u32x4 r;
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const float2_t lo = __builtin_amdgcn_cvt_pk_f32_fp8(int(raw[i]), false);  // b0, b1
-            const float2_t hi = __builtin_amdgcn_cvt_pk_f32_fp8(int(raw[i]), true);   // b2, b3
-            const half2_t x0 = {static_cast<_Float16>(lo[0] * sc), static_cast<_Float16>(lo[1] * sc)};
-            const half2_t x1 = {static_cast<_Float16>(hi[0] * sc), static_cast<_Float16>(hi[1] * sc)};
-            r[2 * i] = __builtin_bit_cast(uint32_t, x0);
-            r[2 * i + 1] = __builtin_bit_cast(uint32_t, x1);
-        }
-        return r;
+    for (int i = 0; i < 2; ++i) {
+        const float2_t lo = __builtin_amdgcn_cvt_pk_f32_fp8(int(raw[i]), false);  // b0, b1
+        const float2_t hi = __builtin_amdgcn_cvt_pk_f32_fp8(int(raw[i]), true);   // b2, b3
+        const half2_t x0 = {static_cast<_Float16>(lo[0] * sc), static_cast<_Float16>(lo[1] * sc)};
+        const half2_t x1 = {static_cast<_Float16>(hi[0] * sc), static_cast<_Float16>(hi[1] * sc)};
+        r[2 * i] = __builtin_bit_cast(uint32_t, x0);
+        r[2 * i + 1] = __builtin_bit_cast(uint32_t, x1);
     }
+    return r;
 }
 
 // Max over lanes l, l ^ 16, l ^ 32, l ^ 48 (the four key groups of one query
@@ -189,296 +137,6 @@ __device__ __forceinline__ u32x2 tr_read(const char* lds) {
     typedef __fp16 fp16x4_t __attribute__((__vector_size__(4 * sizeof(__fp16))));
     typedef __attribute__((address_space(3))) fp16x4_t* lds_ptr;
     return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4f16((lds_ptr)(lds)));
-}
-
-// One work item: query block qb (kBQ tokens) of sequence s against kv head kvh.
-template <int D, int KVT>
-__device__ __forceinline__ void prefill_block(const PrefillArgs& a, const int s, const int qb, const int kvh,
-                                              char* klds, char* vlds, int* btc) {
-    using St = Stage<D, KVT>;
-    constexpr int EB = St::EB;
-    constexpr int kTileBytes = kBK * St::STR;  // one K (or V) tile buffer in LDS
-    constexpr int DT = D / 16;  // output dim tiles
-    constexpr int KS = D / 32;  // MFMA k-steps of Q K^T
-
-    const int tid = threadIdx.x;
-    const int nthr = blockDim.x;
-    const int lane = tid & 63;
-    const int wave = tid >> 6;
-    const int col = lane & 15;   // query row within a 16-row tile
-    const int grp = lane >> 4;   // key group: keys 4 grp .. 4 grp + 3 of a 16-key half
-    const int g = blockIdx.z * a.heads_per_wg + wave;  // head within the GQA group
-    const bool computes = wave < a.heads_per_wg && g < a.group;
-
-    const int q0 = a.qsl[s];
-    const int qlen = a.qsl[s + 1] - q0;
-    if (qlen < 2 || qb * kBQ >= qlen) return;  // (the item list holds none of these)
-    const int prior = a.cl[s] - qlen;
-    const int jmax = min(qlen, qb * kBQ + kBQ);  // query rows j in [qb*kBQ, jmax)
-    int kend = prior + jmax;                     // keys any row of the block may see
-    kend = kend < a.table_tokens ? kend : a.table_tokens;
-    const int ntiles = kend > 0 ? (kend + kBK - 1) / kBK : 0;
-    const int h = kvh * a.group + g;
-
-    // ---------------- Q (B operand of S^T = K Q^T) and per-row context
-    const bool neg_scale = a.scale_log2 < 0.0f;
-    const float sc = neg_scale ? -a.scale_log2 : a.scale_log2;
-    half8_t qop[kRT][KS];
-    int rctx[kRT];
-#pragma unroll
-    for (int r = 0; r < kRT; ++r) {
-        const int j = qb * kBQ + 16 * r + col;
-        int c = prior + j + 1;
-        c = c < 0 ? 0 : (c > a.table_tokens ? a.table_tokens : c);
-        rctx[r] = (j < qlen) ? c : 0;
-#pragma unroll
-        for (int i = 0; i < KS; ++i) {
-            // Unconditional load (row 0 / head 0 stand in for absent rows, then
-            // zeroed): a load under a branch makes the compiler wait for every
-            // outstanding load before the first use of Q inside the key loop,
-            // which would serialise the staging prefetch with the MFMAs.
-            const bool ok = computes && j < qlen;
-            const int64_t qrow = ok ? int64_t(q0) + j : int64_t(q0);
-            const int64_t qcol = ok ? int64_t(h) * D : 0;
-            u32x4 w = load16(a.q + (qrow * a.q_stride + qcol + 32 * i + 8 * grp) * 2);
-            const uint32_t keep = ok ? 0xFFFFFFFFu : 0u;
-            const uint32_t flip = neg_scale ? 0x80008000u : 0u;
-            w = (w ^ u32x4{flip, flip, flip, flip}) & u32x4{keep, keep, keep, keep};
-            qop[r][i] = __builtin_bit_cast(half8_t, w);
-        }
-    }
-
-    // ---------------- staging
-    const int bs_mask = (1 << a.bs_log2) - 1;
-    const int64_t row_bytes = int64_t(a.num_kv_heads) * D * EB;  // one slot (token) of the cache
-    const int32_t* table = a.bt + int64_t(s) * a.max_blocks_per_seq;
-    int win = -1;  // first block id index held in btc
-    auto ensure_window = [&](int first_block) __attribute__((always_inline)) {
-        // uniform across the workgroup; callers are between barriers
-        if (win < 0 || first_block < win || first_block + (kBK >> a.bs_log2) + 1 > win + kBtCache) {
-            __syncthreads();
-            win = first_block;
-            for (int i = tid; i < kBtCache; i += nthr) {
-                const int b = win + i;
-                int id = 0;
-                if (b < a.max_blocks_per_seq) {
-                    id = table[b];
-                    if (a.num_blocks > 0 && unsigned(id) >= unsigned(a.num_blocks)) id = 0;
-                }
-                btc[i] = id;
-            }
-            __syncthreads();
-        }
-    };
-    // Keys past kend (the tail of the last tile) load the row of key kend - 1
-    // instead: every query row masks them, so no branch is needed around the
-    // loads and they all issue back to back.
-    auto fetch = [&](St& st, int k0) __attribute__((always_inline)) {
-        int64_t off[St::UPT];
-#pragma unroll
-        for (int i = 0; i < St::UPT; ++i) {
-            const int u = tid + i * 64 * kMinWaves;
-            int k = k0 + u / St::COLS;
-            k = k < kend ? k : kend - 1;
-            const int blk = btc[(k >> a.bs_log2) - win];
-            off[i] = ((int64_t(blk) << a.bs_log2) + (k & bs_mask));  // slot
-        }
-#pragma unroll
-        for (int i = 0; i < St::UPT; ++i) {
-            const int c = (tid + i * 64 * kMinWaves) % St::COLS;
-            const int64_t bytes = off[i] * row_bytes + int64_t(kvh) * D * EB + c * 8 * EB;
-            const int64_t sidx = off[i] * a.num_kv_heads + kvh;
-            st.k[i] = load8<KVT>(a.kc + bytes, KVT == kFp8 ? a.ks + sidx : nullptr);
-            st.v[i] = load8<KVT>(a.vc + bytes, KVT == kFp8 ? a.vs + sidx : nullptr);
-        }
-    };
-    auto put = [&](const St& st, char* kbuf, char* vbuf) __attribute__((always_inline)) {
-#pragma unroll
-        for (int i = 0; i < St::UPT; ++i) {
-            const int u = tid + i * 64 * kMinWaves;
-            const int off = (u / St::COLS) * St::STR + (u % St::COLS) * 16;
-            store16(kbuf + off, to_half8<KVT>(st.k[i]));
-            store16(vbuf + off, to_half8<KVT>(st.v[i]));
-        }
-    };
-
-    // ---------------- main loop
-    const float lazy = kLazy / sc;  // kLazy in raw (unscaled) logit units
-    float m[kRT];
-    float4_t lsum[kRT];  // row sums (every element the same), see below
-    float4_t o[kRT][DT];
-    const half8_t kOnes = {1.0f16, 1.0f16, 1.0f16, 1.0f16, 1.0f16, 1.0f16, 1.0f16, 1.0f16};
-#pragma unroll
-    for (int r = 0; r < kRT; ++r) {
-        m[r] = -INFINITY;
-        lsum[r] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-        for (int t = 0; t < DT; ++t) o[r][t] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
-    }
-
-    // Two LDS tile buffers and one staging register set: tile kt is computed
-    // from buffer kt & 1 while the registers (tile kt + 1, loaded during the
-    // previous tile) go to the other buffer and are refilled with tile kt + 2.
-    // One barrier per tile: it publishes buffer (kt + 1) & 1, and every wave
-    // has left tile kt - 1 (the previous user of that buffer) before it.
-    St st;
-    const bool stager = tid < 64 * kMinWaves;
-    if (ntiles > 0) {
-        ensure_window(0);
-        if (stager) {
-            fetch(st, 0);
-            put(st, klds, vlds);
-        }
-        if (ntiles > 1) {
-            ensure_window(kBK >> a.bs_log2);
-            if (stager) fetch(st, kBK);
-        }
-        __syncthreads();
-    }
-    // One 32-key step in three parts, so that a tile's second S^T (matrix
-    // pipe) is issued before the first step's softmax (VALU) and overlaps it.
-    auto qk = [&](const char* kb, const int sub, float4_t (&sv)[kRT][2]) __attribute__((always_inline)) {
-        // S^T of both row tiles; each K operand (one LDS read) feeds both.
-#pragma unroll
-        for (int r = 0; r < kRT; ++r) sv[r][0] = sv[r][1] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-        for (int hh = 0; hh < 2; ++hh)
-#pragma unroll
-            for (int i = 0; i < KS; ++i) {
-                const half8_t kop = __builtin_bit_cast(
-                    half8_t, *reinterpret_cast<const u32x4*>(kb + (32 * sub + 16 * hh + col) * St::STR + (32 * i + 8 * grp) * 2));
-#pragma unroll
-                for (int r = 0; r < kRT; ++r)
-                    sv[r][hh] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kop, qop[r][i], sv[r][hh], 0, 0, 0);
-            }
-    };
-    auto softmax = [&](const int kbase, const float4_t (&sv)[kRT][2], half8_t (&pop)[kRT]) __attribute__((always_inline)) {
-#pragma unroll
-        for (int r = 0; r < kRT; ++r) {
-            // causal / context mask (key kbase + 16 hh + 4 grp + e < rctx), only
-            // on tiles that reach past some row's context (wave-uniform test)
-            float x[8];
-#pragma unroll
-            for (int hh = 0; hh < 2; ++hh)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) x[4 * hh + e] = sv[r][hh][e];
-            if (__builtin_amdgcn_ballot_w64(kbase + 32 > rctx[r])) {
-#pragma unroll
-                for (int hh = 0; hh < 2; ++hh)
-#pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        if (kbase + 16 * hh + 4 * grp + e >= rctx[r]) x[4 * hh + e] = -INFINITY;
-            }
-            float mx = fmaxf(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])), fmaxf(fmaxf(x[4], x[5]), fmaxf(x[6], x[7])));
-            mx = row_group_max(mx);
-            // Rescale only when some row's max exceeds the one in use by more
-            // than kLazy (log2 units): below that the weights exp2((x - m) sc)
-            // stay under 2^kLazy, well inside fp16 for P and fp32 for the sums,
-            // and the result is the same softmax.  The first key always sets m.
-            if (__builtin_amdgcn_ballot_w64(mx > m[r] + lazy)) {
-                const float mn = fmaxf(m[r], mx);
-                const float alpha = mn > m[r] ? __builtin_amdgcn_exp2f((m[r] - mn) * sc) : 1.0f;
-                m[r] = mn;
-                lsum[r] *= alpha;
-#pragma unroll
-                for (int t = 0; t < DT; ++t) o[r][t] *= alpha;
-            }
-            const float mref = m[r] == -INFINITY ? 0.0f : m[r];  // rows with no key yet
-            const float msc = mref * sc;
-            // P^T operand: k slot (grp, e) = key 4 grp + e, slot (grp, 4 + e) = key 16 + 4 grp + e
-#pragma unroll
-            for (int e = 0; e < 8; ++e) pop[r][e] = static_cast<_Float16>(__builtin_amdgcn_exp2f(fmaf(x[e], sc, -msc)));
-            // row sums on the matrix pipe: a V^T tile of ones gives sum_k p in every lane
-            lsum[r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kOnes, pop[r], lsum[r], 0, 0, 0);
-        }
-    };
-    auto pv = [&](const char* vb, const int sub, const half8_t (&pop)[kRT]) __attribute__((always_inline)) {
-        // O^T += V^T P^T; each V^T operand (two transpose reads of row-major V:
-        // within each 16-lane group, lane i receives element i % 4 of the 8-byte
-        // chunks addressed by lanes i / 4 + 4 e, e = 0..3, so lane m of group
-        // grp addresses key 4 grp + m / 4 (+16), dims 16 t + 4 (m % 4) .. +3)
-        // feeds both row tiles.
-        const int vrow = 32 * sub + 4 * grp + (col >> 2);
-#pragma unroll
-        for (int t = 0; t < DT; ++t) {
-            const int dcol = (16 * t + 4 * (col & 3)) * 2;
-            const u32x2 lo = tr_read(vb + vrow * St::STR + dcol);
-            const u32x2 hi = tr_read(vb + (16 + vrow) * St::STR + dcol);
-            const half8_t vop = __builtin_bit_cast(half8_t, u32x4{lo[0], lo[1], hi[0], hi[1]});
-#pragma unroll
-            for (int r = 0; r < kRT; ++r) o[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vop, pop[r], o[r][t], 0, 0, 0);
-        }
-    };
-    static_assert(kBK == 64, "the tile loop below computes two 32-key steps");
-    for (int kt = 0; kt < ntiles; ++kt) {
-        const char* kcur = klds + (kt & 1) * kTileBytes;
-        const char* vcur = vlds + (kt & 1) * kTileBytes;
-        if (computes) {
-            const bool second = kt * kBK + 32 < kend;
-            float4_t sa[kRT][2], sb[kRT][2];
-            half8_t pa[kRT], pb[kRT];
-            qk(kcur, 0, sa);
-            if (second) qk(kcur, 1, sb);
-            softmax(kt * kBK, sa, pa);
-            pv(vcur, 0, pa);
-            if (second) {
-                softmax(kt * kBK + 32, sb, pb);
-                pv(vcur, 1, pb);
-            }
-        }
-        if (kt + 1 < ntiles) {
-            if (stager) put(st, klds + ((kt + 1) & 1) * kTileBytes, vlds + ((kt + 1) & 1) * kTileBytes);
-            __syncthreads();
-            if (kt + 2 < ntiles) {
-                ensure_window(((kt + 2) * kBK) >> a.bs_log2);
-                if (stager) fetch(st, (kt + 2) * kBK);
-            }
-        }
-    }
-    __syncthreads();  // LDS is free for the next item
-
-    // ---------------- output: lane (row col) holds dims 16 t + 4 grp + e
-    if (!computes) return;  // (after the loop's last barrier)
-#pragma unroll
-    for (int r = 0; r < kRT; ++r) {
-        const float lt = lsum[r][0];  // already summed over every key of the row
-        const int j = qb * kBQ + 16 * r + col;
-        if (j >= qlen) continue;
-        const float inv = (rctx[r] > 0 && lt > 0.0f) ? 1.0f / lt : 0.0f;
-        _Float16* orow = a.out + ((int64_t(q0) + j) * a.num_heads + h) * D;
-#pragma unroll
-        for (int t = 0; t < DT; ++t) {
-            const half2_t lo = {static_cast<_Float16>(o[r][t][0] * inv), static_cast<_Float16>(o[r][t][1] * inv)};
-            const half2_t hi = {static_cast<_Float16>(o[r][t][2] * inv), static_cast<_Float16>(o[r][t][3] * inv)};
-            *reinterpret_cast<u32x2*>(orow + 16 * t + 4 * grp) =
-                u32x2{__builtin_bit_cast(uint32_t, lo), __builtin_bit_cast(uint32_t, hi)};
-        }
-    }
-}
-
-// Persistent workgroups claim items of the list (built by
-// prefill_items_kernel, longest first) one at a time through a counter, so a
-// workgroup that finishes a short item takes the next one (greedy
-// longest-processing-time balance).  Every item ends with a barrier, so LDS is
-// free for the next one; every workgroup leaves once the list is exhausted.
-template <int D, int KVT>
-__global__ __launch_bounds__(64 * kMaxWaves) void prefill_mfma_kernel(PrefillArgs a) {
-    using St = Stage<D, KVT>;
-    __shared__ __attribute__((aligned(16))) char klds[2 * kBK * St::STR];  // two tile buffers each
-    __shared__ __attribute__((aligned(16))) char vlds[2 * kBK * St::STR];
-    __shared__ int btc[kBtCache];
-    __shared__ int claimed;
-    const int count = a.item_count[0];
-    for (;;) {
-        if (threadIdx.x == 0) claimed = atomicAdd(a.item_count + 1 + blockIdx.z, 1);
-        __syncthreads();
-        const int it = claimed;
-        __syncthreads();  // every thread has read `claimed` before thread 0 may overwrite it
-        if (it >= count) break;
-        const int2 item = a.items[it];
-        prefill_block<D, KVT>(a, item.x, item.y / a.num_kv_heads, item.y % a.num_kv_heads, klds, vlds, btc);
-        __syncthreads();
-    }
 }
 
 // ---------------------------------------------------------------------------
@@ -503,8 +161,7 @@ struct DmaTile {
 // loads in rows of D bytes (same swizzle), the token scales by one 4-byte
 // direct load per wave (waves of one parity load the same 64 K or V scales),
 // and the workgroup converts each tile once into the fp16 tile that the fp16
-// path computes from (code x scale in fp32, rounded to fp16, as the
-// register-staged kernel does).
+// path computes from (code x scale in fp32, rounded to fp16).
 template <int D>
 struct DmaTile8 {
     static constexpr int ROW = D;
@@ -560,7 +217,8 @@ __device__ __forceinline__ float vmax3(float a, float b, float c) {
 constexpr int kWideWaves = 8;  // two per SIMD
 constexpr int kWideStages = 3;
 constexpr int kWideBtc = 2048;  // block ids held in LDS at a time
-// 16-row tiles per wave (what fits 256 registers) and (token, head) rows per item
+// 16-row tiles per wave (what fits 256 registers) and (token, head) rows per
+// item (head_dim 64: of the host-built lists only, its calls order their own)
 template <int D>
 struct Wide {
     static constexpr int RT = D == 128 ? 2 : 4;
@@ -756,10 +414,10 @@ __device__ __forceinline__ void prefill_block_wide(const PrefillArgs& a, const P
         const uint32_t vsb = __builtin_bit_cast(uint32_t, buf.sc[S][64 + r]);
         const u32x4 kw = *reinterpret_cast<const u32x4*>(buf.f8k[S] + src);
         const u32x4 vw = *reinterpret_cast<const u32x4*>(buf.f8v[S] + src);
-        *reinterpret_cast<u32x4*>(buf.k[0] + T::off(r, 2 * c)) = to_half8<kFp8>(u32x4{kw[0], kw[1], ksb, 0u});
-        *reinterpret_cast<u32x4*>(buf.k[0] + T::off(r, 2 * c + 1)) = to_half8<kFp8>(u32x4{kw[2], kw[3], ksb, 0u});
-        *reinterpret_cast<u32x4*>(buf.v[0] + T::off(r, 2 * c)) = to_half8<kFp8>(u32x4{vw[0], vw[1], vsb, 0u});
-        *reinterpret_cast<u32x4*>(buf.v[0] + T::off(r, 2 * c + 1)) = to_half8<kFp8>(u32x4{vw[2], vw[3], vsb, 0u});
+        *reinterpret_cast<u32x4*>(buf.k[0] + T::off(r, 2 * c)) = to_half8(u32x4{kw[0], kw[1], ksb, 0u});
+        *reinterpret_cast<u32x4*>(buf.k[0] + T::off(r, 2 * c + 1)) = to_half8(u32x4{kw[2], kw[3], ksb, 0u});
+        *reinterpret_cast<u32x4*>(buf.v[0] + T::off(r, 2 * c)) = to_half8(u32x4{vw[0], vw[1], vsb, 0u});
+        *reinterpret_cast<u32x4*>(buf.v[0] + T::off(r, 2 * c + 1)) = to_half8(u32x4{vw[2], vw[3], vsb, 0u});
     };
 
     fill_window(0);
@@ -1009,76 +667,110 @@ __device__ __forceinline__ void prefill_block_wide(const PrefillArgs& a, const P
     }
 }
 
-// In-kernel work list of a small call, built by every workgroup of the fp16
-// kernel alike (so no list kernel runs before it): the row blocks are
-// numbered in (sequence, block) order, each block's sort key is (bin, number)
-// and its place in the longest-first order is the count of smaller keys.  The
-// keys are distinct, so every workgroup computes the same order; the ranking
-// is quadratic, which at kInlineBlocks blocks is a few hundred LDS reads per
-// thread.  Returns the number of blocks; lblk holds them in order.
+// In-kernel work list of a small call, built by every workgroup alike (so no
+// list kernel runs before it): the sequences with row blocks, in order, with
+// the number of blocks before each.  A call whose items all start at once needs
+// no more; a larger one orders the blocks: each block's sort key is (bin,
+// number) and its place in the longest-first order is the count of smaller
+// keys.  The keys are distinct, so every workgroup computes the same order;
+// the ranking is quadratic, which at kInlineBlocks blocks is a few hundred LDS
+// reads per thread.  (One thread numbering all the blocks of its sequence, with
+// a 64-bit division per block, took 9 us for the 85 blocks of a prompt.)
 constexpr int kInlineBlocks = 512;
+struct InlineList {
+    int first[kInlineBlocks];  // blocks before the sequence's
+    int s[kInlineBlocks], q0[kInlineBlocks], qlen[kInlineBlocks], prior[kInlineBlocks];
+    int key[kInlineBlocks];
+    int order[kInlineBlocks];  // block numbers, longest first (when ordered)
+    int nseq, total;
+};
+
+// Row block i: its sequence's entry (last with first <= i).
+__device__ __forceinline__ int inline_entry(const InlineList& l, const int i) {
+    int lo = 0, hi = l.nseq - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (l.first[mid] <= i) lo = mid;
+        else hi = mid - 1;
+    }
+    return lo;
+}
+
 template <int NT>
-__device__ int inline_row_blocks(const PrefillArgs& a, int2* lblk) {
+__device__ void inline_row_blocks(const PrefillArgs& a, InlineList& l, const int workgroups) {
     constexpr int NW = NT / 64;
-    constexpr int PER = kInlineBlocks / NT;  // blocks ranked per thread
-    static_assert(kInlineBlocks % NT == 0, "blocks must split evenly over the threads");
-    __shared__ int key[kInlineBlocks];
-    __shared__ int wave_tot[NW];
-    __shared__ int carry;
+    constexpr int PER = (kInlineBlocks + NT - 1) / NT;  // blocks ranked per thread
+    __shared__ int2 wave_tot[NW];
+    __shared__ int2 carry;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    if (tid == 0) carry = 0;
+    if (tid == 0) carry = int2{0, 0};
     __syncthreads();
-    // number the blocks: sequences in chunks of one per thread, block counts
-    // scanned across the workgroup
+    // sequences in chunks of one per thread: block counts, and sequences with
+    // any, scanned across the workgroup (the host bounds the blocks of every
+    // call, and so its entries, by kInlineBlocks)
     for (int s0 = 0; s0 < a.num_seqs; s0 += NT) {
         const int s = s0 + tid;
-        int q = 0, prior = 0, n = 0;
+        int q0 = 0, q = 0, prior = 0, n = 0;
         if (s < a.num_seqs) {
-            q = a.qsl[s + 1] - a.qsl[s];
+            q0 = a.qsl[s];
+            q = a.qsl[s + 1] - q0;
             prior = a.cl[s] - q;
             n = seq_row_blocks(q, a.group, a.rows_per_item, a.qblocks);
         }
-        const int incl = wave_incl_scan(n);
-        if (lane == 63) wave_tot[wave] = incl;
+        const int blocks = wave_incl_scan(n), seqs = wave_incl_scan(n > 0 ? 1 : 0);
+        if (lane == 63) wave_tot[wave] = int2{blocks, seqs};
         __syncthreads();
-        int before = carry;
-        for (int w = 0; w < wave; ++w) before += wave_tot[w];
-        for (int b = 0; b < n; ++b) {
-            const int i = before + incl - n + b;
-            if (i < kInlineBlocks) {  // (the host bound keeps every call within)
-                key[i] = (row_block_bin(prior, q, b, a.group, a.rows_per_item, a.table_tokens, a.nbins) << 9) | i;
-                lblk[i] = int2{s, b};
-            }
+        int first = carry.x + blocks - n, e = carry.y + seqs - 1;
+        for (int w = 0; w < wave; ++w) {
+            first += wave_tot[w].x;
+            e += wave_tot[w].y;
+        }
+        if (n > 0 && e < kInlineBlocks) {
+            l.first[e] = first;
+            l.s[e] = s;
+            l.q0[e] = q0;
+            l.qlen[e] = q;
+            l.prior[e] = prior;
         }
         __syncthreads();
         if (tid == 0) {
-            int t = carry;
-            for (int w = 0; w < NW; ++w) t += wave_tot[w];
+            int2 t = carry;
+            for (int w = 0; w < NW; ++w) {
+                t.x += wave_tot[w].x;
+                t.y += wave_tot[w].y;
+            }
             carry = t;
         }
         __syncthreads();
     }
-    const int total = carry < kInlineBlocks ? carry : kInlineBlocks;
-    // rank, then place (lblk is read before the barrier and written after it)
-    int2 mine[PER];
-    int rank[PER];
+    if (tid == 0) {
+        l.nseq = carry.y < kInlineBlocks ? carry.y : kInlineBlocks;
+        l.total = carry.x < kInlineBlocks ? carry.x : kInlineBlocks;
+    }
+    __syncthreads();
+    const int total = l.total;
+    if (total * a.num_kv_heads <= workgroups) return;
 #pragma unroll
     for (int p = 0; p < PER; ++p) {
         const int i = tid + p * NT;
-        mine[p] = int2{0, 0};
-        rank[p] = 0;
         if (i < total) {
-            const int k = key[i];
-            mine[p] = lblk[i];
-            for (int j = 0; j < total; ++j) rank[p] += key[j] < k ? 1 : 0;
+            const int e = inline_entry(l, i);
+            l.key[i] = (row_block_bin(l.prior[e], l.qlen[e], i - l.first[e], a.group, a.rows_per_item, a.table_tokens,
+                                      a.nbins) << 9) | i;
         }
     }
     __syncthreads();
 #pragma unroll
-    for (int p = 0; p < PER; ++p)
-        if (tid + p * NT < total) lblk[rank[p]] = mine[p];
+    for (int p = 0; p < PER; ++p) {
+        const int i = tid + p * NT;
+        if (i < total) {
+            const int k = l.key[i];
+            int rank = 0;
+            for (int j = 0; j < total; ++j) rank += l.key[j] < k ? 1 : 0;
+            l.order[rank] = i;
+        }
+    }
     __syncthreads();
-    return total;
 }
 
 // Host-built schedule (vkv_prefill_work_list_host): 32 header words ([0] W
@@ -1152,21 +844,24 @@ __device__ __forceinline__ void run_items(const PrefillArgs& a, Item item_fn) {
     // to W - 1 - p when r is odd (W workgroups, all resident: one per CU), so
     // the longest items meet the shortest ones, as a longest-processing-time
     // schedule would put them, with no claims.
-    __shared__ int2 lblk[kInlineBlocks];  // inline list: (s, b) of row block i, then in longest-first order
-    const int count = a.inline_list ? inline_row_blocks<NT>(a, lblk) * a.num_kv_heads : a.item_count[0];
     const int W = gridDim.x, p = blockIdx.x;
+    __shared__ InlineList list;
+    if (a.inline_list) inline_row_blocks<NT>(a, list, W);
+    const int count = a.inline_list ? list.total * a.num_kv_heads : a.item_count[0];
     for (int r = 0;; ++r) {
         const int64_t it = int64_t(r) * W + ((r & 1) ? W - 1 - p : p);
         if (it >= count) break;  // (later rounds are further on)
         // items (row block, kv head), kv head fastest
-        int2 item;
         if (a.inline_list) {
-            const int2 blk = lblk[it / a.num_kv_heads];
-            item = int2{blk.x, blk.y * a.num_kv_heads + int(it % a.num_kv_heads)};
+            const int at = int(it) / a.num_kv_heads;
+            const int i = count > W ? list.order[at] : at;
+            const int e = inline_entry(list, i);
+            item_fn(PrefillItem{list.s[e], i - list.first[e], int(it) % a.num_kv_heads, list.q0[e], list.qlen[e],
+                                list.prior[e]});
         } else {
-            item = a.items[it];
+            const int2 item = a.items[it];
+            item_fn(load_item(a, item.x, item.y / a.num_kv_heads, item.y % a.num_kv_heads));
         }
-        item_fn(load_item(a, item.x, item.y / a.num_kv_heads, item.y % a.num_kv_heads));
     }
 }
 
@@ -1796,12 +1491,378 @@ __global__ __launch_bounds__(64 * kWideWaves) void prefill_wide8_kernel(PrefillA
     wide_items<D, true>(a, buf);
 }
 
+// ---------------------------------------------------------------------------
+// prefill_split_kernel: small row blocks, keys split over groups of waves.
+//
+// A work item is (sequence, kv head, block of ROWS = 16 NR CT (token, head)
+// rows).  Its NR x NG waves are NG key groups of NR waves: wave (g, w) computes
+// rows [16 CT w, 16 CT (w + 1)) of the block over the key tiles t = g (mod NG),
+// and the groups' results are merged in LDS at the end, as decode merges
+// partitions.  So an item is small (a short prompt still fills the chip) and
+// its chain of key tiles is NG times shorter, while the waves of a group share
+// every K/V tile and two waves per SIMD overlap one's softmax with the other's
+// matrix products.  Tiles of TK keys reach LDS by direct loads, ST stages per
+// group, published by one workgroup barrier per round of NG tiles.  FP8: the
+// code tiles (and their scales) are converted once per group into an fp16 tile
+// (code x scale in fp32, rounded to fp16, as the other FP8 kernels do).
+// Tile rows of ROW bytes, unpadded; chunk c of row r sits at slot c ^ key(r).
+// The operand reads take one chunk column of 16 rows: with 256-byte rows the
+// key is r % 16, with 128-byte rows (two to a 256-byte line of banks) r / 2 % 8,
+// with 64-byte rows r / 4 % 4, so the 16 rows meet 16 different bank groups.
+template <int ROW_>
+struct SplitTile {
+    static constexpr int ROW = ROW_, CH = ROW / 16, RPI = 1024 / ROW;
+    __device__ static __forceinline__ int key(int row) { return row / (16 / CH) % CH; }
+    __device__ static __forceinline__ int off(int row, int chunk) { return row * ROW + ((chunk ^ key(row)) << 4); }
+};
+
+template <int D, bool FP8, int NR_, int NG_, int CT_, int TK_, int ST_>
+struct Split {
+    static constexpr int NR = NR_, NG = NG_, CT = CT_, TK = TK_, ST = ST_;
+    static constexpr int WAVES = NR * NG, NT = 64 * WAVES, ROWS = 16 * NR * CT;
+    using T = SplitTile<2 * D>;               // the fp16 tile
+    using L = SplitTile<FP8 ? D : 2 * D>;     // the tile the loads fill
+    static constexpr int INST = TK * L::ROW / 1024;  // wave loads of a K (or V) tile
+    static constexpr int JW = INST / NR;             // of them per wave
+    static constexpr int NLOAD = 2 * JW + (FP8 ? 1 : 0);
+    static constexpr int LBYTES = TK * L::ROW;       // a K (or V) tile as loaded
+    static constexpr int STAGE = 2 * LBYTES + (FP8 ? 8 * TK : 0);  // K, V, then the K and V scales
+    static constexpr int GROUP = ST * STAGE + (FP8 ? 2 * TK * T::ROW : 0);  // stages, then the fp16 tile
+    static constexpr int MERGE = (NG - 1) * NR * CT * (D / 16 * 1024 + 512);
+    static constexpr int OUT = NR * 16 * CT * D * 2;
+    static constexpr int BYTES0 = NG * GROUP > MERGE ? NG * GROUP : MERGE;
+    static constexpr int BYTES = BYTES0 > OUT ? BYTES0 : OUT;
+    static_assert(INST % NR == 0, "the loads of a tile must split evenly over a group's waves");
+    static_assert(TK == 32 || TK == 64, "one or two 32-key steps");
+};
+
+// One 4-byte direct load per lane (LDS address lds + 4 lane).
+__device__ __forceinline__ void dma4(const float* g, const uint32_t lds) {
+    const uint32_t l = __builtin_amdgcn_readfirstlane(lds);
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" : : "v"(g), "s"(l) : "memory", "m0");
+}
+
+template <int D, bool FP8, class C>
+__device__ __forceinline__ void prefill_block_split(const PrefillArgs& a, const PrefillItem& it, char* lds, int* btc) {
+    using T = typename C::T;
+    using L = typename C::L;
+    constexpr int EB = FP8 ? 1 : 2;
+    constexpr int DT = D / 16, KS = D / 32, CT = C::CT, NR = C::NR, NG = C::NG, TK = C::TK, ST = C::ST, JW = C::JW;
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int g = wave / NR, w = wave % NR;  // key group, row wave
+    const int col = lane & 15, grp = lane >> 4;
+    const int G = a.group;
+    const int s = it.s, b = it.b, kvh = it.kvh, q0 = it.q0, qlen = it.qlen, prior = it.prior;
+    const int nrows = qlen * G;
+    if (qlen < 2 || b * C::ROWS >= nrows) return;  // (the item list holds none of these)
+    const int kend = item_kend(a, it, C::ROWS);    // keys any row of the block may see
+    const int ntiles = kend > 0 ? (kend + TK - 1) / TK : 0;
+    const int rounds = (ntiles + NG - 1) / NG;
+
+    // ---------------- loads of this group's tile t
+    const int bs_mask = (1 << a.bs_log2) - 1;
+    const uint32_t row_bytes32 = uint32_t(a.num_kv_heads) * D * EB;
+    uint32_t lane_off[JW];
+#pragma unroll
+    for (int j = 0; j < JW; ++j) {
+        const int row = (w * JW + j) * L::RPI + lane / L::CH;
+        lane_off[j] = uint32_t(kvh) * D * EB + uint32_t(((lane % L::CH) ^ L::key(row)) * 16);
+    }
+    const int32_t* table = a.bt + int64_t(s) * a.max_blocks_per_seq;
+    const int nblk = kend > 0 ? ((kend - 1) >> a.bs_log2) + 1 : 1;
+    int win = 0;
+    auto fill_window = [&](const int first) __attribute__((always_inline)) {
+        win = first;
+        const int n = nblk - first < kWideBtc ? nblk - first : kWideBtc;
+        for (int i = tid; i < n; i += C::NT) {
+            int id = table[first + i];
+            if (a.num_blocks > 0 && unsigned(id) >= unsigned(a.num_blocks)) id = 0;
+            btc[i] = id;
+        }
+    };
+    // the slot of key k (keys past the end: the last one again, masked)
+    auto slot_of = [&](int k) __attribute__((always_inline)) {
+        k = k < kend ? k : kend - 1;
+        k = k > 0 ? k : 0;
+        return (uint32_t(btc[(k >> a.bs_log2) - win]) << a.bs_log2) + uint32_t(k & bs_mask);
+    };
+    char* const base = lds + g * C::GROUP;
+    const uint32_t base_lds = lds_addr(base);
+    auto load_tile = [&](const int st, const int t) __attribute__((always_inline)) {
+        const uint32_t dst = base_lds + uint32_t(st * C::STAGE);
+#pragma unroll
+        for (int j = 0; j < JW; ++j) {
+            const uint64_t off =
+                uint64_t(slot_of(t * TK + (w * JW + j) * L::RPI + lane / L::CH)) * row_bytes32 + lane_off[j];
+            dma16(a.kc + off, dst + (w * JW + j) * 1024);
+            dma16(a.vc + off, dst + C::LBYTES + (w * JW + j) * 1024);
+        }
+        if constexpr (FP8) {
+            // TK = 64: even waves the key scales, odd ones the value scales;
+            // TK = 32: key scales in lanes 0-31, value scales in 32-63
+            const bool v = TK == 64 ? (w & 1) : lane >= 32;
+            const uint64_t at = uint64_t(slot_of(t * TK + (TK == 64 ? lane : lane & 31))) * a.num_kv_heads + kvh;
+            dma4((v ? a.vs : a.ks) + at, dst + 2 * C::LBYTES + (TK == 64 ? 256 * (w & 1) : 0));
+        }
+    };
+    // FP8: this group's stage as an fp16 tile (a unit: 16 codes of a key row)
+    char* const half_tile = base + ST * C::STAGE;
+    auto convert = [&](const int st) __attribute__((always_inline)) {
+        const char* src = base + st * C::STAGE;
+        const float* scale = reinterpret_cast<const float*>(src + 2 * C::LBYTES);
+#pragma unroll
+        for (int u0 = 0; u0 < TK * L::CH; u0 += 64 * NR) {
+            const int u = u0 + 64 * w + lane;
+            const int r = u / L::CH, c = u % L::CH;
+            const uint32_t ks = as_u32(scale[r]), vs = as_u32(scale[TK + r]);
+            const u32x4 k = load16(src + L::off(r, c)), v = load16(src + C::LBYTES + L::off(r, c));
+            char* vd = half_tile + TK * T::ROW;
+            store16(half_tile + T::off(r, 2 * c), to_half8(u32x4{k[0], k[1], ks, 0u}));
+            store16(half_tile + T::off(r, 2 * c + 1), to_half8(u32x4{k[2], k[3], ks, 0u}));
+            store16(vd + T::off(r, 2 * c), to_half8(u32x4{v[0], v[1], vs, 0u}));
+            store16(vd + T::off(r, 2 * c + 1), to_half8(u32x4{v[2], v[3], vs, 0u}));
+        }
+    };
+
+    fill_window(0);
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < ST - 1; ++i)
+        if (i < rounds) load_tile(i, i * NG + g);
+
+    // ---------------- Q (B operand) and per-row context: row rho is (token rho / G, head rho % G)
+    const bool neg_scale = a.scale_log2 < 0.0f;
+    const float sc = neg_scale ? -a.scale_log2 : a.scale_log2;
+    const float lazy = kLazy / sc;
+    const int rho0 = b * C::ROWS + 16 * CT * w;
+    half8_t qop[CT][KS];
+    int rctx[CT];
+    float m[CT], msc[CT];
+    float4_t lsum[CT], o[CT][DT];
+#pragma unroll
+    for (int c = 0; c < CT; ++c) {
+        const int rho = rho0 + 16 * c + col;
+        const bool ok = rho < nrows;
+        const int j = ok ? row_token(a, rho) : 0;
+        const int h = kvh * G + (ok ? rho - j * G : 0);
+        int x = prior + j + 1;
+        x = x < 0 ? 0 : (x > a.table_tokens ? a.table_tokens : x);
+        rctx[c] = ok ? x : 0;
+        const int64_t qbase = (int64_t(q0) + j) * a.q_stride + int64_t(h) * D;
+#pragma unroll
+        for (int i = 0; i < KS; ++i) {
+            u32x4 v = load16(a.q + (qbase + 32 * i + 8 * grp) * 2);
+            const uint32_t keep = ok ? 0xFFFFFFFFu : 0u;
+            const uint32_t flip = neg_scale ? 0x80008000u : 0u;
+            v = (v ^ u32x4{flip, flip, flip, flip}) & u32x4{keep, keep, keep, keep};
+            qop[c][i] = __builtin_bit_cast(half8_t, v);
+        }
+        m[c] = -INFINITY;
+        msc[c] = 0.0f;
+        lsum[c] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int t = 0; t < DT; ++t) o[c][t] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+    const half8_t kOnes = {1.0f16, 1.0f16, 1.0f16, 1.0f16, 1.0f16, 1.0f16, 1.0f16, 1.0f16};
+
+    int koff[KS], voff[DT];
+    const int vrow = 4 * grp + (col >> 2);
+#pragma unroll
+    for (int i = 0; i < KS; ++i) koff[i] = T::off(col, 4 * i + grp);
+#pragma unroll
+    for (int t = 0; t < DT; ++t) voff[t] = T::off(vrow, 2 * t + ((col & 3) >> 1)) + 8 * (col & 1);
+
+    auto qk = [&](const char* kb, float4_t (&sv)[CT][2]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int c = 0; c < CT; ++c) sv[c][0] = sv[c][1] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int i = 0; i < KS; ++i)
+#pragma unroll
+            for (int hh = 0; hh < 2; ++hh) {
+                const half8_t kop = __builtin_bit_cast(half8_t, load16(kb + koff[i] + 16 * hh * T::ROW));
+#pragma unroll
+                for (int c = 0; c < CT; ++c)
+                    sv[c][hh] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kop, qop[c][i], sv[c][hh], 0, 0, 0);
+            }
+    };
+    auto softmax = [&](const int kbase, float4_t (&sv)[CT][2], half8_t (&pop)[CT]) __attribute__((always_inline)) {
+        // key kbase + 16 hh + 4 grp + e < rctx, where the step reaches past some row's context
+        bool edge = false;
+#pragma unroll
+        for (int c = 0; c < CT; ++c) edge = edge || kbase + 32 > rctx[c];
+        if (__builtin_amdgcn_ballot_w64(edge)) {
+#pragma unroll
+            for (int c = 0; c < CT; ++c)
+#pragma unroll
+                for (int hh = 0; hh < 2; ++hh)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        if (kbase + 16 * hh + 4 * grp + e >= rctx[c]) sv[c][hh][e] = -INFINITY;
+        }
+        float lmx[CT];
+        bool over = false;
+#pragma unroll
+        for (int c = 0; c < CT; ++c) {
+            lmx[c] = vmax3(vmax3(sv[c][0][0], sv[c][0][1], sv[c][0][2]), vmax3(sv[c][0][3], sv[c][1][0], sv[c][1][1]),
+                           vmax3(sv[c][1][2], sv[c][1][3], sv[c][1][3]));
+            over = over || lmx[c] > m[c] + lazy;
+        }
+        if (__builtin_amdgcn_ballot_w64(over)) {
+#pragma unroll
+            for (int c = 0; c < CT; ++c) {
+                if (__builtin_amdgcn_ballot_w64(lmx[c] > m[c] + lazy)) {
+                    const float mn = fmaxf(m[c], row_group_max(lmx[c]));
+                    const float alpha = mn > m[c] ? __builtin_amdgcn_exp2f((m[c] - mn) * sc) : 1.0f;
+                    m[c] = mn;
+                    msc[c] = (mn == -INFINITY ? 0.0f : mn) * sc;
+                    lsum[c] *= alpha;
+#pragma unroll
+                    for (int t = 0; t < DT; ++t) o[c][t] *= alpha;
+                }
+            }
+        }
+#pragma unroll
+        for (int c = 0; c < CT; ++c) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                pop[c][e] = static_cast<_Float16>(__builtin_amdgcn_exp2f(fmaf(sv[c][e >> 2][e & 3], sc, -msc[c])));
+            lsum[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kOnes, pop[c], lsum[c], 0, 0, 0);
+        }
+    };
+    auto read_v = [&](const char* vb, half8_t (&vop)[DT]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int t = 0; t < DT; ++t) {
+            const u32x2 lo = tr_read(vb + voff[t]);
+            const u32x2 hi = tr_read(vb + voff[t] + 16 * T::ROW);
+            vop[t] = __builtin_bit_cast(half8_t, u32x4{lo[0], lo[1], hi[0], hi[1]});
+        }
+    };
+    auto pv = [&](const half8_t (&vop)[DT], const half8_t (&pop)[CT]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int t = 0; t < DT; ++t)
+#pragma unroll
+            for (int c = 0; c < CT; ++c) o[c][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vop[t], pop[c], o[c][t], 0, 0, 0);
+    };
+
+    for (int i = 0; i < rounds; ++i) {
+        // round i's tiles published; every wave has left round i - 1
+        if (ST == 2 || i + 1 >= rounds) tile_barrier<0>();
+        else tile_barrier<(ST - 2) * C::NLOAD>();
+        if (i + ST - 1 < rounds) {
+            const int last = min((i + ST) * NG * TK, kend) - 1;
+            if ((last >> a.bs_log2) - win >= kWideBtc) {
+                fill_window(((i + ST - 1) * NG * TK) >> a.bs_log2);
+                __syncthreads();
+            }
+            load_tile((i + ST - 1) % ST, (i + ST - 1) * NG + g);
+        }
+        if constexpr (FP8) {
+            convert(i % ST);
+            lds_barrier();
+        }
+        const int t = i * NG + g;
+        const char* kb = FP8 ? half_tile : base + (i % ST) * C::STAGE;
+        const char* vb = FP8 ? half_tile + TK * T::ROW : kb + C::LBYTES;
+        if (t < ntiles) {
+            float4_t sa[CT][2];
+            half8_t pa[CT];
+            qk(kb, sa);
+            if constexpr (TK == 64) {
+                float4_t sb[CT][2];
+                half8_t pb[CT];
+                const bool second = t * TK + 32 < kend;
+                if (second) qk(kb + 32 * T::ROW, sb);
+                half8_t va[DT];
+                read_v(vb, va);
+                softmax(t * TK, sa, pa);
+                half8_t vb2[DT];
+                if (second) read_v(vb + 32 * T::ROW, vb2);
+                pv(va, pa);
+                if (second) {
+                    softmax(t * TK + 32, sb, pb);
+                    pv(vb2, pb);
+                }
+            } else {
+                half8_t va[DT];
+                read_v(vb, va);
+                softmax(t * TK, sa, pa);
+                pv(va, pa);
+            }
+        }
+    }
+
+    // ---------------- merge of the key groups, into group 0's waves: region
+    // (g - 1, w, c) holds DT x 64 accumulator vectors, then 64 (max, sum) pairs
+    __syncthreads();
+    if constexpr (NG > 1) {
+        constexpr int kPart = DT * 1024 + 512;
+        if (g > 0) {
+#pragma unroll
+            for (int c = 0; c < CT; ++c) {
+                char* part = lds + (((g - 1) * NR + w) * CT + c) * kPart;
+#pragma unroll
+                for (int t = 0; t < DT; ++t) reinterpret_cast<float4_t*>(part)[t * 64 + lane] = o[c][t];
+                reinterpret_cast<float2_t*>(part + DT * 1024)[lane] = float2_t{m[c], lsum[c][0]};
+            }
+        }
+        __syncthreads();
+        if (g == 0) {
+#pragma unroll
+            for (int c = 0; c < CT; ++c) {
+                const char* part0 = lds + (w * CT + c) * kPart;
+                constexpr int kNext = NR * CT * kPart;  // the next group's
+                float mx = m[c], other[NG - 1];
+#pragma unroll
+                for (int x = 0; x < NG - 1; ++x) {
+                    other[x] = reinterpret_cast<const float2_t*>(part0 + x * kNext + DT * 1024)[lane][0];
+                    mx = fmaxf(mx, other[x]);
+                }
+                // (a group without a key of this row: max -inf, weight 0)
+                const float ref = mx == -INFINITY ? 0.0f : mx;
+                float f = __builtin_amdgcn_exp2f((m[c] - ref) * sc);
+                lsum[c] *= f;
+#pragma unroll
+                for (int t = 0; t < DT; ++t) o[c][t] *= f;
+#pragma unroll
+                for (int x = 0; x < NG - 1; ++x) {
+                    f = __builtin_amdgcn_exp2f((other[x] - ref) * sc);
+                    lsum[c] += f * reinterpret_cast<const float2_t*>(part0 + x * kNext + DT * 1024)[lane][1];
+#pragma unroll
+                    for (int t = 0; t < DT; ++t)
+                        o[c][t] += f * reinterpret_cast<const float4_t*>(part0 + x * kNext)[t * 64 + lane];
+                }
+            }
+        }
+        __syncthreads();  // the partials are read: LDS is free for the output rows
+    }
+    if (g == 0) {
+        float inv[CT];
+#pragma unroll
+        for (int c = 0; c < CT; ++c) {
+            const float lt = lsum[c][0];
+            inv[c] = (rctx[c] > 0 && lt > 0.0f) ? 1.0f / lt : 0.0f;
+        }
+        store_rows_lds<D, CT>(a, lds + w * (16 * CT * D * 2), o, inv, rho0, nrows, q0, kvh, lane);
+    }
+    __syncthreads();  // LDS is free for the next item
+}
+
+template <int D, bool FP8, class C>
+__global__ __launch_bounds__(C::NT) void prefill_split_kernel(PrefillArgs a) {
+    __shared__ __attribute__((aligned(1024))) char lds[C::BYTES];
+    __shared__ int btc[kWideBtc];
+    run_items<C::NT>(a, [&](const PrefillItem& it) __attribute__((always_inline)) {
+        prefill_block_split<D, FP8, C>(a, it, lds, btc);
+    });
+}
+
 // Work list of the matrix-core kernels, in one workgroup: items (s, b * Hkv +
 // kvh), row block b of every sequence with >= 2 query tokens, ordered by the
 // number of key tiles they stage, most first, so that persistent workgroups
-// taking them in turn (dealt in a snake by the direct-load kernels, claimed by
-// prefill_mfma_kernel) form a longest-processing-time schedule (short items
-// fill in at the end).  A row block of rows_per_item rows (query tokens
+// taking them in turn (dealt in a snake) form a longest-processing-time
+// schedule (short items fill in at the end).  A row block of rows_per_item rows (query tokens
 // times row_mult heads) sees keys 0 .. kend - 1 with kend = prior + its last
 // token + 1; a histogram over the tile counts (one bin per possible count,
 // at most kMaxLevels: counts past that share the top bin) gives every count's
@@ -1809,7 +1870,6 @@ __global__ __launch_bounds__(64 * kWideWaves) void prefill_wide8_kernel(PrefillA
 // slots through LDS atomics (the order within a bin does not matter to the
 // results).
 constexpr int kMaxLevels = 4096;
-constexpr int kMaxHeadGroups = 63;  // claim counters after the item count (256-byte header)
 
 // Exclusive prefix sum of arr[0, n) in LDS by 256 threads (each a contiguous
 // tile, tiles combined with DPP wave scans and one LDS step); returns the total.
@@ -1861,7 +1921,6 @@ __global__ __launch_bounds__(256) void prefill_items_kernel(const int32_t* qsl, 
     __syncthreads();
     const int total = block_exclusive_scan(off, nbins, wave_tot);
     if (tid == 0) count[0] = total;
-    if (tid < kMaxHeadGroups) count[1 + tid] = 0;  // claim counters of the prefill kernel
     for (int s = tid; s < num_seqs; s += 256) {
         const int q = qsl[s + 1] - qsl[s];
         const int prior = cl[s] - q;
@@ -1891,39 +1950,86 @@ bool prefill_mfma_supported(const vkv_prefill_params* p) {
     return p->io_dtype == VKV_DTYPE_F16 && (p->kv_dtype == VKV_DTYPE_F16 || p->kv_dtype == VKV_DTYPE_FP8_E4M3) &&
            (p->head_dim == 64 || p->head_dim == 128) && p->max_query_len >= 2 && pow2_bs && (align & 15u) == 0 &&
            p->num_kv_heads > 0 && p->num_heads % p->num_kv_heads == 0 &&
-           p->num_heads / p->num_kv_heads <= kMaxHeadGroups * kMaxWaves;
+           p->num_heads / p->num_kv_heads <= kMaxGroup;
 }
 
 namespace {
 
-// D = 128, and fp16 caches at D = 64 with groups below 4 heads, run on the
-// direct-load kernels, whose items are Wide<D>::ROWS (token, head) rows; the
-// rest of D = 64 on prefill_mfma_kernel, whose items are kBQ query tokens of
-// every head of a kv head (a wave per head, at least 4 waves: smaller groups
-// would leave waves idle).  Measured on C3's chunks at D = 64, fp16 cache:
-// groups of 7 73.5 us on the staged kernel against 88.0 on the direct-load
-// one, groups of 4 89.2 against 91.7, groups of 1 138.4 against 101.8.
-bool wide_path(const vkv_prefill_params* p) {
-    if (p->head_dim == 128) return true;
-    const int G = p->num_kv_heads > 0 ? p->num_heads / p->num_kv_heads : 1;
-    return p->kv_dtype == VKV_DTYPE_F16 && (VKV_PREFILL_D64_WIDE || G < kMinWaves);
+// The work items of prefill_split_kernel, by the call's (token, head) rows in
+// blocks of 64 over its kv heads, n64.  Few blocks: 64 rows each, the keys over
+// four groups of waves, so that every CU has one and its chain of key tiles is
+// short.  More of them, or longer calls: 128 rows (each K/V operand read from
+// LDS feeds twice the products), then 256.  At head_dim 128 calls that fill the
+// chip with 256-row blocks run on the one-wave-per-SIMD kernels, whose
+// schedule overlaps more (rows 0).  Measured (us, blocks of 64 / 128 / 256 rows
+// or the latter kernels; "4 x 700" four prompts of 700 tokens, + prior keys):
+//   D 64, 14/2 heads: 1 x 500 (n64 108): 11.4 / 13.4 / 21.3; 1 x 1 000 (218):
+//     14.1 / 20.3 / 32.7; 3 x 700 (458): 20.8 / 16.7 / 27.0; 8 x 512 + 2 000
+//     (896): 59.6 / 46.5 / 62.2; 16 x 500 (1 750): 65.6 / 43.2 / 36.8
+//   D 128, 32/8 heads: 1 x 500 (248): 16.4 / 18.2 / 26.5; 4 x 100 + 2 000
+//     (200): 32.9 / 47.2 / 71.4; 8 x 100 + 1 000 (400): 32.2 / 29.8 / 44.9;
+//     1 x 2 000 (1 000): 76 / 53.9 / 72.2; 4 x 700 (1 400): 67 / 44.0 / 41.6
+//   (FP8 caches alike: 1 x 500: 18.9 / 21.1 / 28.0; 4 x 700: 79 / 49.3 / 41.2)
+template <bool FP8> using Split64S = Split<64, FP8, 4, 4, 1, 64, 2>;
+template <bool FP8> using Split64M = Split<64, FP8, 4, 3, 2, 64, 2>;
+template <bool FP8> using Split64L = Split<64, FP8, 4, 2, 4, 64, 2>;
+template <bool FP8> using Split128S = Split<128, FP8, 2, 4, 2, 32, 2>;
+template <bool FP8> using Split128M = Split<128, FP8, 4, 2, 2, 32, 2>;
+
+int cu_count() {
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) {
+        (void)hipGetLastError();  // (no device: the default, and no error left behind)
+        return kListDefaultCus;
+    }
+    return cus;
 }
+int split_rows(const vkv_prefill_params* p) {
+    const int64_t n64 = int64_t(p->num_query_tokens) * p->num_heads / 64, cus = cu_count();
+    if (p->head_dim == 64) return n64 <= cus * 5 / 4 ? 64 : n64 <= 4 * cus ? 128 : 256;
+    return n64 <= cus ? 64 : n64 <= 4 * cus ? 128 : 0;
+}
+// (token, head) rows of the items of vkv_prefill_work_list_host's lists, and of the call's
+int list_rows(const vkv_prefill_params* p) { return p->head_dim == 128 ? Wide<128>::ROWS : Wide<64>::ROWS; }
 int rows_per_item(const vkv_prefill_params* p) {
-    if (!wide_path(p)) return kBQ;
-    return p->head_dim == 128 ? Wide<128>::ROWS : Wide<64>::ROWS;
+    const int r = split_rows(p);
+    return r > 0 ? r : list_rows(p);
 }
 // Row blocks (work items per kv head) of a sequence, at most: with a group of
-// G heads a token brings G rows to the direct-load kernels.
-int64_t max_row_blocks(const vkv_prefill_params* p) {
-    const int64_t row_mult = wide_path(p) ? p->num_heads / p->num_kv_heads : 1;
-    const int rows = rows_per_item(p);
-    return (int64_t(p->max_query_len) * row_mult + rows - 1) / rows;
+// G heads a token brings G rows.
+int64_t max_row_blocks(const vkv_prefill_params* p, int rows) {
+    return (int64_t(p->max_query_len) * (p->num_heads / p->num_kv_heads) + rows - 1) / rows;
+}
+
+// One workgroup per resident slot (queried once per kernel), at most `items`.
+template <class C, class K>
+void run_split(K kernel, const PrefillArgs& a, int64_t items, int cus, hipStream_t st) {
+    static std::atomic<int> cached{0};
+    int per_cu = cached.load(std::memory_order_relaxed);
+    if (per_cu <= 0) {
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, C::NT, 0) != hipSuccess || per_cu < 1) per_cu = 1;
+        cached.store(per_cu, std::memory_order_relaxed);
+    }
+    const int64_t wgs = std::min(int64_t(cus) * per_cu, items);
+    hipLaunchKernelGGL(kernel, dim3(unsigned(wgs > 0 ? wgs : 1)), dim3(C::NT), 0, st, a);
+}
+template <bool FP8>
+void launch_split(const PrefillArgs& a, int head_dim, int rows, int64_t items, int cus, hipStream_t st) {
+    if (head_dim == 64) {
+        if (rows == 64) run_split<Split64S<FP8>>(prefill_split_kernel<64, FP8, Split64S<FP8>>, a, items, cus, st);
+        else if (rows == 128) run_split<Split64M<FP8>>(prefill_split_kernel<64, FP8, Split64M<FP8>>, a, items, cus, st);
+        else run_split<Split64L<FP8>>(prefill_split_kernel<64, FP8, Split64L<FP8>>, a, items, cus, st);
+    } else {
+        if (rows == 64) run_split<Split128S<FP8>>(prefill_split_kernel<128, FP8, Split128S<FP8>>, a, items, cus, st);
+        else run_split<Split128M<FP8>>(prefill_split_kernel<128, FP8, Split128M<FP8>>, a, items, cus, st);
+    }
 }
 
 }  // namespace
 
 size_t prefill_items_bytes(const vkv_prefill_params* p) {
-    return 256 + size_t(int64_t(p->num_seqs) * max_row_blocks(p) * p->num_kv_heads) * sizeof(int2);
+    return 256 + size_t(int64_t(p->num_seqs) * max_row_blocks(p, rows_per_item(p)) * p->num_kv_heads) * sizeof(int2);
 }
 
 int launch_prefill_mfma(const vkv_prefill_params* p, void* item_space, hipStream_t st) {
@@ -1941,12 +2047,6 @@ int launch_prefill_mfma(const vkv_prefill_params* p, void* item_space, hipStream
     a.num_heads = p->num_heads;
     a.num_kv_heads = p->num_kv_heads;
     a.group = p->num_heads / p->num_kv_heads;
-    // wide_path(): prefill_w64_kernel / prefill_wide_kernel /
-    // prefill_wide8_kernel, Wide<D>::ROWS (token, head) rows per item; else
-    // prefill_mfma_kernel, up to kMaxWaves heads x kBQ tokens per item
-    const bool wide = wide_path(p);
-    const int head_groups = wide ? 1 : (a.group + kMaxWaves - 1) / kMaxWaves;
-    a.heads_per_wg = (a.group + head_groups - 1) / head_groups;
     a.bs_log2 = ilog2i(p->block_size);
     a.max_blocks_per_seq = p->max_blocks_per_seq;
     a.num_blocks = p->num_blocks;
@@ -1954,9 +2054,9 @@ int launch_prefill_mfma(const vkv_prefill_params* p, void* item_space, hipStream
     int64_t tt = int64_t(p->max_blocks_per_seq) * p->block_size;
     if (p->max_context_len > 0 && p->max_context_len < tt) tt = p->max_context_len;
     a.table_tokens = int32_t(tt > 0x7FFFFFFF ? 0x7FFFFFFF : tt);
-    const int row_mult = wide ? a.group : 1;
+    const int split = split_rows(p);
     const int rpi = rows_per_item(p);
-    a.qblocks = int(max_row_blocks(p));
+    a.qblocks = int(max_row_blocks(p, rpi));
     a.num_seqs = p->num_seqs;
     a.scale_log2 = logit_scale_log2(p->scale);
     int32_t* count = static_cast<int32_t*>(item_space);
@@ -1973,9 +2073,9 @@ int launch_prefill_mfma(const vkv_prefill_params* p, void* item_space, hipStream
     // (T query tokens).  Small calls order them in the kernel itself.
     const int64_t T = p->num_query_tokens;
     const int64_t nseq2 = p->num_seqs < T / 2 ? p->num_seqs : T / 2;
-    const int64_t bound = T * row_mult / rpi + nseq2;
-    // a host-built list (wide kernels only) replaces both in-kernel orderings
-    a.work_list = wide && p->work_list && p->work_list_words > kListHeaderWords ? p->work_list : nullptr;
+    const int64_t bound = T * a.group / rpi + nseq2;
+    // a host-built list (of 256-row items) replaces both in-kernel orderings
+    a.work_list = !split && p->work_list && p->work_list_words > kListHeaderWords ? p->work_list : nullptr;
     a.work_list_words = a.work_list ? p->work_list_words : 0;
     a.num_query_tokens = int32_t(p->num_query_tokens);
     {
@@ -1985,43 +2085,38 @@ int launch_prefill_mfma(const vkv_prefill_params* p, void* item_space, hipStream
         a.group_div_m = uint32_t(m - (uint64_t(1) << 32));
         a.group_div_s = sh;
     }
-    a.inline_list = !a.work_list && wide && bound <= kInlineBlocks;
+    a.inline_list = !a.work_list && bound <= kInlineBlocks;
     if (!a.inline_list && !a.work_list)
         hipLaunchKernelGGL(prefill_items_kernel, dim3(1), dim3(256), 0, st, p->query_start_loc, p->context_lens,
-                           p->num_seqs, p->num_kv_heads, row_mult, rpi, a.qblocks, a.table_tokens, nbins,
+                           p->num_seqs, p->num_kv_heads, a.group, rpi, a.qblocks, a.table_tokens, nbins,
                            items, count);
-    // Persistent grid, never more workgroups than there can be items: one per
-    // CU for the wide kernel (its LDS and registers fill a CU); two per CU for
-    // the FP8 kernel (at D = 128 one is resident, the other starts when a CU
-    // frees up).
-    int dev = 0, cus = 256;
-    if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-    const int64_t upper = int64_t(p->num_seqs) * a.qblocks * p->num_kv_heads;
-    const int64_t per_cu = wide ? 1 : 2;
-    const int64_t wgs = int64_t(cus) * per_cu < upper ? int64_t(cus) * per_cu : upper;
-    const bool w64 = VKV_PREFILL_W64 && p->head_dim == 128 && p->kv_dtype == VKV_DTYPE_F16;
-    const int waves = w64 ? kW64Waves : wide ? kWideWaves : (a.heads_per_wg < kMinWaves ? kMinWaves : a.heads_per_wg);
-    const dim3 grid(unsigned(wgs > 0 ? wgs : 1), 1u, unsigned(head_groups));
-    const dim3 block(unsigned(64 * waves));
-    if (p->head_dim == 128) {
-        if (w64) hipLaunchKernelGGL((prefill_w64_kernel<128>), grid, block, 0, st, a);
-        else if (p->kv_dtype == VKV_DTYPE_F16) hipLaunchKernelGGL((prefill_wide_kernel<128>), grid, block, 0, st, a);
-        else hipLaunchKernelGGL(prefill_wide8_kernel, grid, block, 0, st, a);
-    } else {
-        if (wide) hipLaunchKernelGGL((prefill_wide_kernel<64>), grid, block, 0, st, a);
-        else if (p->kv_dtype == VKV_DTYPE_F16) hipLaunchKernelGGL((prefill_mfma_kernel<64, kF16>), grid, block, 0, st, a);
-        else hipLaunchKernelGGL((prefill_mfma_kernel<64, kFp8>), grid, block, 0, st, a);
+    // Persistent grid, never more workgroups than there can be items.
+    const int cus = cu_count();
+    const int64_t upper = std::min(int64_t(p->num_seqs) * a.qblocks, bound) * p->num_kv_heads;
+    if (split) {
+        if (p->kv_dtype == VKV_DTYPE_F16) launch_split<false>(a, p->head_dim, split, upper, cus, st);
+        else launch_split<true>(a, p->head_dim, split, upper, cus, st);
+        return 0;
     }
+    // (one per CU: their LDS and registers fill it)
+    const int64_t wgs = std::min(int64_t(cus), upper);
+    const bool w64 = VKV_PREFILL_W64 && p->kv_dtype == VKV_DTYPE_F16;
+    const dim3 grid(unsigned(wgs > 0 ? wgs : 1));
+    const dim3 block(unsigned(64 * (w64 ? kW64Waves : kWideWaves)));
+    if (w64) hipLaunchKernelGGL((prefill_w64_kernel<128>), grid, block, 0, st, a);
+    else if (p->kv_dtype == VKV_DTYPE_F16) hipLaunchKernelGGL((prefill_wide_kernel<128>), grid, block, 0, st, a);
+    else hipLaunchKernelGGL(prefill_wide8_kernel, grid, block, 0, st, a);
     return 0;
 }
 
 int64_t prefill_work_list_host(const vkv_prefill_params* p, const int32_t* host_qsl, const int32_t* host_cl,
                                int32_t* out, int64_t capacity) {
     if (!p || !host_qsl || !host_cl) return -1;
-    if (p->num_seqs <= 0 || !prefill_mfma_supported(p) || !wide_path(p)) return 0;  // no list for this call
+    if (p->num_seqs <= 0 || !prefill_mfma_supported(p)) return 0;  // no list for this call
     const int G = p->num_heads / p->num_kv_heads, hkv = p->num_kv_heads;
-    const int rpi = rows_per_item(p);
-    const int64_t qblocks = max_row_blocks(p);
+    if (p->head_dim == 64 && (p->kv_dtype != VKV_DTYPE_F16 || G >= 4)) return 0;
+    const int rpi = list_rows(p);
+    const int64_t qblocks = max_row_blocks(p, rpi);
     int64_t tt = int64_t(p->max_blocks_per_seq) * p->block_size;
     if (p->max_context_len > 0 && p->max_context_len < tt) tt = p->max_context_len;
     // items in (s, b, kvh) order with their key tiles
@@ -2045,13 +2140,7 @@ int64_t prefill_work_list_host(const vkv_prefill_params* p, const int32_t* host_
         }
     }
     // one list per workgroup of the persistent grid (one per CU)
-    int dev = 0, cus = 0;
-    hipError_t e = hipGetDevice(&dev);
-    if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-    if (e != hipSuccess || cus <= 0) {
-        cus = kListDefaultCus;
-        (void)hipGetLastError();  // (no device: the default, and no error left behind)
-    }
+    const int cus = cu_count();
     const int64_t n = int64_t(items.size());
     const int64_t lists = n < cus ? (n > 0 ? n : 1) : cus;
     // Longest first (ties in (s, b, kvh) order), each item to the list with
