@@ -1976,13 +1976,17 @@ template <bool FP8> using Split64L = Split<64, FP8, 4, 2, 4, 64, 2>;
 template <bool FP8> using Split128S = Split<128, FP8, 2, 4, 2, 32, 2>;
 template <bool FP8> using Split128M = Split<128, FP8, 4, 2, 2, 32, 2>;
 
+// CUs of the current device (asked once per device).
 int cu_count() {
+    static std::atomic<int> cached[64];
     int dev = 0, cus = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) {
+    const bool known = hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < 64;
+    if (known && (cus = cached[dev].load(std::memory_order_relaxed)) > 0) return cus;
+    if (!known || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) {
         (void)hipGetLastError();  // (no device: the default, and no error left behind)
         return kListDefaultCus;
     }
+    cached[dev].store(cus, std::memory_order_relaxed);
     return cus;
 }
 int split_rows(const vkv_prefill_params* p) {

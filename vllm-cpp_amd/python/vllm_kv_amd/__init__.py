@@ -20,6 +20,7 @@ from typing import Optional, Sequence
 _HERE = os.path.dirname(os.path.abspath(__file__))
 PKG_ROOT = os.path.dirname(os.path.dirname(_HERE))          # vllm-cpp_amd/
 LIB_PATH = os.path.join(PKG_ROOT, "lib", "libvllm_kv_amd.so")
+FASTCALL_PATH = os.path.join(PKG_ROOT, "lib", "_vkv_fastcall.so")
 
 ABI_VERSION = 4  # vkv_abi_version() of the library this binding's structs match
 DTYPE_F32, DTYPE_F16, DTYPE_FP8 = 0, 1, 2
@@ -122,11 +123,38 @@ class BlockPlane(ctypes.Structure):
 
 
 _lib = None
+_fast = None  # the extension of python/src/fastcall.c, bound to the library
+
+
+def _bind_fastcall(lib):
+    """The extension that reads the tensors and fills the parameter structures of
+    the calls a step makes, bound to the library's entry points (None without torch)."""
+    import importlib.machinery
+    import importlib.util
+    try:
+        import torch
+    except ImportError:
+        return None
+    if not os.path.exists(FASTCALL_PATH):
+        raise RuntimeError(f"{FASTCALL_PATH} is missing: build it with __graft_entry__.build() "
+                           "(make -C vllm-cpp_amd)")
+    loader = importlib.machinery.ExtensionFileLoader("_vkv_fastcall", FASTCALL_PATH)
+    fast = importlib.util.module_from_spec(importlib.util.spec_from_file_location("_vkv_fastcall", FASTCALL_PATH,
+                                                                                  loader=loader))
+    loader.exec_module(fast)
+    entry = tuple(ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in (
+        "vkv_reshape_and_cache", "vkv_paged_decode", "vkv_paged_decode_append", "vkv_paged_prefill",
+        "vkv_rope_reshape_and_cache"))
+    current = (getattr(torch._C, "_cuda_getDevice", None), getattr(torch._C, "_cuda_getCurrentRawStream", None))
+    if None in current:
+        current = (lambda: None, lambda _: torch.cuda.current_stream().cuda_stream)
+    fast.bind(entry, (torch.float32, torch.float16, torch.uint8, getattr(torch, "float8_e4m3fn", None)), current)
+    return fast
 
 
 def load(path: str = LIB_PATH) -> ctypes.CDLL:
     """Load the library once; raises if it has not been built."""
-    global _lib
+    global _lib, _fast
     if _lib is not None:
         return _lib
     if not os.path.exists(path):
@@ -184,8 +212,22 @@ def load(path: str = LIB_PATH) -> ctypes.CDLL:
     lib.vkv_prefill_work_list_host.argtypes = [ctypes.POINTER(PrefillParams), ctypes.c_void_p, ctypes.c_void_p,
                                                ctypes.c_void_p, ctypes.c_int64]
     lib.vkv_prefill_work_list_host.restype = ctypes.c_int64
+    _fast = _bind_fastcall(lib)
     _lib = lib
     return lib
+
+
+def _calls():
+    """The bound extension; loads the library on first use."""
+    if _fast is None:
+        load()
+        _torch()  # (the extension is bound whenever torch can be imported)
+    return _fast
+
+
+def _handle(stream):
+    """A raw stream handle, or None for the current stream."""
+    return None if stream is None else _stream(stream)
 
 
 def check(rc: int) -> None:
@@ -244,9 +286,8 @@ def reshape_and_cache(key, value, key_cache, value_cache, slot_mapping,
                       key_scales=None, value_scales=None, stream=None) -> None:
     """key/value [T, Hkv, D] (token stride from the tensor); caches [N, bs, Hkv, D];
     slot_mapping int32 [T]; FP8 caches (uint8) need key_scales/value_scales [N, bs, Hkv]."""
-    _require_cuda(key, value, key_cache, value_cache, slot_mapping, key_scales, value_scales)
-    p = append_params(key, value, key_cache, value_cache, slot_mapping, key_scales, value_scales)
-    check(load().vkv_reshape_and_cache(ctypes.byref(p), _stream(stream)))
+    check((_fast or _calls()).append(key, value, key_cache, value_cache, slot_mapping, key_scales, value_scales,
+                                     _handle(stream)))
 
 
 def append_params(key, value, key_cache, value_cache, slot_mapping, key_scales=None,
@@ -293,24 +334,8 @@ def rope_reshape_and_cache(query, key, value, cos_sin, positions=None, start_pos
     """query [T, H, D], key/value [T, Hkv, D] (f32 or f16); cos_sin [P, D/2, 2] fp32 on the GPU;
     positions int32 [T] or None (start_pos + t).  With caches: query rotated in place, rotated
     key and value stored through slot_mapping.  Without: query and key rotated in place."""
-    _require_cuda(query, key, value, cos_sin, positions, key_cache, value_cache, slot_mapping,
-                  key_scales, value_scales)
-    T, H, D = query.shape
-    Hkv = key.shape[1]
-    N = bs = 0
-    cache_dtype = DTYPE_F16
-    if key_cache is not None:
-        N, bs = key_cache.shape[0], key_cache.shape[1]
-        cache_dtype = _dtype_code(key_cache)
-    p = RopeAppendParams(
-        query=_ptr(query), key=_ptr(key), value=_ptr(value), query_stride=query.stride(0),
-        key_stride=key.stride(0), value_stride=0 if value is None else value.stride(0),
-        cos_sin=_ptr(cos_sin), positions=_ptr(positions), start_pos=start_pos,
-        max_position=cos_sin.shape[0], key_cache=_ptr(key_cache), value_cache=_ptr(value_cache),
-        key_scales=_ptr(key_scales), value_scales=_ptr(value_scales), slot_mapping=_ptr(slot_mapping),
-        num_tokens=T, num_heads=H, num_kv_heads=Hkv, head_dim=D, block_size=bs, num_blocks=N,
-        src_dtype=_dtype_code(query), cache_dtype=cache_dtype)
-    check(load().vkv_rope_reshape_and_cache(ctypes.byref(p), _stream(stream)))
+    check((_fast or _calls()).rope(query, key, value, cos_sin, positions, start_pos, key_cache, value_cache,
+                                   slot_mapping, key_scales, value_scales, _handle(stream)))
 
 
 def decode_params(out, query, key_cache, value_cache, block_tables, context_lens, scale,
@@ -335,11 +360,9 @@ def paged_decode(out, query, key_cache, value_cache, block_tables, context_lens,
                  partition_size=0, workspace=None, stream=None) -> None:
     """out/query [S, H, D] (f32 or f16); caches [N, bs, Hkv, D]; block_tables int32 [S, MB];
     context_lens int32 [S]."""
-    _require_cuda(out, query, key_cache, value_cache, block_tables, context_lens, key_scales,
-                  value_scales, workspace)
-    p = decode_params(out, query, key_cache, value_cache, block_tables, context_lens, scale,
-                      key_scales, value_scales, max_context_len, accumulate, partition_size, workspace)
-    check(load().vkv_paged_decode(ctypes.byref(p), _stream(stream)))
+    check((_fast or _calls()).decode(out, query, key_cache, value_cache, block_tables, context_lens, scale,
+                                     key_scales, value_scales, max_context_len, accumulate, partition_size, workspace,
+                                     _handle(stream)))
 
 
 def paged_decode_append(out, query, key_cache, value_cache, block_tables, context_lens, scale,
@@ -349,12 +372,9 @@ def paged_decode_append(out, query, key_cache, value_cache, block_tables, contex
     """vkv_paged_decode_append: reshape_and_cache(key, value, ..., slot_mapping) then
     paged_decode(...), the append fused into the decode when the shapes allow (key/value
     [num_seqs, Hkv, D], token s being sequence s's new token)."""
-    _require_cuda(out, query, key_cache, value_cache, block_tables, context_lens, key, value, slot_mapping,
-                  key_scales, value_scales, workspace)
-    ap = append_params(key, value, key_cache, value_cache, slot_mapping, key_scales, value_scales)
-    dp = decode_params(out, query, key_cache, value_cache, block_tables, context_lens, scale,
-                       key_scales, value_scales, max_context_len, accumulate, partition_size, workspace)
-    check(load().vkv_paged_decode_append(ctypes.byref(ap), ctypes.byref(dp), _stream(stream)))
+    check((_fast or _calls()).decode_append(out, query, key_cache, value_cache, block_tables, context_lens, scale,
+                                            key_scales, value_scales, max_context_len, accumulate, partition_size,
+                                            workspace, key, value, slot_mapping, _handle(stream)))
 
 
 def paged_decode_noalloc(out, query, key_cache, value_cache, block_tables, context_lens, scale,
@@ -402,15 +422,9 @@ def paged_prefill(out, query, key_cache, value_cache, block_tables, context_lens
     multi_token_only: the caller's promise that no sequence has exactly one query token
     (skips the decode pass that serves those); work_list: a device int32 copy of
     prefill_work_list()'s words for this call (optional)."""
-    _require_cuda(out, query, key_cache, value_cache, block_tables, context_lens, query_start_loc,
-                  key_scales, value_scales, workspace, work_list)
-    p = prefill_params(out, query, key_cache, value_cache, block_tables, context_lens, query_start_loc,
-                       max_query_len, scale, key_scales, value_scales, max_context_len, workspace,
-                       multi_token_only)
-    if work_list is not None and work_list.numel() > 0:
-        p.work_list = work_list.data_ptr()
-        p.work_list_words = int(work_list.numel())
-    check(load().vkv_paged_prefill(ctypes.byref(p), _stream(stream)))
+    check((_fast or _calls()).prefill(out, query, key_cache, value_cache, block_tables, context_lens, query_start_loc,
+                                      max_query_len, scale, key_scales, value_scales, max_context_len, workspace,
+                                      multi_token_only, work_list, _handle(stream)))
 
 
 def prefill_work_list(out, query, key_cache, value_cache, block_tables, context_lens, query_start_loc,
