@@ -102,3 +102,32 @@ def test_stream_noalloc_without_room_for_slices(vkv, oracle, cuda):
     ref = oracle.paged_decode(q.astype(np.float32), np.nan_to_num(k).view(np.uint16), np.nan_to_num(v).view(np.uint16),
                               lay.block_tables, lay.context_lens, D ** -0.5)
     assert_close(to_np(out).astype(np.float32), ref, F16_ATOL, F16_RTOL, "noalloc")
+
+
+@pytest.mark.parametrize("table", [1024, 6000], ids=["rows", "partitions"])
+@pytest.mark.parametrize("H,Hkv,bs", [(28, 4, 32), (32, 8, 16), (8, 8, 16), (16, 2, 64)])
+def test_stream_fp8_edges_vs_oracle(vkv, oracle, cuda, H, Hkv, bs, table):
+    """FP8 caches at head_dim 128: unattended slots hold the NaN code and NaN scales."""
+    import torch
+    D = 128
+    rng = np.random.default_rng(H + bs)
+    lay, (k, v), q = _case(rng, H, Hkv, D, bs, CONTEXTS, table)
+    used = ~np.isnan(k[:, :, 0, 0].astype(np.float32))
+    N = lay.num_blocks
+    codes = [np.zeros((N, bs, Hkv, D), np.uint8) for _ in range(2)]
+    scales = [np.zeros((N, bs, Hkv), np.float32) for _ in range(2)]
+    oracle.reshape_and_cache(np.nan_to_num(k).view(np.uint16).reshape(-1, Hkv, D),
+                             np.nan_to_num(v).view(np.uint16).reshape(-1, Hkv, D), *codes,
+                             np.arange(N * bs, dtype=np.int32), *scales)
+    scale = float(D) ** -0.5
+    ref = oracle.paged_decode(q.astype(np.float32), *codes, lay.block_tables, lay.context_lens, scale,
+                              key_scales=scales[0], value_scales=scales[1])
+    for c, s in zip(codes, scales):
+        c[~used] = 0x7F
+        s[~used] = np.nan
+    out = torch.full((len(CONTEXTS), H, D), 7.0, dtype=torch.float16, device=cuda)
+    vkv.paged_decode(out, to_dev(q, cuda), to_dev(codes[0], cuda), to_dev(codes[1], cuda), to_dev(lay.block_tables, cuda),
+                     to_dev(lay.context_lens, cuda), scale, key_scales=to_dev(scales[0], cuda),
+                     value_scales=to_dev(scales[1], cuda))
+    torch.cuda.synchronize()
+    assert_close(to_np(out).astype(np.float32), ref, F16_ATOL, F16_RTOL, f"FP8 {H}/{Hkv}/bs{bs}")

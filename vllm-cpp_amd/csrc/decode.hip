@@ -54,18 +54,6 @@ constexpr int kUnroll = VKV_DECODE_UNROLL;
 #define VKV_DECODE_MIN_WAVES 3
 #endif
 constexpr int kMinWavesPerSimd = VKV_DECODE_MIN_WAVES;
-// MFMA variant: FP8 groups above kOneChunkAboveGFp8 heads load one 16-token
-// chunk per step instead of two (their chunks carry scales); fp16 groups above
-// kOneChunkAboveG heads keep two chunks at a lower occupancy target.
-// Build-time tuning knobs.
-#ifndef VKV_DECODE_ONE_CHUNK_ABOVE_G
-#define VKV_DECODE_ONE_CHUNK_ABOVE_G 6
-#endif
-#ifndef VKV_DECODE_ONE_CHUNK_ABOVE_G_FP8
-#define VKV_DECODE_ONE_CHUNK_ABOVE_G_FP8 3
-#endif
-constexpr int kOneChunkAboveG = VKV_DECODE_ONE_CHUNK_ABOVE_G;
-constexpr int kOneChunkAboveGFp8 = VKV_DECODE_ONE_CHUNK_ABOVE_G_FP8;
 // Default partition sizing aims at this many (row, partition, kv head) items.
 constexpr int64_t kMinItems = 2048;
 // Small batches stop splitting before a row could have more partitions than this.
@@ -454,349 +442,16 @@ __device__ __forceinline__ void decode_item(const DecodeArgs& a, const int P, co
     }
 }
 
-// MFMA variant of one work item, for fp16 queries over fp16 or FP8 caches with
-// D = 128 and block_size a multiple of 16.  A chunk is 16 tokens of one block.
-//   QK^T on the matrix cores (v_mfma_f32_16x16x32_f16, 4 per chunk): rows =
-//   the chunk's 16 tokens (A operand = K, lane l holds token l%16 and 8 dims
-//   chosen by l/16 and the MFMA index), columns = query heads (B operand = Q,
-//   head l%16 of the group, zero for l%16 >= G, its dims in the same order).
-//   The accumulator gives lane l the logits of head l%16 for tokens
-//   4(l/16)..+3.  fp16 K: lane l loads dims 32i + 8(l/16) for MFMA i.  FP8 K:
-//   lane l loads 16 codes, dims 32(l/16) + 16j (two loads), feeding MFMAs 2j
-//   and 2j+1; codes are converted exactly to fp16 (v_cvt_scalef32_pk_f16_fp8,
-//   scale 1) and the token's scale multiplies the logit.
-//   Softmax on that layout (running max per head, lanes sharing l%16 agree),
-//   probabilities through a 16 x G slice of LDS to the V layout, and p * V as
-//   packed fp16 dot products over token pairs (lane l: token 4u + l/16, dims
-//   8(l%16)..+7), as in the VALU variant; FP8 V scales are folded into p.
-// This moves the 128 VALU instructions of the per-token dot products and their
-// cross-lane sums per chunk onto the matrix pipe.
-template <int G, int KVT>
-__device__ __forceinline__ void decode_item_mfma(const DecodeArgs& a, const int P, const int s, const int kvh,
-                                                 const int part, const int lane, float* plds) {
-    constexpr int D = 128;
-    constexpr int CH = 16;
-    constexpr bool FP8 = KVT == kFp8;
-    constexpr int EB = FP8 ? 1 : 2;
-    typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
-    typedef float float4_t __attribute__((ext_vector_type(4)));
-    typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
-    static_assert(G <= 16, "group size must fit the 16 MFMA columns");
-
-    const int seq = a.row_seq ? a.row_seq[s] : s;
-    const int ctx = row_context(a, s);
-    const int t0 = part * P;
-    if (t0 >= ctx) return;
-    const int n = (ctx - t0) < P ? (ctx - t0) : P;
-    const int bs_mask = (1 << a.bs_log2) - 1;
-    const int col = lane & 15;  // MFMA column (query head) / V dim slice
-    const int quad = lane >> 4; // MFMA k-slice / accumulator row group / V token in a load
-
-    const int nb = (n + bs_mask) >> a.bs_log2;
-    int my_block = 0;
-    if (lane < nb) {
-        my_block = a.bt[int64_t(seq) * a.max_blocks_per_seq + (t0 >> a.bs_log2) + lane];
-        if (a.num_blocks > 0 && unsigned(my_block) >= unsigned(a.num_blocks)) my_block = 0;
-    }
-
-    // Q as the B operand; a negative scale is moved into Q (exact sign flip).
-    // Loads are unconditional (head h0 stands in for the unused columns, which
-    // are then zeroed) so that they overlap instead of each being awaited.
-    const int h0 = kvh * G;
-    const bool neg_scale = a.scale_log2 < 0.0f;
-    const uint32_t qkeep = col < G ? 0xFFFFFFFFu : 0u;
-    const uint32_t qflip = neg_scale ? 0x80008000u : 0u;
-    const char* qrow = static_cast<const char*>(a.q) +
-                       (query_row(a, s) * a.q_stride + int64_t(h0 + (col < G ? col : 0)) * D) * 2;
-    half8_t qb[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        // dims of MFMA i: fp16 32i + 8 quad; FP8 32 quad + 16 (i / 2) + 8 (i % 2)
-        const int d0 = FP8 ? 32 * quad + 16 * (i >> 1) + 8 * (i & 1) : 32 * i + 8 * quad;
-        u32x4 w = load16(qrow + d0 * 2);
-        w = (w ^ u32x4{qflip, qflip, qflip, qflip}) & u32x4{qkeep, qkeep, qkeep, qkeep};
-        qb[i] = __builtin_bit_cast(half8_t, w);
-    }
-    const float sc = neg_scale ? -a.scale_log2 : a.scale_log2;
-
-    const uint32_t slot_stride = uint32_t(a.num_kv_heads) * D * EB;
-    const int64_t block_stride = int64_t(slot_stride) << a.bs_log2;
-    const uint32_t koff = FP8 ? uint32_t(col) * slot_stride + uint32_t(kvh * D + 32 * quad)
-                              : uint32_t(col) * slot_stride + uint32_t(kvh * D + 8 * quad) * 2;
-    const uint32_t voff = uint32_t(quad) * slot_stride + uint32_t(kvh * D + 8 * col) * EB;
-
-    float m = -INFINITY;  // running max of this lane's head (col), raw units
-    float l = 0.0f;       // this lane's share of the head's weight sum
-    float acc[G][8];
-#pragma unroll
-    for (int h = 0; h < G; ++h)
-#pragma unroll
-        for (int e = 0; e < 8; ++e) acc[h][e] = 0.0f;
-
-    struct Chunk {
-        u32x4 k[FP8 ? 2 : 4];
-        u32x4 v[FP8 ? 1 : 4];
-        u32x2 v8[FP8 ? 4 : 1];
-        // FP8: one scale per lane (lanes 0-15: K scale of token l, lanes
-        // 16-31: V scale of token l - 16), shuffled to the lanes that use it;
-        // after compute starts, ks/vs hold the per-lane values.
-        float sc1;
-        float ks[FP8 ? 4 : 1];  // scales of tokens 4 quad + k
-        float vs[FP8 ? 4 : 1];  // scales of tokens 4 u + quad
-    };
-    // Issue the K (A-operand layout) and V (row layout) loads of the 16 tokens
-    // at c.  Addresses are always valid (block ids past the partition are 0).
-    auto load_chunk = [&](Chunk& ch, const int c) __attribute__((always_inline)) {
-        const int blk = __builtin_amdgcn_readlane(my_block, (c >> a.bs_log2) & 63);
-        const int64_t boff = int64_t(blk) * block_stride + int64_t(c & bs_mask) * slot_stride;
-        const char* kb = a.kc + boff;
-        const char* vb = a.vc + boff;
-        // K lines are read in two halves by different instructions: ordinary
-        // loads keep the line for the second half; V rows stream (non-temporal).
-        if constexpr (FP8) {
-#pragma unroll
-            for (int j = 0; j < 2; ++j) ch.k[j] = load16(kb + koff + 16 * j);
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-                ch.v8[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x2*>(vb + voff + u * 4 * slot_stride));
-            const int64_t sbase = ((int64_t(blk) << a.bs_log2) + (c & bs_mask)) * a.num_kv_heads + kvh;
-            ch.sc1 = ((lane & 16) ? a.vs : a.ks)[sbase + int64_t(col) * a.num_kv_heads];
-        } else {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) ch.k[i] = load16(kb + koff + 64 * i);
-#pragma unroll
-            for (int u = 0; u < 4; ++u) ch.v[u] = load16_nt(vb + voff + u * 4 * slot_stride);
-        }
-    };
-
-    auto compute_chunk = [&](Chunk& ch, const int c, auto tail_tag) __attribute__((always_inline)) {
-        constexpr bool TAIL = decltype(tail_tag)::value;
-        u32x4* vr = ch.v;  // (fp16 only)
-        float4_t cc = {0.0f, 0.0f, 0.0f, 0.0f};
-        if constexpr (FP8) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const uint32_t c0 = ch.k[i >> 1][2 * (i & 1)], c1 = ch.k[i >> 1][2 * (i & 1) + 1];
-                const u32x4 w = {fp8x2_to_half2<false>(c0), fp8x2_to_half2<true>(c0), fp8x2_to_half2<false>(c1),
-                                 fp8x2_to_half2<true>(c1)};
-                cc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, w), qb[i], cc, 0, 0, 0);
-            }
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                ch.ks[k] = __shfl(ch.sc1, 4 * quad + k, kWave);
-                ch.vs[k] = __shfl(ch.sc1, 16 + 4 * k + quad, kWave);
-                cc[k] *= ch.ks[k];
-            }
-        } else {
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                cc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, ch.k[i]), qb[i], cc, 0, 0, 0);
-        }
-        float r[4];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) r[k] = (TAIL && c + 4 * quad + k >= n) ? -INFINITY : cc[k];
-        if constexpr (TAIL) {
-            // past n: V zero and (FP8) scale zero, whatever the slots hold
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                if (c + 4 * u + quad >= n) {
-                    if constexpr (FP8) {
-                        ch.v8[u] = u32x2{0u, 0u};  // code 0 widens to +0
-                        ch.vs[u] = 0.0f;
-                    } else {
-                        vr[u] = u32x4{0u, 0u, 0u, 0u};
-                    }
-                }
-            }
-        }
-
-        // running max per head: lanes sharing col hold the same value after the exchange
-        float cm = fmaxf(fmaxf(r[0], r[1]), fmaxf(r[2], r[3]));
-        // (FP8 chunks keep the exchange on the LDS permute: their VALU is the
-        // busier pipe, and the VALU swaps measured C5 1 % slower)
-        if constexpr (FP8) cm = fmaxf(cm, __shfl_xor(cm, 16, kWave)), cm = fmaxf(cm, __shfl_xor(cm, 32, kWave));
-        else cm = xor_max<32>(xor_max<16>(cm));
-        const bool grow = cm > m;
-        if (__builtin_amdgcn_ballot_w64(grow && col < G)) {
-            const float alpha = grow ? __builtin_amdgcn_exp2f((m - cm) * sc) : 1.0f;
-            if (grow) m = cm;
-            l *= alpha;
-#pragma unroll
-            for (int h = 0; h < G; ++h) {
-                // lane h holds column (head) h
-                const float ah = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, alpha), h));
-#pragma unroll
-                for (int e = 0; e < 8; ++e) acc[h][e] *= ah;
-            }
-        }
-        const float msc = m * sc;
-        float pr[4];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            pr[k] = __builtin_amdgcn_exp2f(fmaf(r[k], sc, -msc));
-            if (TAIL && c + 4 * quad + k >= n) pr[k] = 0.0f;
-        }
-        // weights to LDS as [token][head]; the sum uses the fp16-rounded values
-        // that the p * V products use
-        if (col < G) {
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                const float pk = static_cast<float>(static_cast<_Float16>(pr[k]));
-                l += pk;
-                plds[(4 * quad + k) * G + col] = pk;
-            }
-        }
-        wave_lds_sync();
-#pragma unroll
-        for (int u = 0; u < 4; u += 2) {
-            half2_t pp[G];
-            const float v0 = FP8 ? ch.vs[u] : 1.0f;
-            const float v1 = FP8 ? ch.vs[u + 1] : 1.0f;
-#pragma unroll
-            for (int h = 0; h < G; ++h)
-                pp[h] = half2_t{static_cast<_Float16>(plds[(4 * u + quad) * G + h] * v0),
-                                static_cast<_Float16>(plds[(4 * (u + 1) + quad) * G + h] * v1)};
-            u32x4 va, vb;
-            if constexpr (!FP8) {
-                va = vr[u];
-                vb = vr[u + 1];
-            } else {
-                // the two tokens' codes as fp16 in dim order: (b0, b1), (b2, b3)
-#pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    va[2 * h] = fp8x2_to_half2<false>(ch.v8[u][h]);
-                    va[2 * h + 1] = fp8x2_to_half2<true>(ch.v8[u][h]);
-                    vb[2 * h] = fp8x2_to_half2<false>(ch.v8[u + 1][h]);
-                    vb[2 * h + 1] = fp8x2_to_half2<true>(ch.v8[u + 1][h]);
-                }
-            }
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const uint32_t lo = __builtin_amdgcn_perm(vb[i], va[i], 0x05040100u);
-                const uint32_t hi = __builtin_amdgcn_perm(vb[i], va[i], 0x07060302u);
-#pragma unroll
-                for (int h = 0; h < G; ++h) {
-                    acc[h][2 * i] = dot2(pp[h], as_half2(lo), acc[h][2 * i]);
-                    acc[h][2 * i + 1] = dot2(pp[h], as_half2(hi), acc[h][2 * i + 1]);
-                }
-            }
-        }
-        wave_lds_sync();
-    };
-
-    // Two chunks (32 tokens, 16 KiB of K/V per wave at D=128 fp16) are loaded
-    // before either is computed, doubling the bytes in flight per wave.  FP8
-    // groups above 3 heads (their chunks carry scales) load one chunk at a
-    // time so that the 8 G accumulators per lane fit without spilling.
-    const int nc = (n + CH - 1) / CH;
-    const bool ragged = (n % CH) != 0;
-    // Fused append (fp16): the row's last position reads the new token's rows
-    // when the append targets that position's slot.  Applied to the last
-    // chunk right after its loads are issued.
-    auto fuse_last = [&](Chunk& ch, const int c) __attribute__((always_inline)) {
-        if constexpr (!FP8) {
-            if (a.fkey && t0 + n == ctx) {
-                const int pn = n - 1;
-                const int pblk = __builtin_amdgcn_readlane(my_block, (pn >> a.bs_log2) & 63);
-                const int64_t pslot = (int64_t(pblk) << a.bs_log2) + (pn & bs_mask);
-                if (int64_t(a.fslots[s]) == pslot) {
-                    const char* kr = a.fkey + s * a.fkey_stride + kvh * D * 2;
-                    const char* vr = a.fval + s * a.fval_stride + kvh * D * 2;
-                    // K: lane (col, quad) holds token c + col, dims 32 i + 8 quad
-                    if (c + col == pn) {
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) ch.k[i] = load16(kr + (32 * i + 8 * quad) * 2);
-                    }
-                    // V: load u holds token c + 4 u + quad, dims 8 col..+7
-#pragma unroll
-                    for (int u = 0; u < 4; ++u)
-                        if (c + 4 * u + quad == pn) ch.v[u] = load16(vr + 8 * col * 2);
-                }
-            }
-        }
-    };
-    int ci = 0;
-    if constexpr (FP8 && G > kOneChunkAboveGFp8) {
-        for (; ci + 1 < nc; ++ci) {
-            Chunk x;
-            load_chunk(x, ci * CH);
-            compute_chunk(x, ci * CH, std::false_type{});
-        }
-        Chunk x;
-        load_chunk(x, ci * CH);
-        if (ragged) compute_chunk(x, ci * CH, std::true_type{});
-        else compute_chunk(x, ci * CH, std::false_type{});
-    } else {
-    for (; ci + 2 < nc; ci += 2) {
-        Chunk x, y;
-        load_chunk(x, ci * CH);
-        load_chunk(y, (ci + 1) * CH);
-        compute_chunk(x, ci * CH, std::false_type{});
-        compute_chunk(y, (ci + 1) * CH, std::false_type{});
-    }
-    if (ci + 1 < nc) {
-        Chunk x, y;
-        load_chunk(x, ci * CH);
-        load_chunk(y, (ci + 1) * CH);
-        fuse_last(y, (ci + 1) * CH);
-        compute_chunk(x, ci * CH, std::false_type{});
-        if (ragged) compute_chunk(y, (ci + 1) * CH, std::true_type{});
-        else compute_chunk(y, (ci + 1) * CH, std::false_type{});
-    } else {
-        Chunk x;
-        load_chunk(x, ci * CH);
-        fuse_last(x, ci * CH);
-        if (ragged) compute_chunk(x, ci * CH, std::true_type{});
-        else compute_chunk(x, ci * CH, std::false_type{});
-    }
-    }
-
-    // head sums: lanes sharing col; accumulators: lanes sharing col (token groups)
-    l = xor_add<32>(xor_add<16>(l));
-#pragma unroll
-    for (int h = 0; h < G; ++h)
-#pragma unroll
-        for (int e = 0; e < 8; ++e) acc[h][e] = cross_group_sum<16>(acc[h][e]);
-
-    if (quad == 0) {
-#pragma unroll
-        for (int h = 0; h < G; ++h) {
-            const int64_t item = ((int64_t(s) * a.num_kv_heads + kvh) * a.max_parts + part) * G + h;
-            float* o = a.part_o + item * D + col * 8;
-            store16(o, u32x4{as_u32(acc[h][0]), as_u32(acc[h][1]), as_u32(acc[h][2]), as_u32(acc[h][3])});
-            store16(o + 4, u32x4{as_u32(acc[h][4]), as_u32(acc[h][5]), as_u32(acc[h][6]), as_u32(acc[h][7])});
-        }
-        if (col < G) {
-            const int64_t item = ((int64_t(s) * a.num_kv_heads + kvh) * a.max_parts + part) * G + col;
-            a.part_ml[item * 2] = m * sc;
-            a.part_ml[item * 2 + 1] = l;
-        }
-    }
-}
-
 // Persistent partition kernel (the item loop of decode_common.hpp) whose
 // items are (row, partition, kv head), kv head fastest.
-// Register budget per instantiation: the fp16 matrix-core variant with 7-8
-// heads per group keeps two chunks in flight at 2 waves per SIMD (measured
-// faster than one chunk at 3), and FP8 groups of 7-8 fit their one chunk
-// without spilling at 2; everything else targets kMinWavesPerSimd.
-template <int KVT, int G, bool MFMA>
-constexpr int min_waves_per_simd() {
-    return (MFMA && ((KVT == kF16 && G > kOneChunkAboveG) || (KVT == kFp8 && G > 6))) ? 2 : kMinWavesPerSimd;
-}
-
 // STATIC: the small-call variant (a static grid, static_parts > 0).
-template <typename IO, int KVT, int D, int G, bool MFMA, bool STATIC>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(min_waves_per_simd<KVT, G, MFMA>())))
+template <typename IO, int KVT, int D, int G, bool STATIC>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kMinWavesPerSimd)))
 void decode_partition_kernel(const DecodeArgs a) {
-    __shared__ float plds[MFMA ? kWavesPerBlock : 1][MFMA ? 16 * G : 1];
     const int lane = threadIdx.x & (kWave - 1);
-    const int wave = threadIdx.x / kWave;
-    // (matrix-core items are dealt, VALU ones claimed: run_partitions)
-    run_partitions<STATIC, MFMA>(a, a.num_kv_heads, [&](const int P, const int row, const int part, const int kvh)
-                                                  __attribute__((always_inline)) {
-        if constexpr (MFMA) decode_item_mfma<G, KVT>(a, P, row, kvh, part, lane, plds[wave]);
-        else decode_item<IO, KVT, D, G, STATIC>(a, P, row, kvh, part, lane);
+    run_partitions<STATIC>(a, a.num_kv_heads, [&](const int P, const int row, const int part, const int kvh)
+                                          __attribute__((always_inline)) {
+        decode_item<IO, KVT, D, G, STATIC>(a, P, row, kvh, part, lane);
     });
 }
 
@@ -905,8 +560,8 @@ __global__ __launch_bounds__(DT ? DT : 1024) void decode_reduce_kernel(DecodeArg
     *out = static_cast<IO>(r);
 }
 
-// Building with -DVKV_DECODE_MFMA=0 selects the VALU QK^T variant everywhere
-// (an A/B switch for measurements; the shipped library uses matrix cores).
+// Building with -DVKV_DECODE_MFMA=0 runs every shape on the VALU kernels (an
+// A/B switch for measurements; the shipped library uses matrix cores).
 #ifndef VKV_DECODE_MFMA
 #define VKV_DECODE_MFMA 1
 #endif
@@ -914,10 +569,7 @@ constexpr int mfma_enabled() { return VKV_DECODE_MFMA; }
 
 template <typename IO, int KVT, int D, int G>
 void launch_g(DecodeArgs& args, int grid_x, int grid_y, int grid_z, size_t lds, hipStream_t st) {
-    // Matrix-core QK^T for fp16 query and keys at D = 128 with blocks of a
-    // multiple of 16 tokens; the VALU variant covers everything else.
-    constexpr bool kMfmaShape = std::is_same<IO, _Float16>::value && KVT != kF32 && D == 128;
-    // fp16 over fp16 at head_dim 64 and 128 runs on decode_stream.hip otherwise.
+    // (fp16 over fp16 at head_dim 64 and 128 runs on decode_stream.hip)
     constexpr bool kStreamed = mfma_enabled() && std::is_same<IO, _Float16>::value && KVT == kF16 && D <= 128;
     // grid_x arrives as the number of item groups (an upper bound).  One workgroup per resident slot: the variant's workgroups per CU by
     // registers (queried once per variant), bounded by the LDS the rows'
@@ -928,15 +580,15 @@ void launch_g(DecodeArgs& args, int grid_x, int grid_y, int grid_z, size_t lds, 
     // resident wave count also feeds the partition choice.
     // Static small-call variants exist for fp16 queries (the serving case).
     constexpr bool kStatic = std::is_same<IO, _Float16>::value;
-    static std::atomic<int> reg_blocks[2];
-    auto run = [&](auto kernel, auto static_kernel, int variant) {
+    static std::atomic<int> reg_blocks{0};
+    auto run = [&](auto kernel, auto static_kernel) {
         const int cus = device_cu_count();
-        int per_cu = reg_blocks[variant].load(std::memory_order_relaxed);
+        int per_cu = reg_blocks.load(std::memory_order_relaxed);
         if (per_cu <= 0) {
             if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kWave * kWavesPerBlock, 0) !=
                     hipSuccess || per_cu <= 0)
                 per_cu = 1;
-            reg_blocks[variant].store(per_cu, std::memory_order_relaxed);
+            reg_blocks.store(per_cu, std::memory_order_relaxed);
         }
         const int by_lds = kLdsPerCu / int(lds + 4096);  // + an allowance for the static LDS
         if (by_lds < per_cu) per_cu = by_lds > 0 ? by_lds : 1;
@@ -970,13 +622,9 @@ void launch_g(DecodeArgs& args, int grid_x, int grid_y, int grid_z, size_t lds, 
         else
             hipLaunchKernelGGL(kernel, dim3(gx > 0 ? gx : 1, grid_y, grid_z), dim3(kBlockThreads), lds, st, args);
     };
-    if (kMfmaShape && args.bs_log2 >= 4 && args.mfma_enabled)
-        run(decode_partition_kernel<IO, KVT, D, G, kMfmaShape, false>,
-            decode_partition_kernel<IO, KVT, D, G, kMfmaShape, kStatic>, 1);
-    else if constexpr (!kStreamed)
-        run(decode_partition_kernel<IO, KVT, D, G, false, false>, decode_partition_kernel<IO, KVT, D, G, false, kStatic>, 0);
+    if constexpr (!kStreamed)
+        run(decode_partition_kernel<IO, KVT, D, G, false>, decode_partition_kernel<IO, KVT, D, G, kStatic>);
 }
-
 
 template <typename IO, int KVT, int D>
 int dispatch_g(int G, DecodeArgs& args, int grid_x, int Hkv, int S, size_t lds, hipStream_t st) {
@@ -1241,7 +889,6 @@ int launch_rows(const vkv_decode_params* p, const DecodePlan& plan, void* worksp
     a.counters = static_cast<int*>(workspace);
     a.part_o = reinterpret_cast<float*>(static_cast<char*>(workspace) + kWorkspaceHeader);
     a.part_ml = a.part_o + o_elems;
-    a.mfma_enabled = mfma_enabled();
     a.q_stride = p->query_stride ? p->query_stride : int64_t(p->num_heads) * p->head_dim;
     a.num_heads = p->num_heads;
     a.num_kv_heads = p->num_kv_heads;
@@ -1275,6 +922,8 @@ int launch_rows(const vkv_decode_params* p, const DecodePlan& plan, void* worksp
     const bool split_streams = plan.stream && !matrix_split_shape(D, G, p->block_size, p->key_cache, p->value_cache);
     a.row_parts = split_streams ? reinterpret_cast<int32_t*>(a.part_ml + size_t(rows) * p->num_heads * plan.max_parts * 2)
                                 : nullptr;
+    const bool matrix = mfma_enabled() && p->io_dtype == VKV_DTYPE_F16 && p->kv_dtype != VKV_DTYPE_F32 &&
+                        matrix_split_shape(D, G, p->block_size, p->key_cache, p->value_cache);
     a.head_dim = D;
     a.block_size = p->block_size;
     set_block_div(a, p->block_size);
@@ -1332,6 +981,10 @@ int launch_rows(const vkv_decode_params* p, const DecodePlan& plan, void* worksp
         if (streamed) {
             rc = launch_decode_stream(c, whole_rows, (size_t(n) + 1) * sizeof(int), st);
             if (!rc && !whole_rows) rc = launch_reduce<_Float16>(D, c, p->num_heads, n, st);
+        } else if (matrix) {
+            rc = 0;
+            if (!launch_decode_matrix(c, p->kv_dtype == VKV_DTYPE_FP8_E4M3, max_items, lds, st))
+                rc = launch_reduce<_Float16>(D, c, p->num_heads, n, st);
         } else if (!fixed) {
             rc = launch_decode_generic(c, p->kv_dtype, int64_t(n) * plan.max_parts, lds, st);
             if (!rc) rc = p->io_dtype == VKV_DTYPE_F32 ? launch_reduce<float>(D, c, p->num_heads, n, st)

@@ -68,7 +68,6 @@ struct DecodeArgs {
     int32_t accumulate;
     int32_t num_rows;         // sequences (decode) or query rows (prefill)
     int* counters;            // the workspace header ints (claim counters zero between calls)
-    int32_t mfma_enabled;     // use the matrix-core QK^T variant where it applies
     // num_cands > 1: P is the default size, the kernel picks the partition
     // size among cands (ascending) and records it in the workspace header.
     int32_t num_cands;
@@ -131,7 +130,8 @@ inline bool fixed_decode_shape(int head_dim, int group, int block_size, const vo
 // The shapes of decode_stream.hip: fp16 queries over fp16 caches at these head
 // dimensions, groups of up to 32 heads and any block size.  Split-K calls at
 // head_dim 128, groups of up to 8 and power-of-two blocks of 16 tokens and more
-// stay on decode.hip's matrix-core kernel (matrix_split_shape).
+// (matrix_split_shape; FP8 caches too) run in partitions of the size that
+// run_partitions picks, the others in equal slices.
 inline bool stream_decode_shape(int head_dim, int group, const void* kc, const void* vc, bool f16_io, bool f16_kv) {
     const bool aligned = ((reinterpret_cast<uintptr_t>(kc) | reinterpret_cast<uintptr_t>(vc)) & 15u) == 0;
     return f16_io && f16_kv && aligned && head_dim >= 64 && head_dim <= 128 && head_dim % 16 == 0 && group >= 1 &&
@@ -145,6 +145,10 @@ inline bool matrix_split_shape(int head_dim, int group, int block_size, const vo
 bool stream_decode_rows(int num_rows, int num_kv_heads, int head_dim, int max_ctx, bool matrix_split);
 // The call's partition launch (or, with rows, its only launch).  0 or VKV_ERR_*.
 int launch_decode_stream(DecodeArgs& a, bool rows, size_t lds, hipStream_t st);
+
+// The partition launch of a matrix_split_shape call (fp16 queries over an fp16
+// or FP8 cache); true if it wrote the output itself instead of partials.
+bool launch_decode_matrix(DecodeArgs& a, bool fp8, int64_t max_items, size_t lds, hipStream_t st);
 
 // Partition kernel of the generic variant (decode_generic.hip) for one launch
 // of rows; max_pairs bounds the (row, partition) pairs.  0 or VKV_ERR_*.

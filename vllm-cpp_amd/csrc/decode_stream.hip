@@ -1,7 +1,8 @@
 // decode_stream.hip — paged decode attention for fp16 queries over fp16 caches
-// at head_dim 64, 80, 96, 112 or 128 with groups of up to 32 query heads, both
-// products on the matrix cores (gfx950).  Semantics as in decode.hip (the
-// reference's src/attention/paged_attention.cu:13-82).
+// at head_dim 64, 80, 96, 112 or 128 with groups of up to 32 query heads, and
+// over FP8 caches at head_dim 128 with groups of up to 8, both products on the
+// matrix cores (gfx950).  Semantics as in decode.hip (the reference's
+// src/attention/paged_attention.cu:13-82).
 //
 // A wave streams the K and V rows of its tokens through LDS, 32 tokens a step,
 // with direct global->LDS loads (global_load_lds_dwordx4, 1 KiB per wave
@@ -18,8 +19,14 @@
 //                 B = P^T straight from the S^T registers, so the weights
 //                 never leave the lane and the accumulators are head_dim / 4
 //                 registers per 16 heads.
-// The VALU kernels that served these shapes spent ~300 instructions per 16
-// tokens and held 4 KiB of loads per wave, waited for in turn.
+// FP8: codes become fp16 exactly (v_cvt_scalef32_pk_f16_fp8, scale 1) as they
+// are read from LDS, V^T by ds_read_b64_tr_b8; the token's K scale multiplies
+// the logit, its V scale the weight.
+// Before: the VALU kernels of head_dim 64 and the generic shapes spent ~300
+// instructions per 16 tokens and held 4 KiB of loads per wave, waited for in
+// turn; head_dim 128's kernel ran P V on the VALU (packed dot products, 16 G
+// of them and as many accumulators per 16 tokens), which left FP8 groups of 7
+// one chunk in flight at two waves per SIMD: 178 us where it now takes 125.
 #include <atomic>
 #include <type_traits>
 
@@ -41,22 +48,31 @@ constexpr float kLazyLog2 = 8.0f;    // the running max is raised when passed by
 
 // LDS tile of a step's K (or V) rows: row-major, unpadded (a direct load
 // writes lane L's 16 bytes at 16 L).  Where a row is a power of two of 16-byte
-// chunks, chunk c of row r sits at slot c ^ (r % CH): the operand reads take
-// one chunk column of 16 rows, which would otherwise meet in the same banks.
+// chunks, chunk c of row r sits at slot c ^ key(r): the operand reads take one
+// chunk column of 16 rows, which would otherwise meet in the same banks.
 // (Rows of 160, 192 or 224 bytes are spread by their own stride.)
-template <int D>
+template <int D, bool FP8>
 struct Tile {
-    static constexpr int ROW = 2 * D;
+    static constexpr int ROW = FP8 ? D : 2 * D;
     static constexpr int CH = ROW / 16;
     static constexpr int NI = kStep * CH / 64;  // direct loads per tile
     static constexpr int BYTES = kStep * ROW;
+    static constexpr int STAGE = 2 * BYTES + (FP8 ? 8 * kStep : 0);  // K, V, then the K and V scales
+    static constexpr int LOADS = 2 * NI + (FP8 ? 1 : 0);             // wave loads per stage
     static constexpr bool SWZ = (CH & (CH - 1)) == 0;
     static constexpr int KS = D / 32;       // 32-dim MFMA steps of K Q^T
     static constexpr bool HALF = D % 32 != 0;  // and a 16-dim one
     static constexpr int DT = D / 16;       // dim tiles of O^T
     static_assert(D % 16 == 0 && kStep * CH % 64 == 0, "whole loads");
-    __device__ static __forceinline__ int slot(int row, int chunk) { return SWZ ? chunk ^ (row % CH) : chunk; }
+    static_assert(!FP8 || (SWZ && KS % 2 == 0), "FP8 operands are pairs of 8 codes of one chunk");
+    __device__ static __forceinline__ int slot(int row, int chunk) {
+        return SWZ ? chunk ^ (row / (16 / (SWZ ? CH : 16)) % CH) : chunk;
+    }
     __device__ static __forceinline__ int off(int row, int chunk) { return row * ROW + slot(row, chunk) * 16; }
+    // first of the 8 dims that lane group grp holds for MFMA i of K Q^T
+    __device__ static __forceinline__ int dim(int i, int grp) {
+        return FP8 ? 16 * (grp * (KS / 2) + i / 2) + 8 * (i % 2) : 32 * i + 8 * grp;
+    }
 };
 
 __device__ __forceinline__ uint32_t lds_addr(const char* p) {
@@ -75,6 +91,11 @@ __device__ __forceinline__ void dma16(const char* g, const uint32_t lds) {
     else
         asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(g), "s"(l) : "memory", "m0");
 }
+// One 4-byte direct load per lane to LDS bytes lds + 4 lane.
+__device__ __forceinline__ void dma4(const float* g, const uint32_t lds) {
+    const uint32_t l = __builtin_amdgcn_readfirstlane(lds);
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" : : "v"(g), "s"(l) : "memory", "m0");
+}
 template <int N>
 __device__ __forceinline__ void wait_loads() {
     static_assert(N >= 0 && N < 64, "vmcnt is 6 bits");
@@ -89,23 +110,37 @@ __device__ __forceinline__ u32x2 tr_read(const char* lds) {
     return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4f16((lds_ptr)(lds)));
 }
 
+// ds_read_b64_tr_b8: within each 16-lane group, lane i receives byte i % 8 of
+// the 8-byte chunks addressed by lanes i / 8 + 2 e, e = 0..7 (checked on the
+// device).
+__device__ __forceinline__ u32x2 tr_read8(const char* lds) {
+    typedef int i32x2 __attribute__((ext_vector_type(2)));
+    typedef __attribute__((address_space(3))) i32x2* lds_ptr;
+    return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_ptr)(lds)));
+}
+// Eight e4m3fn codes as their exact fp16 values, in order.
+__device__ __forceinline__ half8_t codes8(const uint32_t lo, const uint32_t hi) {
+    return __builtin_bit_cast(half8_t, u32x4{fp8x2_to_half2<false>(lo), fp8x2_to_half2<true>(lo),
+                                             fp8x2_to_half2<false>(hi), fp8x2_to_half2<true>(hi)});
+}
+
 // Attention state of one wave: CT tiles of 16 heads.
-template <int D, int CT>
+template <int D, int CT, bool FP8>
 struct State {
-    using T = Tile<D>;
+    using T = Tile<D, FP8>;
     half8_t q[CT][T::KS];
     half4_t qh[CT];
     float m[CT];              // running max of head 16 ct + l % 16, raw logits
-    float4_t l[CT];           // weight sums (every element the same)
+    float4_t l[CT];           // weight sums (every element the same; FP8: element 0, this lane's keys)
     float4_t o[CT][T::DT];    // O^T: lane l holds dims 16 t + 4 (l / 16) + e of head l % 16
 };
 
 // Q as the B operand and an empty state.  Columns past the group read head 0
 // and are zeroed; a negative scale is moved into Q (exact sign flip).
-template <int D, int CT>
-__device__ __forceinline__ void init_state(const DecodeArgs& a, State<D, CT>& st, const int s, const int kvh,
+template <int D, int CT, bool FP8>
+__device__ __forceinline__ void init_state(const DecodeArgs& a, State<D, CT, FP8>& st, const int s, const int kvh,
                                            const int G, const int lane) {
-    using T = Tile<D>;
+    using T = Tile<D, FP8>;
     const int col = lane & 15, grp = lane >> 4;
     const uint32_t flip = a.scale_log2 < 0.0f ? 0x80008000u : 0u;
 #pragma unroll
@@ -116,7 +151,7 @@ __device__ __forceinline__ void init_state(const DecodeArgs& a, State<D, CT>& st
                            (query_row(a, s) * a.q_stride + int64_t(kvh * G + (h < G ? h : 0)) * D) * 2;
 #pragma unroll
         for (int i = 0; i < T::KS; ++i) {
-            u32x4 w = load16(qrow + (32 * i + 8 * grp) * 2);
+            u32x4 w = load16(qrow + T::dim(i, grp) * 2);
             w = (w ^ u32x4{flip, flip, flip, flip}) & u32x4{keep, keep, keep, keep};
             st.q[c][i] = __builtin_bit_cast(half8_t, w);
         }
@@ -135,18 +170,18 @@ __device__ __forceinline__ void init_state(const DecodeArgs& a, State<D, CT>& st
 // Attends tokens [t0, t0 + n) (n >= 1) of row s at kv head kvh.  ring: NST
 // stages of a K and a V tile, this wave's own.  my_block: block ids of
 // [win, win + 64) in the row's table, one per lane (0 where out of the pool).
-template <int D, int CT, int NST>
-__device__ __forceinline__ void stream_tokens(const DecodeArgs& a, State<D, CT>& st, char* ring, const int s,
+template <int D, int CT, bool FP8, int NST>
+__device__ __forceinline__ void stream_tokens(const DecodeArgs& a, State<D, CT, FP8>& st, char* ring, const int s,
                                               const int32_t* table, const int ctx, const int kvh, const int t0,
                                               const int n, int win, int my_block, const int lane) {
-    using T = Tile<D>;
-    constexpr int kStage = 2 * T::BYTES;
-    constexpr int kLoads = 2 * T::NI;  // vector-memory operations per stage
+    using T = Tile<D, FP8>;
+    constexpr int kStage = T::STAGE;
     const int col = lane & 15, grp = lane >> 4;
     const uint32_t slot_stride = uint32_t(a.num_kv_heads) * T::ROW;
     const uint32_t ring_lds = lds_addr(ring);
     const float sc = a.scale_log2 < 0.0f ? -a.scale_log2 : a.scale_log2;
-    const float lazy = kLazyLog2 / sc;
+    // (FP8 weights carry their token's scale: they stay at most 1 before it)
+    const float lazy = FP8 ? 0.0f : kLazyLog2 / sc;
     const int steps = (n + kStep - 1) / kStep;
     // The fused append: the row's last position reads the new token's rows
     // when the append targets that position's slot.
@@ -183,6 +218,13 @@ __device__ __forceinline__ void stream_tokens(const DecodeArgs& a, State<D, CT>&
             dma16<T::ROW % 128 == 0>(kp, dst + i * 1024);
             dma16<T::ROW % 128 == 0>(vp, dst + T::BYTES + i * 1024);
         }
+        if constexpr (FP8) {
+            // lanes 0-31 the K scales of the step's tokens, 32-63 the V scales
+            const int tok = t0 + min(step * kStep + (lane & 31), n - 1);
+            const int blk = block_div(a, tok);
+            const int64_t slot = int64_t(__shfl(my_block, blk - win, kWave)) * a.block_size + (tok - blk * a.block_size);
+            dma4((lane < 32 ? a.ks : a.vs) + (slot * a.num_kv_heads + kvh), dst + 2 * T::BYTES);
+        }
     };
 
     const half8_t ones = {1.0f16, 1.0f16, 1.0f16, 1.0f16, 1.0f16, 1.0f16, 1.0f16, 1.0f16};
@@ -190,7 +232,7 @@ __device__ __forceinline__ void stream_tokens(const DecodeArgs& a, State<D, CT>&
         char* kb = ring + stage * kStage;
         char* vb = kb + T::BYTES;
         const bool tail = step * kStep + kStep > n;
-        if (tail) {
+        if (!FP8 && tail) {  // (a code of a clamped row times a zero weight is zero)
             // rows past the end: V zero whatever the slots hold (their weight is 0)
 #pragma unroll
             for (int i = 0; i < T::NI; ++i)
@@ -203,12 +245,24 @@ __device__ __forceinline__ void stream_tokens(const DecodeArgs& a, State<D, CT>&
         for (int c = 0; c < CT; ++c) sv[c][0] = sv[c][1] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int hh = 0; hh < 2; ++hh) {
+            if constexpr (FP8) {
 #pragma unroll
-            for (int i = 0; i < T::KS; ++i) {
-                const half8_t k = __builtin_bit_cast(half8_t, load16(kb + T::off(16 * hh + col, 4 * i + grp)));
+                for (int j = 0; j < T::KS / 2; ++j) {
+                    const u32x4 w = load16(kb + T::off(16 * hh + col, grp * (T::KS / 2) + j));
 #pragma unroll
-                for (int c = 0; c < CT; ++c)
-                    sv[c][hh] = __builtin_amdgcn_mfma_f32_16x16x32_f16(k, st.q[c][i], sv[c][hh], 0, 0, 0);
+                    for (int c = 0; c < CT; ++c) {
+                        sv[c][hh] = __builtin_amdgcn_mfma_f32_16x16x32_f16(codes8(w[0], w[1]), st.q[c][2 * j], sv[c][hh], 0, 0, 0);
+                        sv[c][hh] = __builtin_amdgcn_mfma_f32_16x16x32_f16(codes8(w[2], w[3]), st.q[c][2 * j + 1], sv[c][hh], 0, 0, 0);
+                    }
+                }
+            } else {
+#pragma unroll
+                for (int i = 0; i < T::KS; ++i) {
+                    const half8_t k = __builtin_bit_cast(half8_t, load16(kb + T::off(16 * hh + col, 4 * i + grp)));
+#pragma unroll
+                    for (int c = 0; c < CT; ++c)
+                        sv[c][hh] = __builtin_amdgcn_mfma_f32_16x16x32_f16(k, st.q[c][i], sv[c][hh], 0, 0, 0);
+                }
             }
             if constexpr (T::HALF) {
                 // A product of its own, added on the VALU: accumulated onto the
@@ -229,6 +283,19 @@ __device__ __forceinline__ void stream_tokens(const DecodeArgs& a, State<D, CT>&
             for (int c = 0; c < CT; ++c)
 #pragma unroll
                 for (int hh = 0; hh < 2; ++hh) sv[c][hh] += half_sv[c][hh];
+        }
+        // FP8: the token's K scale times the logit, its V scale times the weight
+        // (lane: keys 16 hh + 4 grp + e)
+        [[maybe_unused]] float4_t vsc[2];
+        if constexpr (FP8) {
+            const float* scales = reinterpret_cast<const float*>(kb + 2 * T::BYTES);
+#pragma unroll
+            for (int hh = 0; hh < 2; ++hh) {
+                const float4_t ksc = *reinterpret_cast<const float4_t*>(scales + 16 * hh + 4 * grp);
+                vsc[hh] = *reinterpret_cast<const float4_t*>(scales + kStep + 16 * hh + 4 * grp);
+#pragma unroll
+                for (int c = 0; c < CT; ++c) sv[c][hh] *= ksc;
+            }
         }
         half8_t p[CT];
 #pragma unroll
@@ -253,21 +320,38 @@ __device__ __forceinline__ void stream_tokens(const DecodeArgs& a, State<D, CT>&
                 for (int t = 0; t < T::DT; ++t) st.o[c][t] *= alpha;
             }
             const float msc = st.m[c] == -INFINITY ? 0.0f : st.m[c] * sc;
+if constexpr (FP8) {
 #pragma unroll
-            for (int e = 0; e < 8; ++e) p[c][e] = static_cast<_Float16>(__builtin_amdgcn_exp2f(fmaf(x[e], sc, -msc)));
-            // sums of the rounded weights, on the matrix pipe
-            st.l[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ones, p[c], st.l[c], 0, 0, 0);
+                for (int e = 0; e < 8; ++e) {
+                    const float w = __builtin_amdgcn_exp2f(fmaf(x[e], sc, -msc));
+                    st.l[c][0] += w;
+                    p[c][e] = static_cast<_Float16>(w * vsc[e >> 2][e & 3]);
+                }
+            } else {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) p[c][e] = static_cast<_Float16>(__builtin_amdgcn_exp2f(fmaf(x[e], sc, -msc)));
+                // sums of the rounded weights, on the matrix pipe
+                st.l[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ones, p[c], st.l[c], 0, 0, 0);
+            }
         }
-        // V^T operand: within each 16-lane group, lane i receives element i % 4
-        // of the 8-byte chunks addressed by lanes i / 4 + 4 e, so lane (col,
-        // grp) addresses key 4 grp + col / 4 (+ 16), dims 16 t + 4 (col % 4)
-        const int vrow = 4 * grp + (col >> 2);
+        // V^T operand, weight slots (grp, e) = key 4 grp + e, (grp, 4 + e) = key
+        // 16 + 4 grp + e.  fp16: within each 16-lane group, lane i receives
+        // element i % 4 of the 8-byte chunks addressed by lanes i / 4 + 4 e, so
+        // lane (col, grp) addresses key 4 grp + col / 4 (+ 16), dims 16 t + 4
+        // (col % 4).  FP8 (tr_read8): the key of slot col / 2, dims 16 t + 8 (col % 2).
+        const int vrow = FP8 ? (col < 8 ? 4 * grp + (col >> 1) : 12 + 4 * grp + (col >> 1)) : 4 * grp + (col >> 2);
 #pragma unroll
         for (int t = 0; t < T::DT; ++t) {
-            const int chunk = 2 * t + ((col & 3) >> 1);
-            const u32x2 lo = tr_read(vb + T::off(vrow, chunk) + 8 * (col & 1));
-            const u32x2 hi = tr_read(vb + T::off(16 + vrow, chunk) + 8 * (col & 1));
-            const half8_t v = __builtin_bit_cast(half8_t, u32x4{lo[0], lo[1], hi[0], hi[1]});
+            half8_t v;
+            if constexpr (FP8) {
+                const u32x2 w = tr_read8(vb + T::off(vrow, t) + 8 * (col & 1));
+                v = codes8(w[0], w[1]);
+            } else {
+                const int chunk = 2 * t + ((col & 3) >> 1);
+                const u32x2 lo = tr_read(vb + T::off(vrow, chunk) + 8 * (col & 1));
+                const u32x2 hi = tr_read(vb + T::off(16 + vrow, chunk) + 8 * (col & 1));
+                v = __builtin_bit_cast(half8_t, u32x4{lo[0], lo[1], hi[0], hi[1]});
+            }
 #pragma unroll
             for (int c = 0; c < CT; ++c) st.o[c][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(v, p[c], st.o[c][t], 0, 0, 0);
         }
@@ -288,12 +372,16 @@ __device__ __forceinline__ void stream_tokens(const DecodeArgs& a, State<D, CT>&
             if (step + 1 < steps) {
                 wait_lds();  // (the stage's reads, two steps ago in program order, are done)
                 issue(step + 1, (step + 1) & 1);
-                wait_loads<kLoads>();
+                wait_loads<T::LOADS>();
             } else {
                 wait_loads<0>();
             }
             compute(step, step & 1);
         }
+    }
+    if constexpr (FP8) {
+#pragma unroll
+        for (int c = 0; c < CT; ++c) st.l[c][0] = xor_add<32>(xor_add<16>(st.l[c][0]));
     }
 }
 
@@ -310,10 +398,10 @@ __device__ __forceinline__ int load_block(const DecodeArgs& a, const int32_t* ta
 // A workgroup of W waves per (row, kv head): each wave attends a contiguous
 // share of the context and the shares are merged in LDS, so the call is one
 // launch with no workspace.
-template <int D, int CT, int W, int NST>
+template <int D, int CT, bool FP8, int W, int NST>
 __global__ __launch_bounds__(64 * W) void decode_rows_kernel(const DecodeArgs a) {
-    using T = Tile<D>;
-    constexpr int kRing = NST * 2 * T::BYTES;
+    using T = Tile<D, FP8>;
+    constexpr int kRing = (NST * T::STAGE + 1023) / 1024 * 1024;
     constexpr int kMergeBytes = W * 16 * CT * (D + 2) * 4;
     __shared__ __attribute__((aligned(1024))) char lds[W * kRing > kMergeBytes ? W * kRing : kMergeBytes];
     const int lane = threadIdx.x & (kWave - 1);
@@ -334,7 +422,7 @@ __global__ __launch_bounds__(64 * W) void decode_rows_kernel(const DecodeArgs a)
     // the table fits one id per lane
     const bool whole = a.max_blocks_per_seq <= kWave;
     int ids = whole ? load_block(a, table, lane) : 0;
-    State<D, CT> st;
+    State<D, CT, FP8> st;
     init_state(a, st, s, kvh, G, lane);
     const int ctx = row_context(a, s);
     const int per = ((ctx + W - 1) / W + kStep - 1) / kStep * kStep;
@@ -346,7 +434,7 @@ __global__ __launch_bounds__(64 * W) void decode_rows_kernel(const DecodeArgs a)
             win = block_div(a, t0);
             ids = load_block(a, table, win + lane);
         }
-        stream_tokens<D, CT, NST>(a, st, lds + wave * kRing, s, table, ctx, kvh, t0, n, win, ids, lane);
+        stream_tokens<D, CT, FP8, NST>(a, st, lds + wave * kRing, s, table, ctx, kvh, t0, n, win, ids, lane);
     }
     // ---------------- merge
     const float sc = a.scale_log2 < 0.0f ? -a.scale_log2 : a.scale_log2;
@@ -432,8 +520,9 @@ constexpr int kMinSliceSteps = 2;
 
 template <int D, int CT, int NST>
 __global__ __launch_bounds__(256) void decode_stream_kernel(const DecodeArgs a) {
-    using T = Tile<D>;
-    constexpr int kRing = NST * 2 * T::BYTES;
+    constexpr bool FP8 = false;
+    using T = Tile<D, FP8>;
+    constexpr int kRing = NST * T::STAGE;
     __shared__ __attribute__((aligned(1024))) char lds[kWavesPerBlock * kRing];
     __shared__ int wave_total[kWavesPerBlock], wave_longest[kWavesPerBlock];
     extern __shared__ int prefix[];  // [num_rows + 1] exclusive prefix of the rows' steps
@@ -514,9 +603,9 @@ __global__ __launch_bounds__(256) void decode_stream_kernel(const DecodeArgs a) 
             const int n = min(ctx - t0, (e - at) * kStep);
             const int win = block_div(a, t0);
             const int ids = load_block(a, table, win + lane);
-            State<D, CT> st;
+            State<D, CT, FP8> st;
             init_state(a, st, s, kvh, G, lane);
-            stream_tokens<D, CT, NST>(a, st, lds + wave * kRing, s, table, ctx, kvh, t0, n, win, ids, lane);
+            stream_tokens<D, CT, FP8, NST>(a, st, lds + wave * kRing, s, table, ctx, kvh, t0, n, win, ids, lane);
             const int64_t slot = (int64_t(s) * a.num_kv_heads + kvh) * a.max_parts + (slice - b / R);
 #pragma unroll
             for (int c = 0; c < CT; ++c) {
@@ -535,6 +624,46 @@ __global__ __launch_bounds__(256) void decode_stream_kernel(const DecodeArgs a) 
     }
 }
 
+// Split-K in partitions of a fixed size (decode.hip's items and size choice).
+template <int D, int CT, bool FP8, int NST>
+__global__ __launch_bounds__(256) void decode_parts_kernel(const DecodeArgs a) {
+    using T = Tile<D, FP8>;
+    constexpr int kRing = (NST * T::STAGE + 1023) / 1024 * 1024;
+    __shared__ __attribute__((aligned(1024))) char lds[kWavesPerBlock * kRing];
+    const int lane = threadIdx.x & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int G = a.num_heads / a.num_kv_heads;
+    run_partitions<false, true>(a, a.num_kv_heads, [&](const int P, const int s, const int part, const int kvh)
+                                                __attribute__((always_inline)) {
+        const int seq = a.row_seq ? a.row_seq[s] : s;
+        const int32_t* table = a.bt + int64_t(seq) * a.max_blocks_per_seq;
+        const int ctx = row_context(a, s);
+        const int t0 = part * P;
+        if (t0 >= ctx) return;
+        const int n = min(ctx - t0, P);
+        const int win = block_div(a, t0);
+        const int ids = load_block(a, table, win + lane);
+        State<D, CT, FP8> st;
+        init_state(a, st, s, kvh, G, lane);
+        stream_tokens<D, CT, FP8, NST>(a, st, lds + wave * kRing, s, table, ctx, kvh, t0, n, win, ids, lane);
+        const float sc = a.scale_log2 < 0.0f ? -a.scale_log2 : a.scale_log2;
+        const int col = lane & 15, grp = lane >> 4;
+#pragma unroll
+        for (int c = 0; c < CT; ++c) {
+            const int h = 16 * c + col;
+            if (h >= G) continue;
+            const int64_t item = ((int64_t(s) * a.num_kv_heads + kvh) * a.max_parts + part) * G + h;
+            float* row = a.part_o + item * D;
+#pragma unroll
+            for (int t = 0; t < T::DT; ++t) *reinterpret_cast<float4_t*>(row + 16 * t + 4 * grp) = st.o[c][t];
+            if (grp == 0) {
+                a.part_ml[item * 2] = st.m[c] * sc;
+                a.part_ml[item * 2 + 1] = st.l[c][0];
+            }
+        }
+    });
+}
+
 // One workgroup per resident slot (occupancy queried once per variant).
 template <int D, int CT, int NST>
 void launch_split(DecodeArgs& a, size_t lds, hipStream_t st) {
@@ -545,7 +674,7 @@ void launch_split(DecodeArgs& a, size_t lds, hipStream_t st) {
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kBlockThreads, 0) != hipSuccess || per_cu <= 0) per_cu = 1;
         cached.store(per_cu, std::memory_order_relaxed);
     }
-    const int by_lds = kLdsPerCu / int(lds + 1024 + kWavesPerBlock * NST * 2 * Tile<D>::BYTES);
+    const int by_lds = kLdsPerCu / int(lds + 1024 + kWavesPerBlock * NST * Tile<D, false>::STAGE);
     if (by_lds < per_cu) per_cu = by_lds > 0 ? by_lds : 1;
     hipLaunchKernelGGL(kernel, dim3(device_cu_count() * per_cu), dim3(kBlockThreads), lds, st, a);
 }
@@ -556,9 +685,9 @@ void launch_shape(DecodeArgs& a, bool rows, size_t lds, hipStream_t st) {
         const int64_t pairs = int64_t(a.num_rows) * a.num_kv_heads;
         const dim3 grid{unsigned(pairs)};
         if (pairs <= device_cu_count())
-            hipLaunchKernelGGL((decode_rows_kernel<D, CT, 8, D == 64 ? 2 : 1>), grid, dim3(512), 0, st, a);
+            hipLaunchKernelGGL((decode_rows_kernel<D, CT, false, 8, D == 64 ? 2 : 1>), grid, dim3(512), 0, st, a);
         else
-            hipLaunchKernelGGL((decode_rows_kernel<D, CT, 4, D == 64 ? 2 : 1>), grid, dim3(256), 0, st, a);
+            hipLaunchKernelGGL((decode_rows_kernel<D, CT, false, 4, D == 64 ? 2 : 1>), grid, dim3(256), 0, st, a);
         return;
     }
     // (calls over thousands of rows leave LDS for one stage only)
@@ -601,6 +730,52 @@ bool stream_decode_rows(int num_rows, int num_kv_heads, int head_dim, int max_ct
     if (head_dim % 64 != 0) return max_ctx <= (pairs < 2 * cus ? 1056 : pairs < 8 * cus ? 528 : 264);
     const int64_t row_bytes = int64_t(max_ctx) * head_dim * 4;
     return max_ctx <= 2112 && (row_bytes <= 528 << 10 || (pairs >= cus && !matrix_split));
+}
+
+template <bool FP8, int NST>
+static void launch_parts(DecodeArgs& a, int64_t max_items, size_t lds, hipStream_t st) {
+    static std::atomic<int> cached{0};
+    auto kernel = decode_parts_kernel<128, 1, FP8, NST>;
+    const int cus = device_cu_count();
+    int per_cu = cached.load(std::memory_order_relaxed);
+    if (per_cu <= 0) {
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kBlockThreads, 0) != hipSuccess || per_cu <= 0) per_cu = 1;
+        cached.store(per_cu, std::memory_order_relaxed);
+    }
+    const int by_lds = kLdsPerCu / int(lds + 2048 + kWavesPerBlock * ((NST * Tile<128, FP8>::STAGE + 1023) / 1024 * 1024));
+    if (by_lds < per_cu) per_cu = by_lds > 0 ? by_lds : 1;
+    const int64_t groups = (max_items + kWavesPerBlock - 1) / kWavesPerBlock, wgs = int64_t(cus) * per_cu;
+    const int gx = int(groups < wgs ? (groups > 0 ? groups : 1) : wgs);
+    a.static_parts = 0;
+    a.wave_slots = gx * kWavesPerBlock;
+    a.level_waves = (gx < cus ? gx : cus) * kWavesPerBlock;
+    if (a.num_cands > 1) {
+        const int64_t worst = int64_t(a.num_rows) * ((int64_t(a.max_ctx) + a.P - 1) / a.P) * a.num_kv_heads;
+        if (worst <= a.level_waves) a.num_cands = 1;
+    }
+    hipLaunchKernelGGL(kernel, dim3(gx), dim3(kBlockThreads), lds, st, a);
+}
+
+// Rows of FP8 caches are half the bytes, as head_dim 64 in fp16.  One stage per
+// wave leaves room for two workgroups per CU in fp16 (two stages: one) and is
+// the faster for small FP8 groups; larger ones compute longer per step and keep
+// a second one in flight (us, one stage / two: 64 sequences of C2's lengths,
+// group 4, fp16 105.4 / 110.8; 256 long-tailed ones, group 4, FP8 312.4 / 317.0;
+// 120 of 1 024 to 8 192, group 7, FP8 132.2 / 125.3).
+bool launch_decode_matrix(DecodeArgs& a, bool fp8, int64_t max_items, size_t lds, hipStream_t st) {
+    if (fp8 && stream_decode_rows(a.num_rows, a.num_kv_heads, 64, a.max_ctx, true)) {
+        const int64_t pairs = int64_t(a.num_rows) * a.num_kv_heads;
+        const dim3 grid{unsigned(pairs)};
+        if (pairs <= device_cu_count())
+            hipLaunchKernelGGL((decode_rows_kernel<128, 1, true, 8, 1>), grid, dim3(512), 0, st, a);
+        else
+            hipLaunchKernelGGL((decode_rows_kernel<128, 1, true, 4, 2>), grid, dim3(256), 0, st, a);
+        return true;
+    }
+    if (!fp8) launch_parts<false, 1>(a, max_items, lds, st);
+    else if (a.num_heads / a.num_kv_heads <= 4) launch_parts<true, 1>(a, max_items, lds, st);
+    else launch_parts<true, 2>(a, max_items, lds, st);
+    return false;
 }
 
 int launch_decode_stream(DecodeArgs& a, bool rows, size_t lds, hipStream_t st) {
