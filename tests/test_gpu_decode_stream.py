@@ -131,3 +131,24 @@ def test_stream_fp8_edges_vs_oracle(vkv, oracle, cuda, H, Hkv, bs, table):
                      value_scales=to_dev(scales[1], cuda))
     torch.cuda.synchronize()
     assert_close(to_np(out).astype(np.float32), ref, F16_ATOL, F16_RTOL, f"FP8 {H}/{Hkv}/bs{bs}")
+
+
+@pytest.mark.parametrize("table", [1024, 6000], ids=["rows", "slices"])
+@pytest.mark.parametrize("H,Hkv,bs", [(14, 2, 16), (34, 2, 24), (4, 4, 1), (64, 2, 32)])
+def test_stream_fp32_edges_vs_oracle(vkv, oracle, cuda, H, Hkv, bs, table):
+    """All in fp32 at head_dim 64 (fp32 bounds: weights, sums and products stay fp32)."""
+    import torch
+    from helpers import F32_ATOL, F32_RTOL
+    D = 64
+    rng = np.random.default_rng(H + bs)
+    lay, (k, v), q = _case(rng, H, Hkv, D, bs, CONTEXTS, table)
+    # (full fp32 mantissas; the unattended slots stay NaN)
+    k, v, q = ((x.astype(np.float32) * np.float32(1.0001)) for x in (k, v, q))
+    scale = -float(D) ** -0.5 if bs == 24 else float(D) ** -0.5
+    ref = oracle.paged_decode(q, np.nan_to_num(k), np.nan_to_num(v), lay.block_tables, lay.context_lens, scale)
+    for size in (0, 64):
+        out = torch.full((len(CONTEXTS), H, D), 7.0, dtype=torch.float32, device=cuda)
+        vkv.paged_decode(out, to_dev(q, cuda), to_dev(k, cuda), to_dev(v, cuda), to_dev(lay.block_tables, cuda),
+                         to_dev(lay.context_lens, cuda), scale, partition_size=size)
+        torch.cuda.synchronize()
+        assert_close(to_np(out), ref, F32_ATOL, F32_RTOL, f"fp32 {H}/{Hkv}/bs{bs} size {size}")

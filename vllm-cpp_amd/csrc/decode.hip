@@ -569,8 +569,9 @@ constexpr int mfma_enabled() { return VKV_DECODE_MFMA; }
 
 template <typename IO, int KVT, int D, int G>
 void launch_g(DecodeArgs& args, int grid_x, int grid_y, int grid_z, size_t lds, hipStream_t st) {
-    // (fp16 over fp16 at head_dim 64 and 128 runs on decode_stream.hip)
-    constexpr bool kStreamed = mfma_enabled() && std::is_same<IO, _Float16>::value && KVT == kF16 && D <= 128;
+    // (fp16 over fp16 at head_dim 64 and 128, and all-fp32 at 64, run on decode_stream.hip)
+    constexpr bool kStreamed = mfma_enabled() && (std::is_same<IO, _Float16>::value ? KVT == kF16 && D <= 128
+                                                                                    : KVT == kF32 && D == 64);
     // grid_x arrives as the number of item groups (an upper bound).  One workgroup per resident slot: the variant's workgroups per CU by
     // registers (queried once per variant), bounded by the LDS the rows'
     // prefix takes, and never more than there are item groups.  Groups
@@ -675,9 +676,14 @@ __global__ __launch_bounds__(kWave) void decode_reduce_wave_kernel(DecodeArgs a)
     const float* ml = a.part_ml + slot0 * 2;
     const float* o = a.part_o + slot0 * DT + d;
     if (a.qsl && a.qsl[s + 1] - a.qsl[s] != 1) return;
-    const int ctx = row_context(a, s);
-    const int P = a.num_cands > 1 && !a.row_parts ? __builtin_amdgcn_readfirstlane(a.counters[kChosenPartitionSlot]) : a.P;
-    const int np = a.row_parts ? a.row_parts[s] : ctx > 0 ? (ctx + P - 1) / P : 0;
+    int np;
+    if (a.row_parts) {
+        np = a.row_parts[s];
+    } else {
+        const int ctx = row_context(a, s);
+        const int P = a.num_cands > 1 ? __builtin_amdgcn_readfirstlane(a.counters[kChosenPartitionSlot]) : a.P;
+        np = ctx > 0 ? (ctx + P - 1) / P : 0;
+    }
     // partials of batch i0 (slots past np are neither loaded nor read)
     float bm[B], bl[B];
     fE bo[B];
@@ -742,6 +748,8 @@ int launch_reduce_b(int D, const DecodeArgs& args, int H, int S, hipStream_t st)
 
 template <typename IO>
 int launch_reduce(int D, const DecodeArgs& args, int H, int S, hipStream_t st) {
+    // Few rows cut into many slices: more of a row's partials per round.
+    if (args.row_parts && D == 64 && args.max_parts > 16 && H * S <= 2048) return launch_reduce_b<IO, 32>(D, args, H, S, st);
     // Small (static) calls split finely load every partial in one round;
     // the others keep batches of 8 (their rows have few partitions, and
     // wider batches measured slower at C2's batch).
@@ -753,7 +761,13 @@ int launch_reduce(int D, const DecodeArgs& args, int H, int S, hipStream_t st) {
 
 bool stream_shape(const vkv_decode_params* p) {
     return mfma_enabled() && stream_decode_shape(p->head_dim, p->num_heads / p->num_kv_heads, p->key_cache, p->value_cache,
-                                                 p->io_dtype == VKV_DTYPE_F16, p->kv_dtype == VKV_DTYPE_F16);
+                                                 p->io_dtype, p->kv_dtype);
+}
+
+// fp16 queries over fp16 or FP8 caches in a matrix_split_shape.
+bool split_in_partitions(const vkv_decode_params* p) {
+    return mfma_enabled() && p->io_dtype == VKV_DTYPE_F16 && p->kv_dtype != VKV_DTYPE_F32 &&
+           matrix_split_shape(p->head_dim, p->num_heads / p->num_kv_heads, p->block_size, p->key_cache, p->value_cache);
 }
 
 int ilog2(int x) {
@@ -831,7 +845,7 @@ DecodePlan plan_decode(const vkv_decode_params* p) {
     plan.base_bytes = plan.workspace_bytes = kWorkspaceHeader + part_bytes * plan.max_parts;
     plan.whole_rows = false;
     plan.stream = stream_shape(p);
-    if (plan.stream && !matrix_split_shape(p->head_dim, p->num_heads / p->num_kv_heads, bs, p->key_cache, p->value_cache)) {
+    if (plan.stream && !split_in_partitions(p)) {
         // Equal slices (decode_stream.hip): partials for slices of down to
         // kSliceTokens tokens, at most kMaxSplitParts of a row and one more (a
         // row's first and last slice are shared with its neighbours).  A
@@ -919,11 +933,10 @@ int launch_rows(const vkv_decode_params* p, const DecodePlan& plan, void* worksp
     const int D = p->head_dim;
     const int io_eb = p->io_dtype == VKV_DTYPE_F32 ? 4 : 2;
     const bool fixed = fixed_decode_shape(D, G, p->block_size, p->key_cache, p->value_cache);
-    const bool split_streams = plan.stream && !matrix_split_shape(D, G, p->block_size, p->key_cache, p->value_cache);
+    const bool split_streams = plan.stream && !split_in_partitions(p);
     a.row_parts = split_streams ? reinterpret_cast<int32_t*>(a.part_ml + size_t(rows) * p->num_heads * plan.max_parts * 2)
                                 : nullptr;
-    const bool matrix = mfma_enabled() && p->io_dtype == VKV_DTYPE_F16 && p->kv_dtype != VKV_DTYPE_F32 &&
-                        matrix_split_shape(D, G, p->block_size, p->key_cache, p->value_cache);
+    const bool matrix = split_in_partitions(p);
     a.head_dim = D;
     a.block_size = p->block_size;
     set_block_div(a, p->block_size);
@@ -940,7 +953,7 @@ int launch_rows(const vkv_decode_params* p, const DecodePlan& plan, void* worksp
         const int n = p->num_seqs - r0 < kMaxRowsPerLaunch ? p->num_seqs - r0 : kMaxRowsPerLaunch;
         DecodeArgs c = a;
         c.num_rows = n;
-        const bool whole_rows = plan.stream && (plan.whole_rows || stream_decode_rows(n, p->num_kv_heads, D, c.max_ctx, !split_streams));
+        const bool whole_rows = plan.stream && (plan.whole_rows || stream_decode_rows(n, p->num_kv_heads, io_eb == 4 ? 2 * D : D, c.max_ctx, !split_streams));
         const bool streamed = whole_rows || split_streams;
         // Small plain decode calls (at most one (row, kv head) pair per CU):
         // a static grid over the partitions of the default size, if its waves
@@ -979,8 +992,9 @@ int launch_rows(const vkv_decode_params* p, const DecodePlan& plan, void* worksp
         const size_t lds = (size_t(n) + 1) * sizeof(int) + lpt_lds_bytes(n);
         int rc;
         if (streamed) {
-            rc = launch_decode_stream(c, whole_rows, (size_t(n) + 1) * sizeof(int), st);
-            if (!rc && !whole_rows) rc = launch_reduce<_Float16>(D, c, p->num_heads, n, st);
+            rc = launch_decode_stream(c, io_eb == 4, whole_rows, (size_t(n) + 1) * sizeof(int), st);
+            if (!rc && !whole_rows) rc = io_eb == 4 ? launch_reduce<float>(D, c, p->num_heads, n, st)
+                                                    : launch_reduce<_Float16>(D, c, p->num_heads, n, st);
         } else if (matrix) {
             rc = 0;
             if (!launch_decode_matrix(c, p->kv_dtype == VKV_DTYPE_FP8_E4M3, max_items, lds, st))

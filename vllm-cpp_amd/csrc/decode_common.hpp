@@ -128,23 +128,27 @@ inline bool fixed_decode_shape(int head_dim, int group, int block_size, const vo
 }
 
 // The shapes of decode_stream.hip: fp16 queries over fp16 caches at these head
-// dimensions, groups of up to 32 heads and any block size.  Split-K calls at
-// head_dim 128, groups of up to 8 and power-of-two blocks of 16 tokens and more
-// (matrix_split_shape; FP8 caches too) run in partitions of the size that
-// run_partitions picks, the others in equal slices.
-inline bool stream_decode_shape(int head_dim, int group, const void* kc, const void* vc, bool f16_io, bool f16_kv) {
+// dimensions, or all in fp32 at head_dim 64; groups of up to 32 heads and any
+// block size.  Split-K calls in fp16 at head_dim 128, groups of up to 8 and
+// power-of-two blocks of 16 tokens and more (matrix_split_shape; FP8 caches too)
+// run in partitions of the size that run_partitions picks, the others in equal
+// slices.
+inline bool stream_decode_shape(int head_dim, int group, const void* kc, const void* vc, int io_dtype, int kv_dtype) {
     const bool aligned = ((reinterpret_cast<uintptr_t>(kc) | reinterpret_cast<uintptr_t>(vc)) & 15u) == 0;
-    return f16_io && f16_kv && aligned && head_dim >= 64 && head_dim <= 128 && head_dim % 16 == 0 && group >= 1 &&
+    const bool f16 = io_dtype == VKV_DTYPE_F16 && kv_dtype == VKV_DTYPE_F16;
+    const bool f32 = io_dtype == VKV_DTYPE_F32 && kv_dtype == VKV_DTYPE_F32 && head_dim == 64;
+    return (f16 || f32) && aligned && head_dim >= 64 && head_dim <= 128 && head_dim % 16 == 0 && group >= 1 &&
            group <= 32;
 }
 inline bool matrix_split_shape(int head_dim, int group, int block_size, const void* kc, const void* vc) {
     return head_dim == 128 && block_size >= 16 && fixed_decode_shape(head_dim, group, block_size, kc, vc);
 }
 // Whether a launch of num_rows rows runs as one workgroup per (row, kv head),
-// merged in LDS, instead of split-K.
-bool stream_decode_rows(int num_rows, int num_kv_heads, int head_dim, int max_ctx, bool matrix_split);
+// merged in LDS, instead of split-K.  half_dims: a head's row in fp16 elements'
+// bytes (head_dim; twice that in fp32, half in FP8).
+bool stream_decode_rows(int num_rows, int num_kv_heads, int half_dims, int max_ctx, bool matrix_split);
 // The call's partition launch (or, with rows, its only launch).  0 or VKV_ERR_*.
-int launch_decode_stream(DecodeArgs& a, bool rows, size_t lds, hipStream_t st);
+int launch_decode_stream(DecodeArgs& a, bool f32, bool rows, size_t lds, hipStream_t st);
 
 // The partition launch of a matrix_split_shape call (fp16 queries over an fp16
 // or FP8 cache); true if it wrote the output itself instead of partials.

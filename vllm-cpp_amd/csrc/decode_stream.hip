@@ -1,8 +1,9 @@
 // decode_stream.hip — paged decode attention for fp16 queries over fp16 caches
 // at head_dim 64, 80, 96, 112 or 128 with groups of up to 32 query heads, and
 // over FP8 caches at head_dim 128 with groups of up to 8, both products on the
-// matrix cores (gfx950).  Semantics as in decode.hip (the reference's
-// src/attention/paged_attention.cu:13-82).
+// matrix cores (gfx950); and all in fp32 at head_dim 64, groups of up to 32.
+// Semantics as in decode.hip (the reference's src/attention/
+// paged_attention.cu:13-82).
 //
 // A wave streams the K and V rows of its tokens through LDS, 32 tokens a step,
 // with direct global->LDS loads (global_load_lds_dwordx4, 1 KiB per wave
@@ -13,8 +14,7 @@
 //                 an odd multiple of 16): A = K rows from LDS, B = Q in
 //                 registers (columns = the group's heads, 16 per tile);
 //   softmax       lane-local on the S^T layout (lane l: head l % 16, keys
-//                 4 (l / 16) + e of each 16-key half), the running max raised
-//                 lazily (only when a score passes it by 2^8);
+//                 4 (l / 16) + e of each 16-key half);
 //   O^T += V^T P^T  A = V^T by ds_read_b64_tr_b16 from the row-major tile,
 //                 B = P^T straight from the S^T registers, so the weights
 //                 never leave the lane and the accumulators are head_dim / 4
@@ -22,6 +22,9 @@
 // FP8: codes become fp16 exactly (v_cvt_scalef32_pk_f16_fp8, scale 1) as they
 // are read from LDS, V^T by ds_read_b64_tr_b8; the token's K scale multiplies
 // the logit, its V scale the weight.
+// fp32: v_mfma_f32_16x16x4_f32 for both products, its k slots chosen so that a
+// lane's 16 bytes of a row feed four of them and the weights stay in place;
+// weights and sums in fp32.
 // Before: the VALU kernels of head_dim 64 and the generic shapes spent ~300
 // instructions per 16 tokens and held 4 KiB of loads per wave, waited for in
 // turn; head_dim 128's kernel ran P V on the VALU (packed dot products, 16 G
@@ -44,16 +47,17 @@ typedef float float4_t __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kStep = 32;            // tokens per step (the k of the P V products)
-constexpr float kLazyLog2 = 8.0f;    // the running max is raised when passed by 2^8
 
 // LDS tile of a step's K (or V) rows: row-major, unpadded (a direct load
 // writes lane L's 16 bytes at 16 L).  Where a row is a power of two of 16-byte
 // chunks, chunk c of row r sits at slot c ^ key(r): the operand reads take one
 // chunk column of 16 rows, which would otherwise meet in the same banks.
 // (Rows of 160, 192 or 224 bytes are spread by their own stride.)
-template <int D, bool FP8>
+template <int D, int KVT>
 struct Tile {
-    static constexpr int ROW = FP8 ? D : 2 * D;
+    static constexpr bool FP8 = KVT == kFp8;
+    static constexpr bool F32 = KVT == kF32;
+    static constexpr int ROW = D * KvTraits<KVT>::bytes;
     static constexpr int CH = ROW / 16;
     static constexpr int NI = kStep * CH / 64;  // direct loads per tile
     static constexpr int BYTES = kStep * ROW;
@@ -65,6 +69,7 @@ struct Tile {
     static constexpr int DT = D / 16;       // dim tiles of O^T
     static_assert(D % 16 == 0 && kStep * CH % 64 == 0, "whole loads");
     static_assert(!FP8 || (SWZ && KS % 2 == 0), "FP8 operands are pairs of 8 codes of one chunk");
+    static_assert(!F32 || D == 64, "the fp32 dim tiles hold dims 4 m + t, m < 16");
     __device__ static __forceinline__ int slot(int row, int chunk) {
         return SWZ ? chunk ^ (row / (16 / (SWZ ? CH : 16)) % CH) : chunk;
     }
@@ -125,37 +130,53 @@ __device__ __forceinline__ half8_t codes8(const uint32_t lo, const uint32_t hi) 
 }
 
 // Attention state of one wave: CT tiles of 16 heads.
-template <int D, int CT, bool FP8>
+template <int D, int CT, int KVT>
 struct State {
-    using T = Tile<D, FP8>;
-    half8_t q[CT][T::KS];
+    using T = Tile<D, KVT>;
+    half8_t q[CT][T::F32 ? 1 : T::KS];
     half4_t qh[CT];
+    float4_t qf[CT][T::F32 ? D / 16 : 1];
     float m[CT];              // running max of head 16 ct + l % 16, raw logits
-    float4_t l[CT];           // weight sums (every element the same; FP8: element 0, this lane's keys)
+    float4_t l[CT];           // weight sums (every element the same; FP8, fp32: element 0, this lane's keys)
     float4_t o[CT][T::DT];    // O^T: lane l holds dims 16 t + 4 (l / 16) + e of head l % 16
+                              // (fp32: dims 16 (l / 16) + 4 e + t)
+    // Four consecutive dims of head 16 c + l % 16, from dim() on.
+    __device__ __forceinline__ float4_t out4(const int c, const int i) const {
+        if constexpr (T::F32) return float4_t{o[c][0][i], o[c][1][i], o[c][2][i], o[c][3][i]};
+        else return o[c][i];
+    }
+    __device__ static __forceinline__ int dim(const int i, const int grp) {
+        return T::F32 ? 16 * grp + 4 * i : 16 * i + 4 * grp;
+    }
 };
 
 // Q as the B operand and an empty state.  Columns past the group read head 0
 // and are zeroed; a negative scale is moved into Q (exact sign flip).
-template <int D, int CT, bool FP8>
-__device__ __forceinline__ void init_state(const DecodeArgs& a, State<D, CT, FP8>& st, const int s, const int kvh,
+template <int D, int CT, int KVT>
+__device__ __forceinline__ void init_state(const DecodeArgs& a, State<D, CT, KVT>& st, const int s, const int kvh,
                                            const int G, const int lane) {
-    using T = Tile<D, FP8>;
+    using T = Tile<D, KVT>;
     const int col = lane & 15, grp = lane >> 4;
-    const uint32_t flip = a.scale_log2 < 0.0f ? 0x80008000u : 0u;
+    const uint32_t flip = a.scale_log2 < 0.0f ? (T::F32 ? 0x80000000u : 0x80008000u) : 0u;
 #pragma unroll
     for (int c = 0; c < CT; ++c) {
         const int h = 16 * c + col;
         const uint32_t keep = h < G ? 0xFFFFFFFFu : 0u;
         const char* qrow = static_cast<const char*>(a.q) +
-                           (query_row(a, s) * a.q_stride + int64_t(kvh * G + (h < G ? h : 0)) * D) * 2;
+                           (query_row(a, s) * a.q_stride + int64_t(kvh * G + (h < G ? h : 0)) * D) * (T::F32 ? 4 : 2);
 #pragma unroll
-        for (int i = 0; i < T::KS; ++i) {
+        for (int i = 0; i < (T::F32 ? D / 16 : 0); ++i) {
+            u32x4 w = load16(qrow + (16 * i + 4 * grp) * 4);
+            w = (w ^ u32x4{flip, flip, flip, flip}) & u32x4{keep, keep, keep, keep};
+            st.qf[c][i] = __builtin_bit_cast(float4_t, w);
+        }
+#pragma unroll
+        for (int i = 0; i < (T::F32 ? 0 : T::KS); ++i) {
             u32x4 w = load16(qrow + T::dim(i, grp) * 2);
             w = (w ^ u32x4{flip, flip, flip, flip}) & u32x4{keep, keep, keep, keep};
             st.q[c][i] = __builtin_bit_cast(half8_t, w);
         }
-        if constexpr (T::HALF) {
+        if constexpr (T::HALF && !T::F32) {
             u32x2 w = *reinterpret_cast<const u32x2*>(qrow + (32 * T::KS + 4 * grp) * 2);
             w = (w ^ u32x2{flip, flip}) & u32x2{keep, keep};
             st.qh[c] = __builtin_bit_cast(half4_t, w);
@@ -170,18 +191,17 @@ __device__ __forceinline__ void init_state(const DecodeArgs& a, State<D, CT, FP8
 // Attends tokens [t0, t0 + n) (n >= 1) of row s at kv head kvh.  ring: NST
 // stages of a K and a V tile, this wave's own.  my_block: block ids of
 // [win, win + 64) in the row's table, one per lane (0 where out of the pool).
-template <int D, int CT, bool FP8, int NST>
-__device__ __forceinline__ void stream_tokens(const DecodeArgs& a, State<D, CT, FP8>& st, char* ring, const int s,
+template <int D, int CT, int KVT, int NST>
+__device__ __forceinline__ void stream_tokens(const DecodeArgs& a, State<D, CT, KVT>& st, char* ring, const int s,
                                               const int32_t* table, const int ctx, const int kvh, const int t0,
                                               const int n, int win, int my_block, const int lane) {
-    using T = Tile<D, FP8>;
+    using T = Tile<D, KVT>;
+    constexpr bool FP8 = T::FP8;
     constexpr int kStage = T::STAGE;
     const int col = lane & 15, grp = lane >> 4;
     const uint32_t slot_stride = uint32_t(a.num_kv_heads) * T::ROW;
     const uint32_t ring_lds = lds_addr(ring);
     const float sc = a.scale_log2 < 0.0f ? -a.scale_log2 : a.scale_log2;
-    // (FP8 weights carry their token's scale: they stay at most 1 before it)
-    const float lazy = FP8 ? 0.0f : kLazyLog2 / sc;
     const int steps = (n + kStep - 1) / kStep;
     // The fused append: the row's last position reads the new token's rows
     // when the append targets that position's slot.
@@ -245,7 +265,27 @@ __device__ __forceinline__ void stream_tokens(const DecodeArgs& a, State<D, CT, 
         for (int c = 0; c < CT; ++c) sv[c][0] = sv[c][1] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int hh = 0; hh < 2; ++hh) {
-            if constexpr (FP8) {
+            if constexpr (T::F32) {
+                // v_mfma_f32_16x16x4_f32: lane (col, grp) holds one k slot, dim
+                // 16 i + 4 grp + e of product (i, e).  Each 16 dims a sum of
+                // their own, added in pairs: one chain over the 64 dims (and
+                // one over all tokens below) doubled the error against 64 bits
+                // of the lane-wise sums of the VALU kernel.
+                float4_t part[CT][D / 16];
+#pragma unroll
+                for (int i = 0; i < D / 16; ++i) {
+                    const float4_t k = __builtin_bit_cast(float4_t, load16(kb + T::off(16 * hh + col, 4 * i + grp)));
+#pragma unroll
+                    for (int c = 0; c < CT; ++c) part[c][i] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+#pragma unroll
+                        for (int c = 0; c < CT; ++c)
+                            part[c][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(k[e], st.qf[c][i][e], part[c][i], 0, 0, 0);
+                }
+#pragma unroll
+                for (int c = 0; c < CT; ++c) sv[c][hh] = (part[c][0] + part[c][1]) + (part[c][2] + part[c][3]);
+            } else if constexpr (FP8) {
 #pragma unroll
                 for (int j = 0; j < T::KS / 2; ++j) {
                     const u32x4 w = load16(kb + T::off(16 * hh + col, grp * (T::KS / 2) + j));
@@ -264,7 +304,7 @@ __device__ __forceinline__ void stream_tokens(const DecodeArgs& a, State<D, CT, 
                         sv[c][hh] = __builtin_amdgcn_mfma_f32_16x16x32_f16(k, st.q[c][i], sv[c][hh], 0, 0, 0);
                 }
             }
-            if constexpr (T::HALF) {
+            if constexpr (T::HALF && !T::F32) {
                 // A product of its own, added on the VALU: accumulated onto the
                 // 16x16x32 result right behind it (no wait state between the
                 // two shapes in the compiler's code), head_dim 112 gave wrong
@@ -298,6 +338,7 @@ __device__ __forceinline__ void stream_tokens(const DecodeArgs& a, State<D, CT, 
             }
         }
         half8_t p[CT];
+        [[maybe_unused]] float pf[CT][8];
 #pragma unroll
         for (int c = 0; c < CT; ++c) {
             float x[8];
@@ -309,9 +350,10 @@ __device__ __forceinline__ void stream_tokens(const DecodeArgs& a, State<D, CT, 
                     if (step * kStep + 16 * (e >> 2) + 4 * grp + (e & 3) >= n) x[e] = -INFINITY;
             }
             const float mx = fmaxf(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])), fmaxf(fmaxf(x[4], x[5]), fmaxf(x[6], x[7])));
-            // Below m + lazy the weights stay under 2^8, exact enough in fp16
-            // as any others; the first step always sets m.
-            if (__builtin_amdgcn_ballot_w64(mx > st.m[c] + lazy)) {
+            // The running max follows every score that passes it, so that weights
+            // are at most 1 (letting it lag by 2^8 is no faster here, and its
+            // weights round more: error against 64 bits 2.9e-4 for 2.7e-4).
+            if (__builtin_amdgcn_ballot_w64(mx > st.m[c])) {
                 const float mn = fmaxf(st.m[c], xor_max<32>(xor_max<16>(mx)));
                 const float alpha = mn > st.m[c] ? __builtin_amdgcn_exp2f((st.m[c] - mn) * sc) : 1.0f;
                 st.m[c] = mn;
@@ -320,7 +362,11 @@ __device__ __forceinline__ void stream_tokens(const DecodeArgs& a, State<D, CT, 
                 for (int t = 0; t < T::DT; ++t) st.o[c][t] *= alpha;
             }
             const float msc = st.m[c] == -INFINITY ? 0.0f : st.m[c] * sc;
-if constexpr (FP8) {
+            if constexpr (T::F32) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) pf[c][e] = __builtin_amdgcn_exp2f(fmaf(x[e], sc, -msc));
+                st.l[c][0] += ((pf[c][0] + pf[c][1]) + (pf[c][2] + pf[c][3])) + ((pf[c][4] + pf[c][5]) + (pf[c][6] + pf[c][7]));
+            } else if constexpr (FP8) {
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
                     const float w = __builtin_amdgcn_exp2f(fmaf(x[e], sc, -msc));
@@ -339,6 +385,35 @@ if constexpr (FP8) {
         // element i % 4 of the 8-byte chunks addressed by lanes i / 4 + 4 e, so
         // lane (col, grp) addresses key 4 grp + col / 4 (+ 16), dims 16 t + 4
         // (col % 4).  FP8 (tr_read8): the key of slot col / 2, dims 16 t + 8 (col % 2).
+        if constexpr (T::F32) {
+            // product (hh, e): the k slot of lane (col, grp) is key 16 hh + 4 grp
+            // + e, whose weight it holds; dims 4 col + t of that key's row.  Each
+            // half's sum of its own, added to the running sums.
+            float4_t part[CT][2][T::DT];
+#pragma unroll
+            for (int c = 0; c < CT; ++c)
+#pragma unroll
+                for (int hh = 0; hh < 2; ++hh)
+#pragma unroll
+                    for (int t = 0; t < T::DT; ++t) part[c][hh][t] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int hh = 0; hh < 2; ++hh) {
+                    const float4_t v = __builtin_bit_cast(float4_t, load16(vb + T::off(16 * hh + 4 * grp + e, col)));
+#pragma unroll
+                    for (int t = 0; t < T::DT; ++t)
+#pragma unroll
+                        for (int c = 0; c < CT; ++c)
+                            part[c][hh][t] =
+                                __builtin_amdgcn_mfma_f32_16x16x4f32(v[t], pf[c][4 * hh + e], part[c][hh][t], 0, 0, 0);
+                }
+#pragma unroll
+            for (int c = 0; c < CT; ++c)
+#pragma unroll
+                for (int t = 0; t < T::DT; ++t) st.o[c][t] += part[c][0][t] + part[c][1][t];
+            return;
+        }
         const int vrow = FP8 ? (col < 8 ? 4 * grp + (col >> 1) : 12 + 4 * grp + (col >> 1)) : 4 * grp + (col >> 2);
 #pragma unroll
         for (int t = 0; t < T::DT; ++t) {
@@ -379,7 +454,7 @@ if constexpr (FP8) {
             compute(step, step & 1);
         }
     }
-    if constexpr (FP8) {
+    if constexpr (FP8 || T::F32) {
 #pragma unroll
         for (int c = 0; c < CT; ++c) st.l[c][0] = xor_add<32>(xor_add<16>(st.l[c][0]));
     }
@@ -398,9 +473,10 @@ __device__ __forceinline__ int load_block(const DecodeArgs& a, const int32_t* ta
 // A workgroup of W waves per (row, kv head): each wave attends a contiguous
 // share of the context and the shares are merged in LDS, so the call is one
 // launch with no workspace.
-template <int D, int CT, bool FP8, int W, int NST>
+template <int D, int CT, int KVT, int W, int NST>
 __global__ __launch_bounds__(64 * W) void decode_rows_kernel(const DecodeArgs a) {
-    using T = Tile<D, FP8>;
+    using T = Tile<D, KVT>;
+    using IO = typename std::conditional<T::F32, float, _Float16>::type;
     constexpr int kRing = (NST * T::STAGE + 1023) / 1024 * 1024;
     constexpr int kMergeBytes = W * 16 * CT * (D + 2) * 4;
     __shared__ __attribute__((aligned(1024))) char lds[W * kRing > kMergeBytes ? W * kRing : kMergeBytes];
@@ -422,7 +498,7 @@ __global__ __launch_bounds__(64 * W) void decode_rows_kernel(const DecodeArgs a)
     // the table fits one id per lane
     const bool whole = a.max_blocks_per_seq <= kWave;
     int ids = whole ? load_block(a, table, lane) : 0;
-    State<D, CT, FP8> st;
+    State<D, CT, KVT> st;
     init_state(a, st, s, kvh, G, lane);
     const int ctx = row_context(a, s);
     const int per = ((ctx + W - 1) / W + kStep - 1) / kStep * kStep;
@@ -434,7 +510,7 @@ __global__ __launch_bounds__(64 * W) void decode_rows_kernel(const DecodeArgs a)
             win = block_div(a, t0);
             ids = load_block(a, table, win + lane);
         }
-        stream_tokens<D, CT, FP8, NST>(a, st, lds + wave * kRing, s, table, ctx, kvh, t0, n, win, ids, lane);
+        stream_tokens<D, CT, KVT, NST>(a, st, lds + wave * kRing, s, table, ctx, kvh, t0, n, win, ids, lane);
     }
     // ---------------- merge
     const float sc = a.scale_log2 < 0.0f ? -a.scale_log2 : a.scale_log2;
@@ -449,7 +525,7 @@ __global__ __launch_bounds__(64 * W) void decode_rows_kernel(const DecodeArgs a)
             if (h >= G) continue;
             float* row = mo + (wave * 16 * CT + h) * D;
 #pragma unroll
-            for (int t = 0; t < T::DT; ++t) *reinterpret_cast<float4_t*>(row + 16 * t + 4 * grp) = st.o[c][t];
+            for (int t = 0; t < T::DT; ++t) *reinterpret_cast<float4_t*>(row + st.dim(t, grp)) = st.out4(c, t);
             if (grp == 0) {
                 mml[(wave * 16 * CT + h) * 2] = st.m[c] * sc;
                 mml[(wave * 16 * CT + h) * 2 + 1] = st.l[c][0];
@@ -460,7 +536,7 @@ __global__ __launch_bounds__(64 * W) void decode_rows_kernel(const DecodeArgs a)
         mml[(wave * 16 * CT + lane) * 2 + 1] = 0.0f;
     }
     __syncthreads();
-    _Float16* out = static_cast<_Float16*>(a.out) + (query_row(a, s) * a.num_heads + kvh * G) * D;
+    IO* out = static_cast<IO*>(a.out) + (query_row(a, s) * a.num_heads + kvh * G) * D;
     const int shares = ctx > 0 ? (ctx + per - 1) / per : 0;
     for (int i = threadIdx.x; i < G * (D / 2); i += 64 * W) {
         const int h = i / (D / 2), d = (i - h * (D / 2)) * 2;
@@ -479,13 +555,13 @@ __global__ __launch_bounds__(64 * W) void decode_rows_kernel(const DecodeArgs a)
             }
         }
         float r0 = shares > 0 ? x0 / l : 0.0f, r1 = shares > 0 ? x1 / l : 0.0f;
-        _Float16* o = out + h * D + d;
+        IO* o = out + h * D + d;
         if (a.accumulate) {
             r0 += static_cast<float>(o[0]);
             r1 += static_cast<float>(o[1]);
         }
-        o[0] = static_cast<_Float16>(r0);
-        o[1] = static_cast<_Float16>(r1);
+        o[0] = static_cast<IO>(r0);
+        o[1] = static_cast<IO>(r1);
     }
     // Fused append: this workgroup alone reads the new token's slot at this kv
     // head, and has.
@@ -518,10 +594,9 @@ constexpr int kMinSliceSteps = 2;
 #define VKV_STREAM_ROWS 0
 #endif
 
-template <int D, int CT, int NST>
+template <int D, int CT, int KVT, int NST>
 __global__ __launch_bounds__(256) void decode_stream_kernel(const DecodeArgs a) {
-    constexpr bool FP8 = false;
-    using T = Tile<D, FP8>;
+    using T = Tile<D, KVT>;
     constexpr int kRing = NST * T::STAGE;
     __shared__ __attribute__((aligned(1024))) char lds[kWavesPerBlock * kRing];
     __shared__ int wave_total[kWavesPerBlock], wave_longest[kWavesPerBlock];
@@ -603,9 +678,9 @@ __global__ __launch_bounds__(256) void decode_stream_kernel(const DecodeArgs a) 
             const int n = min(ctx - t0, (e - at) * kStep);
             const int win = block_div(a, t0);
             const int ids = load_block(a, table, win + lane);
-            State<D, CT, FP8> st;
+            State<D, CT, KVT> st;
             init_state(a, st, s, kvh, G, lane);
-            stream_tokens<D, CT, FP8, NST>(a, st, lds + wave * kRing, s, table, ctx, kvh, t0, n, win, ids, lane);
+            stream_tokens<D, CT, KVT, NST>(a, st, lds + wave * kRing, s, table, ctx, kvh, t0, n, win, ids, lane);
             const int64_t slot = (int64_t(s) * a.num_kv_heads + kvh) * a.max_parts + (slice - b / R);
 #pragma unroll
             for (int c = 0; c < CT; ++c) {
@@ -613,7 +688,7 @@ __global__ __launch_bounds__(256) void decode_stream_kernel(const DecodeArgs a) 
                 if (h >= G) continue;
                 float* row = a.part_o + (slot * G + h) * D;
 #pragma unroll
-                for (int t = 0; t < T::DT; ++t) *reinterpret_cast<float4_t*>(row + 16 * t + 4 * grp) = st.o[c][t];
+                for (int t = 0; t < T::DT; ++t) *reinterpret_cast<float4_t*>(row + st.dim(t, grp)) = st.out4(c, t);
                 if (grp == 0) {
                     a.part_ml[(slot * G + h) * 2] = st.m[c] * sc;
                     a.part_ml[(slot * G + h) * 2 + 1] = st.l[c][0];
@@ -625,9 +700,9 @@ __global__ __launch_bounds__(256) void decode_stream_kernel(const DecodeArgs a) 
 }
 
 // Split-K in partitions of a fixed size (decode.hip's items and size choice).
-template <int D, int CT, bool FP8, int NST>
+template <int D, int CT, int KVT, int NST>
 __global__ __launch_bounds__(256) void decode_parts_kernel(const DecodeArgs a) {
-    using T = Tile<D, FP8>;
+    using T = Tile<D, KVT>;
     constexpr int kRing = (NST * T::STAGE + 1023) / 1024 * 1024;
     __shared__ __attribute__((aligned(1024))) char lds[kWavesPerBlock * kRing];
     const int lane = threadIdx.x & (kWave - 1);
@@ -643,9 +718,9 @@ __global__ __launch_bounds__(256) void decode_parts_kernel(const DecodeArgs a) {
         const int n = min(ctx - t0, P);
         const int win = block_div(a, t0);
         const int ids = load_block(a, table, win + lane);
-        State<D, CT, FP8> st;
+        State<D, CT, KVT> st;
         init_state(a, st, s, kvh, G, lane);
-        stream_tokens<D, CT, FP8, NST>(a, st, lds + wave * kRing, s, table, ctx, kvh, t0, n, win, ids, lane);
+        stream_tokens<D, CT, KVT, NST>(a, st, lds + wave * kRing, s, table, ctx, kvh, t0, n, win, ids, lane);
         const float sc = a.scale_log2 < 0.0f ? -a.scale_log2 : a.scale_log2;
         const int col = lane & 15, grp = lane >> 4;
 #pragma unroll
@@ -655,7 +730,7 @@ __global__ __launch_bounds__(256) void decode_parts_kernel(const DecodeArgs a) {
             const int64_t item = ((int64_t(s) * a.num_kv_heads + kvh) * a.max_parts + part) * G + h;
             float* row = a.part_o + item * D;
 #pragma unroll
-            for (int t = 0; t < T::DT; ++t) *reinterpret_cast<float4_t*>(row + 16 * t + 4 * grp) = st.o[c][t];
+            for (int t = 0; t < T::DT; ++t) *reinterpret_cast<float4_t*>(row + st.dim(t, grp)) = st.out4(c, t);
             if (grp == 0) {
                 a.part_ml[item * 2] = st.m[c] * sc;
                 a.part_ml[item * 2 + 1] = st.l[c][0];
@@ -665,45 +740,53 @@ __global__ __launch_bounds__(256) void decode_parts_kernel(const DecodeArgs a) {
 }
 
 // One workgroup per resident slot (occupancy queried once per variant).
-template <int D, int CT, int NST>
+template <int D, int CT, int KVT, int NST>
 void launch_split(DecodeArgs& a, size_t lds, hipStream_t st) {
     static std::atomic<int> cached{0};
-    auto kernel = decode_stream_kernel<D, CT, NST>;
+    auto kernel = decode_stream_kernel<D, CT, KVT, NST>;
     int per_cu = cached.load(std::memory_order_relaxed);
     if (per_cu <= 0) {
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kBlockThreads, 0) != hipSuccess || per_cu <= 0) per_cu = 1;
         cached.store(per_cu, std::memory_order_relaxed);
     }
-    const int by_lds = kLdsPerCu / int(lds + 1024 + kWavesPerBlock * NST * Tile<D, false>::STAGE);
+    const int by_lds = kLdsPerCu / int(lds + 1024 + kWavesPerBlock * NST * Tile<D, KVT>::STAGE);
     if (by_lds < per_cu) per_cu = by_lds > 0 ? by_lds : 1;
     hipLaunchKernelGGL(kernel, dim3(device_cu_count() * per_cu), dim3(kBlockThreads), lds, st, a);
 }
 
-template <int D, int CT>
+// Eight waves per row while every (row, kv head) has a CU, else four, so that
+// two workgroups share a CU; two stages per wave where a stage is 8 KiB.
+template <int D, int CT, int KVT>
+void launch_row_groups(DecodeArgs& a, hipStream_t st) {
+    constexpr int NST = Tile<D, KVT>::STAGE <= 8192 + 256 ? 2 : 1;
+    const int64_t pairs = int64_t(a.num_rows) * a.num_kv_heads;
+    const dim3 grid{unsigned(pairs)};
+    if (pairs <= device_cu_count())
+        hipLaunchKernelGGL((decode_rows_kernel<D, CT, KVT, 8, NST == 2 && KVT == kFp8 ? 1 : NST>), grid, dim3(512), 0, st, a);
+    else
+        hipLaunchKernelGGL((decode_rows_kernel<D, CT, KVT, 4, NST>), grid, dim3(256), 0, st, a);
+}
+
+template <int D, int CT, int KVT>
 void launch_shape(DecodeArgs& a, bool rows, size_t lds, hipStream_t st) {
     if (rows) {
-        const int64_t pairs = int64_t(a.num_rows) * a.num_kv_heads;
-        const dim3 grid{unsigned(pairs)};
-        if (pairs <= device_cu_count())
-            hipLaunchKernelGGL((decode_rows_kernel<D, CT, false, 8, D == 64 ? 2 : 1>), grid, dim3(512), 0, st, a);
-        else
-            hipLaunchKernelGGL((decode_rows_kernel<D, CT, false, 4, D == 64 ? 2 : 1>), grid, dim3(256), 0, st, a);
+        launch_row_groups<D, CT, KVT>(a, st);
         return;
     }
     // (calls over thousands of rows leave LDS for one stage only)
     if constexpr (D > 80) {
-        if (lds > (16 << 10)) {
-            launch_split<D, CT, 1>(a, lds, st);
+        if (lds <= (16 << 10)) {
+            launch_split<D, CT, KVT, 2>(a, lds, st);
             return;
         }
     }
-    launch_split<D, CT, D == 80 ? 1 : 2>(a, lds, st);
+    launch_split<D, CT, KVT, D == 64 && KVT == kF16 ? 2 : 1>(a, lds, st);
 }
 
-template <int D>
+template <int D, int KVT = kF16>
 void launch_dim(DecodeArgs& a, int G, bool rows, size_t lds, hipStream_t st) {
-    if (G <= 16) launch_shape<D, 1>(a, rows, lds, st);
-    else launch_shape<D, 2>(a, rows, lds, st);
+    if (G <= 16) launch_shape<D, 1, KVT>(a, rows, lds, st);
+    else launch_shape<D, 2, KVT>(a, rows, lds, st);
 }
 
 }  // namespace
@@ -722,27 +805,27 @@ void launch_dim(DecodeArgs& a, int G, bool rows, size_t lds, hipStream_t st) {
 //                2048 pairs:       256: 27.8 / 28.2     512: 48.1 / 47.6
 // Against decode.hip's split (head_dim 128, group 4): 256 pairs, 1 024: 18.6 /
 // 24.3; 2 048: 36.3 / 36.8; 1 024 pairs, 1 024: 53.9 / 79.1.
-bool stream_decode_rows(int num_rows, int num_kv_heads, int head_dim, int max_ctx, bool matrix_split) {
+bool stream_decode_rows(int num_rows, int num_kv_heads, int half_dims, int max_ctx, bool matrix_split) {
 #if VKV_STREAM_ROWS
     return VKV_STREAM_ROWS == 1;
 #endif
     const int64_t pairs = int64_t(num_rows) * num_kv_heads, cus = device_cu_count();
-    if (head_dim % 64 != 0) return max_ctx <= (pairs < 2 * cus ? 1056 : pairs < 8 * cus ? 528 : 264);
-    const int64_t row_bytes = int64_t(max_ctx) * head_dim * 4;
+    if (half_dims % 64 != 0) return max_ctx <= (pairs < 2 * cus ? 1056 : pairs < 8 * cus ? 528 : 264);
+    const int64_t row_bytes = int64_t(max_ctx) * half_dims * 4;
     return max_ctx <= 2112 && (row_bytes <= 528 << 10 || (pairs >= cus && !matrix_split));
 }
 
-template <bool FP8, int NST>
+template <int KVT, int NST>
 static void launch_parts(DecodeArgs& a, int64_t max_items, size_t lds, hipStream_t st) {
     static std::atomic<int> cached{0};
-    auto kernel = decode_parts_kernel<128, 1, FP8, NST>;
+    auto kernel = decode_parts_kernel<128, 1, KVT, NST>;
     const int cus = device_cu_count();
     int per_cu = cached.load(std::memory_order_relaxed);
     if (per_cu <= 0) {
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kBlockThreads, 0) != hipSuccess || per_cu <= 0) per_cu = 1;
         cached.store(per_cu, std::memory_order_relaxed);
     }
-    const int by_lds = kLdsPerCu / int(lds + 2048 + kWavesPerBlock * ((NST * Tile<128, FP8>::STAGE + 1023) / 1024 * 1024));
+    const int by_lds = kLdsPerCu / int(lds + 2048 + kWavesPerBlock * ((NST * Tile<128, KVT>::STAGE + 1023) / 1024 * 1024));
     if (by_lds < per_cu) per_cu = by_lds > 0 ? by_lds : 1;
     const int64_t groups = (max_items + kWavesPerBlock - 1) / kWavesPerBlock, wgs = int64_t(cus) * per_cu;
     const int gx = int(groups < wgs ? (groups > 0 ? groups : 1) : wgs);
@@ -764,22 +847,22 @@ static void launch_parts(DecodeArgs& a, int64_t max_items, size_t lds, hipStream
 // 120 of 1 024 to 8 192, group 7, FP8 132.2 / 125.3).
 bool launch_decode_matrix(DecodeArgs& a, bool fp8, int64_t max_items, size_t lds, hipStream_t st) {
     if (fp8 && stream_decode_rows(a.num_rows, a.num_kv_heads, 64, a.max_ctx, true)) {
-        const int64_t pairs = int64_t(a.num_rows) * a.num_kv_heads;
-        const dim3 grid{unsigned(pairs)};
-        if (pairs <= device_cu_count())
-            hipLaunchKernelGGL((decode_rows_kernel<128, 1, true, 8, 1>), grid, dim3(512), 0, st, a);
-        else
-            hipLaunchKernelGGL((decode_rows_kernel<128, 1, true, 4, 2>), grid, dim3(256), 0, st, a);
+        launch_row_groups<128, 1, kFp8>(a, st);
         return true;
     }
-    if (!fp8) launch_parts<false, 1>(a, max_items, lds, st);
-    else if (a.num_heads / a.num_kv_heads <= 4) launch_parts<true, 1>(a, max_items, lds, st);
-    else launch_parts<true, 2>(a, max_items, lds, st);
+    if (!fp8) launch_parts<kF16, 1>(a, max_items, lds, st);
+    else if (a.num_heads / a.num_kv_heads <= 4) launch_parts<kFp8, 1>(a, max_items, lds, st);
+    else launch_parts<kFp8, 2>(a, max_items, lds, st);
     return false;
 }
 
-int launch_decode_stream(DecodeArgs& a, bool rows, size_t lds, hipStream_t st) {
+int launch_decode_stream(DecodeArgs& a, bool f32, bool rows, size_t lds, hipStream_t st) {
     const int G = a.num_heads / a.num_kv_heads;
+    if (f32) {
+        if (a.head_dim != 64) return VKV_ERR_UNSUPPORTED;
+        launch_dim<64, kF32>(a, G, rows, lds, st);
+        return 0;
+    }
     switch (a.head_dim) {
         case 64: launch_dim<64>(a, G, rows, lds, st); return 0;
         case 80: launch_dim<80>(a, G, rows, lds, st); return 0;
