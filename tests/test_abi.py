@@ -217,6 +217,17 @@ def test_prefill_argument_errors_and_workspace(vkv):
     assert lib.vkv_paged_prefill_workspace_size(ctypes.byref(_prefill_params(vkv, head_dim=0))) == 0
 
 
+@pytest.mark.parametrize("head_dim,kv_dtype", [(64, 1), (64, 2), (128, 1), (128, 2)])
+def test_prefill_workspace_serves_smaller_steps(vkv, head_dim, kv_dtype):
+    """A workspace sized for a server's largest step (same sequences and longest
+    query) is enough for every step with fewer tokens, whatever row blocks they run in."""
+    lib = vkv.load()
+    over = dict(num_seqs=64, head_dim=head_dim, kv_dtype=kv_dtype, key_scales=16, value_scales=16)
+    size = [lib.vkv_paged_prefill_workspace_size(ctypes.byref(_prefill_params(vkv, num_query_tokens=t, **over)))
+            for t in (130, 600, 1500, 3000, 8192, 32768)]
+    assert size[0] > 0 and max(size[:-1]) <= size[-1], size
+
+
 @pytest.mark.parametrize("shape", [(28, 4, 128, 32, 1, 1), (32, 8, 128, 16, 1, 2), (16, 8, 64, 16, 1, 1),
                                    (32, 2, 128, 16, 1, 1)])
 def test_prefill_work_list_host(vkv, shape):

@@ -1989,6 +1989,7 @@ int cu_count() {
     cached[dev].store(cus, std::memory_order_relaxed);
     return cus;
 }
+constexpr int kSmallestRows = 64;
 int split_rows(const vkv_prefill_params* p) {
     const int64_t n64 = int64_t(p->num_query_tokens) * p->num_heads / 64, cus = cu_count();
     if (p->head_dim == 64) return n64 <= cus * 5 / 4 ? 64 : n64 <= 4 * cus ? 128 : 256;
@@ -2032,8 +2033,10 @@ void launch_split(const PrefillArgs& a, int head_dim, int rows, int64_t items, i
 
 }  // namespace
 
+// Room for the smallest row blocks, whatever the call's token count picks, so
+// that a workspace sized for a server's largest step serves every smaller one.
 size_t prefill_items_bytes(const vkv_prefill_params* p) {
-    return 256 + size_t(int64_t(p->num_seqs) * max_row_blocks(p, rows_per_item(p)) * p->num_kv_heads) * sizeof(int2);
+    return 256 + size_t(int64_t(p->num_seqs) * max_row_blocks(p, kSmallestRows) * p->num_kv_heads) * sizeof(int2);
 }
 
 int launch_prefill_mfma(const vkv_prefill_params* p, void* item_space, hipStream_t st) {
