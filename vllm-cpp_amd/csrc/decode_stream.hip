@@ -267,21 +267,24 @@ __device__ __forceinline__ void stream_tokens(const DecodeArgs& a, State<D, CT, 
         for (int hh = 0; hh < 2; ++hh) {
             if constexpr (T::F32) {
                 // v_mfma_f32_16x16x4_f32: lane (col, grp) holds one k slot, dim
-                // 16 i + 4 grp + e of product (i, e).  Each 16 dims a sum of
-                // their own, added in pairs: one chain over the 64 dims (and
-                // one over all tokens below) doubled the error against 64 bits
-                // of the lane-wise sums of the VALU kernel.
+                // 16 i + 4 grp + e of product (i, e).  Each product's 4 dims a
+                // sum of their own, added in pairs, as the VALU kernel's lanes
+                // of 4 dims were: one chain over the 64 dims (and one over all
+                // tokens below) doubled its error against 64 bits, chains of
+                // 16 still added a tenth to it at contexts of 1 to 300.
                 float4_t part[CT][D / 16];
 #pragma unroll
                 for (int i = 0; i < D / 16; ++i) {
                     const float4_t k = __builtin_bit_cast(float4_t, load16(kb + T::off(16 * hh + col, 4 * i + grp)));
-#pragma unroll
-                    for (int c = 0; c < CT; ++c) part[c][i] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+                    float4_t four[CT][4];
 #pragma unroll
                     for (int e = 0; e < 4; ++e)
 #pragma unroll
                         for (int c = 0; c < CT; ++c)
-                            part[c][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(k[e], st.qf[c][i][e], part[c][i], 0, 0, 0);
+                            four[c][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(k[e], st.qf[c][i][e],
+                                                                              float4_t{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+#pragma unroll
+                    for (int c = 0; c < CT; ++c) part[c][i] = (four[c][0] + four[c][1]) + (four[c][2] + four[c][3]);
                 }
 #pragma unroll
                 for (int c = 0; c < CT; ++c) sv[c][hh] = (part[c][0] + part[c][1]) + (part[c][2] + part[c][3]);
@@ -388,30 +391,31 @@ __device__ __forceinline__ void stream_tokens(const DecodeArgs& a, State<D, CT, 
         if constexpr (T::F32) {
             // product (hh, e): the k slot of lane (col, grp) is key 16 hh + 4 grp
             // + e, whose weight it holds; dims 4 col + t of that key's row.  Each
-            // half's sum of its own, added to the running sums.
-            float4_t part[CT][2][T::DT];
+            // product's 4 keys a sum of their own, added in pairs.
+            float4_t half[CT][2][T::DT];
 #pragma unroll
-            for (int c = 0; c < CT; ++c)
+            for (int hh = 0; hh < 2; ++hh) {
+                float4_t four[CT][4][T::DT];
 #pragma unroll
-                for (int hh = 0; hh < 2; ++hh)
-#pragma unroll
-                    for (int t = 0; t < T::DT; ++t) part[c][hh][t] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-#pragma unroll
-                for (int hh = 0; hh < 2; ++hh) {
+                for (int e = 0; e < 4; ++e) {
                     const float4_t v = __builtin_bit_cast(float4_t, load16(vb + T::off(16 * hh + 4 * grp + e, col)));
 #pragma unroll
                     for (int t = 0; t < T::DT; ++t)
 #pragma unroll
                         for (int c = 0; c < CT; ++c)
-                            part[c][hh][t] =
-                                __builtin_amdgcn_mfma_f32_16x16x4f32(v[t], pf[c][4 * hh + e], part[c][hh][t], 0, 0, 0);
+                            four[c][e][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[t], pf[c][4 * hh + e],
+                                                                                 float4_t{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
                 }
+#pragma unroll
+                for (int c = 0; c < CT; ++c)
+#pragma unroll
+                    for (int t = 0; t < T::DT; ++t)
+                        half[c][hh][t] = (four[c][0][t] + four[c][1][t]) + (four[c][2][t] + four[c][3][t]);
+            }
 #pragma unroll
             for (int c = 0; c < CT; ++c)
 #pragma unroll
-                for (int t = 0; t < T::DT; ++t) st.o[c][t] += part[c][0][t] + part[c][1][t];
+                for (int t = 0; t < T::DT; ++t) st.o[c][t] += half[c][0][t] + half[c][1][t];
             return;
         }
         const int vrow = FP8 ? (col < 8 ? 4 * grp + (col >> 1) : 12 + 4 * grp + (col >> 1)) : 4 * grp + (col >> 2);
