@@ -152,3 +152,29 @@ def test_stream_fp32_edges_vs_oracle(vkv, oracle, cuda, H, Hkv, bs, table):
                          to_dev(lay.context_lens, cuda), scale, partition_size=size)
         torch.cuda.synchronize()
         assert_close(to_np(out), ref, F32_ATOL, F32_RTOL, f"fp32 {H}/{Hkv}/bs{bs} size {size}")
+
+
+@pytest.mark.parametrize("dtype", ["f16", "f32"])
+@pytest.mark.parametrize("D", [64, 80, 112, 128])
+def test_stream_query_rows_of_any_alignment(vkv, cuda, D, dtype):
+    """Queries at an odd element and with an odd row stride: bit for bit the
+    result of the same queries in aligned rows."""
+    import torch
+    if dtype == "f32" and D != 64:
+        pytest.skip("fp32 streams at head_dim 64 only")
+    H, Hkv, bs = 6, 2, 16
+    rng = np.random.default_rng(D)
+    lay, (k, v), q = _case(rng, H, Hkv, D, bs, CONTEXTS, 1024)
+    t = np.float16 if dtype == "f16" else np.float32
+    q, n = to_dev(q.astype(t), cuda), len(CONTEXTS)
+    odd = torch.empty(1 + n * (H * D + 3), dtype=q.dtype, device=cuda)
+    odd = odd[1:].view(n, H * D + 3)[:, :H * D].unflatten(1, (H, D))
+    odd.copy_(q)
+    assert odd.data_ptr() % 16 != 0 and odd.stride(0) % 2 == 1
+    rest = (to_dev(k.astype(t), cuda), to_dev(v.astype(t), cuda), to_dev(lay.block_tables, cuda),
+            to_dev(lay.context_lens, cuda), float(D) ** -0.5)
+    outs = [torch.zeros((n, H, D), dtype=q.dtype, device=cuda) for _ in range(2)]
+    vkv.paged_decode(outs[0], q, *rest)
+    vkv.paged_decode(outs[1], odd, *rest)
+    torch.cuda.synchronize()
+    assert torch.equal(outs[0], outs[1])

@@ -150,6 +150,17 @@ struct State {
     }
 };
 
+// Queries need only their element's alignment (any row stride): loads that say
+// so (the compiler takes whole-vector loads where the target allows them).
+__device__ __forceinline__ u32x4 load_q16(const char* p) {
+    typedef u32x4 any_u32x4 __attribute__((aligned(2)));
+    return *reinterpret_cast<const any_u32x4*>(p);
+}
+__device__ __forceinline__ u32x2 load_q8(const char* p) {
+    typedef u32x2 any_u32x2 __attribute__((aligned(2)));
+    return *reinterpret_cast<const any_u32x2*>(p);
+}
+
 // Q as the B operand and an empty state.  Columns past the group read head 0
 // and are zeroed; a negative scale is moved into Q (exact sign flip).
 template <int D, int CT, int KVT>
@@ -166,18 +177,18 @@ __device__ __forceinline__ void init_state(const DecodeArgs& a, State<D, CT, KVT
                            (query_row(a, s) * a.q_stride + int64_t(kvh * G + (h < G ? h : 0)) * D) * (T::F32 ? 4 : 2);
 #pragma unroll
         for (int i = 0; i < (T::F32 ? D / 16 : 0); ++i) {
-            u32x4 w = load16(qrow + (16 * i + 4 * grp) * 4);
+            u32x4 w = load_q16(qrow + (16 * i + 4 * grp) * 4);
             w = (w ^ u32x4{flip, flip, flip, flip}) & u32x4{keep, keep, keep, keep};
             st.qf[c][i] = __builtin_bit_cast(float4_t, w);
         }
 #pragma unroll
         for (int i = 0; i < (T::F32 ? 0 : T::KS); ++i) {
-            u32x4 w = load16(qrow + T::dim(i, grp) * 2);
+            u32x4 w = load_q16(qrow + T::dim(i, grp) * 2);
             w = (w ^ u32x4{flip, flip, flip, flip}) & u32x4{keep, keep, keep, keep};
             st.q[c][i] = __builtin_bit_cast(half8_t, w);
         }
         if constexpr (T::HALF && !T::F32) {
-            u32x2 w = *reinterpret_cast<const u32x2*>(qrow + (32 * T::KS + 4 * grp) * 2);
+            u32x2 w = load_q8(qrow + (32 * T::KS + 4 * grp) * 2);
             w = (w ^ u32x2{flip, flip}) & u32x2{keep, keep};
             st.qh[c] = __builtin_bit_cast(half4_t, w);
         }
