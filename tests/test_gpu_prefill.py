@@ -570,3 +570,29 @@ def test_prefill_multi_token_only(vkv, oracle, cuda, kvt):
     ref2 = oracle.paged_prefill(q2.astype(np.float32), hk2, hv2, lay2.block_tables, ctx2, qsl2, scale,
                                 key_scales=hks2, value_scales=hvs2, nthreads=_threads())
     assert_close(to_np(out_c).astype(np.float32), ref2, F16_ATOL, F16_RTOL, f"mixed prefill after ({kvt})")
+
+
+@pytest.mark.parametrize("H,Hkv,D,bs", [(28, 4, 128, 16), (14, 2, 64, 16)])
+def test_prefill_inline_order_many_sequences(vkv, oracle, cuda, H, Hkv, D, bs):
+    """The in-kernel work list at its limits: 400 short sequences with single-token
+    ones between them, so entries run past 8 bits while the row blocks (at most
+    512) still order in LDS, and more items than workgroups, so that they are
+    ordered at all.  Every row against the oracle."""
+    import torch
+    rng = np.random.default_rng(23)
+    S = 400
+    q_lens = np.full(S, 2)
+    q_lens[rng.permutation(S)[:30]] = 1
+    q_lens[[0, 217, S - 1]] = [20, 33, 9]
+    prior = rng.integers(0, 60, S)
+    prior[[5, 300, S - 2]] = [700, 900, 400]
+    lay, ctx, qsl, q, k, v, scale = _case(H, Hkv, D, bs, q_lens, prior, 71)
+    Tq, G = q.shape[0], H // Hkv
+    assert Tq * G // 64 + S <= 512 and S * Hkv > 512  # ordered in LDS whatever the blocks; more than the grid
+    ref = oracle.paged_prefill(q.astype(np.float32), k.view(np.uint16), v.view(np.uint16), lay.block_tables, ctx, qsl,
+                               scale, nthreads=_threads())
+    out = torch.full((Tq, H, D), 7.0, dtype=torch.float16, device=cuda)
+    vkv.paged_prefill(out, to_dev(q, cuda), to_dev(k, cuda), to_dev(v, cuda), to_dev(lay.block_tables, cuda),
+                      to_dev(ctx, cuda), to_dev(qsl, cuda), int(max(q_lens)), scale)
+    torch.cuda.synchronize()
+    assert_close(to_np(out).astype(np.float32), ref, F16_ATOL, F16_RTOL, "400 sequences ordered in the kernel")

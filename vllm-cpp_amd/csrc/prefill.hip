@@ -676,12 +676,12 @@ __device__ __forceinline__ void prefill_block_wide(const PrefillArgs& a, const P
 // the ranking is quadratic, which at kInlineBlocks blocks is a few hundred LDS
 // reads per thread.  (One thread numbering all the blocks of its sequence, with
 // a 64-bit division per block, took 9 us for the 85 blocks of a prompt.)
-constexpr int kInlineBlocks = 512;
+constexpr int kInlineBlocks = 512;  // (9 bits in the keys and in order)
 struct InlineList {
     int first[kInlineBlocks];  // blocks before the sequence's
     int s[kInlineBlocks], q0[kInlineBlocks], qlen[kInlineBlocks], prior[kInlineBlocks];
     int key[kInlineBlocks];
-    int order[kInlineBlocks];  // block numbers, longest first (when ordered)
+    int order[kInlineBlocks];  // (entry << 9) | block number, longest first (when ordered)
     int nseq, total;
 };
 
@@ -750,11 +750,13 @@ __device__ void inline_row_blocks(const PrefillArgs& a, InlineList& l, const int
     __syncthreads();
     const int total = l.total;
     if (total * a.num_kv_heads <= workgroups) return;
+    int entry[PER];
 #pragma unroll
     for (int p = 0; p < PER; ++p) {
         const int i = tid + p * NT;
+        entry[p] = 0;
         if (i < total) {
-            const int e = inline_entry(l, i);
+            const int e = entry[p] = inline_entry(l, i);
             l.key[i] = (row_block_bin(l.prior[e], l.qlen[e], i - l.first[e], a.group, a.rows_per_item, a.table_tokens,
                                       a.nbins) << 9) | i;
         }
@@ -767,7 +769,7 @@ __device__ void inline_row_blocks(const PrefillArgs& a, InlineList& l, const int
             const int k = l.key[i];
             int rank = 0;
             for (int j = 0; j < total; ++j) rank += l.key[j] < k ? 1 : 0;
-            l.order[rank] = i;
+            l.order[rank] = (entry[p] << 9) | i;
         }
     }
     __syncthreads();
@@ -790,86 +792,112 @@ constexpr int kListItemWords = 8;
 constexpr int kListItemStartTiles = 5;
 constexpr int kListDefaultCus = 256;  // lists when the builder finds no device
 
-// The sequence fields of item (s, b, kvh), read from the call's arrays.
-__device__ __forceinline__ PrefillItem load_item(const PrefillArgs& a, const int s, const int b, const int kvh) {
-    const int q0 = a.qsl[s];
-    const int qlen = a.qsl[s + 1] - q0;
-    return PrefillItem{s, b, kvh, q0, qlen, a.cl[s] - qlen};
-}
-
-// Persistent loop of the direct-load kernels (NT threads): work items from the
-// host-built schedule, the in-kernel list (small calls) or the list kernel's;
-// item_fn(it) runs one.  No item is claimed, so no counter needs resetting.
-template <int NT, typename Item>
-__device__ __forceinline__ void run_items(const PrefillArgs& a, Item item_fn) {
-    if (a.work_list) {
-        // Workgroup w runs list w (and w + grid, ...), no claims.  Every index
-        // read from the list is bounded by its length, and items outside the
-        // call's sequences, kv heads and query rows are skipped, so a list
-        // from another call gives wrong rows but reads nothing out of bounds.
-        const int32_t* wl = a.work_list;
-        const int32_t* slots = wl + kListHeaderWords;
-        const int64_t cap = (int64_t(a.work_list_words) - kListHeaderWords) / kListItemWords;
-        PrefillItem nx;
-        auto fetch = [&](const int64_t k) __attribute__((always_inline)) {
-            const int32_t* e = slots + k * kListItemWords;
-            nx = PrefillItem{e[0], e[1], e[2], e[3], e[4], e[5]};
-        };
-        auto valid = [&](const PrefillItem& it) __attribute__((always_inline)) {
-            return unsigned(it.s) < unsigned(a.num_seqs) && unsigned(it.kvh) < unsigned(a.num_kv_heads) &&
-                   it.b >= 0 && it.q0 >= 0 && it.qlen >= 2 && int64_t(it.q0) + it.qlen <= a.num_query_tokens &&
-                   int64_t(it.b) * a.rows_per_item < int64_t(it.qlen) * a.group;
-        };
-        for (int w = blockIdx.x; w < cap; w += gridDim.x) {
-            fetch(w);  // (slot 0 of list w, beside the header)
-            const int lists = wl[0], len = wl[1];
-            if (wl[2] != kListFormat || lists < 1 || len < 0 || int64_t(lists) * len > cap || w >= lists) break;
-            for (int k = 0; k < len; ++k) {
-                const PrefillItem it = nx;
-                if (it.s < 0) break;  // (the list has ended)
-                const bool ok = valid(it);
-                // the next slot, requested after this one is checked (waiting
-                // for this one then waits for nothing else), arrives while
-                // this item runs
-                asm volatile("" ::: "memory");
-                if (k + 1 < len) fetch(int64_t(k + 1) * lists + w);
-                if (ok) item_fn(it);
-            }
-        }
-        return;
+// The items of a workgroup of the persistent kernels, one after the other (no item
+// is claimed, so no counter needs resetting).  The fields are scalars in both
+// sources: the item's code keeps its addresses out of the vector registers.
+//
+// ListedItems: the host-built schedule.  Workgroup w runs list w (and w + grid,
+// ...).  Every index read from the list is bounded by its length, and items
+// outside the call's sequences, kv heads and query rows are skipped, so a list
+// from another call gives wrong rows but reads nothing out of bounds.
+struct ListedItems {
+    const PrefillArgs& a;
+    const int32_t* const slots;
+    int lists = 0, len = 0, w, k = 0;
+    PrefillItem nx{};
+    __device__ __forceinline__ explicit ListedItems(const PrefillArgs& args)
+        : a(args), slots(args.work_list + kListHeaderWords), w(int(blockIdx.x)) {}
+    __device__ __forceinline__ void fetch(const int64_t i) {
+        const int32_t* e = slots + i * kListItemWords;
+        nx = PrefillItem{e[0], e[1], e[2], e[3], e[4], e[5]};
     }
-    // The in-kernel list (every workgroup orders a small call's row blocks
-    // itself) or the list kernel's, longest first, dealt to the workgroups in
-    // a snake: round r gives item r W + p to workgroup p when r is even and
-    // to W - 1 - p when r is odd (W workgroups, all resident: one per CU), so
-    // the longest items meet the shortest ones, as a longest-processing-time
-    // schedule would put them, with no claims.
-    const int W = gridDim.x, p = blockIdx.x;
-    __shared__ InlineList list;
-    if (a.inline_list) inline_row_blocks<NT>(a, list, W);
-    const int count = a.inline_list ? list.total * a.num_kv_heads : a.item_count[0];
-    for (int r = 0;; ++r) {
+    __device__ __forceinline__ void start() {
+        const int64_t cap = (int64_t(a.work_list_words) - kListHeaderWords) / kListItemWords;
+        if (w >= cap) return;
+        fetch(w);  // (slot 0 of list w, beside the header)
+        const int n = a.work_list[0], m = a.work_list[1];
+        if (a.work_list[2] != kListFormat || n < 1 || m < 1 || int64_t(n) * m > cap) return;
+        lists = n;
+        len = m;
+    }
+    // The next item of the workgroup's lists; false when they have ended.
+    __device__ __forceinline__ bool next(PrefillItem& it) {
+        for (;;) {
+            if (w >= lists) return false;
+            if (k >= len || nx.s < 0) {  // (list w has ended)
+                w += int(gridDim.x);
+                k = 0;
+                if (w >= lists) return false;
+                fetch(w);
+                continue;
+            }
+            it = nx;
+            const bool ok = unsigned(it.s) < unsigned(a.num_seqs) && unsigned(it.kvh) < unsigned(a.num_kv_heads) &&
+                            it.b >= 0 && it.q0 >= 0 && it.qlen >= 2 &&
+                            int64_t(it.q0) + it.qlen <= a.num_query_tokens &&
+                            int64_t(it.b) * a.rows_per_item < int64_t(it.qlen) * a.group;
+            // the next slot, requested after this one is checked (waiting for
+            // this one then waits for nothing else), arrives while this item runs
+            asm volatile("" ::: "memory");
+            if (++k < len) fetch(int64_t(k) * lists + w);
+            if (ok) return true;
+        }
+    }
+};
+
+// InKernelItems: the in-kernel list (every workgroup orders a small call's row
+// blocks itself) or the list kernel's, longest first, dealt to the workgroups in
+// a snake: round r gives item r W + p to workgroup p when r is even and to
+// W - 1 - p when r is odd (W workgroups, all resident), so the longest items meet
+// the shortest ones, as a longest-processing-time schedule would put them, with
+// no claims.
+struct InKernelItems {
+    const PrefillArgs& a;
+    InlineList& list;
+    int count = 0, r = 0;
+    __device__ __forceinline__ InKernelItems(const PrefillArgs& args, InlineList& lds) : a(args), list(lds) {}
+    template <int NT>
+    __device__ __forceinline__ void start() {
+        if (a.inline_list) inline_row_blocks<NT>(a, list, int(gridDim.x));
+        count = a.inline_list ? list.total * a.num_kv_heads : a.item_count[0];
+    }
+    __device__ __forceinline__ bool next(PrefillItem& item) {
+        const int W = int(gridDim.x), p = int(blockIdx.x);
         const int64_t it = int64_t(r) * W + ((r & 1) ? W - 1 - p : p);
-        if (it >= count) break;  // (later rounds are further on)
+        if (it >= count) return false;  // (later rounds are further on)
+        ++r;
+        auto u = [](const int x) __attribute__((always_inline)) { return __builtin_amdgcn_readfirstlane(x); };
         // items (row block, kv head), kv head fastest
         if (a.inline_list) {
             const int at = int(it) / a.num_kv_heads;
-            const int i = count > W ? list.order[at] : at;
-            const int e = inline_entry(list, i);
-            item_fn(PrefillItem{list.s[e], i - list.first[e], int(it) % a.num_kv_heads, list.q0[e], list.qlen[e],
-                                list.prior[e]});
+            const int o = count > W ? list.order[at] : (inline_entry(list, at) << 9) | at;
+            const int i = o & 511, e = o >> 9;
+            item = PrefillItem{u(list.s[e]), u(i - list.first[e]), int(it) % a.num_kv_heads,
+                               u(list.q0[e]), u(list.qlen[e]), u(list.prior[e])};
         } else {
-            const int2 item = a.items[it];
-            item_fn(load_item(a, item.x, item.y / a.num_kv_heads, item.y % a.num_kv_heads));
+            const int2 x = a.items[it];
+            const int s = u(x.x), q0 = a.qsl[s], qlen = a.qsl[s + 1] - q0;
+            item = PrefillItem{s, u(x.y) / a.num_kv_heads, u(x.y) % a.num_kv_heads, q0, qlen, a.cl[s] - qlen};
         }
+        return true;
     }
-}
+};
 
+// One copy of the item's code per source: at two waves per SIMD a single copy for
+// both took 4.5 % longer on calls without a host-built list.
 template <int D, bool FP8>
 __device__ __forceinline__ void wide_items(const PrefillArgs& a, const WideBuffers& buf) {
-    run_items<64 * kWideWaves>(a, [&](const PrefillItem& it) __attribute__((always_inline)) {
-        prefill_block_wide<D, FP8>(a, it, buf);
-    });
+    __shared__ InlineList list;
+    PrefillItem it;
+    if (a.work_list) {
+        ListedItems items(a);
+        items.start();
+        while (items.next(it)) prefill_block_wide<D, FP8>(a, it, buf);
+    } else {
+        InKernelItems items(a, list);
+        items.start<64 * kWideWaves>();
+        while (items.next(it)) prefill_block_wide<D, FP8>(a, it, buf);
+    }
 }
 
 template <int D>
@@ -1455,11 +1483,20 @@ __device__ __forceinline__ void prefill_block_w64(const PrefillArgs& a, const Pr
     store_rows_lds<D, RT>(a, buf.tiles + wave * (64 * D * EB), o, inv, b * kRows + 64 * wave, nrows, q0, kvh, lane);
 }
 
+// One copy of the item's code for every source: at 512 registers three copies
+// (listed, ordered in the kernel, ordered by the list kernel) spilled 28 of them
+// for 3, and calls with more items than workgroups took up to 15 % longer (24
+// prompts of 180 tokens, 28/4 heads: 51.4 us for 44.4; 24 of 180 + 256 keys:
+// 65.8 for 58.8).
 template <int D>
 __device__ __forceinline__ void w64_items(const PrefillArgs& a, const W64Buffers& buf) {
-    run_items<64 * kW64Waves>(a, [&](const PrefillItem& it) __attribute__((always_inline)) {
-        prefill_block_w64<D>(a, it, buf);
-    });
+    __shared__ InlineList list;
+    ListedItems listed(a);
+    InKernelItems ordered(a, list);
+    if (a.work_list) listed.start();
+    else ordered.start<64 * kW64Waves>();
+    PrefillItem it;
+    while (a.work_list ? listed.next(it) : ordered.next(it)) prefill_block_w64<D>(a, it, buf);
 }
 
 template <int D>
@@ -1853,9 +1890,11 @@ template <int D, bool FP8, class C>
 __global__ __launch_bounds__(C::NT) void prefill_split_kernel(PrefillArgs a) {
     __shared__ __attribute__((aligned(1024))) char lds[C::BYTES];
     __shared__ int btc[kWideBtc];
-    run_items<C::NT>(a, [&](const PrefillItem& it) __attribute__((always_inline)) {
-        prefill_block_split<D, FP8, C>(a, it, lds, btc);
-    });
+    __shared__ InlineList list;
+    InKernelItems items(a, list);
+    items.start<C::NT>();
+    PrefillItem it;
+    while (items.next(it)) prefill_block_split<D, FP8, C>(a, it, lds, btc);
 }
 
 // Work list of the matrix-core kernels, in one workgroup: items (s, b * Hkv +
