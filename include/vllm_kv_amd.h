@@ -360,14 +360,17 @@ int vkv_paged_prefill(const vkv_prefill_params* p, vkv_stream_t stream);
  * items and knows its next item while it computes the current one.  With the words
  * copied to device memory and passed as p->work_list / work_list_words, the
  * kernels skip ordering the items themselves: an engine builds it once per
- * step beside its other metadata, for every layer of the step.  The list must
- * come from the same lengths and shape as the call (items outside the call's
- * sequences, kv heads and query rows are skipped, so a stale list gives wrong
- * rows but reads nothing out of bounds; a grid smaller than the number of
- * lists runs the extra lists in turn).  Returns the number of int32 words; writes them when out is not
- * NULL and capacity_words suffices (else returns -2); 0 when the call's shape
- * runs without a list (everything but fp16 queries at head_dim 64/128 over fp16
- * caches or FP8 caches at 128); -1 for a NULL argument. */
+ * step beside its other metadata, for every layer of the step.  A call with a
+ * list runs the list's items (head_dim 128; elsewhere it is not read), so it
+ * must come from the same lengths and shape as the call (items outside the
+ * call's sequences, kv heads and query rows are skipped, so a stale list gives
+ * wrong rows but reads nothing out of bounds; a grid smaller than the number of
+ * lists runs the extra lists in turn).  Returns the number of int32 words;
+ * writes them when out is not NULL and capacity_words suffices (else returns
+ * -2); 0 when the call runs without a list: everything but fp16 queries at
+ * head_dim 128 over fp16 or FP8 caches, and there the lengths for which the
+ * kernels' smaller blocks, which need no list, are estimated to be faster (few
+ * rows, or long contexts before them); -1 for a NULL argument. */
 int64_t vkv_prefill_work_list_host(const vkv_prefill_params* p, const int32_t* host_query_start_loc,
                                    const int32_t* host_context_lens, int32_t* out, int64_t capacity_words);
 

@@ -190,6 +190,34 @@ def test_kv_pool_sizing_with_element_type(vkv):
         vkv.kv_block_bytes(L, bs, Hkv, D, 7)
 
 
+# (query lengths, keys before them, whether the 256-row items of a list are the faster
+# blocks), 28/4 heads at head_dim 128.  Steps of a dozen or more prompts without a
+# long context give those items enough work in one round of the CUs (measured at 12 x
+# 128 tokens: 18.2 us listed, 20.3 in blocks of 128 rows); a prompt alone, or chunks
+# that bring little work to long contexts, do not (4 x 100 + 2 048 keys: 125, 56.2).
+LISTED = {
+    "12 short prompts": ([100, 110, 125, 130, 140, 150, 160, 175, 190, 200, 225, 250], 0, True),
+    "16 x 100": ([100] * 16, 0, True),
+    "8 x 512, long contexts": ([512] * 8, 1024, True),
+    "one prompt": ([1000], 0, False),
+    "4 x 100, long contexts": ([100] * 4, 2048, False),
+}
+
+
+@pytest.mark.parametrize("kv_dtype", [1, 2])
+@pytest.mark.parametrize("step", list(LISTED))
+def test_prefill_list_where_it_is_read(vkv, step, kv_dtype):
+    """Words only for lengths whose call runs the list's items."""
+    import numpy as np
+    q_lens, prior, listed = LISTED[step]
+    qsl = np.concatenate([[0], np.cumsum(q_lens)]).astype(np.int32)
+    ctx = (np.array(q_lens) + prior).astype(np.int32)
+    p = _prefill_params(vkv, num_seqs=len(q_lens), num_query_tokens=int(qsl[-1]), max_query_len=max(q_lens),
+                        kv_dtype=kv_dtype, key_scales=16, value_scales=16)
+    n = vkv.load().vkv_prefill_work_list_host(ctypes.byref(p), qsl.ctypes.data, ctx.ctypes.data, None, 0)
+    assert (n > 0) == listed
+
+
 def _prefill_params(vkv, **over):
     p = vkv.PrefillParams(output=16, query=16, key_cache=16, value_cache=16, block_tables=16, context_lens=16,
                           query_start_loc=16, num_seqs=3, num_query_tokens=600, max_query_len=512, num_heads=28,
@@ -228,18 +256,19 @@ def test_prefill_workspace_serves_smaller_steps(vkv, head_dim, kv_dtype):
     assert size[0] > 0 and max(size[:-1]) <= size[-1], size
 
 
-@pytest.mark.parametrize("shape", [(28, 4, 128, 32, 1, 1), (32, 8, 128, 16, 1, 2), (16, 8, 64, 16, 1, 1),
+@pytest.mark.parametrize("shape", [(28, 4, 128, 32, 1, 1), (32, 8, 128, 16, 1, 2), (16, 8, 128, 16, 1, 1),
                                    (32, 2, 128, 16, 1, 1)])
 def test_prefill_work_list_host(vkv, shape):
     """vkv_prefill_work_list_host (no GPU): every work item (sequence, row block,
     kv head) of the call exactly once, with its sequence's query rows and prior
     context, dealt to one list per workgroup longest first, each to the least
-    loaded list; no list for shapes the matrix-core kernels do not run;
-    capacity and argument errors."""
+    loaded list; no list for shapes and lengths that run without one; capacity
+    and argument errors.  (40 prompts: with 9 of these lengths the call runs in
+    smaller blocks, which take no list.)"""
     import numpy as np
     H, Hkv, D, bs, io, kv = shape
     rng = np.random.default_rng(H + D)
-    q_lens = np.concatenate([rng.integers(2, 700, 9), [1, 1, 1]]).astype(np.int32)
+    q_lens = np.concatenate([rng.integers(2, 700, 40), [1, 1, 1]]).astype(np.int32)
     prior = rng.integers(0, 3000, q_lens.size).astype(np.int32)
     qsl = np.concatenate([[0], np.cumsum(q_lens)]).astype(np.int32)
     ctx = (prior + q_lens).astype(np.int32)
@@ -250,7 +279,7 @@ def test_prefill_work_list_host(vkv, shape):
     lib = vkv.load()
     n = lib.vkv_prefill_work_list_host(ctypes.byref(p), qsl.ctypes.data, ctx.ctypes.data, None, 0)
     G = H // Hkv
-    rows = 256 if D == 128 else 512
+    rows = 256
     want = {}
     for s in range(q_lens.size):
         if q_lens[s] < 2:
@@ -294,15 +323,16 @@ def test_prefill_work_list_host(vkv, shape):
         load[w] += want[key][3] + 5
         dealt[w].append(key)
     assert dealt == [[(int(e[0]), int(e[1]), int(e[2])) for e in c] for c in per_list]
-    # shapes without the list: fp32 queries, FP8 at head_dim 64, and fp16 at
-    # head_dim 64 with groups of 4 heads or more (the register-staged kernel)
+    # without the list: fp32 queries, head_dim 64 (any cache and group)
     p32 = _prefill_params(vkv, io_dtype=0, kv_dtype=0)
     assert lib.vkv_prefill_work_list_host(ctypes.byref(p32), qsl.ctypes.data, ctx.ctypes.data, None, 0) == 0
     p8 = _prefill_params(vkv, head_dim=64, kv_dtype=2)
     assert lib.vkv_prefill_work_list_host(ctypes.byref(p8), qsl.ctypes.data, ctx.ctypes.data, None, 0) == 0
     p64 = _prefill_params(vkv, num_seqs=q_lens.size, num_query_tokens=int(qsl[-1]), max_query_len=int(q_lens.max()),
                           num_heads=16, num_kv_heads=4, head_dim=64, block_size=16, max_blocks_per_seq=mb)
-    assert lib.vkv_prefill_work_list_host(ctypes.byref(p64), qsl.ctypes.data, ctx.ctypes.data, None, 0) == 0
+    for kv_heads in (4, 8, 16):
+        p64.num_kv_heads = kv_heads
+        assert lib.vkv_prefill_work_list_host(ctypes.byref(p64), qsl.ctypes.data, ctx.ctypes.data, None, 0) == 0
     assert lib.vkv_prefill_work_list_host(ctypes.byref(p), None, ctx.ctypes.data, None, 0) == -1
     # a negative length is refused before any launch
     assert lib.vkv_paged_prefill(ctypes.byref(_prefill_params(vkv, work_list_words=-1)), None) == -2

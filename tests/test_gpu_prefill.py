@@ -53,6 +53,30 @@ def _threads():
     return max(1, min(16, os.cpu_count() or 1))
 
 
+def whole_items_list(qsl, ctx, group, kv_heads, lists=256):
+    """A host-built schedule of the 256-row items (the words that
+    vkv_prefill_work_list_host documents), whatever the lengths: a call at head_dim 128
+    that is given one runs these items, on the kernels that serve the large steps."""
+    items = []
+    for s in range(len(ctx)):
+        q = int(qsl[s + 1] - qsl[s])
+        prior = int(ctx[s]) - q
+        for b in range((q * group + 255) // 256 if q >= 2 else 0):
+            last = min(q, ((b + 1) * 256 - 1) // group + 1)
+            tiles = max(0, (prior + last + 63) // 64)
+            items += [[s, b, h, int(qsl[s]), q, prior, tiles, 0] for h in range(kv_heads)]
+    items.sort(key=lambda e: -e[6])
+    lists = max(1, min(lists, len(items)))
+    L = max(1, -(-len(items) // lists))
+    words = np.zeros(32 + 8 * lists * L, np.int32)
+    words[:4] = [lists, L, 3, len(items)]
+    slots = words[32:].reshape(L, lists, 8)
+    slots[:, :, 0] = -1
+    for n, e in enumerate(items):
+        slots[n // lists, n % lists] = e
+    return words
+
+
 # fp16 queries at head_dim 64/128 run sequences with >= 2 query tokens on the
 # matrix-core kernels and single-token ones through split-K decode; each case
 # runs over an fp16 cache and over its FP8 quantisation (against the oracle
@@ -76,8 +100,9 @@ def _threads():
     (32, 1, 64, 16, [200, 2], [30, 0]),
 ])
 def test_prefill_vs_oracle(vkv, oracle, cuda, kvt, H, Hkv, D, bs, q_lens, prior):
-    """Against the oracle, with the kernels' own work ordering and with the
-    host-built work list (vkv_prefill_work_list_host) of the same call."""
+    """Against the oracle, with the kernels' own work ordering and with a host-built
+    work list of the same call (at head_dim 128 a list makes it run the 256-row items,
+    where vkv_prefill_work_list_host would give none for lengths this short)."""
     import torch
     lay, ctx, qsl, q, k, v, scale = _case(H, Hkv, D, bs, q_lens, prior, sum(q_lens) + H)
     Tq = q.shape[0]
@@ -90,8 +115,7 @@ def test_prefill_vs_oracle(vkv, oracle, cuda, kvt, H, Hkv, D, bs, q_lens, prior)
         out = torch.zeros((Tq, H, D), dtype=torch.float16, device=cuda)
         wl = None
         if listed:
-            words = vkv.prefill_work_list(out, *args, qsl, ctx, key_scales=ks, value_scales=vs)
-            wl = to_dev(words, cuda) if words.size else None
+            wl = to_dev(whole_items_list(qsl, ctx, H // Hkv, Hkv), cuda)
         vkv.paged_prefill(out, *args, key_scales=ks, value_scales=vs, work_list=wl)
         torch.cuda.synchronize()
         assert_close(to_np(out).astype(np.float32), ref, F16_ATOL, F16_RTOL,
@@ -115,7 +139,7 @@ def test_prefill_work_list_relaid(vkv, oracle, cuda, kvt):
     args = (to_dev(q, cuda), kc, vc, to_dev(lay.block_tables, cuda), to_dev(ctx, cuda), to_dev(qsl, cuda),
             int(max(q_lens)), scale)
     out = torch.zeros((Tq, H, D), dtype=torch.float16, device=cuda)
-    words = vkv.prefill_work_list(out, *args, qsl, ctx, key_scales=ks, value_scales=vs)
+    words = whole_items_list(qsl, ctx, H // Hkv, Hkv)
     lists, L = int(words[0]), int(words[1])
     slots = words[32:].reshape(L, lists, 8)
     items = [slots[kk, w].copy() for w in range(lists) for kk in range(L) if slots[kk, w, 0] >= 0]
@@ -137,6 +161,31 @@ def test_prefill_work_list_relaid(vkv, oracle, cuda, kvt):
     vkv.paged_prefill(out, *args, key_scales=ks, value_scales=vs, work_list=to_dev(relaid, cuda))
     torch.cuda.synchronize()
     assert_close(to_np(out).astype(np.float32), ref, F16_ATOL, F16_RTOL, f"prefill, re-laid list ({kvt} cache)")
+
+
+@pytest.mark.parametrize("kvt", ["f16", "fp8"])
+def test_prefill_list_is_read(vkv, cuda, kvt):
+    """Where vkv_prefill_work_list_host gives words, the call runs the list: a dozen
+    short prompts with the list of the host write every row, and nothing with one
+    whose entries have all ended."""
+    import torch
+    H, Hkv, D, bs = 28, 4, 128, 32
+    q_lens = [100, 110, 125, 130, 140, 150, 160, 175, 190, 200, 225, 250]
+    lay, ctx, qsl, q, k, v, scale = _case(H, Hkv, D, bs, q_lens, [0] * len(q_lens), 37)
+    (kc, vc, ks, vs), _ = _cache(vkv, cuda, kvt, k, v)
+    args = (to_dev(q, cuda), kc, vc, to_dev(lay.block_tables, cuda), to_dev(ctx, cuda), to_dev(qsl, cuda),
+            int(max(q_lens)), scale)
+    out = torch.full((q.shape[0], H, D), float("nan"), dtype=torch.float16, device=cuda)
+    words = vkv.prefill_work_list(out, *args, qsl, ctx, key_scales=ks, value_scales=vs)
+    assert words.size > 0
+    empty = words.copy()
+    empty[32::8] = -1
+    vkv.paged_prefill(out, *args, key_scales=ks, value_scales=vs, multi_token_only=True, work_list=to_dev(empty, cuda))
+    torch.cuda.synchronize()
+    assert torch.isnan(out).all()
+    vkv.paged_prefill(out, *args, key_scales=ks, value_scales=vs, multi_token_only=True, work_list=to_dev(words, cuda))
+    torch.cuda.synchronize()
+    assert torch.isfinite(out).all()
 
 
 @pytest.mark.parametrize("bs", [1, 2])

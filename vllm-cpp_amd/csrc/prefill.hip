@@ -26,6 +26,7 @@
 // The output tile is O^T, again one row per lane, normalised at the end.
 #include <algorithm>
 #include <atomic>
+#include <cmath>
 #include <functional>
 #include <queue>
 #include <utility>
@@ -217,12 +218,12 @@ __device__ __forceinline__ float vmax3(float a, float b, float c) {
 constexpr int kWideWaves = 8;  // two per SIMD
 constexpr int kWideStages = 3;
 constexpr int kWideBtc = 2048;  // block ids held in LDS at a time
-// 16-row tiles per wave (what fits 256 registers) and (token, head) rows per
-// item (head_dim 64: of the host-built lists only, its calls order their own)
+// 16-row tiles per wave (what fits 256 registers) and (token, head) rows per item
 template <int D>
 struct Wide {
-    static constexpr int RT = D == 128 ? 2 : 4;
+    static constexpr int RT = 2;
     static constexpr int ROWS = kWideWaves * RT * 16;
+    static_assert(D == 128, "head_dim 64 runs on prefill_split_kernel");
 };
 
 // K and V tile buffers of the three stages: six LDS objects, so that the
@@ -621,50 +622,29 @@ __device__ __forceinline__ void prefill_block_wide(const PrefillArgs& a, const P
     }
     wait_vmcnt<0>();  // no load of this item may land in the next item's buffers
 
-    if constexpr (D == 128) {
-        // ---------------- output through LDS, 8 KiB per wave: FP8, the six
-        // code buffers and the two fp16 tiles; fp16, the halves of the six
-        // tile buffers
-        static_assert(16 * RT * D * 2 == 8192 && DmaTile8<D>::BYTES == 8192 && T::BYTES == 16384,
-                      "8 KiB of output rows per wave");
-        __syncthreads();  // every wave's loads have landed and no wave reads a tile
-        // (constant indices only: a buffer array indexed by a variable would
-        // be materialised in memory)
-        char* ob;
-        if constexpr (FP8) {
-            ob = wave == 0 ? buf.f8k[0] : wave == 1 ? buf.f8k[1] : wave == 2 ? buf.f8k[2] : wave == 3 ? buf.f8v[0]
-               : wave == 4 ? buf.f8v[1] : wave == 5 ? buf.f8v[2] : wave == 6 ? buf.k[0] : buf.v[0];
-        } else {
-            const int h2 = wave >> 1;
-            ob = (h2 == 0 ? buf.k[0] : h2 == 1 ? buf.k[1] : h2 == 2 ? buf.k[2] : buf.v[0]) + (wave & 1) * 8192;
-        }
-        float inv[RT];
-#pragma unroll
-        for (int r = 0; r < RT; ++r) {
-            const float lt = lsum[r][0];
-            inv[r] = (rctx[r] > 0 && lt > 0.0f) ? 1.0f / lt : 0.0f;
-        }
-        store_rows_lds<D, RT>(a, ob, o, inv, b * kWideRows + 16 * RT * wave, nrows, q0, kvh, lane);
-        return;
+    // ---------------- output through LDS, 8 KiB per wave: FP8, the six
+    // code buffers and the two fp16 tiles; fp16, the halves of the six
+    // tile buffers
+    static_assert(16 * RT * D * 2 == 8192 && DmaTile8<D>::BYTES == 8192 && T::BYTES == 16384,
+                  "8 KiB of output rows per wave");
+    __syncthreads();  // every wave's loads have landed and no wave reads a tile
+    // (constant indices only: a buffer array indexed by a variable would
+    // be materialised in memory)
+    char* ob;
+    if constexpr (FP8) {
+        ob = wave == 0 ? buf.f8k[0] : wave == 1 ? buf.f8k[1] : wave == 2 ? buf.f8k[2] : wave == 3 ? buf.f8v[0]
+           : wave == 4 ? buf.f8v[1] : wave == 5 ? buf.f8v[2] : wave == 6 ? buf.k[0] : buf.v[0];
+    } else {
+        const int h2 = wave >> 1;
+        ob = (h2 == 0 ? buf.k[0] : h2 == 1 ? buf.k[1] : h2 == 2 ? buf.k[2] : buf.v[0]) + (wave & 1) * 8192;
     }
-    // ---------------- output: lane (row col) holds dims 16 t + 4 grp + e
+    float inv[RT];
 #pragma unroll
     for (int r = 0; r < RT; ++r) {
-        const int rho = b * kWideRows + 16 * RT * wave + 16 * r + col;
-        if (rho >= nrows) continue;
-        const int j = rho / G;
-        const int h = kvh * G + rho - j * G;
         const float lt = lsum[r][0];
-        const float inv = (rctx[r] > 0 && lt > 0.0f) ? 1.0f / lt : 0.0f;
-        _Float16* orow = a.out + ((int64_t(q0) + j) * a.num_heads + h) * D;
-#pragma unroll
-        for (int t = 0; t < DT; ++t) {
-            const half2_t lo = {static_cast<_Float16>(o[r][t][0] * inv), static_cast<_Float16>(o[r][t][1] * inv)};
-            const half2_t hi = {static_cast<_Float16>(o[r][t][2] * inv), static_cast<_Float16>(o[r][t][3] * inv)};
-            *reinterpret_cast<u32x2*>(orow + 16 * t + 4 * grp) =
-                u32x2{__builtin_bit_cast(uint32_t, lo), __builtin_bit_cast(uint32_t, hi)};
-        }
+        inv[r] = (rctx[r] > 0 && lt > 0.0f) ? 1.0f / lt : 0.0f;
     }
+    store_rows_lds<D, RT>(a, ob, o, inv, b * kWideRows + 16 * RT * wave, nrows, q0, kvh, lane);
 }
 
 // In-kernel work list of a small call, built by every workgroup alike (so no
@@ -790,6 +770,7 @@ constexpr int kListItemWords = 8;
 // Cost of an item in the host's schedule: its key tiles plus this many for
 // its start (the chain of loads before its first tile can be computed).
 constexpr int kListItemStartTiles = 5;
+constexpr int kListRows = 256;       // (token, head) rows of a listed item
 constexpr int kListDefaultCus = 256;  // lists when the builder finds no device
 
 // The items of a workgroup of the persistent kernels, one after the other (no item
@@ -1994,24 +1975,19 @@ bool prefill_mfma_supported(const vkv_prefill_params* p) {
 
 namespace {
 
-// The work items of prefill_split_kernel, by the call's (token, head) rows in
-// blocks of 64 over its kv heads, n64.  Few blocks: 64 rows each, the keys over
-// four groups of waves, so that every CU has one and its chain of key tiles is
-// short.  More of them, or longer calls: 128 rows (each K/V operand read from
-// LDS feeds twice the products), then 256.  At head_dim 128 calls that fill the
-// chip with 256-row blocks run on the one-wave-per-SIMD kernels, whose
-// schedule overlaps more (rows 0).  Measured (us, blocks of 64 / 128 / 256 rows
-// or the latter kernels; "4 x 700" four prompts of 700 tokens, + prior keys):
-//   D 64, 14/2 heads: 1 x 500 (n64 108): 11.4 / 13.4 / 21.3; 1 x 1 000 (218):
-//     14.1 / 20.3 / 32.7; 3 x 700 (458): 20.8 / 16.7 / 27.0; 8 x 512 + 2 000
-//     (896): 59.6 / 46.5 / 62.2; 16 x 500 (1 750): 65.6 / 43.2 / 36.8
-//   D 128, 32/8 heads: 1 x 500 (248): 16.4 / 18.2 / 26.5; 4 x 100 + 2 000
-//     (200): 32.9 / 47.2 / 71.4; 8 x 100 + 1 000 (400): 32.2 / 29.8 / 44.9;
-//     1 x 2 000 (1 000): 76 / 53.9 / 72.2; 4 x 700 (1 400): 67 / 44.0 / 41.6
-//   (FP8 caches alike: 1 x 500: 18.9 / 21.1 / 28.0; 4 x 700: 79 / 49.3 / 41.2)
+// prefill_split_kernel's blocks.  Few items: 64 rows each, the keys over four groups
+// of waves, so that every CU has one and its chain of key tiles is short.  More of
+// them: 128 rows (each K/V operand read from LDS feeds twice the products), then
+// 256; at head_dim 128 the 256-row items of the one-wave-per-SIMD kernels, whose
+// schedule overlaps more.  Split64W: 256 rows in one key group, two workgroups to a
+// CU, for steps of short contexts (a chain of at most four tiles), whose items are
+// mostly start and end: 48 prompts of 100 tokens, 14/2 heads, fp16 / FP8 cache: 21.1
+// / 21.2 us, Split64L 25.2 / 28.2; 32 of 180: 25.2 / 26.4 for 26.7 / 30.2; but with
+// 256 keys before them 43.1 / 43.3 for 35.4 / 39.1.
 template <bool FP8> using Split64S = Split<64, FP8, 4, 4, 1, 64, 2>;
 template <bool FP8> using Split64M = Split<64, FP8, 4, 3, 2, 64, 2>;
 template <bool FP8> using Split64L = Split<64, FP8, 4, 2, 4, 64, 2>;
+template <bool FP8> using Split64W = Split<64, FP8, 4, 1, 4, 64, 2>;
 template <bool FP8> using Split128S = Split<128, FP8, 2, 4, 2, 32, 2>;
 template <bool FP8> using Split128M = Split<128, FP8, 4, 2, 2, 32, 2>;
 
@@ -2029,16 +2005,143 @@ int cu_count() {
     return cus;
 }
 constexpr int kSmallestRows = 64;
-int split_rows(const vkv_prefill_params* p) {
-    const int64_t n64 = int64_t(p->num_query_tokens) * p->num_heads / 64, cus = cu_count();
-    if (p->head_dim == 64) return n64 <= cus * 5 / 4 ? 64 : n64 <= 4 * cus ? 128 : 256;
-    return n64 <= cus ? 64 : n64 <= 4 * cus ? 128 : 0;
+
+// Which blocks a call runs in: those with the least estimated time.
+//
+// A kernel's time is `once` plus the work of its busiest workgroup (one per CU),
+// `start` per item and `tile` per 64 keys of it (us); in blocks that the kernels do
+// not order in LDS, the list kernel's before it.  The figures are fits to 600 steps
+// per row: 1 to 48 prompts of 16 to 2 048 tokens with 0, 256 or 2 048 keys before
+// them, 28/4 and 32/8 heads at head_dim 128 and 14/2 at 64 (median error 2 to 3 %,
+// 5 % of the steps off by 7 to 20 %).  Measured (us; blocks of 64 / 128 / 256 rows):
+//   D 128, 28/4 heads, fp16: 1 x 1 024 tokens 28.9 / 25.9 / 39.8; 4 x 100 + 2 048
+//     keys 56.2 / 86.2 / 125; 16 x 100 29.9 / 20.2 / 18.9; 8 x 512 + 256 96.9 / 62.7 /
+//     54.8; FP8 cache: 24 x 64 30.8 / 20.2 / 16.0; 6 x 400 + 256 75.0 / 52.8 / 49.8
+//   D 64, 14/2 heads, fp16: 1 x 700 12.1 / 15.6 / 24.0; 3 x 700 21.0 / 20.1 / 30.6;
+//     16 x 400 61.5 / 32.4 / 29.1
+// Over the 1 900 steps the choice costs 0.3 % against the best of the three each time.
+struct ItemCost {
+    int rows;
+    float once, start, tile;
+};
+constexpr ItemCost kItemCosts[2][2][3] = {
+    // head_dim 64: fp16, FP8 cache
+    {{{64, 1.2f, 6.4f, 0.41f}, {128, 0.5f, 7.5f, 0.70f}, {256, -0.8f, 10.0f, 1.36f}},
+     {{64, 1.4f, 6.3f, 0.59f}, {128, 0.8f, 7.6f, 0.89f}, {256, -0.8f, 10.8f, 1.63f}}},
+    // head_dim 128
+    {{{64, 3.1f, 6.8f, 0.68f}, {128, 2.4f, 5.9f, 1.14f}, {kListRows, 0.7f, 11.0f, 1.73f}},
+     {{64, 3.2f, 7.1f, 0.99f}, {128, 2.4f, 6.1f, 1.49f}, {kListRows, 0.2f, 9.2f, 2.19f}}}};
+constexpr float kSplitMargin = 1.06f;      // smaller blocks where they are clearly faster
+constexpr float kListSaves = 1.5f;         // ordering that a host-built list spares
+constexpr float kListKernel = 5.0f;        // the list kernel's launch, and
+constexpr float kListKernelItem = 0.15f;   // per item of the sequence with the most (one thread writes them)
+constexpr int kShortContext = 256;         // Split64W's
+
+// The items of a call: their number, the longest's and the mean's key tiles, the
+// call's row blocks at most, and the items of the sequence with the most.
+struct ItemLoad {
+    float items, longest, mean;
+    int64_t blocks;
+    float of_one;
+};
+float estimated_us(const ItemCost& c, const ItemLoad& l, int cus) {
+    const float once = c.once + (l.blocks > kInlineBlocks ? kListKernel + kListKernelItem * l.of_one : 0.0f);
+    const float R = l.items / float(cus);
+    if (R <= 1.0f) return once + c.start + c.tile * l.longest;
+    // Longest first, dealt in a snake: the workgroups with one item less hold the
+    // longest of the first round, those with one more the shortest of the last.
+    const float m = std::ceil(R);
+    const float longest = std::max(l.longest, (m - 1) * l.mean + (l.longest - l.mean) * (1 - (m - 1) / R));
+    const float most = std::max(l.mean * std::sqrt(m * R), l.mean * R);
+    return once + std::max((m - 1) * c.start + c.tile * longest, m * c.start + c.tile * most);
 }
-// (token, head) rows of the items of vkv_prefill_work_list_host's lists, and of the call's
-int list_rows(const vkv_prefill_params* p) { return p->head_dim == 128 ? Wide<128>::ROWS : Wide<64>::ROWS; }
-int rows_per_item(const vkv_prefill_params* p) {
-    const int r = split_rows(p);
-    return r > 0 ? r : list_rows(p);
+
+int64_t key_bound(const vkv_prefill_params* p) {
+    const int64_t table = int64_t(p->max_blocks_per_seq) * p->block_size;
+    return p->max_context_len > 0 && p->max_context_len < table ? p->max_context_len : table;
+}
+
+// Row blocks of a call, at most: a sequence of q >= 2 tokens has ceil(q G / rows) <=
+// q G / rows + 1 of them, and there are at most min(S, T / 2) such sequences (T
+// query tokens).
+int64_t block_bound(const vkv_prefill_params* p, int rows) {
+    const int64_t T = p->num_query_tokens;
+    return T * (p->num_heads / p->num_kv_heads) / rows + (p->num_seqs < T / 2 ? p->num_seqs : T / 2);
+}
+
+// The load of a call whose lengths are on the device, from what the host knows of
+// them.  Sequences: all, or (with single-token ones among them) as many as bring
+// the tokens at three quarters of the longest chunk.  Keys before the chunks:
+// none to the bound the table (or max_context_len) leaves, evenly; a bound of
+// more than 8 192 says how long a sequence may grow and not how long the step's
+// are: 512.
+ItemLoad expected_load(const vkv_prefill_params* p, int rows) {
+    const float G = float(p->num_heads / p->num_kv_heads), longest = float(p->max_query_len);
+    float seqs = float(p->num_seqs), T = float(p->num_query_tokens);
+    if (!p->multi_token_only && p->num_seqs > 1) {
+        const float more = T - seqs;  // tokens beyond one per sequence
+        seqs = std::min(seqs, std::max(1.0f, std::ceil(more / (0.75f * (longest - 1)))));
+        T = more + seqs;
+    }
+    const float q = std::max(1.0f, std::min(T / seqs, longest));
+    float prior = std::max(0.0f, float(key_bound(p)) - longest);
+    if (prior > 8192.0f) prior = 512.0f;
+    const float most = std::ceil(longest * G / float(rows)), heads = float(p->num_kv_heads);
+    const float blocks = seqs == 1.0f ? most
+                         : std::min(most, std::max(1.0f, q * G / float(rows) + (longest > 1.05f * q ? 0.5f : 0.0f)));
+    const float before = seqs == 1.0f ? prior : 0.5f * prior;
+    return ItemLoad{heads * seqs * blocks, (prior + longest) / 64.0f + 0.5f,
+                    (before + 0.5f * (q + std::min(q, float(rows) / G))) / 64.0f + 0.5f, block_bound(p, rows), heads * most};
+}
+
+// The load of a call whose lengths the host has.
+ItemLoad known_load(const vkv_prefill_params* p, int rows, const int32_t* qsl, const int32_t* cl) {
+    const int G = p->num_heads / p->num_kv_heads;
+    const int64_t bound = key_bound(p);
+    int64_t n = 0, most = 0;
+    float longest = 0.0f, sum = 0.0f;
+    for (int32_t s = 0; s < p->num_seqs; ++s) {
+        const int64_t q = int64_t(qsl[s + 1]) - qsl[s];
+        if (q < 2) continue;
+        const int64_t prior = int64_t(cl[s]) - q, nb = (q * G + rows - 1) / rows;
+        const float first = float(std::max<int64_t>(0, std::min(prior + std::min<int64_t>(q, rows / G), bound)) + 63) / 64.0f;
+        const float last = float(std::max<int64_t>(0, std::min(prior + q, bound)) + 63) / 64.0f;
+        n += nb;
+        most = std::max(most, nb);
+        sum += float(nb) * 0.5f * (first + last);
+        longest = std::max(longest, last);
+    }
+    const float heads = float(p->num_kv_heads);
+    return ItemLoad{heads * float(n), longest, n > 0 ? sum / float(n) : 0.0f, block_bound(p, rows), heads * float(most)};
+}
+
+// The items of a call: rows of prefill_split_kernel's, or 0: the 256-row items of the
+// one-wave-per-SIMD kernels (head_dim 128), the only ones that read a host-built list.
+int split_rows(const vkv_prefill_params* p) {
+    const ItemCost* const c = kItemCosts[p->head_dim == 128][p->kv_dtype != VKV_DTYPE_F16];
+    const int cus = cu_count();
+    int best = 2;
+    float least = 0.0f;
+    for (int i = 2; i >= 0; --i) {
+        const float t = estimated_us(c[i], expected_load(p, c[i].rows), cus) * (i < 2 ? kSplitMargin : 1.0f);
+        if (i == 2 || t < least) {
+            least = t;
+            best = i;
+        }
+    }
+    return best < 2 || p->head_dim == 64 ? c[best].rows : 0;
+}
+// Whether a call of these lengths runs faster on the 256-row items in the order of
+// a host-built list than in smaller blocks without one (head_dim 128).
+bool list_pays(const vkv_prefill_params* p, const int32_t* qsl, const int32_t* cl) {
+    const ItemCost* const c = kItemCosts[1][p->kv_dtype != VKV_DTYPE_F16];
+    const int cus = cu_count();
+    ItemLoad whole = known_load(p, c[2].rows, qsl, cl);
+    whole.blocks = 0;  // (nothing left to order)
+    const float listed = estimated_us(c[2], whole, cus) - kListSaves;
+    for (int i = 0; i < 2; ++i)
+        if (estimated_us(c[i], known_load(p, c[i].rows, qsl, cl), cus) * kSplitMargin < listed) return false;
+    return true;
 }
 // Row blocks (work items per kv head) of a sequence, at most: with a group of
 // G heads a token brings G rows.
@@ -2063,6 +2166,7 @@ void launch_split(const PrefillArgs& a, int head_dim, int rows, int64_t items, i
     if (head_dim == 64) {
         if (rows == 64) run_split<Split64S<FP8>>(prefill_split_kernel<64, FP8, Split64S<FP8>>, a, items, cus, st);
         else if (rows == 128) run_split<Split64M<FP8>>(prefill_split_kernel<64, FP8, Split64M<FP8>>, a, items, cus, st);
+        else if (a.table_tokens <= kShortContext) run_split<Split64W<FP8>>(prefill_split_kernel<64, FP8, Split64W<FP8>>, a, items, cus, st);
         else run_split<Split64L<FP8>>(prefill_split_kernel<64, FP8, Split64L<FP8>>, a, items, cus, st);
     } else {
         if (rows == 64) run_split<Split128S<FP8>>(prefill_split_kernel<128, FP8, Split128S<FP8>>, a, items, cus, st);
@@ -2097,11 +2201,12 @@ int launch_prefill_mfma(const vkv_prefill_params* p, void* item_space, hipStream
     a.max_blocks_per_seq = p->max_blocks_per_seq;
     a.num_blocks = p->num_blocks;
     // keys any row may see: the table, and the caller's max_context_len clamp
-    int64_t tt = int64_t(p->max_blocks_per_seq) * p->block_size;
-    if (p->max_context_len > 0 && p->max_context_len < tt) tt = p->max_context_len;
+    const int64_t tt = key_bound(p);
     a.table_tokens = int32_t(tt > 0x7FFFFFFF ? 0x7FFFFFFF : tt);
-    const int split = split_rows(p);
-    const int rpi = rows_per_item(p);
+    // a host-built list (of 256-row items) replaces both in-kernel orderings
+    const bool listed = p->head_dim == 128 && p->work_list && p->work_list_words > kListHeaderWords;
+    const int split = listed ? 0 : split_rows(p);
+    const int rpi = split ? split : kListRows;
     a.qblocks = int(max_row_blocks(p, rpi));
     a.num_seqs = p->num_seqs;
     a.scale_log2 = logit_scale_log2(p->scale);
@@ -2114,15 +2219,10 @@ int launch_prefill_mfma(const vkv_prefill_params* p, void* item_space, hipStream
     const int nbins = int(max_tiles + 1 < kMaxLevels ? max_tiles + 1 : kMaxLevels);
     a.rows_per_item = rpi;
     a.nbins = nbins;
-    // Row blocks, at most: a sequence of q >= 2 tokens has ceil(q G / R) <=
-    // q G / R + 1 of them, and there are at most min(S, T / 2) such sequences
-    // (T query tokens).  Small calls order them in the kernel itself.
-    const int64_t T = p->num_query_tokens;
-    const int64_t nseq2 = p->num_seqs < T / 2 ? p->num_seqs : T / 2;
-    const int64_t bound = T * a.group / rpi + nseq2;
-    // a host-built list (of 256-row items) replaces both in-kernel orderings
-    a.work_list = !split && p->work_list && p->work_list_words > kListHeaderWords ? p->work_list : nullptr;
-    a.work_list_words = a.work_list ? p->work_list_words : 0;
+    // (small calls order their row blocks in the kernel itself)
+    const int64_t bound = block_bound(p, rpi);
+    a.work_list = listed ? p->work_list : nullptr;
+    a.work_list_words = listed ? p->work_list_words : 0;
     a.num_query_tokens = int32_t(p->num_query_tokens);
     {
         int sh = 0;
@@ -2160,11 +2260,10 @@ int64_t prefill_work_list_host(const vkv_prefill_params* p, const int32_t* host_
     if (!p || !host_qsl || !host_cl) return -1;
     if (p->num_seqs <= 0 || !prefill_mfma_supported(p)) return 0;  // no list for this call
     const int G = p->num_heads / p->num_kv_heads, hkv = p->num_kv_heads;
-    if (p->head_dim == 64 && (p->kv_dtype != VKV_DTYPE_F16 || G >= 4)) return 0;
-    const int rpi = list_rows(p);
+    if (p->head_dim != 128 || !list_pays(p, host_qsl, host_cl)) return 0;
+    const int rpi = kListRows;
     const int64_t qblocks = max_row_blocks(p, rpi);
-    int64_t tt = int64_t(p->max_blocks_per_seq) * p->block_size;
-    if (p->max_context_len > 0 && p->max_context_len < tt) tt = p->max_context_len;
+    const int64_t tt = key_bound(p);
     // items in (s, b, kvh) order with their key tiles
     struct Item {
         int32_t s, b, kvh, q0, qlen, prior, tiles;
