@@ -284,8 +284,10 @@ int vkv_release_workspace(vkv_stream_t stream);
  * object: every process that runs any of this library's kernels on a device
  * holds those 64 MiB of HBM on it, from the library's first use there until
  * the process ends, whether or not it ever calls this entry point.  A call whose
- * vkv_paged_decode_workspace_size() exceeds 64 MiB fails with
- * VKV_ERR_WORKSPACE before any launch.  All calls on one device share the
+ * partials, in partitions of the size that the library (or partition_size)
+ * takes, exceed 64 MiB fails with VKV_ERR_WORKSPACE before any launch; one whose
+ * equal slices (below that, the kernels of fp16 at head_dim 64 to 128 and fp32 at
+ * 64 split finer) would exceed it runs in fewer.  All calls on one device share the
  * array: calls that overlap on one device (other streams, other threads) race
  * and give wrong results; serialise them.  Calls no hipMalloc or hipFree. */
 int vkv_paged_decode_noalloc(const vkv_decode_params* p, vkv_stream_t stream);

@@ -256,6 +256,37 @@ def test_prefill_workspace_serves_smaller_steps(vkv, head_dim, kv_dtype):
     assert size[0] > 0 and max(size[:-1]) <= size[-1], size
 
 
+# Workspaces of partitions of a fixed size (bytes): the equal slices of
+# decode_stream.hip's shapes need fewer partials than that in calls over many rows,
+# whose slices are an equal share of the resident waves.  (sequences or, "prefill",
+# query tokens that run as rows; H, Hkv, D, table tokens, block size, dtype)
+PARTITIONED = [
+    ("decode", 256, 14, 2, 64, 8192, 16, 1, 14193664),
+    ("decode", 64, 32, 1, 128, 32768, 16, 1, 45794304),
+    ("decode", 8192, 28, 4, 128, 8192, 24, 1, 1312031744),
+    ("decode", 64, 32, 32, 96, 32768, 16, 1, 34522112),
+    ("prefill", 8192, 32, 32, 80, 4096, 16, 1, 515965952),
+    ("prefill", 8192, 32, 32, 96, 32768, 16, 1, 4418765824),
+    ("prefill", 8192, 14, 2, 64, 8192, 16, 0, 333120512),
+]
+
+
+@pytest.mark.parametrize("call", PARTITIONED, ids=lambda c: "-".join(map(str, c[:6])))
+def test_workspace_of_many_rows(vkv, call):
+    kind, rows, H, Hkv, D, tokens, bs, dtype, most = call
+    lib = vkv.load()
+    shape = dict(num_heads=H, num_kv_heads=Hkv, head_dim=D, block_size=bs, max_blocks_per_seq=-(-tokens // bs),
+                 num_blocks=100000, io_dtype=dtype, kv_dtype=dtype)
+    if kind == "decode":
+        p = vkv.DecodeParams(output=16, query=16, key_cache=16, value_cache=16, block_tables=16, context_lens=16,
+                             num_seqs=rows, max_context_len=tokens, scale=0.1, **shape)
+        need = lib.vkv_paged_decode_workspace_size(ctypes.byref(p))
+    else:
+        p = _prefill_params(vkv, num_seqs=8, num_query_tokens=rows, max_query_len=1024, **shape)
+        need = lib.vkv_paged_prefill_workspace_size(ctypes.byref(p))
+    assert 0 < need <= most
+
+
 @pytest.mark.parametrize("shape", [(28, 4, 128, 32, 1, 1), (32, 8, 128, 16, 1, 2), (16, 8, 128, 16, 1, 1),
                                    (32, 2, 128, 16, 1, 1)])
 def test_prefill_work_list_host(vkv, shape):

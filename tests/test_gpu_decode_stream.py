@@ -85,23 +85,58 @@ def test_stream_fused_append(vkv, cuda, H, Hkv, D, bs, table):
         assert np.array_equal(a, b)
 
 
-def test_stream_noalloc_without_room_for_slices(vkv, oracle, cuda):
-    """A call whose slices would not fit the library's array, but whose plain
-    partitions do: accepted, and as right as the call with a workspace."""
+# (rows, contexts, caller's partition size): a call whose finer partials once did not
+# fit the library's array, so that it ran unsplit; many rows of short contexts; and
+# a caller's size whose slices, with one of each row more, do not fit (coarser ones do)
+@pytest.mark.parametrize("S,Hkv,lo,hi,table,size", [(64, 1, 900, 1100, 32768, 0), (400, 2, 1, 40, 4096, 0),
+                                                    (63, 2, 4096, 4096, 4096, 64)])
+def test_stream_noalloc_fits_its_array(vkv, oracle, cuda, S, Hkv, lo, hi, table, size):
+    """Accepted like the call with a workspace and as right, whatever the array holds."""
     import torch
-    H, Hkv, D, bs, S = 32, 2, 128, 16, 400
+    H, D, bs = 32, 128, 16
     rng = np.random.default_rng(3)
-    ctx = rng.integers(1, 40, S)
-    lay, (k, v), q = _case(rng, H, Hkv, D, bs, ctx, 4096)
-    out = torch.zeros((S, H, D), dtype=torch.float16, device=cuda)
-    args = (out, to_dev(q, cuda), to_dev(k, cuda), to_dev(v, cuda), to_dev(lay.block_tables, cuda),
+    ctx = rng.integers(lo, hi + 1, S)
+    lay, (k, v), q = _case(rng, H, Hkv, D, bs, ctx, table)
+    outs = [torch.zeros((S, H, D), dtype=torch.float16, device=cuda) for _ in range(2)]
+    args = (to_dev(q, cuda), to_dev(k, cuda), to_dev(v, cuda), to_dev(lay.block_tables, cuda),
             to_dev(lay.context_lens, cuda), D ** -0.5)
-    assert vkv.decode_workspace_size(*args) > 64 << 20
-    vkv.paged_decode_noalloc(*args)
+    if size:
+        assert vkv.decode_workspace_size(outs[0], *args, partition_size=size) > 64 << 20
+    vkv.paged_decode_noalloc(outs[0], *args, partition_size=size)
+    vkv.paged_decode(outs[1], *args, partition_size=size)
     torch.cuda.synchronize()
+    if not size:  # the same slices
+        assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
+    rows = np.unique(np.linspace(0, S - 1, 12).astype(int))
+    ref = oracle.paged_decode(q[rows].astype(np.float32), np.nan_to_num(k).view(np.uint16),
+                              np.nan_to_num(v).view(np.uint16), np.ascontiguousarray(lay.block_tables[rows]),
+                              np.ascontiguousarray(lay.context_lens[rows]), D ** -0.5)
+    for out in outs:
+        assert_close(to_np(out)[rows].astype(np.float32), ref, F16_ATOL, F16_RTOL, "noalloc and workspace")
+
+
+@pytest.mark.parametrize("S,H,Hkv,D,table", [(17000, 8, 2, 64, 6000), (9000, 4, 2, 96, 6000), (5000, 16, 1, 128, 6000),
+                                             (300, 4, 4, 80, 6000)])
+def test_stream_slices_of_many_rows(vkv, oracle, cuda, S, H, Hkv, D, table):
+    """Equal slices over several launches (8 192 rows each) that share the partials and
+    the rows' places, several rows to a thread of the scan, prefixes too long for two
+    stages per wave, fewer slices than rows, rows without keys: every row against the
+    oracle, and the same bits twice."""
+    import torch
+    rng = np.random.default_rng(S)
+    ctx = rng.integers(0, 40, S)
+    ctx[[0, S // 2, S - 1]] = [700, 1500, 333]
+    lay, (k, v), q = _case(rng, H, Hkv, D, 16, ctx, table)
+    outs = [torch.full((S, H, D), 7.0, dtype=torch.float16, device=cuda) for _ in range(2)]
+    args = (to_dev(q, cuda), to_dev(k, cuda), to_dev(v, cuda), to_dev(lay.block_tables, cuda),
+            to_dev(lay.context_lens, cuda), float(D) ** -0.5)
+    for out in outs:
+        vkv.paged_decode(out, *args)
+    torch.cuda.synchronize()
+    assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
     ref = oracle.paged_decode(q.astype(np.float32), np.nan_to_num(k).view(np.uint16), np.nan_to_num(v).view(np.uint16),
-                              lay.block_tables, lay.context_lens, D ** -0.5)
-    assert_close(to_np(out).astype(np.float32), ref, F16_ATOL, F16_RTOL, "noalloc")
+                              lay.block_tables, lay.context_lens, float(D) ** -0.5, nthreads=8)
+    assert_close(to_np(outs[0]).astype(np.float32), ref, F16_ATOL, F16_RTOL, f"{S} rows in slices")
 
 
 @pytest.mark.parametrize("table", [1024, 6000], ids=["rows", "partitions"])

@@ -512,14 +512,18 @@ __global__ __launch_bounds__(DT ? DT : 1024) void decode_reduce_kernel(DecodeArg
     const int G = a.num_heads / a.num_kv_heads;
     const int kvh = h / G;
     if (a.fkey && h == kvh * G) store_new_token<1>(a, s, kvh, d, D);
-    const int64_t slot0 = (int64_t(s) * a.num_kv_heads + kvh) * a.max_parts * G + (h - kvh * G);
+    // (equal slices: the row's place comes first, and only its own partials)
+    const int2 slices = a.row_parts ? a.row_parts[s] : int2{0, 0};
+    const int last = a.row_parts ? (slices.y > 0 ? slices.y - 1 : 0) : a.max_parts - 1;  // in-bounds slots
+    const int64_t slot0 = (a.row_parts ? int64_t(kvh) * a.part_slots + slices.x
+                                       : (int64_t(s) * a.num_kv_heads + kvh) * a.max_parts) * G + (h - kvh * G);
     const float* ml = a.part_ml + slot0 * 2;
     const float* o = a.part_o + slot0 * D + d;
     float bm[kMergeBatch], bl[kMergeBatch], bo[kMergeBatch];
     auto load_batch = [&](int i0) __attribute__((always_inline)) {
 #pragma unroll
         for (int k = 0; k < kMergeBatch; ++k) {
-            const int i = i0 + k < a.max_parts ? i0 + k : a.max_parts - 1;  // in-bounds slot
+            const int i = i0 + k < last ? i0 + k : last;
             bm[k] = ml[int64_t(i) * G * 2];
             bl[k] = ml[int64_t(i) * G * 2 + 1];
             bo[k] = o[int64_t(i) * G * D];
@@ -532,7 +536,7 @@ __global__ __launch_bounds__(DT ? DT : 1024) void decode_reduce_kernel(DecodeArg
     load_batch(0);
     const int ctx = row_context(a, s);
     const int P = a.num_cands > 1 && !a.row_parts ? __builtin_amdgcn_readfirstlane(a.counters[kChosenPartitionSlot]) : a.P;
-    const int np = a.row_parts ? a.row_parts[s] : ctx > 0 ? (ctx + P - 1) / P : 0;
+    const int np = a.row_parts ? slices.y : ctx > 0 ? (ctx + P - 1) / P : 0;
     float m = -INFINITY, l = 0.0f, acc = 0.0f;
     for (int i0 = 0; i0 < np; i0 += kMergeBatch) {
         if (i0 > 0) load_batch(i0);
@@ -672,18 +676,22 @@ __global__ __launch_bounds__(kWave) void decode_reduce_wave_kernel(DecodeArgs a)
     const int G = a.num_heads / a.num_kv_heads;
     const int kvh = h / G;
     if (a.fkey && h == kvh * G) store_new_token<E>(a, s, kvh, d, DT);
-    const int64_t slot0 = (int64_t(s) * a.num_kv_heads + kvh) * a.max_parts * G + (h - kvh * G);
-    const float* ml = a.part_ml + slot0 * 2;
-    const float* o = a.part_o + slot0 * DT + d;
     if (a.qsl && a.qsl[s + 1] - a.qsl[s] != 1) return;
     int np;
+    int64_t slot0;
     if (a.row_parts) {
-        np = a.row_parts[s];
+        const int2 slices = a.row_parts[s];
+        np = slices.y;
+        slot0 = int64_t(kvh) * a.part_slots + slices.x;
     } else {
         const int ctx = row_context(a, s);
         const int P = a.num_cands > 1 ? __builtin_amdgcn_readfirstlane(a.counters[kChosenPartitionSlot]) : a.P;
         np = ctx > 0 ? (ctx + P - 1) / P : 0;
+        slot0 = (int64_t(s) * a.num_kv_heads + kvh) * a.max_parts;
     }
+    slot0 = slot0 * G + (h - kvh * G);
+    const float* ml = a.part_ml + slot0 * 2;
+    const float* o = a.part_o + slot0 * DT + d;
     // partials of batch i0 (slots past np are neither loaded nor read)
     float bm[B], bl[B];
     fE bo[B];
@@ -748,6 +756,9 @@ int launch_reduce_b(int D, const DecodeArgs& args, int H, int S, hipStream_t st)
 
 template <typename IO>
 int launch_reduce(int D, const DecodeArgs& args, int H, int S, hipStream_t st) {
+    // Many rows to a slice: nearly all have a partial or two (8 192 rows of 1 to 256
+    // tokens, 4/4 heads, head_dim 80, ~310 us: batches of 8 took 7 % longer).
+    if (args.row_parts && S / 8 >= args.max_slices) return launch_reduce_b<IO, 2>(D, args, H, S, st);
     // Few rows cut into many slices: more of a row's partials per round.
     if (args.row_parts && D == 64 && args.max_parts > 16 && H * S <= 2048) return launch_reduce_b<IO, 32>(D, args, H, S, st);
     // Small (static) calls split finely load every partial in one round;
@@ -770,6 +781,13 @@ bool split_in_partitions(const vkv_decode_params* p) {
            matrix_split_shape(p->head_dim, p->num_heads / p->num_kv_heads, p->block_size, p->key_cache, p->value_cache);
 }
 
+// Bytes of one partial of every query head, and of a call in equal slices.
+size_t slot_bytes(const vkv_decode_params* p) { return size_t(p->num_heads) * (p->head_dim + 2) * sizeof(float); }
+size_t stream_bytes(const vkv_decode_params* p, int max_slices) {
+    const size_t rows = size_t(launch_rows_max(p->num_seqs));
+    return kWorkspaceHeader + (rows + max_slices) * slot_bytes(p) + rows * sizeof(int2);
+}
+
 int ilog2(int x) {
     int r = 0;
     while ((1 << r) < x) ++r;
@@ -777,6 +795,16 @@ int ilog2(int x) {
 }
 
 }  // namespace
+
+void fit_decode_plan(const vkv_decode_params* p, size_t bytes, DecodePlan& plan) {
+    if (plan.max_slices <= 0 || stream_bytes(p, plan.max_slices) <= bytes) return;
+    // The slices whose partials, with one of each row more, fit; where the rows
+    // alone are as many, one workgroup per (row, kv head) splits the call as far.
+    const int64_t rows = launch_rows_max(p->num_seqs);
+    const int64_t fit = (int64_t(bytes) - int64_t(stream_bytes(p, 0))) / int64_t(slot_bytes(p));
+    if (fit > rows) plan.max_slices = int(fit);
+    else plan.whole_rows = true;
+}
 
 DecodePlan plan_decode(const vkv_decode_params* p) {
     DecodePlan plan;
@@ -840,26 +868,36 @@ DecodePlan plan_decode(const vkv_decode_params* p) {
     }
     plan.max_parts = int((max_ctx + smallest - 1) / smallest);
     if (plan.max_parts < 1) plan.max_parts = 1;
-    const size_t rows = size_t(launch_rows_max(p->num_seqs));
-    const size_t part_bytes = rows * p->num_heads * (p->head_dim + 2) * sizeof(float);  // one partial of every row
-    plan.base_bytes = plan.workspace_bytes = kWorkspaceHeader + part_bytes * plan.max_parts;
+    const int64_t rows = launch_rows_max(p->num_seqs);
+    plan.base_bytes = plan.workspace_bytes = kWorkspaceHeader + size_t(rows) * plan.max_parts * slot_bytes(p);
     plan.whole_rows = false;
+    plan.max_slices = 0;
     plan.stream = stream_shape(p);
     if (plan.stream && !split_in_partitions(p)) {
-        // Equal slices (decode_stream.hip): partials for slices of down to
-        // kSliceTokens tokens, at most kMaxSplitParts of a row and one more (a
-        // row's first and last slice are shared with its neighbours).  A
-        // caller's size is rounded up to whole steps of 32 tokens.
+        // Equal slices (decode_stream.hip) of down to kSliceTokens tokens, at most
+        // kMaxSplitParts of a row and one more (a row's first and last slice are
+        // shared with its neighbours), and no more of the call than its resident
+        // waves could run together.  A caller's size is rounded up to whole steps
+        // of 32 tokens.
         const bool own = p->partition_size <= 0;
         const int64_t slice = own ? kSliceTokens : (int64_t(P) + 31) / 32 * 32;
         int64_t parts = (max_ctx + slice - 1) / slice;
         if (own && parts > kMaxSplitParts) parts = kMaxSplitParts;
         parts = parts < 1 ? 2 : parts + 1;
         if (own && parts < plan.max_parts) parts = plan.max_parts;
+        int64_t slices = rows * (parts - 1);
+        if (own) {
+            const int64_t together = stream_split_waves(p->head_dim, p->io_dtype == VKV_DTYPE_F32) / p->num_kv_heads;
+            slices = slices < together ? slices : (together > 0 ? together : 1);
+        }
         plan.partition_size = int(slice);
         plan.num_candidates = own ? 2 : 1;  // 2: the kernel sizes the slices
         plan.max_parts = int(parts);
-        plan.workspace_bytes = kWorkspaceHeader + part_bytes * plan.max_parts + rows * sizeof(int32_t);
+        plan.max_slices = int(slices < (int64_t(1) << 30) ? slices : int64_t(1) << 30);
+        // (never less than the partitions' workspace: a size asked for with
+        // 16-byte aligned caches serves others too)
+        const size_t bytes = stream_bytes(p, plan.max_slices);
+        if (bytes > plan.workspace_bytes) plan.workspace_bytes = bytes;
     }
     return plan;
 }
@@ -899,7 +937,9 @@ int launch_rows(const vkv_decode_params* p, const DecodePlan& plan, void* worksp
     a.row_ctx = row_ctx;
     a.qsl = qsl;
     const int rows = launch_rows_max(p->num_seqs);
-    const size_t o_elems = size_t(rows) * p->num_heads * plan.max_parts * p->head_dim;
+    const bool split_streams = plan.max_slices > 0;
+    const size_t slots = split_streams ? size_t(plan.max_slices) + rows : size_t(rows) * plan.max_parts;
+    const size_t o_elems = slots * p->num_heads * p->head_dim;
     a.counters = static_cast<int*>(workspace);
     a.part_o = reinterpret_cast<float*>(static_cast<char*>(workspace) + kWorkspaceHeader);
     a.part_ml = a.part_o + o_elems;
@@ -933,9 +973,9 @@ int launch_rows(const vkv_decode_params* p, const DecodePlan& plan, void* worksp
     const int D = p->head_dim;
     const int io_eb = p->io_dtype == VKV_DTYPE_F32 ? 4 : 2;
     const bool fixed = fixed_decode_shape(D, G, p->block_size, p->key_cache, p->value_cache);
-    const bool split_streams = plan.stream && !split_in_partitions(p);
-    a.row_parts = split_streams ? reinterpret_cast<int32_t*>(a.part_ml + size_t(rows) * p->num_heads * plan.max_parts * 2)
-                                : nullptr;
+    a.row_parts = split_streams ? reinterpret_cast<int2*>(a.part_ml + slots * p->num_heads * 2) : nullptr;
+    a.max_slices = plan.max_slices;
+    a.part_slots = split_streams ? int32_t(slots) : 0;
     const bool matrix = split_in_partitions(p);
     a.head_dim = D;
     a.block_size = p->block_size;

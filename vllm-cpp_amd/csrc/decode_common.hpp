@@ -89,10 +89,15 @@ struct DecodeArgs {
     // prefix scan, no claims, and items request their block ids together with
     // the context length.  0: the persistent claim loop.
     int32_t static_parts;
-    // decode_stream.hip's split calls: partials of each row (written by the
-    // partition launch, read by the merge), nullptr for the other kernels
-    // (whose rows have ceil(context / P)).
-    int32_t* row_parts;
+    // decode_stream.hip's split calls: each row's first partial and their number
+    // (written by the partition launch, read by the merge), nullptr for the
+    // other kernels (whose rows have ceil(context / P), max_parts apart).  The
+    // partial of (slice, row, kv head) is number kvh * part_slots + slice + row:
+    // from one of a kv head's partials to the next the slice or the row goes up,
+    // so part_slots = max_slices + rows hold them all.
+    int2* row_parts;
+    int32_t max_slices;
+    int32_t part_slots;
     // Append fused into the call (source rows in the cache's element type,
     // fp16 or fp32; fixed shapes): row s's new token is fkey / fval + s *
     // stride (bytes), bound for cache slot fslots[s].  The partition kernel
@@ -147,6 +152,9 @@ inline bool matrix_split_shape(int head_dim, int group, int block_size, const vo
 // merged in LDS, instead of split-K.  half_dims: a head's row in fp16 elements'
 // bytes (head_dim; twice that in fp32, half in FP8).
 bool stream_decode_rows(int num_rows, int num_kv_heads, int half_dims, int max_ctx, bool matrix_split);
+// Waves that a split launch of decode_stream.hip keeps resident, at most: slices of
+// the kv heads together beyond that would not start sooner.
+int stream_split_waves(int head_dim, bool f32);
 // The call's partition launch (or, with rows, its only launch).  0 or VKV_ERR_*.
 int launch_decode_stream(DecodeArgs& a, bool f32, bool rows, size_t lds, hipStream_t st);
 

@@ -56,8 +56,7 @@ extern "C" int vkv_paged_decode_noalloc(const vkv_decode_params* p, vkv_stream_t
                                  "vkv_paged_decode_noalloc: the call needs %zu bytes of split-K scratch, more than "
                                  "the %zu the library holds; use vkv_paged_decode with a workspace",
                                  plan.base_bytes, kScratchBytes);
-    // a finer split than the array holds: one workgroup per (row, kv head), which needs no scratch
-    plan.whole_rows = plan.workspace_bytes > kScratchBytes;
+    vkv::fit_decode_plan(p, kScratchBytes, plan);
     void* ws = nullptr;
     rc = scratch_address(&ws);
     if (rc != VKV_OK) return rc;

@@ -600,8 +600,9 @@ __global__ __launch_bounds__(64 * W) void decode_rows_kernel(const DecodeArgs a)
 // context lengths, where partitions of a fixed size leave some waves a second
 // one (256 rows of head_dim 64, contexts up to 4 096: 66 to 78 us over sizes
 // 128 to 512, 57 at the best of them).  A row's partials are its slices in
-// order; row_parts holds their number for the merge kernel.  Slices are at
-// least so long that no row has more than max_parts of them.
+// order; row_parts holds the first one and their number for the merge kernel.
+// Slices are at least so long that no row has more than max_parts of them, and the
+// call no more than max_slices.
 constexpr int kMinSliceSteps = 2;
 // Building with -DVKV_STREAM_ROWS=1 (2) runs every launch as one workgroup per
 // (row, kv head) (in equal slices): an A/B switch.
@@ -657,16 +658,18 @@ __global__ __launch_bounds__(256) void decode_stream_kernel(const DecodeArgs a) 
     int longest = 0;
     for (int w = 0; w < kWavesPerBlock; ++w) longest = max(longest, wave_longest[w]);
     // Steps per slice: an equal share of every resident wave (a size the
-    // caller asked for instead, a.P), within max_parts partials per row.
+    // caller asked for instead, a.P), within max_parts partials per row and
+    // max_slices slices.
     const int waves = int(gridDim.x) * kWavesPerBlock;
     const int share = waves / a.num_kv_heads > 0 ? waves / a.num_kv_heads : 1;
     int R = a.num_cands > 1 ? max((total + share - 1) / share, kMinSliceSteps) : a.P / kStep;
     R = max(R, (longest + a.max_parts - 2) / (a.max_parts - 1));
+    R = max(R, (total + a.max_slices - 1) / a.max_slices);
     R = __builtin_amdgcn_readfirstlane(max(R, 1));
     if (blockIdx.x == 0) {
         for (int r = int(threadIdx.x); r < nrows; r += kBlockThreads) {
             const int b = prefix[r], e = prefix[r + 1];
-            a.row_parts[r] = e > b ? (e - 1) / R - b / R + 1 : 0;
+            a.row_parts[r] = int2{b / R + r, e > b ? (e - 1) / R - b / R + 1 : 0};
         }
     }
     const int items = (total + R - 1) / R * a.num_kv_heads;
@@ -696,7 +699,7 @@ __global__ __launch_bounds__(256) void decode_stream_kernel(const DecodeArgs a) 
             State<D, CT, KVT> st;
             init_state(a, st, s, kvh, G, lane);
             stream_tokens<D, CT, KVT, NST>(a, st, lds + wave * kRing, s, table, ctx, kvh, t0, n, win, ids, lane);
-            const int64_t slot = (int64_t(s) * a.num_kv_heads + kvh) * a.max_parts + (slice - b / R);
+            const int64_t slot = int64_t(kvh) * a.part_slots + slice + s;
 #pragma unroll
             for (int c = 0; c < CT; ++c) {
                 const int h = 16 * c + col;
@@ -828,6 +831,12 @@ bool stream_decode_rows(int num_rows, int num_kv_heads, int half_dims, int max_c
     if (half_dims % 64 != 0) return max_ctx <= (pairs < 2 * cus ? 1056 : pairs < 8 * cus ? 528 : 264);
     const int64_t row_bytes = int64_t(max_ctx) * half_dims * 4;
     return max_ctx <= 2112 && (row_bytes <= 528 << 10 || (pairs >= cus && !matrix_split));
+}
+
+int stream_split_waves(int head_dim, bool f32) {
+    // (stages as launch_shape takes them; two stages at the wider heads: fewer)
+    const int stage = 2 * kStep * head_dim * (f32 ? 4 : 2) * (head_dim == 64 && !f32 ? 2 : 1);
+    return device_cu_count() * (kLdsPerCu / (1024 + kWavesPerBlock * stage)) * kWavesPerBlock;
 }
 
 template <int KVT, int NST>

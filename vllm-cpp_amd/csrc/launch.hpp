@@ -33,14 +33,18 @@ struct DecodePlan {
     size_t workspace_bytes;
     int num_candidates;
     int candidates[kMaxPartitionCandidates];
-    // decode_stream.hip's shapes.  base_bytes: the workspace without their
-    // finer split (workspace_bytes for every other shape); whole_rows: run
-    // every launch as one workgroup per (row, kv head), which needs none.
+    // decode_stream.hip's shapes.  base_bytes: the workspace of partitions of a
+    // fixed size (every other shape's); max_slices > 0: the call's equal slices, at
+    // most; whole_rows: run every launch as one workgroup per (row, kv head), which
+    // needs no partials.
     bool stream;
     bool whole_rows;
+    int max_slices;
     size_t base_bytes;
 };
 DecodePlan plan_decode(const vkv_decode_params* p);
+// Fewer slices, so that the plan's partials take at most `bytes` (>= base_bytes).
+void fit_decode_plan(const vkv_decode_params* p, size_t bytes, DecodePlan& plan);
 int launch_decode(const vkv_decode_params* p, const DecodePlan& plan, void* workspace, hipStream_t st);
 // An append of one new token per sequence fused into the decode (fp16 source
 // and cache, fixed shapes, the same pool and geometry on both sides): the
