@@ -254,13 +254,18 @@ int vkv_paged_decode(const vkv_decode_params* p, vkv_stream_t stream);
  * — token s of ap is sequence s's new token (ap->num_tokens == dp->num_seqs),
  * both name the same fp16 or fp32 caches with the same geometry and pool,
  * source rows of the cache's type, 16-byte aligned with token strides a
- * multiple of 16 bytes, and a shape the tuned decode kernels run — the append
- * is fused into the decode
- * launches (one launch fewer per step): each sequence's last position is read
- * from its new rows when ap's slot for the token is that position's slot, and
- * the merge kernel stores the rows.  The fused form assumes what a decode step
- * guarantees: the slot of an appended token is read in this call only as its
- * own sequence's last position (a slot of no other sequence's context).
+ * multiple of 16 bytes, and a shape the tuned decode kernels run (16-byte
+ * aligned caches at head_dim 64, 128 or 256 with groups of up to 8 and blocks of
+ * a power of two up to 1 024, or fp16 at head_dim 64 to 128 in steps of 16 and
+ * fp32 at 64 with groups of up to 32 and any blocks) — the append is fused into
+ * the decode launches (one launch fewer per step): each sequence's last position
+ * is read from its new rows when ap's slot for the token is that position's
+ * slot, and the rows are stored in the same launches: by the merge kernel where
+ * the call splits, by the workgroup that has read that position where one
+ * workgroup attends a whole (sequence, kv head).  The fused form assumes what a
+ * decode step guarantees: the slot of an appended token is read in this call
+ * only as its own sequence's last position (a slot of no other sequence's
+ * context; another sequence that reads it may see it before or after the store).
  * Otherwise the two calls run as they are. */
 int vkv_paged_decode_append(const vkv_append_params* ap, const vkv_decode_params* dp, vkv_stream_t stream);
 

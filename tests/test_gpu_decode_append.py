@@ -14,12 +14,12 @@ from helpers import to_dev
 pytestmark = pytest.mark.gpu
 
 
-def _case(rng, H, Hkv, D, bs, prev, extra_blocks=4, sigma=0.5):
+def _case(rng, H, Hkv, D, bs, prev, extra_blocks=4, sigma=0.5, table_tokens=0):
     from vllm_kv_amd import workloads
     prev = np.asarray(prev, np.int32)
     ctx = prev + 1
     need = int(sum((c + bs - 1) // bs for c in ctx))
-    lay = workloads.make_layout(ctx, bs, rng, num_blocks=need + extra_blocks)
+    lay = workloads.make_layout(ctx, bs, rng, num_blocks=need + extra_blocks, max_blocks_per_seq=table_tokens // bs)
     N = lay.num_blocks
     k = (rng.standard_normal((N, bs, Hkv, D), dtype=np.float32) * sigma).astype(np.float16)
     v = (rng.standard_normal((N, bs, Hkv, D), dtype=np.float32) * sigma).astype(np.float16)
@@ -58,12 +58,12 @@ def _assert_same(vkv, cuda, case, **kw):
 
 CASES = [
     # (H, Hkv, D, bs, previous context per sequence): kernels reached
-    (32, 8, 128, 16, None),                        # C2's 64 sequences: matrix-core claim loop
-    (14, 2, 64, 16, [0, 15, 16, 300]),             # small call: static grid, VALU items at D 64
+    (32, 8, 128, 16, None),                        # C2's 64 sequences: partitions
+    (14, 2, 64, 16, [0, 15, 16, 300]),             # small call: one workgroup per row and kv head
     (28, 4, 128, 32, [0, 31, 32, 700, 2047]),      # new token opening a block; bs 32
-    (16, 8, 256, 8, [8, 64, 519]),                 # D 256, blocks of 8 (VALU items), wave merge of 4 per lane
+    (16, 8, 256, 8, [8, 64, 519]),                 # D 256, blocks of 8 (VALU items, static grid), wave merge of 4 per lane
     (8, 8, 128, 16, list(range(5, 3000, 75))),     # group 1, many partitions per row
-    (32, 4, 128, 64, [3, 900, 4000]),              # group 8, blocks larger than a chunk
+    (32, 4, 128, 64, [3, 900, 4000]),              # group 8, blocks larger than a step
 ]
 
 
@@ -79,7 +79,7 @@ def test_decode_append_matches_two_calls(vkv, cuda, H, Hkv, D, bs, prev):
 @pytest.mark.parametrize("H,Hkv,D,bs,prev", [(32, 8, 128, 16, [4, 299, 1000]), (14, 2, 64, 16, [0, 15, 16, 300]),
                                                (16, 8, 256, 8, [8, 64, 519])])
 def test_decode_append_f32_cache(vkv, cuda, H, Hkv, D, bs, prev):
-    """The reference's own dtype: fp32 query, rows, cache and output (VALU items)."""
+    """The reference's own dtype: fp32 query, rows, cache and output."""
     rng = np.random.default_rng(H + D)
     lay, k, v, q, nk, nv, slots = _case(rng, H, Hkv, D, bs, prev)
     case = (lay, k.astype(np.float32), v.astype(np.float32), q.astype(np.float32), nk.astype(np.float32),
@@ -139,15 +139,18 @@ def test_decode_append_fp8_cache_runs_both_calls(vkv, cuda):
     assert res[0] == res[1]
 
 
-@pytest.mark.parametrize("prev", [[100, 50, 300], [100, 50] + list(range(300, 1060, 20))])  # static grid, claim loop
-def test_decode_append_is_fused(vkv, cuda, prev):
+# Tables past the lengths that run as one launch, whose workgroups store the rows
+# while others still read: in the calls that split, the merge launch stores them.
+@pytest.mark.parametrize("prev", [[100, 50, 300], [100, 50] + list(range(300, 1060, 20))])
+@pytest.mark.parametrize("H,Hkv,D", [(32, 8, 128), (32, 2, 128), (14, 2, 64), (8, 8, 256)])
+def test_decode_append_is_fused(vkv, cuda, H, Hkv, D, prev):
     """The fused form reads an appended slot from the new rows only at its own
     sequence's last position: a token bound for a slot inside another
     sequence's context (outside what a decode step does) is seen there by the
     two calls but not by the fused call.  So the outputs differ exactly for
     that other sequence, which shows the fused launches ran."""
     rng = np.random.default_rng(17)
-    lay, k, v, q, nk, nv, slots = _case(rng, 32, 8, 128, 16, prev)
+    lay, k, v, q, nk, nv, slots = _case(rng, H, Hkv, D, 16, prev, table_tokens=6000)
     slots = slots.copy()
     slots[1] = int(lay.block_tables[0, 2]) * 16 + 3  # position 35 of sequence 0
     a = _run(vkv, cuda, lay, k, v, q, nk, nv, slots, fused=False)
@@ -165,14 +168,15 @@ def test_decode_append_rows_beyond_one_launch(vkv, cuda):
     _assert_same(vkv, cuda, _case(rng, 4, 2, 64, 16, prev))
 
 
-@pytest.mark.parametrize("prev", [[3, 60, 300], [100, 50] + list(range(300, 1060, 20))])  # static grid, claim loop
-def test_decode_append_graph_replays(vkv, cuda, prev):
+@pytest.mark.parametrize("table", [0, 6000], ids=["rows", "partitions"])
+@pytest.mark.parametrize("prev", [[3, 60, 300], [100, 50] + list(range(300, 1060, 20))])
+def test_decode_append_graph_replays(vkv, cuda, prev, table):
     """The fused call captured in a HIP graph replays to the eager result (the
     append stores the same rows each time), with eager calls on the capture
     stream's library workspace and synchronisations between the replays."""
     import torch
     rng = np.random.default_rng(23)
-    lay, k, v, q, nk, nv, slots = _case(rng, 32, 8, 128, 16, prev)
+    lay, k, v, q, nk, nv, slots = _case(rng, 32, 8, 128, 16, prev, table_tokens=table)
     kc, vc = to_dev(k, cuda), to_dev(v, cuda)
     args = (to_dev(q, cuda), kc, vc, to_dev(lay.block_tables, cuda), to_dev(lay.context_lens, cuda),
             1.0 / np.sqrt(128), to_dev(nk, cuda), to_dev(nv, cuda), to_dev(slots, cuda))

@@ -99,11 +99,13 @@ struct DecodeArgs {
     int32_t max_slices;
     int32_t part_slots;
     // Append fused into the call (source rows in the cache's element type,
-    // fp16 or fp32; fixed shapes): row s's new token is fkey / fval + s *
+    // fp16 or fp32; fixed and streamed shapes): row s's new token is fkey / fval + s *
     // stride (bytes), bound for cache slot fslots[s].  The partition kernel
     // reads row s's last position from these rows when that position's slot
-    // is fslots[s] (its K/V as the append would leave them); the merge kernel
-    // stores the rows into slots in [0, fnum_slots).  fkey == NULL: no append.
+    // is fslots[s] (its K/V as the append would leave them); the rows are stored
+    // into slots in [0, fnum_slots) by the merge kernel, or, where one workgroup
+    // attends a (row, kv head), by that workgroup at its end.  fkey == NULL: no
+    // append.
     const char* fkey;
     const char* fval;
     int64_t fkey_stride;

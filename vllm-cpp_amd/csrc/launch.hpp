@@ -46,10 +46,11 @@ DecodePlan plan_decode(const vkv_decode_params* p);
 // Fewer slices, so that the plan's partials take at most `bytes` (>= base_bytes).
 void fit_decode_plan(const vkv_decode_params* p, size_t bytes, DecodePlan& plan);
 int launch_decode(const vkv_decode_params* p, const DecodePlan& plan, void* workspace, hipStream_t st);
-// An append of one new token per sequence fused into the decode (fp16 source
-// and cache, fixed shapes, the same pool and geometry on both sides): the
-// partition kernel reads each row's last position from the new rows when the
-// append targets that position's slot, and the merge kernel stores the rows.
+// An append of one new token per sequence fused into the decode (source and cache
+// both fp16 or both fp32, fixed and streamed shapes, the same pool and geometry on
+// both sides): each row's last position is read from the new rows when the append
+// targets that position's slot, and the decode launches store the rows
+// (DecodeArgs::fkey).
 bool decode_append_fusable(const vkv_append_params* ap, const vkv_decode_params* p);
 int launch_decode_append(const vkv_append_params* ap, const vkv_decode_params* p, const DecodePlan& plan,
                          void* workspace, hipStream_t st);
