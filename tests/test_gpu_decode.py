@@ -21,11 +21,11 @@ def _pool(rng, N, bs, Hkv, D, sigma):
     return k, v
 
 
-def _layout(rng, ctx, bs, extra_blocks=3):
+def _layout(rng, ctx, bs, extra_blocks=3, table_tokens=0):
     from vllm_kv_amd import workloads
     need = int(sum((c + bs - 1) // bs for c in ctx))
     return workloads.make_layout(np.asarray(ctx, np.int32), bs, rng, num_blocks=max(need + extra_blocks, 1),
-                                 max_blocks_per_seq=max(1, max((c + bs - 1) // bs for c in ctx)))
+                                 max_blocks_per_seq=max(1, table_tokens // bs, max((c + bs - 1) // bs for c in ctx)))
 
 
 def _run_decode(vkv, cuda, q, k, v, lay, scale, io, **kw):
@@ -546,14 +546,15 @@ def test_decode_library_workspace_capture_rules(vkv, cuda):
         assert torch.equal(scratch.view(torch.int16), ref.view(torch.int16)), i
 
 
-def test_decode_rows_beyond_one_launch(vkv, oracle, cuda):
+@pytest.mark.parametrize("table", [0, 6000], ids=["rows", "slices"])
+def test_decode_rows_beyond_one_launch(vkv, oracle, cuda, table):
     """More sequences than one partition launch holds (8192 rows): the library
     splits the call into consecutive row ranges; every row against the oracle."""
     import torch
     S, H, Hkv, D, bs = 17000, 8, 2, 64, 16
     rng = np.random.default_rng(8)
     ctx = rng.integers(1, 40, size=S).astype(np.int32)
-    lay = _layout(rng, ctx, bs)
+    lay = _layout(rng, ctx, bs, table_tokens=table)
     k, v = _pool(rng, lay.num_blocks, bs, Hkv, D, 0.5)
     q = (rng.standard_normal((S, H, D), dtype=np.float32) * 0.5).astype(np.float16)
     ref = oracle.paged_decode(q.astype(np.float32), k.view(np.uint16), v.view(np.uint16), lay.block_tables,
@@ -562,19 +563,20 @@ def test_decode_rows_beyond_one_launch(vkv, oracle, cuda):
     assert_close(got, ref, F16_ATOL, F16_RTOL, "17000 sequences")
 
 
-@pytest.mark.parametrize("H,Hkv,D", [(8, 8, 64), (32, 8, 128)])
+@pytest.mark.parametrize("H,Hkv,D", [(8, 8, 64), (32, 8, 128), (8, 4, 256)])
 def test_decode_more_groups_than_grid(vkv, oracle, cuda, H, Hkv, D):
     """A batch with many more work groups (4 kv-head items each) than the grid,
     which holds one workgroup per resident slot (at most 8 per CU): the groups
-    past the grid are dealt to the workgroups in later rounds (matrix-core
-    kernel, D 128) or claimed through the workspace counters (VALU kernel,
-    D 64).  Sampled sequences against the oracle; a second call must agree bit
+    past the grid are taken in later rounds (equal slices, D 64), dealt to the
+    workgroups in a snake (partitions on the matrix cores, D 128) or claimed
+    through the workspace counters (VALU kernel, D 256).  (Tables past the
+    lengths that run as one workgroup per row and kv head.)  Sampled sequences against the oracle; a second call must agree bit
     for bit (the counters return to zero)."""
     import torch
     S, bs, P = 2048, 16, 64
     rng = np.random.default_rng(D + H)
     ctx = rng.integers(150, 260, size=S).astype(np.int32)
-    lay = _layout(rng, ctx, bs)
+    lay = _layout(rng, ctx, bs, table_tokens=6000)
     groups = int(sum((c + P - 1) // P for c in ctx)) * Hkv // 4
     cus = torch.cuda.get_device_properties(cuda).multi_processor_count
     assert groups > 16 * cus, (groups, cus)

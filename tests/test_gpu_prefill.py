@@ -87,8 +87,8 @@ def whole_items_list(qsl, ctx, group, kv_heads, lists=256):
     (28, 4, 128, 32, [64, 1, 1, 33], [100, 500, 0, 7]),
     (14, 2, 64, 16, [40], [0]),
     (16, 2, 128, 16, [40, 3, 1], [10, 0, 77]),      # group 8
-    (8, 8, 64, 8, [70, 2], [9000, 5]),              # MHA; 1131 blocks: FP8 D 64 kernel's 1024-id window reloads
-    (8, 8, 64, 8, [40, 3], [17000, 9]),             # 2130 blocks: the wide kernels' 2048-id window refills
+    (8, 8, 64, 8, [70, 2], [9000, 5]),              # MHA; 1 131 blocks
+    (8, 8, 64, 8, [40, 3], [17000, 9]),             # 2 130 blocks: the 2 048-id window refills
     (8, 2, 128, 8, [20, 1], [16500, 40]),           # the same at D 128
     (16, 4, 128, 64, [33, 1, 100], [64, 0, 129]),   # blocks larger than a key tile
     (12, 4, 128, 16, [2, 31, 32, 65], [0, 1, 15, 300]),
@@ -197,11 +197,12 @@ def test_prefill_small_blocks_vs_oracle(vkv, oracle, cuda, bs):
     import torch
     ref = oracle.paged_prefill(q.astype(np.float32), k.view(np.uint16), v.view(np.uint16), lay.block_tables,
                                ctx, qsl, scale)
-    out = torch.zeros(q.shape, dtype=torch.float16, device=cuda)
-    vkv.paged_prefill(out, to_dev(q, cuda), to_dev(k, cuda), to_dev(v, cuda), to_dev(lay.block_tables, cuda),
-                      to_dev(ctx, cuda), to_dev(qsl, cuda), int(np.diff(qsl).max()), scale)
-    torch.cuda.synchronize()
-    assert_close(to_np(out).astype(np.float32), ref, F16_ATOL, F16_RTOL, f"prefill bs{bs}")
+    for wl in (None, to_dev(whole_items_list(qsl, ctx, H // Hkv, Hkv), cuda)):
+        out = torch.zeros(q.shape, dtype=torch.float16, device=cuda)
+        vkv.paged_prefill(out, to_dev(q, cuda), to_dev(k, cuda), to_dev(v, cuda), to_dev(lay.block_tables, cuda),
+                          to_dev(ctx, cuda), to_dev(qsl, cuda), int(np.diff(qsl).max()), scale, work_list=wl)
+        torch.cuda.synchronize()
+        assert_close(to_np(out).astype(np.float32), ref, F16_ATOL, F16_RTOL, f"prefill bs{bs}")
 
 
 @pytest.mark.parametrize("H,Hkv,D,bs", [(28, 4, 128, 32), (16, 2, 64, 16)])  # groups 7 and 8
@@ -229,13 +230,14 @@ def test_prefill_scale_zero(vkv, oracle, cuda, kvt, H, Hkv, D, bs):
     (kc, vc, ks, vs), (hk, hv, hks, hvs) = _cache(vkv, cuda, kvt, k, v)
     ref = oracle.paged_prefill(q.astype(np.float32), hk, hv, lay.block_tables, ctx, qsl, 0.0,
                                key_scales=hks, value_scales=hvs, nthreads=_threads())
-    out = torch.zeros((q.shape[0], H, D), dtype=torch.float16, device=cuda)
-    vkv.paged_prefill(out, to_dev(q, cuda), kc, vc, to_dev(lay.block_tables, cuda), to_dev(ctx, cuda),
-                      to_dev(qsl, cuda), 200, 0.0, key_scales=ks, value_scales=vs)
-    torch.cuda.synchronize()
-    got = to_np(out).astype(np.float32)
-    assert np.isfinite(got).all()
-    assert_close(got, ref, F16_ATOL, F16_RTOL, f"scale 0 prefill ({kvt} cache)")
+    for wl in (None, to_dev(whole_items_list(qsl, ctx, H // Hkv, Hkv), cuda)):  # (read at head_dim 128)
+        out = torch.zeros((q.shape[0], H, D), dtype=torch.float16, device=cuda)
+        vkv.paged_prefill(out, to_dev(q, cuda), kc, vc, to_dev(lay.block_tables, cuda), to_dev(ctx, cuda),
+                          to_dev(qsl, cuda), 200, 0.0, key_scales=ks, value_scales=vs, work_list=wl)
+        torch.cuda.synchronize()
+        got = to_np(out).astype(np.float32)
+        assert np.isfinite(got).all()
+        assert_close(got, ref, F16_ATOL, F16_RTOL, f"scale 0 prefill ({kvt} cache)")
 
 
 def test_prefill_many_items(vkv, oracle, cuda):
@@ -345,24 +347,27 @@ def test_prefill_large_call_list_kernel(vkv, oracle, cuda, kvt):
     assert_close(got[rows], ref, F16_ATOL, F16_RTOL, f"720-block call ({kvt} cache), every row of 4 sequences")
 
 
-def _mixed_inputs(cuda):
+def _mixed_inputs(cuda, blocks):
+    """blocks: "split", few rows beside long contexts (blocks of 64 rows), or "whole",
+    enough prompts to fill the 256-row items of the one-wave kernels."""
     import torch
     rng = np.random.default_rng(31)
     H, Hkv, D, bs = 28, 4, 128, 32
-    q_lens = [300, 1, 1, 77, 1, 1, 1, 200] + [1] * 40
-    prior = rng.integers(0, 3000, len(q_lens)).tolist()
+    q_lens = [300, 1, 1, 77, 1, 1, 1, 200] + [260, 130, 90, 300] * (4 if blocks == "whole" else 0) + [1] * 40
+    prior = rng.integers(0, 600 if blocks == "whole" else 3000, len(q_lens)).tolist()
     lay, ctx, qsl, q, k, v, scale = _case(H, Hkv, D, bs, q_lens, prior, 9)
     args = [to_dev(x, cuda) for x in (q, k, v, lay.block_tables, ctx, qsl)]
     out = torch.zeros((q.shape[0], H, D), dtype=torch.float16, device=cuda)
     return out, args, int(max(q_lens)), scale
 
 
-def test_prefill_mixed_on_caller_stream(vkv, cuda):
+@pytest.mark.parametrize("blocks", ["split", "whole"])
+def test_prefill_mixed_on_caller_stream(vkv, cuda, blocks):
     """A mixed call (matrix-core rows and single-token decode rows) issued on a
     non-default stream: after synchronising only that stream the output is
     complete and equals a call on the default stream bit for bit."""
     import torch
-    out, args, mql, scale = _mixed_inputs(cuda)
+    out, args, mql, scale = _mixed_inputs(cuda, blocks)
     vkv.paged_prefill(out, *args, mql, scale)
     torch.cuda.synchronize()
     s = torch.cuda.Stream()
@@ -376,14 +381,15 @@ def test_prefill_mixed_on_caller_stream(vkv, cuda):
         assert torch.equal(out.view(torch.int16), out2.view(torch.int16))
 
 
-def test_prefill_mixed_graph_replays(vkv, cuda):
+@pytest.mark.parametrize("blocks", ["split", "whole"])
+def test_prefill_mixed_graph_replays(vkv, cuda, blocks):
     """A mixed call captured in a graph (work-list, prefill, decode and merge
     kernels; the claim counters are reset by kernels, not memsets) replays to
     the eager result, with eager calls on the capture stream's library
     workspace and synchronisations between the replays.  The capture stream's
     workspace is sized by one eager call first (it cannot grow under capture)."""
     import torch
-    out, args, mql, scale = _mixed_inputs(cuda)
+    out, args, mql, scale = _mixed_inputs(cuda, blocks)
     vkv.paged_prefill(out, *args, mql, scale)
     torch.cuda.synchronize()
     ref = out.clone()
@@ -424,11 +430,12 @@ def test_prefill_context_shorter_than_chunk(vkv, oracle, cuda):
     ref = oracle.paged_prefill(q.astype(np.float32), k.view(np.uint16), v.view(np.uint16), lay.block_tables,
                                ctx, qsl, scale)
     assert not ref[:29].any() and not ref[40:73].any()  # no key before position 0
-    out = torch.full((q.shape[0], H, D), 7.0, dtype=torch.float16, device=cuda)
-    vkv.paged_prefill(out, to_dev(q, cuda), to_dev(k, cuda), to_dev(v, cuda), to_dev(lay.block_tables, cuda),
-                      to_dev(ctx, cuda), to_dev(qsl, cuda), int(q_lens.max()), scale)
-    torch.cuda.synchronize()
-    assert_close(to_np(out).astype(np.float32), ref, F16_ATOL, F16_RTOL, "prefill")
+    for wl in (None, to_dev(whole_items_list(qsl, ctx, H // Hkv, Hkv), cuda)):
+        out = torch.full((q.shape[0], H, D), 7.0, dtype=torch.float16, device=cuda)
+        vkv.paged_prefill(out, to_dev(q, cuda), to_dev(k, cuda), to_dev(v, cuda), to_dev(lay.block_tables, cuda),
+                          to_dev(ctx, cuda), to_dev(qsl, cuda), int(q_lens.max()), scale, work_list=wl)
+        torch.cuda.synchronize()
+        assert_close(to_np(out).astype(np.float32), ref, F16_ATOL, F16_RTOL, "prefill")
 
 
 def test_prefill_f32_rows(vkv, oracle, cuda):
@@ -485,29 +492,31 @@ def test_prefill_growing_logits(vkv, oracle, cuda, kvt):
                               slots, ks, vs)
         torch.cuda.synchronize()
         hk, hv, hks, hvs = to_np(kc), to_np(vc), to_np(ks), to_np(vs)
-    out = torch.zeros((q.shape[0], H, D), dtype=torch.float16, device=cuda)
-    vkv.paged_prefill(out, tq, kc, vc, to_dev(lay.block_tables, cuda), to_dev(ctx, cuda), to_dev(qsl, cuda),
-                      int(q_lens.max()), scale, key_scales=ks, value_scales=vs)
-    torch.cuda.synchronize()
     ref = oracle.paged_prefill(q.astype(np.float32), hk, hv, lay.block_tables, ctx, qsl, scale,
                                key_scales=hks, value_scales=hvs)
-    got = to_np(out).astype(np.float32)
-    assert np.isfinite(got).all()
-    if kvt == "f16":
-        assert_close(got, ref, F16_ATOL, F16_RTOL, "prefill with growing logits")
-    else:
-        # The kernel stages dequantised keys as fp16 (2^-12 relative), which at
-        # logits near 50 moves single weights by about 1 %: held to the FP8
-        # contract (3e-2 relative) per output row instead of element-wise.
-        err = np.linalg.norm(got - ref, axis=-1) / np.maximum(np.linalg.norm(ref, axis=-1), 1e-6)
-        assert err.max() <= 3e-2, f"FP8 prefill with growing logits: row error {err.max():.3e}"
+    for wl in (None, to_dev(whole_items_list(qsl, ctx, H // Hkv, Hkv), cuda)):
+        out = torch.zeros((q.shape[0], H, D), dtype=torch.float16, device=cuda)
+        vkv.paged_prefill(out, tq, kc, vc, to_dev(lay.block_tables, cuda), to_dev(ctx, cuda), to_dev(qsl, cuda),
+                          int(q_lens.max()), scale, key_scales=ks, value_scales=vs, work_list=wl)
+        torch.cuda.synchronize()
+        got = to_np(out).astype(np.float32)
+        assert np.isfinite(got).all()
+        if kvt == "f16":
+            assert_close(got, ref, F16_ATOL, F16_RTOL, "prefill with growing logits")
+        else:
+            # The kernel stages dequantised keys as fp16 (2^-12 relative), which at
+            # logits near 50 moves single weights by about 1 %: held to the FP8
+            # contract (3e-2 relative) per output row instead of element-wise.
+            err = np.linalg.norm(got - ref, axis=-1) / np.maximum(np.linalg.norm(ref, axis=-1), 1e-6)
+            assert err.max() <= 3e-2, f"FP8 prefill with growing logits: row error {err.max():.3e}"
 
 
-def test_prefill_caller_workspace(vkv, cuda):
+@pytest.mark.parametrize("blocks", ["split", "whole"])
+def test_prefill_caller_workspace(vkv, cuda, blocks):
     """A caller workspace of vkv_paged_prefill_workspace_size() bytes (header
     zeroed) gives the library workspace's result bit for bit, twice in a row."""
     import torch
-    out, args, mql, scale = _mixed_inputs(cuda)
+    out, args, mql, scale = _mixed_inputs(cuda, blocks)
     vkv.paged_prefill(out, *args, mql, scale)
     need = vkv.prefill_workspace_size(out, *args, mql, scale)
     assert need > 1024
@@ -550,10 +559,12 @@ def test_prefill_max_context_len_clamp(vkv, oracle, cuda, io):
     else:
         qd, out = to_dev(qf, cuda), torch.zeros((q.shape[0], H, D), dtype=torch.float32, device=cuda)
         tol = (F32_ATOL, 1e-3)
-    vkv.paged_prefill(out, qd, to_dev(k, cuda), to_dev(v, cuda), to_dev(lay.block_tables, cuda), to_dev(ctx, cuda),
-                      to_dev(qsl, cuda), max(q_lens), scale, max_context_len=max_ctx)
-    torch.cuda.synchronize()
-    assert_close(to_np(out).astype(np.float32), ref, *tol, f"prefill clamped to {max_ctx} keys ({io})")
+    for wl in (None, to_dev(whole_items_list(qsl, ctx, H // Hkv, Hkv), cuda)):
+        out.fill_(7.0)
+        vkv.paged_prefill(out, qd, to_dev(k, cuda), to_dev(v, cuda), to_dev(lay.block_tables, cuda), to_dev(ctx, cuda),
+                          to_dev(qsl, cuda), max(q_lens), scale, max_context_len=max_ctx, work_list=wl)
+        torch.cuda.synchronize()
+        assert_close(to_np(out).astype(np.float32), ref, *tol, f"prefill clamped to {max_ctx} keys ({io})")
 
 
 def test_prefill_group16_list_kernel(vkv, oracle, cuda):
