@@ -189,6 +189,39 @@ def test_stream_fp32_edges_vs_oracle(vkv, oracle, cuda, H, Hkv, bs, table):
         assert_close(to_np(out), ref, F32_ATOL, F32_RTOL, f"fp32 {H}/{Hkv}/bs{bs} size {size}")
 
 
+# All in fp32 at head_dim 64, groups of 1 to 5: by pairs, group and table the call
+# runs on the VALU kernel, as one workgroup per (row, kv head) or in equal slices
+@pytest.mark.parametrize("table", [128, 256, 512, 1024, 2048, 6000])
+@pytest.mark.parametrize("S,H,Hkv", [(12, 8, 8), (12, 4, 2), (12, 8, 2), (12, 10, 2), (70, 4, 4), (70, 16, 4), (300, 4, 4),
+                                     (300, 8, 4)])
+def test_fp32_small_groups_vs_oracle(vkv, oracle, cuda, S, H, Hkv, table):
+    """Against the oracle, and the fused append against the two calls bit for bit."""
+    import torch
+    from helpers import F32_ATOL, F32_RTOL
+    D, bs = 64, 16
+    rng = np.random.default_rng(S + H + table)
+    ctx = rng.integers(1, min(table, 700 if S < 100 else 60) + 1, S)
+    ctx[:2] = [min(table, 900), 1]
+    lay, (k, v), q = _case(rng, H, Hkv, D, bs, ctx, table)
+    k, v, q = ((x.astype(np.float32) * np.float32(1.0001)) for x in (k, v, q))
+    ref = oracle.paged_decode(q, np.nan_to_num(k), np.nan_to_num(v), lay.block_tables, lay.context_lens, D ** -0.5)
+    rest = (to_dev(lay.block_tables, cuda), to_dev(lay.context_lens, cuda), D ** -0.5)
+    kc, vc = to_dev(k, cuda), to_dev(v, cuda)
+    out = torch.full((S, H, D), 7.0, device=cuda)
+    vkv.paged_decode(out, to_dev(q, cuda), kc, vc, *rest)
+    torch.cuda.synchronize()
+    assert_close(to_np(out), ref, F32_ATOL, F32_RTOL, f"fp32 {S} rows {H}/{Hkv}, table {table}")
+    slots = lay.slots(lay.context_lens - 1, np.arange(S))
+    new = [to_dev(rng.standard_normal((S, Hkv, D), dtype=np.float32), cuda) for _ in range(2)]
+    two = [torch.empty_like(out), kc.clone(), vc.clone()]
+    vkv.reshape_and_cache(*new, two[1], two[2], to_dev(slots, cuda))
+    vkv.paged_decode(two[0], to_dev(q, cuda), two[1], two[2], *rest)
+    vkv.paged_decode_append(out, to_dev(q, cuda), kc, vc, *rest, *new, to_dev(slots, cuda))
+    torch.cuda.synchronize()
+    for a, b in zip((out, kc, vc), two):
+        assert torch.equal(a.view(torch.int32), b.view(torch.int32))
+
+
 @pytest.mark.parametrize("dtype", ["f16", "f32"])
 @pytest.mark.parametrize("D", [64, 80, 112, 128])
 def test_stream_query_rows_of_any_alignment(vkv, cuda, D, dtype):

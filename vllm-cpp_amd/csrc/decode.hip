@@ -573,9 +573,8 @@ constexpr int mfma_enabled() { return VKV_DECODE_MFMA; }
 
 template <typename IO, int KVT, int D, int G>
 void launch_g(DecodeArgs& args, int grid_x, int grid_y, int grid_z, size_t lds, hipStream_t st) {
-    // (fp16 over fp16 at head_dim 64 and 128, and all-fp32 at 64, run on decode_stream.hip)
-    constexpr bool kStreamed = mfma_enabled() && (std::is_same<IO, _Float16>::value ? KVT == kF16 && D <= 128
-                                                                                    : KVT == kF32 && D == 64);
+    // (fp16 over fp16 at head_dim 64 and 128 runs on decode_stream.hip)
+    constexpr bool kStreamed = mfma_enabled() && std::is_same<IO, _Float16>::value && KVT == kF16 && D <= 128;
     // grid_x arrives as the number of item groups (an upper bound).  One workgroup per resident slot: the variant's workgroups per CU by
     // registers (queried once per variant), bounded by the LDS the rows'
     // prefix takes, and never more than there are item groups.  Groups
@@ -873,7 +872,10 @@ DecodePlan plan_decode(const vkv_decode_params* p) {
     plan.whole_rows = false;
     plan.max_slices = 0;
     plan.stream = stream_shape(p);
-    if (plan.stream && !split_in_partitions(p)) {
+    if (plan.stream && p->io_dtype == VKV_DTYPE_F32 && fixed &&
+        !stream_f32_pays(int(rows), p->num_kv_heads, p->num_heads / p->num_kv_heads, int(max_ctx)))
+        plan.stream = false;
+    if (stream_shape(p) && !split_in_partitions(p)) {
         // Equal slices (decode_stream.hip) of down to kSliceTokens tokens, at most
         // kMaxSplitParts of a row and one more (a row's first and last slice are
         // shared with its neighbours), and no more of the call than its resident
@@ -890,14 +892,18 @@ DecodePlan plan_decode(const vkv_decode_params* p) {
             const int64_t together = stream_split_waves(p->head_dim, p->io_dtype == VKV_DTYPE_F32) / p->num_kv_heads;
             slices = slices < together ? slices : (together > 0 ? together : 1);
         }
-        plan.partition_size = int(slice);
-        plan.num_candidates = own ? 2 : 1;  // 2: the kernel sizes the slices
-        plan.max_parts = int(parts);
-        plan.max_slices = int(slices < (int64_t(1) << 30) ? slices : int64_t(1) << 30);
-        // (never less than the partitions' workspace: a size asked for with
-        // 16-byte aligned caches serves others too)
-        const size_t bytes = stream_bytes(p, plan.max_slices);
+        slices = slices < (int64_t(1) << 30) ? slices : int64_t(1) << 30;
+        // (the larger of both splits' workspaces, whichever this call takes: a size
+        // asked for with 16-byte aligned caches serves others too, and one asked
+        // for a larger batch this one)
+        const size_t bytes = stream_bytes(p, int(slices));
         if (bytes > plan.workspace_bytes) plan.workspace_bytes = bytes;
+        if (plan.stream) {
+            plan.partition_size = int(slice);
+            plan.num_candidates = own ? 2 : 1;  // 2: the kernel sizes the slices
+            plan.max_parts = int(parts);
+            plan.max_slices = int(slices);
+        }
     }
     return plan;
 }
@@ -993,7 +999,7 @@ int launch_rows(const vkv_decode_params* p, const DecodePlan& plan, void* worksp
         const int n = p->num_seqs - r0 < kMaxRowsPerLaunch ? p->num_seqs - r0 : kMaxRowsPerLaunch;
         DecodeArgs c = a;
         c.num_rows = n;
-        const bool whole_rows = plan.stream && (plan.whole_rows || stream_decode_rows(n, p->num_kv_heads, io_eb == 4 ? 2 * D : D, c.max_ctx, !split_streams));
+        const bool whole_rows = plan.stream && (plan.whole_rows || stream_decode_rows(n, p->num_kv_heads, io_eb == 4 ? 2 * D : D, c.max_ctx, !split_streams, io_eb == 4));
         const bool streamed = whole_rows || split_streams;
         // Small plain decode calls (at most one (row, kv head) pair per CU):
         // a static grid over the partitions of the default size, if its waves

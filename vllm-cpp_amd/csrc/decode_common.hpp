@@ -135,8 +135,8 @@ inline bool fixed_decode_shape(int head_dim, int group, int block_size, const vo
 }
 
 // The shapes of decode_stream.hip: fp16 queries over fp16 caches at these head
-// dimensions, or all in fp32 at head_dim 64; groups of up to 32 heads and any
-// block size.  Split-K calls in fp16 at head_dim 128, groups of up to 8 and
+// dimensions, or all in fp32 at head_dim 64 (small groups where stream_f32_pays
+// says so); groups of up to 32 heads and any block size.  Split-K calls in fp16 at head_dim 128, groups of up to 8 and
 // power-of-two blocks of 16 tokens and more (matrix_split_shape; FP8 caches too)
 // run in partitions of the size that run_partitions picks, the others in equal
 // slices.
@@ -153,7 +153,11 @@ inline bool matrix_split_shape(int head_dim, int group, int block_size, const vo
 // Whether a launch of num_rows rows runs as one workgroup per (row, kv head),
 // merged in LDS, instead of split-K.  half_dims: a head's row in fp16 elements'
 // bytes (head_dim; twice that in fp32, half in FP8).
-bool stream_decode_rows(int num_rows, int num_kv_heads, int half_dims, int max_ctx, bool matrix_split);
+bool stream_decode_rows(int num_rows, int num_kv_heads, int half_dims, int max_ctx, bool matrix_split, bool f32);
+// All in fp32 at head_dim 64: whether decode_stream.hip is faster than decode.hip's
+// VALU kernel (groups of up to 8, blocks of a power of two), which computes a group's
+// heads alone where a matrix tile holds 16.
+bool stream_f32_pays(int num_rows, int num_kv_heads, int group, int max_ctx);
 // Waves that a split launch of decode_stream.hip keeps resident, at most: slices of
 // the kv heads together beyond that would not start sooner.
 int stream_split_waves(int head_dim, bool f32);

@@ -812,22 +812,29 @@ void launch_dim(DecodeArgs& a, int G, bool rows, size_t lds, hipStream_t st) {
 // One workgroup per (row, kv head) saves the merge launch and the scan of the
 // rows, but the longest row's workgroup streams alone at the end, at about 54
 // bytes per ns.  Measured both ways over contexts U[1, max_ctx] (us per
-// appending step, workgroup per row against equal slices; host-bound at ~13):
-//   head_dim 64,   64 pairs: max 2 048: 15.6 / 16.7   4 096: 26.1 / 21.8
-//                 512 pairs:     2 048: 33.1 / 36.3   4 096: 57.3 / 53.9
-//                2048 pairs:     2 048: 102 / 110     4 096: 189 / 192
-//   head_dim 128,  64 pairs:     1 024: 16.7 / 18.7   2 048: 27.8 / 22.7
-//     (group 16) 1024 pairs:     1 024: 63.0 / 74.6   2 048: 114 / 119     4 096: 207 / 205
-//   head_dim 80,   64 pairs:     1 024: 13.2 / 16.9   2 048: 20.6 / 18.6
-//                1024 pairs:       512: 23.8 / 25.4   1 024: 42.6 / 38.9
-//                2048 pairs:       256: 27.8 / 28.2     512: 48.1 / 47.6
-// Against decode.hip's split (head_dim 128, group 4): 256 pairs, 1 024: 18.6 /
-// 24.3; 2 048: 36.3 / 36.8; 1 024 pairs, 1 024: 53.9 / 79.1.
-bool stream_decode_rows(int num_rows, int num_kv_heads, int half_dims, int max_ctx, bool matrix_split) {
+// appending step, FP8 per decode; workgroup per row against equal slices):
+//   head_dim 64,   64 pairs: max 1 024: 9.3 / 13.4   2 048: 14.4 / 14.3   4 096: 26.5 / 20.9
+//                 512 pairs:     1 024: 17.8 / 24.7   2 048: 32.3 / 34.7   4 096: 62.5 / 55.4
+//                2048 pairs:     1 024: 52.9 / 65.3   2 048: 95 / 108      4 096: 185 / 191
+//   head_dim 128,  64 pairs:       512: 11.3 / 14.7   1 024: 16.2 / 15.9   2 048: 28.9 / 20.2
+//     (group 16)  256 pairs:     1 024: 19.1 / 27.1   2 048: 35.3 / 38.9   4 096: 63.9 / 60.4
+//                1024 pairs:     1 024: 58.5 / 68.8   2 048: 109 / 115     4 096: 207 / 207
+//   head_dim 80,   64 pairs:       512: 7.1 / 10.7    1 024: 9.4 / 11.3    2 048: 19.1 / 16.5
+//                1024 pairs:       512: 19.4 / 23.2   1 024: 32.8 / 33.2   2 048: 73.6 / 63.6
+//                2048 pairs:       256: 21.7 / 25.8     512: 34.7 / 37.4   1 024: 85.1 / 75.6
+//   fp32, group 7, 64 pairs:       512: 13.4 / 18.6   1 024: 22.5 / 19.1   2 048: 40.3 / 20.6
+//     head_dim 64 512 pairs:       512: 26.7 / 31.1   1 024: 47.8 / 41.5   2 048: 86.5 / 63.1
+// Against partitions (matrix_split; head_dim 128, group 4): 32 pairs, 1 024: 14.4 /
+// 14.3; 256 pairs, 1 024: 17.9 / 22.7; 2 048: 32.8 / 34.4; 1 024 pairs, 1 024: 54.0 /
+// 79.9; 2 048: 114 / 109.  FP8: 32 pairs, 1 024: 11.3 / 13.1; 2 048: 19.4 / 16.5; 256
+// pairs, 2 048: 24.1 / 28.0; 1 024 pairs, 1 024: 37.7 / 63.7; 2 048: 77.3 / 67.2.
+bool stream_decode_rows(int num_rows, int num_kv_heads, int half_dims, int max_ctx, bool matrix_split, bool f32) {
 #if VKV_STREAM_ROWS
     return VKV_STREAM_ROWS == 1;
 #endif
     const int64_t pairs = int64_t(num_rows) * num_kv_heads, cus = device_cu_count();
+    if (f32) return max_ctx <= (pairs < cus ? 528 : pairs < 4 * cus ? 1056 : 264);
+    if (matrix_split && half_dims == 64) return max_ctx <= (2 * pairs >= cus && pairs <= cus ? 2112 : 1056);
     if (half_dims % 64 != 0) return max_ctx <= (pairs < 2 * cus ? 1056 : pairs < 8 * cus ? 528 : 264);
     const int64_t row_bytes = int64_t(max_ctx) * half_dims * 4;
     return max_ctx <= 2112 && (row_bytes <= 528 << 10 || (pairs >= cus && !matrix_split));
@@ -837,6 +844,20 @@ int stream_split_waves(int head_dim, bool f32) {
     // (stages as launch_shape takes them; two stages at the wider heads: fewer)
     const int stage = 2 * kStep * head_dim * (f32 ? 4 : 2) * (head_dim == 64 && !f32 ? 2 : 1);
     return device_cu_count() * (kLdsPerCu / (1024 + kWavesPerBlock * stage)) * kWavesPerBlock;
+}
+
+// Contexts U[1, max_ctx], us per appending step (VALU kernel / workgroup per row /
+// equal slices):
+//   group 1,   64 pairs: 256 tokens: 10 / 11 / 18     1 024: 13 / 22 / 20   4 096: 23 / 73 / 33
+//            1 024 pairs: 64: 15 / 18 / 19    512: 44 / 45 / 40   1 024: 75 / 77 / 61   4 096: 190 / 296 / 206
+//   group 4,  256 pairs:  512: 20 / 16 / 23   1 024: 27 / 25 / 29   2 048: 48 / 44 / 42   4 096: 73 / 80 / 65
+//   group 5,   64 pairs:  512: 16 / 14 / 19   1 024: 18 / 23 / 20   2 048: 26 / 41 / 22   4 096: 38 / 74 / 33
+bool stream_f32_pays(int num_rows, int num_kv_heads, int group, int max_ctx) {
+    if (group > 4) return true;
+    const int64_t pairs = int64_t(num_rows) * num_kv_heads, cus = device_cu_count();
+    if (pairs < cus) return max_ctx <= (group > 2 ? 264 : 132);
+    if (pairs < 4 * cus) return max_ctx <= (group > 2 ? 528 : 264) || (group == 4 && max_ctx > 1056);
+    return max_ctx > 264 && max_ctx <= (group > 1 ? 2112 : pairs < 8 * cus ? 1056 : 0);
 }
 
 template <int KVT, int NST>
@@ -870,7 +891,7 @@ static void launch_parts(DecodeArgs& a, int64_t max_items, size_t lds, hipStream
 // group 4, fp16 105.4 / 110.8; 256 long-tailed ones, group 4, FP8 312.4 / 317.0;
 // 120 of 1 024 to 8 192, group 7, FP8 132.2 / 125.3).
 bool launch_decode_matrix(DecodeArgs& a, bool fp8, int64_t max_items, size_t lds, hipStream_t st) {
-    if (fp8 && stream_decode_rows(a.num_rows, a.num_kv_heads, 64, a.max_ctx, true)) {
+    if (fp8 && stream_decode_rows(a.num_rows, a.num_kv_heads, 64, a.max_ctx, true, false)) {
         launch_row_groups<128, 1, kFp8>(a, st);
         return true;
     }
