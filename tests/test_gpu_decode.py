@@ -802,6 +802,64 @@ def test_decode_partition_choice_batches(vkv, oracle, cuda, idx):
         assert_close(got[s_:s_ + 1], ref, F16_ATOL, F16_RTOL, f"row {s_} (partition {chosen}, {kv})")
 
 
+# (rows, context range, kv dtype, default size P0 the host halves to, the size a 256-CU device picks)
+_SMALL_BATCHES = [(64, 2048, 2048, "f16", 384, 512), (16, 8192, 8192, "f16", 384, 512), (16, 8192, 8192, "fp8", 384, 512),
+                  (8, 2500, 4096, "f16", 96, 112)]
+
+
+@pytest.mark.parametrize("idx", range(len(_SMALL_BATCHES)))
+def test_decode_partition_choice_small_batches(vkv, oracle, cuda, idx):
+    """Batches whose default size the host halves below 768 tokens (8 kv heads, G = 4,
+    D = 128, 16-token blocks): the least ceil(items / 1 024) x (P + 128) of 2/3, 3/4, 1,
+    5/4, 4/3 and 2 x P0, at most one level of waves or not.  The output is
+    bit-identical to an explicit call at the recorded size; two rows against the
+    oracle."""
+    import torch
+    from vllm_kv_amd import workloads
+    S, lo, hi, kv, p0, want = _SMALL_BATCHES[idx]
+    H, Hkv, D, bs = 32, 8, 128, 16
+    rng = np.random.default_rng(300 + idx)
+    ctx = rng.integers(lo, hi + 1, size=S).astype(np.int32)
+    ctx[0] = hi
+    lay = workloads.make_layout(ctx, bs, rng, slack=0.05)
+    cands = sorted({p0 * n // d // bs * bs for n, d in ((2, 3), (3, 4), (1, 1), (5, 4), (4, 3), (2, 1))})
+    items = {c: int(((ctx.astype(np.int64) + c - 1) // c).sum()) * Hkv for c in cands}
+    assert min(cands, key=lambda c: (-(-items[c] // 1024) * (c + 128), c)) == want
+    shape = (lay.num_blocks, bs, Hkv, D)
+    k = (rng.standard_normal(shape, dtype=np.float32) * 0.5).astype(np.float16)
+    v = (rng.standard_normal(shape, dtype=np.float32) * 0.5).astype(np.float16)
+    if kv == "f16":
+        kc, vc, ks, vs = to_dev(k, cuda), to_dev(v, cuda), None, None
+        hk, hv, hks, hvs = k.view(np.uint16), v.view(np.uint16), None, None
+    else:
+        kc = torch.empty(shape, dtype=torch.uint8, device=cuda)
+        vc = torch.empty_like(kc)
+        ks = torch.empty(shape[:3], dtype=torch.float32, device=cuda)
+        vs = torch.empty_like(ks)
+        vkv.reshape_and_cache(to_dev(k, cuda).view(-1, Hkv, D), to_dev(v, cuda).view(-1, Hkv, D), kc, vc,
+                              torch.arange(lay.num_blocks * bs, dtype=torch.int32, device=cuda), ks, vs)
+        hk, hv, hks, hvs = to_np(kc), to_np(vc), to_np(ks), to_np(vs)
+    q = (rng.standard_normal((S, H, D), dtype=np.float32) * 0.5).astype(np.float16)
+    args = (to_dev(q, cuda), kc, vc, to_dev(lay.block_tables, cuda), to_dev(lay.context_lens, cuda), D ** -0.5)
+    out = torch.zeros((S, H, D), dtype=torch.float16, device=cuda)
+    need = vkv.decode_workspace_size(out, *args, key_scales=ks, value_scales=vs)
+    ws = torch.zeros(need // 4 + 4, dtype=torch.int32, device=cuda)
+    vkv.paged_decode(out, *args, key_scales=ks, value_scales=vs, workspace=ws)
+    torch.cuda.synchronize()
+    chosen = int(ws[1].item())
+    assert chosen in cands
+    if torch.cuda.get_device_properties(cuda).multi_processor_count == 256:
+        assert chosen == want, (chosen, want)
+    out2 = torch.zeros_like(out)
+    vkv.paged_decode(out2, *args, key_scales=ks, value_scales=vs, partition_size=chosen)
+    torch.cuda.synchronize()
+    assert torch.equal(out.view(torch.int16), out2.view(torch.int16)), chosen
+    rows = [0, S - 1]
+    ref = oracle.paged_decode(q[rows].astype(np.float32), hk, hv, np.ascontiguousarray(lay.block_tables[rows]),
+                              np.ascontiguousarray(ctx[rows]), D ** -0.5, key_scales=hks, value_scales=hvs)
+    assert_close(to_np(out)[rows].astype(np.float32), ref, F16_ATOL, F16_RTOL, f"partition {chosen} ({kv})")
+
+
 def test_decode_config5_all_rows(vkv, oracle, cuda):
     """Full C5 (Llama-3-8B shape, FP8 e4m3 cache with per-(token, head) scales, B=256,
     lognormal contexts up to 22.6k tokens): the pool, N(0,1) with 1 % of the values

@@ -66,18 +66,21 @@ constexpr int64_t kSliceTokens = 128;
 // 32-token blocks; with 16-token blocks the last two are both 1 024).  The
 // sizes below P0 let a batch whose items almost fill a whole
 // number of waves per SIMD take shorter partitions that keep that number.
-// Six, because the counts per candidate take registers in the kernels'
-// prologue: with ten, the compiler reloaded a kernel argument and added a
-// load wait inside the partition kernels' token loop (C5's batch: 354 us
-// against 343 us at the same partition size).  Calls over more rows than
-// kAdaptMaxRows keep P0.
+// Calls over more rows than kAdaptMaxRows keep P0.
 constexpr int kCandNum[kMaxPartitionCandidates] = {3, 7, 1, 5, 5, 2};
 constexpr int kCandDen[kMaxPartitionCandidates] = {4, 8, 1, 4, 3, 1};
+// Small batches on the matrix cores (P0 halved below 768): 2/3, 3/4, 1, 5/4, 4/3 and
+// 2 x P0.  The halving leaves gaps of a third between sizes that fill a level of
+// waves: 64 rows of 2 048 tokens, 32/8 heads (P0 384): 88 us at 512, 99 to 102 at 256,
+// 384 and 640.  (Six of nine sizes tried over 524 such batches; all nine counted in
+// the kernel cost its FP8 form 13 % in registers: the counts are taken in the
+// prologue, and loads of the token loop had to wait.)
+constexpr int kSmallNum[kMaxPartitionCandidates] = {2, 3, 1, 5, 4, 2};
+constexpr int kSmallDen[kMaxPartitionCandidates] = {3, 4, 1, 4, 3, 1};
 // When the 64-block cap merges candidates (at 16-token blocks and P0 = 768,
 // 5/3 and 2 x P0 are both 1 024), the freed slots take these, in order: 55/64,
 // 15/16, 13/16 x P0 (656, 720, 624 tokens there).  C2's batch then takes 656
-// (2 016 items, still two waves per SIMD): 97.1 us explicit against 98.0 at
-// 672.
+// (2 016 items, still two waves per SIMD).
 constexpr int kFillCandidates = 3;
 constexpr int kFillNum[kFillCandidates] = {55, 15, 13};
 constexpr int kFillDen[kFillCandidates] = {64, 16, 16};
@@ -613,6 +616,8 @@ void launch_g(DecodeArgs& args, int grid_x, int grid_y, int grid_z, size_t lds, 
         }
         args.wave_slots = (gx > 0 ? gx : 1) * kWavesPerBlock;
         args.level_waves = (gx > 0 ? (gx < cus ? gx : cus) : 1) * kWavesPerBlock;
+        args.keep_below = args.level_waves;
+        args.keep_above = 2 * args.wave_slots;
         // When even the longest possible contexts give at most one wave of
         // default-size items per SIMD, the default stands and the kernels
         // (this one and the merge, which reads these args) skip the choice.
@@ -813,15 +818,16 @@ DecodePlan plan_decode(const vkv_decode_params* p) {
     if (max_ctx > table_tokens) max_ctx = table_tokens;
     if (max_ctx < 0) max_ctx = 0;
     // Default 768 tokens: the best of a 384..1024 sweep for both the C2
-    // (B=64, ctx U[512,4096]) and C5 (B=256, lognormal ctx) decode batches.
-    // Small batches split finer (halving, not below 16 tokens, then down to a
-    // block multiple) until the longest possible contexts would give kMinItems
-    // work items, or a row more than kMaxSplitParts partitions: a wave walks
-    // its partition serially, so 8 items of 512 tokens (C1) leave the GPU idle
-    // while short items finish together (C1's decode: 15.3 us at 48 tokens,
-    // 14.2 at 32, 13.9 at 16, 32.8 at 256), but the merge walks a row's
-    // partitions in batches, one after the other (one sequence of 4 096
-    // tokens: 29.6 us at 16 tokens, 19.7 at 32, 16.5 at 64 and 128).
+    // (B=64, ctx U[512,4096]) and C5 (B=256, lognormal ctx) decode batches on the
+    // VALU kernels.  Small batches split finer (halving, not below 16 tokens, then
+    // down to a block multiple) until the longest possible contexts would give
+    // kMinItems work items, or a row more than kMaxSplitParts partitions: a wave
+    // walks its partition serially, so few items of 512 tokens leave the GPU idle
+    // while short items finish together (4 sequences of 512 tokens, 14/2 heads,
+    // head_dim 64, FP8 cache: 13.5 us at 16 tokens, 13.8 at 32, 15.4 at 48, 36.1 at
+    // 256), but the merge walks a row's partitions in batches, one after the other
+    // (one sequence of 4 096 tokens there: 41.1 us at 16 tokens, 28.4 at 32, 23.2 at
+    // 64, 25.6 at 128).
     int P = p->partition_size > 0 ? p->partition_size : 768;
     if (p->partition_size <= 0) {
         const int64_t per_part = int64_t(p->num_seqs) * p->num_kv_heads;
@@ -846,9 +852,10 @@ DecodePlan plan_decode(const vkv_decode_params* p) {
             const int c = (P * num / den) / bs * bs;
             return c < bs ? bs : (c > 64 * bs ? 64 * bs : c);
         };
+        const bool small = split_in_partitions(p) && P < 768 && P < 64 * bs;
         int n = 0;
         for (int i = 0; i < kMaxPartitionCandidates; ++i) {
-            const int c = block_multiple(kCandNum[i], kCandDen[i]);
+            const int c = small ? block_multiple(kSmallNum[i], kSmallDen[i]) : block_multiple(kCandNum[i], kCandDen[i]);
             if (n == 0 || c != plan.candidates[n - 1]) plan.candidates[n++] = c;
         }
         // Slots freed by the 64-block cap take finer sizes just below the default.
@@ -964,6 +971,8 @@ int launch_rows(const vkv_decode_params* p, const DecodePlan& plan, void* worksp
     for (int i = 0; i < kMaxPartitionCandidates; ++i) a.cands[i] = plan.candidates[i];
     a.wave_slots = 0;  // set per variant at launch
     a.level_waves = 0;
+    a.keep_below = 0;
+    a.keep_above = 0x7FFFFFFF;
     a.scale_log2 = logit_scale_log2(p->scale);
     a.accumulate = p->accumulate;
     a.static_parts = 0;

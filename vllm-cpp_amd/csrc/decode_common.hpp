@@ -72,6 +72,7 @@ struct DecodeArgs {
     // size among cands (ascending) and records it in the workspace header.
     int32_t num_cands;
     int32_t cands[kMaxPartitionCandidates];
+    int32_t keep_below, keep_above;  // items of size P up to (past) which P is kept
     int32_t wave_slots;       // waves of this launch resident at once (estimate)
     int32_t level_waves;      // waves of one workgroup per CU (one wave per SIMD)
     // generic variant (any head_dim / group size / block size) only
@@ -260,21 +261,18 @@ __device__ __forceinline__ void unpack_lane(const uint32_t* w, float* v) {
 // about ceil(items / level_waves) x (P + kItemOverheadTokens), the cost the
 // candidates compete on (ties: the smaller size).  Items beyond the
 // wave_slots resident waves wait for a wave to finish, which the same count
-// covers.  C2's batch (8 kv heads, 64 rows; 1 024 waves per level) measured
-// 97.8 us at 656 tokens (2 016 items, cost 2 x 784), 98.4 at 672, 99.5 at
-// 688, 102.2 at 448 (2 840 items, 3 x 576), 102.8 at 768 (1 784 items,
-// 2 x 896), 106.4 at 512, 110.5 at 544, 113.5 at 576 and 117.7 at 608
-// (2 160 items, 3 x 736): time rises with the cost throughout, except that a
-// nearly empty extra level costs less (107.5 us at 640: 2 064 items); among
-// the candidates it takes 656 (2 016 items, 2 x 784).  C3's decode rows (two
-// waves per SIMD resident) take 1 280 tokens (2 044 items, 2 x 1 408), the
-// fastest of a sweep: 198.8 us, against 200.7 at 1 152, 210.0 at 768, 212.2
-// at 1 536, 223.3 at 960 and 238.0 at 2 048.  Two cases keep the
-// default: default-size items of at most one level (small batches, which the
+// covers.  On the matrix cores (DEAL): C2's batch (8 kv heads, 64 rows; 1 024
+// waves per level) 96.6 us at 656 tokens (2 016 items, cost 2 x 784), 96.9 at
+// 672, 98.3 at 768 (1 784 items, 2 x 896), 112 at 448 (2 840 items, 3 x 576),
+// 118 at 512 and 109 at 1 024; C3's decode rows (fp16) 186 at 1 280 tokens (2 044
+// items, 2 x 1 408), 189 at 1 152, 209 at 768, 191 at 1 536 and 211 at 2 048.
+// Over 524 small batches (2 to 256 rows, groups 1, 4 and 7, contexts up to 16 384,
+// uniform, equal, lognormal; fp16 and FP8) the choice costs 3.3 % against the best
+// of nine sizes (10.7 % keeping the default in the two cases below).  The VALU kernels (claims) keep the default in two
+// cases: default-size items of at most one level (small batches, which the
 // host already split finer), and beyond two rounds of resident waves, where
 // waves that claim items as they finish fill the last round with the short
-// final partitions of the rows (C5's batch, 3.3 rounds at 768 tokens:
-// 345 us at 768 against 356 at 640 and 354-356 at 896 to 1 536).
+// final partitions of the rows.
 __device__ inline int choose_partition(const DecodeArgs& a, const int (&cnt)[kMaxPartitionCandidates]) {
     __shared__ int sums[kWavesPerBlock][kMaxPartitionCandidates];
     const int lane = threadIdx.x & (kWave - 1);
@@ -285,7 +283,6 @@ __device__ inline int choose_partition(const DecodeArgs& a, const int (&cnt)[kMa
         if (lane == 0) sums[wave][c] = v;
     }
     __syncthreads();
-    const unsigned W = a.wave_slots > 0 ? unsigned(a.wave_slots) : 1u;
     const unsigned L = a.level_waves > 0 ? unsigned(a.level_waves) : 1u;
     const unsigned cap = 0x7FFFFFFFu / unsigned(a.num_kv_heads);
     unsigned items0 = 0;
@@ -305,7 +302,7 @@ __device__ inline int choose_partition(const DecodeArgs& a, const int (&cnt)[kMa
             best = a.cands[c];
         }
     }
-    return (items0 <= L || items0 > 2 * W) ? a.P : best;
+    return (items0 <= unsigned(a.keep_below) || items0 > unsigned(a.keep_above)) ? a.P : best;
 }
 
 // Longest-first order of the pairs of a call whose items take more than one

@@ -355,6 +355,8 @@ void launch_variant_q(DecodeArgs& a, int64_t max_pairs, size_t lds, hipStream_t 
     a.wave_slots = int(gx > 0 ? gx : 1) * kWavesPerBlock;
     const int64_t cus = device_cu_count();
     a.level_waves = int(gx > 0 ? (gx < cus ? gx : cus) : 1) * kWavesPerBlock;
+    a.keep_below = a.level_waves;
+    a.keep_above = 2 * a.wave_slots;
     hipLaunchKernelGGL((decode_generic_kernel<KVT, DP, GC, HQ>), dim3(unsigned(gx > 0 ? gx : 1)),
                        dim3(kBlockThreads), lds, st, a);
 }

@@ -877,10 +877,6 @@ static void launch_parts(DecodeArgs& a, int64_t max_items, size_t lds, hipStream
     a.static_parts = 0;
     a.wave_slots = gx * kWavesPerBlock;
     a.level_waves = (gx < cus ? gx : cus) * kWavesPerBlock;
-    if (a.num_cands > 1) {
-        const int64_t worst = int64_t(a.num_rows) * ((int64_t(a.max_ctx) + a.P - 1) / a.P) * a.num_kv_heads;
-        if (worst <= a.level_waves) a.num_cands = 1;
-    }
     hipLaunchKernelGGL(kernel, dim3(gx), dim3(kBlockThreads), lds, st, a);
 }
 
