@@ -72,7 +72,6 @@ struct DecodeArgs {
     // size among cands (ascending) and records it in the workspace header.
     int32_t num_cands;
     int32_t cands[kMaxPartitionCandidates];
-    int32_t keep_below, keep_above;  // items of size P up to (past) which P is kept
     int32_t wave_slots;       // waves of this launch resident at once (estimate)
     int32_t level_waves;      // waves of one workgroup per CU (one wave per SIMD)
     // generic variant (any head_dim / group size / block size) only
@@ -97,8 +96,6 @@ struct DecodeArgs {
     // from one of a kv head's partials to the next the slice or the row goes up,
     // so part_slots = max_slices + rows hold them all.
     int2* row_parts;
-    int32_t max_slices;
-    int32_t part_slots;
     // Append fused into the call (source rows in the cache's element type,
     // fp16 or fp32; fixed and streamed shapes): row s's new token is fkey / fval + s *
     // stride (bytes), bound for cache slot fslots[s].  The partition kernel
@@ -114,6 +111,11 @@ struct DecodeArgs {
     int32_t fbytes;  // element bytes of the rows and the cache (2 or 4)
     const int32_t* fslots;
     int64_t fnum_slots;
+    // (last: read once or not at all by the kernels whose start these loads are part
+    // of; among the fields above they cost the smallest step 0.2 us)
+    int32_t max_slices;              // see row_parts
+    int32_t part_slots;
+    int32_t keep_below, keep_above;  // items of size P up to (past) which P is kept
 };
 
 // The new token of an appending decode call (see DecodeArgs::fkey).
@@ -268,11 +270,11 @@ __device__ __forceinline__ void unpack_lane(const uint32_t* w, float* v) {
 // items, 2 x 1 408), 189 at 1 152, 209 at 768, 191 at 1 536 and 211 at 2 048.
 // Over 524 small batches (2 to 256 rows, groups 1, 4 and 7, contexts up to 16 384,
 // uniform, equal, lognormal; fp16 and FP8) the choice costs 3.3 % against the best
-// of nine sizes (10.7 % keeping the default in the two cases below).  The VALU kernels (claims) keep the default in two
-// cases: default-size items of at most one level (small batches, which the
-// host already split finer), and beyond two rounds of resident waves, where
-// waves that claim items as they finish fill the last round with the short
-// final partitions of the rows.
+// of nine sizes (10.7 % keeping the default in the two cases below).  The default
+// stands (keep_below, keep_above) in default-size items of at most one level on the
+// VALU kernels (small batches, which the host already split finer), and beyond two
+// rounds of resident waves there and at full-size partitions on the matrix cores:
+// the short final partitions of the rows fill the last round.
 __device__ inline int choose_partition(const DecodeArgs& a, const int (&cnt)[kMaxPartitionCandidates]) {
     __shared__ int sums[kWavesPerBlock][kMaxPartitionCandidates];
     const int lane = threadIdx.x & (kWave - 1);

@@ -841,9 +841,10 @@ bool stream_decode_rows(int num_rows, int num_kv_heads, int half_dims, int max_c
 }
 
 int stream_split_waves(int head_dim, bool f32) {
-    // (stages as launch_shape takes them; two stages at the wider heads: fewer)
+    // (256 CUs: asking for the device takes 0.1 us of a small call's 6.  Stages as
+    // launch_shape takes them; two stages at the wider heads: fewer)
     const int stage = 2 * kStep * head_dim * (f32 ? 4 : 2) * (head_dim == 64 && !f32 ? 2 : 1);
-    return device_cu_count() * (kLdsPerCu / (1024 + kWavesPerBlock * stage)) * kWavesPerBlock;
+    return 256 * (kLdsPerCu / (1024 + kWavesPerBlock * stage)) * kWavesPerBlock;
 }
 
 // Contexts U[1, max_ctx], us per appending step (VALU kernel / workgroup per row /
@@ -877,6 +878,9 @@ static void launch_parts(DecodeArgs& a, int64_t max_items, size_t lds, hipStream
     a.static_parts = 0;
     a.wave_slots = gx * kWavesPerBlock;
     a.level_waves = (gx < cus ? gx : cus) * kWavesPerBlock;
+    // (beyond two rounds of full-size partitions the default stands: 256 long-tailed
+    // rows, FP8: 311 us at 768 tokens, 335 at the least cost)
+    if (a.P >= 768) a.keep_above = 2 * a.wave_slots;
     hipLaunchKernelGGL(kernel, dim3(gx), dim3(kBlockThreads), lds, st, a);
 }
 
