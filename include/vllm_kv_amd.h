@@ -237,7 +237,9 @@ typedef struct vkv_decode_params {
     int32_t io_dtype;
     int32_t kv_dtype;
     int32_t accumulate;
-    int32_t partition_size;     /* tokens per split-K partition; 0 = the library picks it per call on the device */
+    int32_t partition_size;     /* tokens per split-K partition (a call that runs as one workgroup per (sequence,
+                                 * kv head) does not split; equal slices round it up to 32); 0 = the library
+                                 * picks it per call on the device */
     void* workspace;            /* optional, see above */
     size_t workspace_bytes;
 } vkv_decode_params;
