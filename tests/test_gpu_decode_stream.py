@@ -191,14 +191,15 @@ def test_stream_fp32_edges_vs_oracle(vkv, oracle, cuda, H, Hkv, bs, table):
 
 # All in fp32 at head_dim 64, groups of 1 to 5: by pairs, group and table the call
 # runs on the VALU kernel, as one workgroup per (row, kv head) or in equal slices
+@pytest.mark.parametrize("bs", [16, 24])  # (24: the generic kernel instead of the VALU one)
 @pytest.mark.parametrize("table", [128, 256, 512, 1024, 2048, 6000])
 @pytest.mark.parametrize("S,H,Hkv", [(12, 8, 8), (12, 4, 2), (12, 8, 2), (12, 10, 2), (70, 4, 4), (70, 16, 4), (300, 4, 4),
                                      (300, 8, 4)])
-def test_fp32_small_groups_vs_oracle(vkv, oracle, cuda, S, H, Hkv, table):
+def test_fp32_small_groups_vs_oracle(vkv, oracle, cuda, S, H, Hkv, table, bs):
     """Against the oracle, and the fused append against the two calls bit for bit."""
     import torch
     from helpers import F32_ATOL, F32_RTOL
-    D, bs = 64, 16
+    D = 64
     rng = np.random.default_rng(S + H + table)
     ctx = rng.integers(1, min(table, 700 if S < 100 else 60) + 1, S)
     ctx[:2] = [min(table, 900), 1]

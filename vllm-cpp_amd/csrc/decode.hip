@@ -779,6 +779,14 @@ bool stream_shape(const vkv_decode_params* p) {
                                                  p->io_dtype, p->kv_dtype);
 }
 
+// Whether a call runs on decode_stream.hip.
+bool streams(const vkv_decode_params* p) {
+    if (!stream_shape(p) || p->io_dtype != VKV_DTYPE_F32) return stream_shape(p);
+    const int64_t table = int64_t(p->max_blocks_per_seq) * p->block_size;
+    return stream_f32_pays(launch_rows_max(p->num_seqs), p->num_kv_heads, p->num_heads / p->num_kv_heads,
+                           int(p->max_context_len < table ? p->max_context_len : table));
+}
+
 // fp16 queries over fp16 or FP8 caches in a matrix_split_shape.
 bool split_in_partitions(const vkv_decode_params* p) {
     return mfma_enabled() && p->io_dtype == VKV_DTYPE_F16 && p->kv_dtype != VKV_DTYPE_F32 &&
@@ -878,10 +886,7 @@ DecodePlan plan_decode(const vkv_decode_params* p) {
     plan.base_bytes = plan.workspace_bytes = kWorkspaceHeader + size_t(rows) * plan.max_parts * slot_bytes(p);
     plan.whole_rows = false;
     plan.max_slices = 0;
-    plan.stream = stream_shape(p);
-    if (plan.stream && p->io_dtype == VKV_DTYPE_F32 && fixed &&
-        !stream_f32_pays(int(rows), p->num_kv_heads, p->num_heads / p->num_kv_heads, int(max_ctx)))
-        plan.stream = false;
+    plan.stream = streams(p);
     if (stream_shape(p) && !split_in_partitions(p)) {
         // Equal slices (decode_stream.hip) of down to kSliceTokens tokens, at most
         // kMaxSplitParts of a row and one more (a row's first and last slice are
@@ -1008,7 +1013,7 @@ int launch_rows(const vkv_decode_params* p, const DecodePlan& plan, void* worksp
         const int n = p->num_seqs - r0 < kMaxRowsPerLaunch ? p->num_seqs - r0 : kMaxRowsPerLaunch;
         DecodeArgs c = a;
         c.num_rows = n;
-        const bool whole_rows = plan.stream && (plan.whole_rows || stream_decode_rows(n, p->num_kv_heads, io_eb == 4 ? 2 * D : D, c.max_ctx, !split_streams, io_eb == 4));
+        const bool whole_rows = plan.stream && (plan.whole_rows || stream_decode_rows(n, p->num_kv_heads, io_eb == 4 ? 2 * D : D, c.max_ctx, !split_streams, io_eb == 4 ? G : 0));
         const bool streamed = whole_rows || split_streams;
         // Small plain decode calls (at most one (row, kv head) pair per CU):
         // a static grid over the partitions of the default size, if its waves
@@ -1096,8 +1101,8 @@ bool decode_append_fusable(const vkv_append_params* ap, const vkv_decode_params*
            ap->num_kv_heads == p->num_kv_heads && ap->head_dim == p->head_dim &&
            ap->block_size == p->block_size && ap->num_blocks == p->num_blocks && (src & 15u) == 0 &&
            ks % 16 == 0 && vs % 16 == 0 &&
-           (stream_shape(p) || fixed_decode_shape(p->head_dim, p->num_heads / p->num_kv_heads, p->block_size,
-                                                  p->key_cache, p->value_cache));
+           (streams(p) || fixed_decode_shape(p->head_dim, p->num_heads / p->num_kv_heads, p->block_size, p->key_cache,
+                                             p->value_cache));
 }
 
 int launch_decode_append(const vkv_append_params* ap, const vkv_decode_params* p, const DecodePlan& plan,

@@ -156,10 +156,11 @@ inline bool matrix_split_shape(int head_dim, int group, int block_size, const vo
 // Whether a launch of num_rows rows runs as one workgroup per (row, kv head),
 // merged in LDS, instead of split-K.  half_dims: a head's row in fp16 elements'
 // bytes (head_dim; twice that in fp32, half in FP8).
-bool stream_decode_rows(int num_rows, int num_kv_heads, int half_dims, int max_ctx, bool matrix_split, bool f32);
-// All in fp32 at head_dim 64: whether decode_stream.hip is faster than decode.hip's
-// VALU kernel (groups of up to 8, blocks of a power of two), which computes a group's
-// heads alone where a matrix tile holds 16.
+// f32_group: the group of a call in fp32, 0 otherwise.
+bool stream_decode_rows(int num_rows, int num_kv_heads, int half_dims, int max_ctx, bool matrix_split, int f32_group);
+// All in fp32 at head_dim 64: whether decode_stream.hip is faster than the VALU
+// kernels (decode.hip, decode_generic.hip), which compute a group's heads alone where
+// a matrix tile holds 16.
 bool stream_f32_pays(int num_rows, int num_kv_heads, int group, int max_ctx);
 // Waves that a split launch of decode_stream.hip keeps resident, at most: slices of
 // the kv heads together beyond that would not start sooner.
