@@ -44,14 +44,15 @@ def source_blob(rel):
     return hashlib.sha1(b"blob %d\0" % len(data) + data).hexdigest()
 
 
-DECODE_SRC = "vllm-cpp_amd/csrc/decode.hip"
+# the sources of the headline decode's kernels
+DECODE_SRC = ("vllm-cpp_amd/csrc/decode.hip", "vllm-cpp_amd/csrc/decode_stream.hip", "vllm-cpp_amd/csrc/decode_common.hpp")
 
 
 def measured_traffic():
     """HBM bytes per decode call from the committed rocprofv3 PMC summary
     (profiles/decode_c2_traffic.json: FETCH_SIZE and WRITE_SIZE, calibrated on a
     1 GiB copy), or None with the reason when that summary is absent or was
-    measured on another decode.hip than the one built here."""
+    measured on other decode sources than those built here."""
     path = os.path.join(ROOT, "profiles", "decode_c2_traffic.json")
     try:
         with open(path) as f:
@@ -59,8 +60,8 @@ def measured_traffic():
         traffic = int(d["traffic_bytes_per_launch"])
     except (OSError, ValueError, KeyError):
         return None, "no committed traffic summary"
-    if d.get("decode_hip_blob") != source_blob(DECODE_SRC):
-        return None, "the committed traffic summary measured another decode.hip"
+    if d.get("source_blobs") != {os.path.basename(p): source_blob(p) for p in DECODE_SRC}:
+        return None, "the committed traffic summary measured other decode sources"
     return traffic, f"profiles/decode_c2_traffic.json (commit {d.get('commit', '?')})"
 
 
