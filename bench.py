@@ -581,8 +581,8 @@ def suite_c1(dev, steps, warmup):
             "step_us_p10_p90": [round(t[1] * 1e3, 2), round(t[2] * 1e3, 2)],
             "fused_step_us_median": round(tf[0] * 1e3, 2),
             "fused_step_us_p10_p90": [round(tf[1] * 1e3, 2), round(tf[2] * 1e3, 2)],
-            "note": "launch-bound: three kernels (append, partition, merge) for 0.6 MB of KV; "
-                    "vkv_paged_decode_append fuses the append into the decode's two",
+            "note": "launch-bound: two kernels (append, decode) for 0.6 MB of KV; "
+                    "vkv_paged_decode_append is the one with the append in it",
             "graph_step_us_median": round(tg[0] * 1e3, 2), "graph_output_equals_eager": graph_equal,
             "native_caller": native,
             "cpu_baseline": {"us_per_step": round(sec * 1e6, 1), "cores": 1, "kind": "port",
@@ -1142,19 +1142,19 @@ def suite_shapes(dev, steps, warmup):
     S = ctx.shape[0]
     stream = torch.cuda.current_stream()
     rows = []
-    # (label, H, Hkv, D, block size, tensor dtype, kernel family)
-    shapes = [("reference API: fp32 q / KV / out", 32, 8, 128, 16, torch.float32, "fixed"),
-              ("head_dim 80", 32, 8, 80, 16, torch.float16, "generic"),
-              ("head_dim 96", 32, 8, 96, 16, torch.float16, "generic"),
-              ("head_dim 112", 32, 8, 112, 16, torch.float16, "generic"),
-              ("head_dim 80, MHA (Phi-2's heads: H32 / Hkv32)", 32, 32, 80, 16, torch.float16, "generic"),
-              ("head_dim 96, MHA (Phi-3-mini's heads: H32 / Hkv32)", 32, 32, 96, 16, torch.float16, "generic"),
-              ("group 16 (H32 / Hkv2)", 32, 2, 128, 16, torch.float16, "generic"),
-              ("MQA (H32 / Hkv1)", 32, 1, 128, 16, torch.float16, "generic"),
-              ("block size 12", 32, 8, 128, 12, torch.float16, "generic"),
-              ("block size 24", 32, 8, 128, 24, torch.float16, "generic"),
-              ("fixed shape for comparison (C2: H32 / Hkv8 / D128 / bs16)", 32, 8, 128, 16, torch.float16, "fixed")]
-    for label, H, Hkv, D, bs, dt, fam in shapes:
+    # (label, H, Hkv, D, block size, tensor dtype)
+    shapes = [("reference API: fp32 q / KV / out", 32, 8, 128, 16, torch.float32),
+              ("head_dim 80", 32, 8, 80, 16, torch.float16),
+              ("head_dim 96", 32, 8, 96, 16, torch.float16),
+              ("head_dim 112", 32, 8, 112, 16, torch.float16),
+              ("head_dim 80, MHA (Phi-2's heads: H32 / Hkv32)", 32, 32, 80, 16, torch.float16),
+              ("head_dim 96, MHA (Phi-3-mini's heads: H32 / Hkv32)", 32, 32, 96, 16, torch.float16),
+              ("group 16 (H32 / Hkv2)", 32, 2, 128, 16, torch.float16),
+              ("MQA (H32 / Hkv1)", 32, 1, 128, 16, torch.float16),
+              ("block size 12", 32, 8, 128, 12, torch.float16),
+              ("block size 24", 32, 8, 128, 24, torch.float16),
+              ("C2's shape for comparison (H32 / Hkv8 / D128 / bs16)", 32, 8, 128, 16, torch.float16)]
+    for label, H, Hkv, D, bs, dt in shapes:
         lay = workloads.make_layout(ctx, bs, np.random.default_rng(1))
         g = torch.Generator(device=dev).manual_seed(1)
         kc = (torch.randn((lay.num_blocks, bs, Hkv, D), generator=g, device=dev) * c2.sigma).to(dt)
@@ -1173,7 +1173,7 @@ def suite_shapes(dev, steps, warmup):
         kvb = int(ctx.astype(np.int64).sum()) * Hkv * 2 * D * kc.element_size()
         gbs = kvb / (t[0] * 1e-3) / 1e9
         rows.append({"shape": label, "H": H, "Hkv": Hkv, "D": D, "block_size": bs,
-                     "dtype": "f32" if dt == torch.float32 else "f16", "kernels": fam,
+                     "dtype": "f32" if dt == torch.float32 else "f16",
                      "us_median": round(t[0] * 1e3, 2), "us_p10_p90": [round(t[1] * 1e3, 2), round(t[2] * 1e3, 2)],
                      "kv_bytes": kvb, "gbs": round(gbs, 1), "frac_of_hbm_peak": round(gbs / HBM_PEAK_GBS, 4)})
         log(f"[shapes] {label}: {t[0] * 1e3:.1f} us, {gbs:.0f} GB/s")

@@ -29,6 +29,11 @@
 //
 // FP8 lanes load 8 bytes (8 codes) so that fp8 and fp16 share one lane layout
 // (D=128: 16 lanes per token) and one register footprint.
+//
+// These VALU kernels serve head_dim 256, FP8 caches at 64, fp32 queries, and all in
+// fp32 at 64 in the small groups where they are the faster; fp16 and FP8 at 128 and
+// fp16 at 64 run on decode_stream.hip.  The merge, the plan and the launches here are
+// common to both and to decode_generic.hip.
 #include <atomic>
 #include <cstdint>
 #include <cstdlib>
@@ -578,13 +583,14 @@ template <typename IO, int KVT, int D, int G>
 void launch_g(DecodeArgs& args, int grid_x, int grid_y, int grid_z, size_t lds, hipStream_t st) {
     // (fp16 over fp16 at head_dim 64 and 128 runs on decode_stream.hip)
     constexpr bool kStreamed = mfma_enabled() && std::is_same<IO, _Float16>::value && KVT == kF16 && D <= 128;
-    // grid_x arrives as the number of item groups (an upper bound).  One workgroup per resident slot: the variant's workgroups per CU by
-    // registers (queried once per variant), bounded by the LDS the rows'
-    // prefix takes, and never more than there are item groups.  Groups
-    // beyond the grid are claimed through the counters as workgroups finish
-    // (each workgroup scans the rows once, where a grid of every group pays
-    // that scan per group: C5's batch measured 361 us against 382 us).  The
-    // resident wave count also feeds the partition choice.
+    // grid_x arrives as the number of item groups (an upper bound).  One workgroup
+    // per resident slot: the variant's workgroups per CU by registers (queried once
+    // per variant), bounded by the LDS the rows' prefix takes, and never more than
+    // there are item groups.  Groups beyond the grid are claimed through the
+    // counters as workgroups finish (each workgroup scans the rows once, where a
+    // grid of every group pays that scan per group: 256 long-tailed rows, FP8 at
+    // head_dim 128 on a kernel since replaced, 361 us against 382).  The resident
+    // wave count also feeds the partition choice.
     // Static small-call variants exist for fp16 queries (the serving case).
     constexpr bool kStatic = std::is_same<IO, _Float16>::value;
     static std::atomic<int> reg_blocks{0};

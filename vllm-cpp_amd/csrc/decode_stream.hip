@@ -1,7 +1,8 @@
 // decode_stream.hip — paged decode attention for fp16 queries over fp16 caches
 // at head_dim 64, 80, 96, 112 or 128 with groups of up to 32 query heads, and
 // over FP8 caches at head_dim 128 with groups of up to 8, both products on the
-// matrix cores (gfx950); and all in fp32 at head_dim 64, groups of up to 32.
+// matrix cores (gfx950); and all in fp32 at head_dim 64, groups of up to 32 (of up to
+// four where stream_f32_pays says so).
 // Semantics as in decode.hip (the reference's src/attention/
 // paged_attention.cu:13-82).
 //
