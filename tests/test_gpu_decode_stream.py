@@ -85,6 +85,67 @@ def test_stream_fused_append(vkv, cuda, H, Hkv, D, bs, table):
         assert np.array_equal(a, b)
 
 
+@pytest.mark.parametrize("S,table", [(520, 32), (520, 64), (520, 80), (520, 384), (520, 400), (1030, 128), (1030, 144),
+                                     (2060, 528), (2060, 544)])
+@pytest.mark.parametrize("H,Hkv,D,dtype", [(2, 2, 64, "f16"), (14, 2, 64, "f32"), (8, 2, 80, "f16"), (2, 2, 112, "f16"),
+                                           (6, 2, 128, "f16"), (4, 2, 128, "fp8")])
+def test_stream_many_short_rows(vkv, oracle, cuda, S, table, H, Hkv, D, dtype):
+    """Over 4, 8 and 16 (row, kv head) pairs per CU at the edges of the tables that one
+    wave and two attend: rows of every length against the oracle, and the fused append
+    against the two calls bit for bit."""
+    import torch
+    from helpers import F32_ATOL, F32_RTOL
+    bs = 16
+    rng = np.random.default_rng(S + table + D)
+    ctx = rng.integers(0, min(table, 400 if S < 2000 else 48) + 1, S)
+    ctx[:9] = [table, 0, 1, 31, 32, table - 1, table // 2, table // 2 + 1, min(33, table)]
+    lay, (k, v), q = _case(rng, H, Hkv, D, bs, ctx, table)
+    rows = np.unique(np.concatenate([np.arange(9), np.linspace(9, S - 1, 24).astype(int)]))
+    args = [to_dev(lay.block_tables, cuda), to_dev(lay.context_lens, cuda), D ** -0.5]
+    if dtype == "fp8":
+        hole = np.isnan(k)
+        codes = [rng.integers(0, 0x70, k.shape).astype(np.uint8) for _ in range(2)]
+        sc = [rng.uniform(0.005, 0.02, k.shape[:3]).astype(np.float32) for _ in range(2)]
+        ref = oracle.paged_decode(q[rows].astype(np.float32), *codes, lay.block_tables[rows], lay.context_lens[rows], D ** -0.5,
+                                  key_scales=sc[0], value_scales=sc[1])
+        for c, x in zip(codes, sc):
+            c[hole] = 0x7F
+            x[hole[..., 0]] = np.nan
+        out = torch.zeros((S, H, D), dtype=torch.float16, device=cuda)
+        vkv.paged_decode(out, to_dev(q, cuda), *[to_dev(c, cuda) for c in codes], *args,
+                         key_scales=to_dev(sc[0], cuda), value_scales=to_dev(sc[1], cuda))
+        torch.cuda.synchronize()
+        assert_close(to_np(out)[rows].astype(np.float32), ref, F16_ATOL, F16_RTOL, f"table {table}")
+        return
+    if dtype == "f32":
+        k, v, q = (x.astype(np.float32) * np.float32(1.0001) for x in (k, v, q))
+        pools = [np.nan_to_num(x) for x in (k, v)]
+    else:
+        pools = [np.nan_to_num(x).view(np.uint16) for x in (k, v)]
+    ref = oracle.paged_decode(q[rows].astype(np.float32), *pools, lay.block_tables[rows], lay.context_lens[rows], D ** -0.5)
+    out = torch.zeros(q.shape, dtype=torch.float32 if dtype == "f32" else torch.float16, device=cuda)
+    vkv.paged_decode(out, to_dev(q, cuda), to_dev(k, cuda), to_dev(v, cuda), *args)
+    torch.cuda.synchronize()
+    tol = (F32_ATOL, F32_RTOL) if dtype == "f32" else (F16_ATOL, F16_RTOL)
+    assert_close(to_np(out)[rows].astype(np.float32), ref, *tol, f"table {table}")
+    new = [(rng.standard_normal((S, Hkv, D)) * 0.7).astype(q.dtype) for _ in range(2)]
+    slots = lay.slots(np.maximum(lay.context_lens - 1, 0), np.arange(S))
+    slots[lay.context_lens == 0] = -1
+    got = []
+    for fused in (True, False):
+        kc, vc = to_dev(k, cuda), to_dev(v, cuda)
+        out = torch.zeros_like(out)
+        call, nw = (out, to_dev(q, cuda), kc, vc, *args), [to_dev(x, cuda) for x in new]
+        if fused:
+            vkv.paged_decode_append(*call, *nw, to_dev(slots, cuda))
+        else:
+            vkv.reshape_and_cache(*nw, kc, vc, to_dev(slots, cuda))
+            vkv.paged_decode(*call)
+        torch.cuda.synchronize()
+        got.append([to_np(x).tobytes() for x in (out, kc, vc)])
+    assert got[0] == got[1]
+
+
 # (rows, contexts, caller's partition size): a call whose finer partials once did not
 # fit the library's array, so that it ran unsplit; many rows of short contexts; and
 # a caller's size whose slices, with one of each row more, do not fit (coarser ones do)

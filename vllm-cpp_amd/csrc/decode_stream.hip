@@ -774,13 +774,38 @@ void launch_split(DecodeArgs& a, size_t lds, hipStream_t st) {
 }
 
 // Eight waves per row while every (row, kv head) has a CU, else four, so that
-// two workgroups share a CU; two stages per wave where a stage is 8 KiB.
+// two workgroups share a CU; two stages per wave where a stage is 8 KiB.  Many
+// pairs of short tables: two waves or one, of one stage.  LDS bounds what a CU
+// holds, and a wave of a row that has no step for it (contexts shorter than 32
+// tokens a wave) holds its ring for nothing; with four pairs to a CU the others
+// cover a wave's loads.  Measured over contexts U[1, max] (us per appending step,
+// FP8 per decode; four waves / two / one):
+//   head_dim 64,   512 pairs: max 64: 8.4 / 7.4 / 7.3   128: 7.5 / 7.9 / 9.7    256: 10.1 / 10.6 / 14.7
+//                 1280 pairs:     64: 13.7 / 8.0 / 7.9  128: 15.2 / 9.5 / 10.8  384: 21.0 / 18.0 / 21.3
+//                 8192 pairs:     64: 66.6 / 24.2 / 21.0  128: 73.7 / 32.7 / 30.5  512: 121 / 102 / 107
+//   head_dim 112, 2048 pairs:     64: 20.7 / 14.1 / 10.3  128: 25.0 / 18.4 / 16.2  256: 32.0 / 25.8 / 28.4
+//   head_dim 128, 1280 pairs:     64: 17.5 / 13.6 / 11.2  256: 26.2 / 24.1 / 25.1  512: 40.4 / 42.1 / 43.4
+//                 8192 pairs:     64: 83.8 / 54.3 / 41.5  128: 96.4 / 73.3 / 63.8  512: 221 / 201 / 206
+//   FP8,          1280 pairs:     64: 14.6 / 8.8 / 9.5  256: 20.2 / 16.4 / 20.7  1 024: 44.5 / 51.3 / 61.7
+//                 8192 pairs:     64: 69.5 / 33.7 / 27.1  128: 77.0 / 44.7 / 39.5  512: 143 / 127 / 130
+//     (every row of 512 tokens, 2048 pairs: 61.5 / 65.3; head_dim 128: 95.1 / 100.7)
+//   fp32, group 7, 2048 pairs:    64: 33.6 / 23.1 / 18.3  128: 35.8 / 32.2 / 28.7  256: 52.1 / 50.8 / 49.7
 template <int D, int CT, int KVT>
 void launch_row_groups(DecodeArgs& a, hipStream_t st) {
     constexpr int NST = Tile<D, KVT>::STAGE <= 8192 + 256 ? 2 : 1;
-    const int64_t pairs = int64_t(a.num_rows) * a.num_kv_heads;
+    const int64_t pairs = int64_t(a.num_rows) * a.num_kv_heads, cus = device_cu_count();
     const dim3 grid{unsigned(pairs)};
-    if (pairs <= device_cu_count())
+    if constexpr (CT == 1) {
+        if (pairs >= 4 * cus && a.max_ctx <= (pairs >= 8 * cus ? 132 : 66)) {
+            hipLaunchKernelGGL((decode_rows_kernel<D, CT, KVT, 1, 1>), grid, dim3(64), 0, st, a);
+            return;
+        }
+        if (pairs >= 4 * cus && a.max_ctx <= (pairs >= 16 * cus ? 528 : 396)) {
+            hipLaunchKernelGGL((decode_rows_kernel<D, CT, KVT, 2, 1>), grid, dim3(128), 0, st, a);
+            return;
+        }
+    }
+    if (pairs <= cus)
         hipLaunchKernelGGL((decode_rows_kernel<D, CT, KVT, 8, NST == 2 && KVT == kFp8 ? 1 : NST>), grid, dim3(512), 0, st, a);
     else
         hipLaunchKernelGGL((decode_rows_kernel<D, CT, KVT, 4, NST>), grid, dim3(256), 0, st, a);
@@ -813,7 +838,8 @@ void launch_dim(DecodeArgs& a, int G, bool rows, size_t lds, hipStream_t st) {
 // One workgroup per (row, kv head) saves the merge launch and the scan of the
 // rows, but the longest row's workgroup streams alone at the end, at about 54
 // bytes per ns.  Measured both ways over contexts U[1, max_ctx] (us per
-// appending step, FP8 per decode; workgroup per row against equal slices):
+// appending step, FP8 per decode; workgroup per row, of four waves beyond 256 pairs,
+// against equal slices):
 //   head_dim 64,   64 pairs: max 1 024: 9.3 / 13.4   2 048: 14.4 / 14.3   4 096: 26.5 / 20.9
 //                 512 pairs:     1 024: 17.8 / 24.7   2 048: 32.3 / 34.7   4 096: 62.5 / 55.4
 //                2048 pairs:     1 024: 52.9 / 65.3   2 048: 95 / 108      4 096: 185 / 191
@@ -849,14 +875,14 @@ int stream_split_waves(int head_dim, bool f32) {
     return 256 * (kLdsPerCu / (1024 + kWavesPerBlock * stage)) * kWavesPerBlock;
 }
 
-// Contexts U[1, max_ctx], us per appending step (VALU kernel / workgroup per row /
-// equal slices):
+// Contexts U[1, max_ctx], us per appending step (VALU kernel / workgroup per row, of
+// four waves beyond 256 pairs / equal slices):
 //   group 1,   64 pairs: 256 tokens: 10 / 11 / 18     1 024: 13 / 22 / 20   4 096: 23 / 73 / 33
 //            1 024 pairs: 64: 15 / 18 / 19    512: 44 / 45 / 40   1 024: 75 / 77 / 61   4 096: 190 / 296 / 206
 //   group 4,  256 pairs:  512: 20 / 16 / 23   1 024: 27 / 25 / 29   2 048: 48 / 44 / 42   4 096: 73 / 80 / 65
 //   group 5,   64 pairs:  512: 16 / 14 / 19   1 024: 18 / 23 / 20   2 048: 26 / 41 / 22   4 096: 38 / 74 / 33
 // (Blocks of no power of two alike: 8/8 heads, 24-token blocks, 256 rows of 1 to 64
-// tokens: 18.8 us on the generic kernel, 32.1 streamed.)
+// tokens: 18.8 us on the generic kernel, 32.1 streamed by four waves.)
 bool stream_f32_pays(int num_rows, int num_kv_heads, int group, int max_ctx) {
     if (group > 4) return true;
     const int64_t pairs = int64_t(num_rows) * num_kv_heads, cus = device_cu_count();
